@@ -1,0 +1,787 @@
+// int4 `linear` for a chunk of rows on the gfx950 matrix cores: eight waves split K.
+//
+// out[m, n] = sum_k x[m,k] * dequant(w)[n,k] + bias[n]
+// (packages/runtime/src/kernels/linear.ts:34-64, packages/runtime/src/kernels/gemm.ts:1187-1237).
+// The weights enter the matrix cores as the exact integers (u - 8) in fp16, products are exact,
+// sums are f32 (v_mfma_f32_32x32x16_f16) and the group scale multiplies the f32 sum of each scale
+// group.  Three forms of x:
+//   kX16     fp16 activations as they are;
+//   kX32     f32 activations, each rounded to fp16 once where it is read from LDS;
+//   kXSplit  f32 activations as x * 2^e = hi + lo (both fp16, e per row), written once per call
+//            by split_rows_kernel below: two matrix instructions a step, 22 bits of x.
+//
+// A workgroup owns a tile of 32 MT rows x 32 NT columns; its eight waves take an eighth of K each
+// and run on their own: a wave streams its slice of x and of the packed weights from memory
+// straight into its own LDS rings (global_load_lds, no registers, no parking instructions), so
+// the K loop has no barrier, every LDS byte is read once and every weight word is turned into
+// integers once per 32 MT rows.  The waves' sums meet in LDS and are added in wave order.  How K
+// is cut depends on K and the group size alone, and every tile size adds in the same order: a
+// row's bits depend neither on M nor on the tile picked for the shape.
+//
+// LDS rings: x in stages of 64 or 32 codes, weights in units of 64 to 256 codes; the 16-byte pieces
+// of a row are permuted by the row number, so that the fragment reads of 32 consecutive rows spread
+// over all banks.
+//
+// What bounds it: what the second-level cache delivers to a CU (tiles of 64 x 96: 2 * 64 + 96 / 2
+// bytes a code), then the conversion of the weights on the vector ALUs (12 operations a word).
+// Measured on cold weights, fp16 x (f32 class in brackets), against the kernel that loaded through
+// registers, one 32 x 32 or 32 x 64 tile a workgroup: 128 x 2560 x 2048 6.6 us, 9.6 before (11.8,
+// 14.5); 128 x 2048 x 2048 5.4, 7.0 (10.1, 12.5); 128 x 11264 x 2048 15.1, 27.0 (25.9, 38.6); 128 x
+// 2048 x 5632 10.6, 13.0 (19.7, 26.2); 77 x 3000 x 2080 with groups of 32 in the f32 class 13.8 us,
+// 221 before (sixteen rows at a time through the GEMV).
+#include "krm_internal.h"
+
+#include <type_traits>
+
+using namespace krm;
+
+namespace {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kX16 = 0, kXSplit = 1, kX32 = 2;
+constexpr int kWaves = 8;
+
+template <typename T>
+__device__ inline float to_f32(T v);
+template <>
+__device__ inline float to_f32<float>(float v) { return v; }
+template <>
+__device__ inline float to_f32<__half>(__half v) { return __half2float(v); }
+template <typename T>
+__device__ inline T from_f32(float v);
+template <>
+__device__ inline float from_f32<float>(float v) { return v; }
+template <>
+__device__ inline __half from_f32<__half>(float v) { return __float2half_rn(v); }
+
+// (a & mask) | bits in one VALU op (the compiler emits two when both constants are literals).
+__device__ inline uint32_t and_or(uint32_t a, uint32_t mask, uint32_t bits) {
+  uint32_t d;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(mask), "v"(bits));
+  return d;
+}
+
+// 8 codes of a word -> 8 fp16 integers (u - 8).  1024 + u (or 1024 + 16 u) is built in the fp16
+// mantissa, one packed op removes the offset.
+// Order (c0,c4,c1,c5,c2,c6,c3,c7): two ops a pair, for activations stored in the same order.
+__device__ inline half8_t ints_paired(uint32_t word) {
+  const uint32_t magic = 0x64006400u;  // (1024, 1024)
+  const half2_t off_lo = {(_Float16)1032.0f, (_Float16)1032.0f};
+  const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
+  const half2_t off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
+  const uint32_t upper = word >> 8;
+  const half2_t q0 = __builtin_bit_cast(half2_t, and_or(word, 0x000F000Fu, magic)) - off_lo;
+  const half2_t q1 = __builtin_elementwise_fma(
+      __builtin_bit_cast(half2_t, and_or(word, 0x00F000F0u, magic)), sixteenth, off_hi);
+  const half2_t q2 = __builtin_bit_cast(half2_t, and_or(upper, 0x000F000Fu, magic)) - off_lo;
+  const half2_t q3 = __builtin_elementwise_fma(
+      __builtin_bit_cast(half2_t, and_or(upper, 0x00F000F0u, magic)), sixteenth, off_hi);
+  return half8_t{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
+}
+// Natural order c0..c7: a byte of the word is copied to both halves, the even code is read from
+// its low nibble and the odd one from its high nibble (three ops a pair).
+__device__ inline half8_t ints_natural(uint32_t word) {
+  const uint32_t magic = 0x64006400u;
+  const half2_t factor = {(_Float16)1.0f, (_Float16)0.0625f};
+  const half2_t offset = {(_Float16)-1032.0f, (_Float16)-72.0f};
+  half2_t q[4];
+  const uint32_t twice[4] = {__builtin_amdgcn_perm(word, word, 0x0c000c00u),
+                             __builtin_amdgcn_perm(word, word, 0x0c010c01u),
+                             __builtin_amdgcn_perm(word, word, 0x0c020c02u),
+                             __builtin_amdgcn_perm(word, word, 0x0c030c03u)};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    q[i] = __builtin_elementwise_fma(
+        __builtin_bit_cast(half2_t, and_or(twice[i], 0x00F0000Fu, magic)), factor, offset);
+  return half8_t{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+}
+
+// ------------------------------------------------------------------- memory -> LDS, counted waits
+//
+// The loads below do not pass through registers and the compiler does not see them; the waits are
+// counted by hand (vector memory operations of a wave complete in order).  Nothing else of the K
+// loop loads from memory through the compiler.
+
+// 16 bytes a lane from base + offset to LDS at lds + 16 * lane.
+__device__ inline void stream_to_lds(uint32_t lds, uint32_t offset, const void* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds),
+               "v"(offset), "s"(base)
+               : "memory");
+}
+// The same for a dword or a zero-extended ushort a lane, to LDS at lds + 4 * lane.
+__device__ inline void stream_word_to_lds(uint32_t lds, uint32_t offset, const void* base, bool half) {
+  if (half)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" ::"s"(lds),
+                 "v"(offset), "s"(base)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds),
+                 "v"(offset), "s"(base)
+                 : "memory");
+}
+template <int N>
+__device__ inline void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// Columns (col, col + 1) of output row `row`, summed: bias, then what the call asked for.
+template <typename T>
+__device__ inline void finish_pair(float v0, float v1, uint32_t row, uint32_t col, uint32_t m,
+                                   uint32_t n, const T* __restrict__ bias, T* __restrict__ out,
+                                   const RowsFusion& fuse) {
+  const T* residual = static_cast<const T*>(fuse.residual);
+  const bool two = col + 1 < n;
+  if (bias) {
+    v0 += to_f32<T>(bias[col]);
+    if (two) v1 += to_f32<T>(bias[col + 1]);
+  }
+  if (fuse.mode == 1) {
+    // (gate, up) -> silu(gate) * up, the roundings of the decode row's epilogue
+    const float t = __builtin_amdgcn_exp2f(-fabsf(v0) * 1.4426950408889634f);
+    const float r = __builtin_amdgcn_rcpf(1.0f + t);
+    const float sig = v0 < 0.f ? t * r : r;
+    float value = __fmul_rn(__fmul_rn(v0, sig), v1);
+    const size_t at = (size_t)row * (n >> 1) + (col >> 1);
+    if (residual) value += to_f32<T>(residual[at]);
+    out[at] = from_f32<T>(value);
+  } else if (fuse.mode == 2) {
+    // what a separate linear would have stored, then the rotation of krm_rope_half
+    const float x0 = to_f32<T>(from_f32<T>(v0)), x1 = to_f32<T>(from_f32<T>(v1));
+    const uint32_t half = fuse.depth >> 1, pair = col >> 1;
+    const uint32_t rope_pairs = (fuse.heads + fuse.kv_heads) * half;
+    if (pair < rope_pairs) {
+      const uint32_t head = pair / half, j = pair - head * half;
+      const int32_t pos = fuse.positions[row];
+      float o0 = NAN, o1 = NAN;  // a position outside the table is never a valid rotation
+      if (pos >= 0 && (uint32_t)pos < fuse.table_rows) {
+        const size_t t = (size_t)pos * fuse.depth + j;
+        o0 = __fadd_rn(__fmul_rn(x0, fuse.cos_table[t]), __fmul_rn(-x1, fuse.sin_table[t]));
+        o1 = __fadd_rn(__fmul_rn(x1, fuse.cos_table[t + half]),
+                       __fmul_rn(x0, fuse.sin_table[t + half]));
+      }
+      T* dst = head < fuse.heads
+                   ? static_cast<T*>(fuse.q_out) + ((size_t)head * m + row) * fuse.depth
+                   : static_cast<T*>(fuse.k_out) + ((size_t)(head - fuse.heads) * m + row) * fuse.depth;
+      dst[j] = from_f32<T>(o0);
+      dst[j + half] = from_f32<T>(o1);
+    } else {
+      const uint32_t e = (pair - rope_pairs) * 2u;  // the v section keeps its natural order
+      const uint32_t plane = e / fuse.depth, d = e - plane * fuse.depth;
+      T* dst = static_cast<T*>(fuse.v_out) + ((size_t)plane * m + row) * fuse.depth;
+      dst[d] = from_f32<T>(x0);
+      dst[d + 1] = from_f32<T>(x1);
+    }
+  } else {
+    const size_t at = (size_t)row * n + col;
+    if (residual) {
+      v0 += to_f32<T>(residual[at]);
+      if (two) v1 += to_f32<T>(residual[at + 1]);
+    }
+    out[at] = from_f32<T>(v0);
+    if (two) out[at + 1] = from_f32<T>(v1);
+  }
+}
+
+// ------------------------------------------------------------------------------- x = hi + lo
+//
+// Row r of the split form: for every 32 codes, 64 bytes of hi and 64 bytes of lo (one line), eight
+// codes at a time in the order (x0,x4,x1,x5,x2,x6,x3,x7); scale[2r] = 2^e with max|x[r, :]| * 2^e in [2^13, 2^14) (no
+// overflow, small entries keep a resolution of 2^-38 of the row's maximum), scale[2r + 1] = 2^-e.
+// A row of zeros, or whose maximum is not finite, gets 1 / 1: what is not finite stays so.
+// One trip over memory up to 16384 codes a row (kept in registers between the maximum and the
+// split), two beyond.
+__global__ __launch_bounds__(512) void split_rows_kernel(const float* __restrict__ x,
+                                                         uint4* __restrict__ planes,
+                                                         float* __restrict__ scale, uint32_t k) {
+  constexpr uint32_t kHeld = 4;
+  __shared__ uint32_t s_max[8];
+  const uint4* row = reinterpret_cast<const uint4*>(x + (size_t)blockIdx.x * k);
+  const uint32_t pieces = k >> 3;
+  uint4 a[kHeld], b[kHeld];
+#pragma unroll
+  for (uint32_t i = 0; i < kHeld; ++i) {
+    const uint32_t p = threadIdx.x + 512u * i;
+    const uint32_t at = p < pieces ? p : 0u;
+    a[i] = row[2 * at];
+    b[i] = row[2 * at + 1];
+  }
+  auto larger = [](uint32_t top, const uint4& v) {
+    return max(max(top, v.x & 0x7fffffffu),
+               max(v.y & 0x7fffffffu, max(v.z & 0x7fffffffu, v.w & 0x7fffffffu)));
+  };
+  uint32_t top = 0;  // largest |x| as raw bits (monotonic for non-negative floats; NaN on top)
+#pragma unroll
+  for (uint32_t i = 0; i < kHeld; ++i) top = larger(larger(top, a[i]), b[i]);
+  for (uint32_t p = threadIdx.x + 512u * kHeld; p < pieces; p += 512u)
+    top = larger(larger(top, row[2 * p]), row[2 * p + 1]);
+  for (int off = 32; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off, kWave));
+  if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = top;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 8; ++i) top = max(top, s_max[i]);
+  const uint32_t biased = top >> 23;  // exponent of the maximum
+  uint32_t up = 127u, down = 127u;    // 2^0
+  if (top != 0 && biased != 255u) {
+    // e = 13 - (biased - 127), kept inside the normal range of both 2^e and 2^-e
+    int e = 13 - ((int)biased - 127);
+    e = e > 126 ? 126 : (e < -126 ? -126 : e);
+    up = (uint32_t)(127 + e);
+    down = (uint32_t)(127 - e);
+  }
+  const float factor = __uint_as_float(up << 23);
+  if (threadIdx.x == 0) {
+    scale[2 * (size_t)blockIdx.x] = factor;
+    scale[2 * (size_t)blockIdx.x + 1] = __uint_as_float(down << 23);
+  }
+  uint4* dst = planes + (size_t)blockIdx.x * (2 * pieces);
+  auto split = [&](uint32_t p, const uint4& va, const uint4& vb) {
+    const uint32_t raw[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
+    _Float16 h[8], l[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float xs = __uint_as_float(raw[i]) * factor;  // exact: a power of two
+      h[i] = (_Float16)xs;                                // round to nearest even
+      l[i] = (_Float16)(xs - (float)h[i]);                // the difference is exact in f32
+    }
+    auto pack = [](_Float16 p0, _Float16 p1) {
+      const half2_t t = {p0, p1};
+      return __builtin_bit_cast(uint32_t, t);
+    };
+    const uint32_t at = (p >> 2) * 8u + (p & 3u);
+    dst[at] = make_uint4(pack(h[0], h[4]), pack(h[1], h[5]), pack(h[2], h[6]), pack(h[3], h[7]));
+    dst[at + 4] =
+        make_uint4(pack(l[0], l[4]), pack(l[1], l[5]), pack(l[2], l[6]), pack(l[3], l[7]));
+  };
+#pragma unroll
+  for (uint32_t i = 0; i < kHeld; ++i) {
+    const uint32_t p = threadIdx.x + 512u * i;
+    if (p < pieces) split(p, a[i], b[i]);
+  }
+  for (uint32_t p = threadIdx.x + 512u * kHeld; p < pieces; p += 512u)
+    split(p, row[2 * p], row[2 * p + 1]);
+}
+
+// ------------------------------------------------------------------------------------ the product
+template <typename T>
+struct type_tag { using type = T; };
+
+struct SliceTail {         // what the end of the kernel needs
+  const void* bias;
+  void* out;
+  const float* row_scale;  // kXSplit
+  RowsFusion fuse;
+};
+
+// STEPS: matrix steps (16 codes) of a scale group inside a flush block: 8 (blocks of 128 codes,
+// groups of 128 and more), or 4, 2, 1 (blocks of 64 codes, groups of 64, 32, 16).
+template <int XKIND, int MT, int NT, int STEPS>
+struct SliceGeometry {
+  static constexpr int kPlanes = XKIND == kXSplit ? 2 : 1;
+  static constexpr int kArea = 20 * 1024;            // a wave's share of the LDS
+  // An x stage holds whole 128-byte lines where the LDS has room: what the second-level cache
+  // delivers counts lines and half lines alike (127 GB/s a CU in 128-byte segments, 80 in 64-byte,
+  // 40 in 32-byte ones).  64 fp16 codes, 32 codes of hi and lo or of f32; the largest tiles take
+  // stages of 32 fp16 codes.
+  static constexpr int kStage = XKIND == kX16 && MT * NT <= (STEPS == 8 ? 4 : 2) ? 64 : 32;
+  static constexpr int kRowBytes = kStage * (XKIND == kX16 ? 2 : 4);
+  static constexpr int kXBytes = 32 * MT * kRowBytes;
+  static constexpr int kXLoads = kXBytes / 1024;
+  static constexpr int kScales = STEPS == 8 ? 1 : 4 / STEPS;  // of a column in a flush block
+  static constexpr int kSLoads = STEPS == 8 ? 0 : (32 * NT * kScales + 63) / 64;  // a unit
+  // codes of a weight unit: the most whose two copies leave room for two stages
+  static constexpr int unit_bytes(int codes) { return NT * 16 * codes + kSLoads * 256; }
+  static constexpr int kUnit =
+      STEPS < 8 ? 64
+                : (2 * unit_bytes(256) + 2 * kXBytes <= kArea
+                       ? 256
+                       : (2 * unit_bytes(128) + 2 * kXBytes <= kArea ? 128 : 64));
+  static constexpr int kWBytes = unit_bytes(kUnit);
+  static constexpr int kWLoads = NT * kUnit / 64;
+  static constexpr int kStagesPerUnit = kUnit / kStage;
+  // ring depths: at stage g, stages g .. g + DX - 1 are in LDS or on their way, and the units
+  // they belong to
+  static constexpr int units_of(int depth) { return (depth - 1 + kStagesPerUnit - 1) / kStagesPerUnit + 1; }
+  static constexpr bool fits(int depth) { return depth * kXBytes + units_of(depth) * kWBytes <= kArea; }
+  static constexpr int kDepthX = fits(4) ? 4 : fits(3) ? 3 : 2;
+  static constexpr int kDepthW = units_of(kDepthX);
+  static_assert(fits(kDepthX), "the rings fit a wave's area");
+  // output columns (in tiles of 32) that are summed at once at the end
+  static constexpr int kSumTiles = MT * NT * 4096 <= kArea ? NT : kArea / (MT * 4096);
+};
+
+template <int XKIND, int MT, int NT, int STEPS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_i4_slices_kernel(
+    // (the leading 14 dwords of the arguments arrive in scalar registers with the wave)
+    const uint8_t* __restrict__ x,  // kX16 / kX32: [m][k]; kXSplit: [m][k / 32][hi, lo][32] fp16
+    const uint8_t* __restrict__ w, const uint8_t* __restrict__ scales, uint32_t row_begin,
+    uint32_t row_end, uint32_t n, uint32_t k, uint32_t group_shift, uint32_t m_blocks, uint32_t tiles, uint32_t scale_f16_arg,
+    uint32_t io_f16, uint32_t m, SliceTail tail) {
+  using G = SliceGeometry<XKIND, MT, NT, STEPS>;
+  constexpr int kPlanes = G::kPlanes, kStage = G::kStage, kRowBytes = G::kRowBytes;
+  constexpr int kLanesPerRow = kRowBytes / 16, kRowsPerLoad = 64 / kLanesPerRow;
+  constexpr int BM = 32 * MT, BN = 32 * NT;
+  constexpr int kScales = G::kScales;
+  constexpr int DX = G::kDepthX, DW = G::kDepthW;
+  __shared__ __align__(1024) uint8_t s_area[kWaves][G::kArea];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int frag_row = lane & 31, frag_h = lane >> 5;
+  // blockIdx & 7 is the XCD: each XCD takes a contiguous range of tiles, the row tiles of a
+  // column tile next to each other, so the weights of a column tile come from memory once
+  const uint32_t per_xcd = (tiles + 7u) >> 3;
+  const uint32_t tile = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+  if (tile >= tiles || (blockIdx.x >> 3) >= per_xcd) return;
+  const uint32_t nb = tile / m_blocks, mb = tile - nb * m_blocks;
+  const uint32_t m0 = row_begin + mb * BM, n0 = nb * BN;
+
+  // K in flush blocks of 128 codes (64 below groups of 128), dealt to the waves in order.  A K
+  // that ends half-way through a block of 64 codes is loaded as its last 64 and only the second
+  // half of those is used.
+  constexpr int kBlock = STEPS == 8 ? 128 : 64;
+  const uint32_t blocks = (k + kBlock - 1u) / kBlock;
+  const uint32_t b0 = (uint32_t)wave * blocks / kWaves, b1 = ((uint32_t)wave + 1u) * blocks / kWaves;
+  const uint32_t k0 = b0 * kBlock, k1 = min(b1 * kBlock, k);
+  const bool ends_early = STEPS < 4 && (k1 & 63u) != 0;  // this slice's last 64 codes are 32
+
+  uint8_t* const area = s_area[wave];
+  const uint32_t x_ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)area;
+  const uint32_t w_ring = x_ring + DX * G::kXBytes;
+
+  // offsets of this lane's pieces inside the tile: rows past M or N re-read the last row
+  constexpr uint32_t kXSize = XKIND == kX16 ? 2 : 4;
+  const uint32_t x_row_bytes = k * kXSize;
+  uint32_t x_off[G::kXLoads];
+#pragma unroll
+  for (int i = 0; i < G::kXLoads; ++i) {
+    const uint32_t row = kRowsPerLoad * i + lane / kLanesPerRow;
+    const uint32_t turn = kRowBytes == 128 ? (row & 7u) : ((row >> 1) & 3u);
+    const uint32_t piece = (lane % kLanesPerRow) ^ turn;
+    x_off[i] = min(row, row_end - 1u - m0) * x_row_bytes + piece * 16u;
+  }
+  // weights: kUnit / 32 pieces of 16 bytes a row
+  constexpr uint32_t kPieces = G::kUnit / 32, kWRows = 64 / kPieces;
+  constexpr int kWRowLoads = 32 * NT / kWRows;
+  static_assert(kWRowLoads == G::kWLoads, "a unit is whole loads");
+  auto w_turn_of = [](uint32_t row) { return kPieces == 2 ? (row >> 2) & 1u : kPieces == 4 ? (row >> 1) & 3u : row & 7u; };
+  uint32_t w_row[kWRowLoads];
+#pragma unroll
+  for (int i = 0; i < kWRowLoads; ++i)
+    w_row[i] = min(kWRows * i + lane / kPieces, n - 1u - n0) * (k >> 1);
+  const uint32_t w_piece = ((lane % kPieces) ^ w_turn_of(lane / kPieces)) * 16u;
+  static_assert(kWRows % 8 == 0, "the turn of a row is the same in every load");
+  // (the planes of the split form hold rows row_begin.. only)
+  const uint8_t* const x_tile =
+      x + (size_t)(XKIND == kXSplit ? m0 - row_begin : m0) * x_row_bytes;
+  const uint8_t* const w_tile = w + (size_t)n0 * (k >> 1);
+
+  // Group scales.  Blocks of 128 codes: one a column, requested into a register at the block's
+  // start and used behind its last step.  Smaller groups: the scales of a unit travel with its
+  // weights, entry e * 32 NT + column.
+  const uint32_t groups = k >> group_shift;
+  const bool scale_f16 = scale_f16_arg != 0;
+  const uint32_t scale_size = scale_f16 ? 2u : 4u;
+  constexpr int kSOff = STEPS == 8 ? NT : G::kSLoads;
+  uint32_t s_off[kSOff];
+#pragma unroll
+  for (int i = 0; i < kSOff; ++i) {
+    const uint32_t entry = STEPS == 8 ? 32u * i + (uint32_t)frag_row
+                                      : min(64u * i + (uint32_t)lane, 32u * NT * kScales - 1u);
+    s_off[i] = (min(entry % (32u * NT), n - 1u - n0) * groups + entry / (32u * NT)) * scale_size;
+  }
+  const uint8_t* const s_tile = scales + (size_t)n0 * groups * scale_size;
+
+  // Stage g of the slice (relative to its first): the weight unit, if it opens one, then x.
+  constexpr int X = G::kXLoads, W = G::kWLoads + G::kSLoads, R = G::kStagesPerUnit;
+  auto stage_code = [&](uint32_t g) {
+    const uint32_t code = k0 + g * kStage;
+    return STEPS < 4 ? min(code, k - kStage) : code;  // (a last half stage of 64: its last 64 codes)
+  };
+  auto request = [&](uint32_t g) {
+    if (g % R == 0) {
+      const uint32_t code = k0 + g * kStage;
+      const uint32_t from = STEPS < 4 ? min(code, k - 64u) : code;  // (the last 64 codes likewise)
+      const uint32_t dst = w_ring + (g / R % DW) * G::kWBytes;
+      // a unit that reaches past the row's end re-reads its last piece, unused
+      const uint32_t piece = G::kUnit > kBlock || STEPS == 8 ? min((from >> 1) + w_piece, (k >> 1) - 16u) : (from >> 1) + w_piece;
+#pragma unroll
+      for (int i = 0; i < kWRowLoads; ++i) stream_to_lds(dst + 1024u * i, w_row[i] + piece, w_tile);
+      if constexpr (STEPS < 8) {
+        const uint8_t* src = s_tile + (size_t)(from >> group_shift) * scale_size;
+#pragma unroll
+        for (int i = 0; i < G::kSLoads; ++i)
+          stream_word_to_lds(dst + NT * 1024u + 256u * i, s_off[i], src, scale_f16);
+      }
+    }
+    const uint8_t* src = x_tile + (size_t)stage_code(g) * kXSize;
+    const uint32_t dst = x_ring + (g % DX) * G::kXBytes;
+#pragma unroll
+    for (int i = 0; i < X; ++i) stream_to_lds(dst + 1024u * i, x_off[i], src);
+  };
+  uint32_t scale_raw[NT];
+  auto load_scales = [&](uint32_t first_code) {
+    if constexpr (STEPS == 8) {
+      const uint8_t* src = s_tile + (size_t)(first_code >> group_shift) * scale_size;
+      if (scale_f16) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          asm volatile("global_load_ushort %0, %1, %2"
+                       : "=v"(scale_raw[nt]) : "v"(s_off[nt]), "s"(src) : "memory");
+      } else {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          asm volatile("global_load_dword %0, %1, %2"
+                       : "=v"(scale_raw[nt]) : "v"(s_off[nt]), "s"(src) : "memory");
+      }
+    }
+  };
+
+  float16_t total[MT][NT], acc[MT][NT];
+  float16_t zero16;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zero16[r] = 0.f;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) total[mt][nt] = acc[mt][nt] = zero16;
+
+  // fragment addresses inside a stage / a unit.  Step j of 32 codes covers the 8-code pieces
+  // 2 h + j (one 8-byte read of weights); groups of 16 need the two pieces of a step next to each
+  // other: 2 j + h.
+  const uint32_t x_turn = kRowBytes == 128 ? (frag_row & 7u) : ((frag_row >> 1) & 3u);
+  const uint8_t* const x_frag = area + frag_row * kRowBytes;
+  const uint8_t* const w_frag =
+      area + DX * G::kXBytes + frag_row * (16 * kPieces) + (STEPS == 1 ? 4u : 8u) * frag_h;
+  const uint32_t w_turn = w_turn_of(frag_row);
+
+  auto flush = [&](uint32_t unit_slot, int e) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      uint32_t bits;
+      if constexpr (STEPS == 8) {
+        bits = scale_raw[nt];
+      } else {
+        bits = *reinterpret_cast<const uint32_t*>(area + DX * G::kXBytes + unit_slot * G::kWBytes + 1024 * NT +
+                                                  4u * (e * 32 * NT + nt * 32 + frag_row));
+      }
+      const float s = scale_f16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)bits) : __uint_as_float(bits);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          total[mt][nt][r] = fmaf(acc[mt][nt][r], s, total[mt][nt][r]);
+    }
+  };
+  // 32 codes: quarter `wq` of the weight unit in slot `unit_slot`, half `xq` of the stage in slot
+  // `slot`; `opens`: the first step starts a scale group (its sums start from zero); `e`: the
+  // unit's scale entry (half of 64 codes) for groups below 64
+  auto half = [&](uint32_t unit_slot, uint32_t wq, uint32_t slot, int xq, bool opens, int e) {
+    const uint8_t* xs = x_frag + slot * G::kXBytes;
+    const uint8_t* ws = w_frag + unit_slot * G::kWBytes + ((wq ^ w_turn) * 16u);
+    uint2 words[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const uint8_t* at = ws + nt * (512 * kPieces);
+      if constexpr (STEPS == 1) {
+        words[nt].x = *reinterpret_cast<const uint32_t*>(at);
+        words[nt].y = *reinterpret_cast<const uint32_t*>(at + 8);
+      } else {
+        words[nt] = *reinterpret_cast<const uint2*>(at);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t piece = STEPS == 1 ? 2u * j + frag_h : 2u * frag_h + j;
+      half8_t a[kPlanes][MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const uint8_t* row = xs + mt * (32 * kRowBytes);
+        if constexpr (XKIND == kX32) {
+          const float4 lo = *reinterpret_cast<const float4*>(row + (((2u * piece) ^ x_turn) * 16u));
+          const float4 hi = *reinterpret_cast<const float4*>(row + (((2u * piece + 1u) ^ x_turn) * 16u));
+          a[0][mt] = half8_t{(_Float16)lo.x, (_Float16)lo.y, (_Float16)lo.z, (_Float16)lo.w,
+                             (_Float16)hi.x, (_Float16)hi.y, (_Float16)hi.z, (_Float16)hi.w};
+        } else {
+#pragma unroll
+          for (int p = 0; p < kPlanes; ++p)
+            a[p][mt] = *reinterpret_cast<const half8_t*>(
+                row + (((4u * (kStage == 64 ? xq : p) + piece) ^ x_turn) * 16u));
+        }
+      }
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const uint32_t word = j == 0 ? words[nt].x : words[nt].y;
+        const half8_t b = XKIND == kXSplit ? ints_paired(word) : ints_natural(word);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int p = 0; p < kPlanes; ++p) {
+            const bool zero = p == 0 && (STEPS == 1 || (j == 0 && opens));
+            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                a[p][mt], b, zero ? zero16 : acc[mt][nt], 0, 0, 0);
+          }
+      }
+      if constexpr (STEPS == 1) flush(unit_slot, 2 * e + j);
+    }
+    if constexpr (STEPS == 2) flush(unit_slot, e);
+  };
+  constexpr int kRegScales = STEPS == 8 ? NT : 0;  // loads of a block's scales
+
+  if (k0 < k1) {
+    const uint32_t stages = (k1 - k0 + kStage - 1u) / kStage;
+    constexpr int kStages = kBlock / kStage;  // of a flush block
+    // At most the stages younger than g (and, `more`, other loads) are on their way.
+    auto wait_for = [&](uint32_t g, auto more_tag) {
+      constexpr int MORE = decltype(more_tag)::value;
+      const uint32_t left = min((uint32_t)(DX - 1), stages - 1u - g);
+      auto wait_n = [&](auto n_tag) {
+        constexpr int N = decltype(n_tag)::value;
+        if constexpr (R == 1) {
+          wait_vm<N * (X + W) + MORE>();
+        } else if constexpr (N == 0) {
+          wait_vm<MORE>();
+        } else if constexpr (N == R) {
+          wait_vm<N * X + W + MORE>();
+        } else {  // does one of the N younger stages open a unit?
+          static_assert(N < R || (R == 2 && N == 3), "at most one or two units");
+          constexpr int kBase = R == 2 && N == 3 ? 1 : 0;
+          if ((g + N) / R - g / R > (uint32_t)kBase) wait_vm<N * X + (kBase + 1) * W + MORE>();
+          else wait_vm<N * X + kBase * W + MORE>();
+        }
+      };
+      if (DX >= 4 && left == 3u) wait_n(std::integral_constant<int, DX >= 4 ? 3 : 0>{});
+      else if (DX >= 3 && left == 2u) wait_n(std::integral_constant<int, DX >= 3 ? 2 : 0>{});
+      else if (left == 1u) wait_n(std::integral_constant<int, 1>{});
+      else wait_n(std::integral_constant<int, 0>{});
+    };
+#pragma unroll
+    for (int i = 0; i < DX - 1; ++i)
+      if ((uint32_t)i < stages) request(i);
+    for (uint32_t b = b0; b < b1; ++b) {
+      load_scales(b * kBlock);
+#pragma unroll
+      for (int i = 0; i < kStages; ++i) {
+        const uint32_t g = (b - b0) * kStages + i;
+        if (kStages == 1 || STEPS >= 4 || g < stages) {
+          if (g + DX - 1 < stages) request(g + DX - 1);
+          // stage g was requested before the block's scales while i < DX - 1
+          if (i < DX - 1 && i < kStages - 1) wait_for(g, std::integral_constant<int, kRegScales>{});
+          else wait_for(g, std::integral_constant<int, 0>{});
+          const uint32_t unit_slot = g / R % DW, slot = g % DX, wq = (g % R) * (kStage / 32);
+          if constexpr (kStage == 64) {
+            const bool early = ends_early && g + 1 == stages;
+            if (!early) half(unit_slot, wq, slot, 0, i == 0, 0);
+            half(unit_slot, wq + 1, slot, 1, STEPS <= 2, 1);
+          } else {
+            const bool early = ends_early && g + 1 == stages;  // the last 64 codes: second half
+            half(unit_slot, early ? 1u : wq, slot, 0, STEPS <= 2 || i == 0, early ? 1 : i % 2);
+          }
+          if constexpr (STEPS == 4) { if (i == kStages - 1) flush(unit_slot, 0); }
+          // the reads of a slot are over before it is filled again
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+      }
+      if constexpr (STEPS == 8) {
+        // requested before the block's last DX - 1 stages were
+        if constexpr (kStages <= DX - 1) {
+          const uint32_t g = (b - b0) * kStages + kStages - 1;
+          if (g + DX - 1 < stages) wait_vm<kStages * X>(); else wait_vm<0>();
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(scale_raw[nt])::"memory");
+        flush(0, 0);
+      }
+    }
+  }
+  wait_vm<0>();
+
+  // The waves' sums, [row][column] in their own areas, kSumTiles column tiles at a time; every
+  // thread adds four columns of a row in wave order and finishes them.
+  constexpr int kCols = 32 * G::kSumTiles;
+#pragma unroll
+  for (int t0 = 0; t0 < NT; t0 += G::kSumTiles) {
+    const int cols = 32 * (NT - t0 < G::kSumTiles ? NT - t0 : G::kSumTiles);
+    float* sums = reinterpret_cast<float*>(area);
+    if (t0 > 0) __syncthreads();
+#pragma unroll
+    for (int t = 0; t < G::kSumTiles; ++t)
+      if (t0 + t < NT) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            sums[(mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4)) * kCols + t * 32 + frag_row] =
+                total[mt][t0 + t][r];
+      }
+    __syncthreads();
+    auto finish = [&](auto type_tag) {
+      using T = typename decltype(type_tag)::type;
+      const int quads = cols / 4, work = BM * quads;
+#pragma unroll
+      for (int i = 0; i < (work + 511) / 512; ++i) {
+        const int p = threadIdx.x + 512 * i;
+        const int local = p / quads, c4 = p % quads;
+        const uint32_t row = m0 + local, col = n0 + 32u * t0 + 4u * c4;
+        if ((work % 512 == 0 || p < work) && row < row_end && col < n) {
+          float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+          for (int wv = 0; wv < kWaves; ++wv) {
+            const float4 part =
+                *reinterpret_cast<const float4*>(s_area[wv] + (size_t)(local * kCols + 4 * c4) * 4);
+            v.x += part.x; v.y += part.y; v.z += part.z; v.w += part.w;
+          }
+          if constexpr (XKIND == kXSplit) {  // exact: a power of two
+            const float inv = tail.row_scale[2 * (size_t)row + 1];
+            v.x *= inv; v.y *= inv; v.z *= inv; v.w *= inv;
+          }
+          finish_pair<T>(v.x, v.y, row, col, m, n, static_cast<const T*>(tail.bias),
+                         static_cast<T*>(tail.out), tail.fuse);
+          if (col + 2 < n)
+            finish_pair<T>(v.z, v.w, row, col + 2, m, n, static_cast<const T*>(tail.bias),
+                           static_cast<T*>(tail.out), tail.fuse);
+        }
+      }
+    };
+    if (io_f16) finish(type_tag<__half>{}); else finish(type_tag<float>{});
+  }
+}
+
+struct SliceCall {
+  const void *x, *w, *scales;
+  uint32_t row_begin, row_end, m, n, k, group_shift, scale_f16, io_f16;
+  SliceTail tail;
+};
+
+template <int XKIND, int MT, int NT, int STEPS>
+int32_t launch_slices(krm_ctx* ctx, const SliceCall& c) {
+  const uint32_t m_blocks = (c.row_end - c.row_begin + 32 * MT - 1) / (32 * MT);
+  const uint32_t tiles = m_blocks * ((c.n + 32 * NT - 1) / (32 * NT));
+  gemm_i4_slices_kernel<XKIND, MT, NT, STEPS>
+      <<<dim3(((tiles + 7) / 8) * 8), dim3(512), 0, ctx->stream>>>(
+          static_cast<const uint8_t*>(c.x), static_cast<const uint8_t*>(c.w),
+          static_cast<const uint8_t*>(c.scales), c.row_begin, c.row_end, c.n, c.k, c.group_shift,
+          m_blocks, tiles, c.scale_f16, c.io_f16, c.m, c.tail);
+  return launched(ctx, "gemm_i4_slices_kernel");
+}
+
+// The tile of a shape.  One workgroup fills a CU (160 KB of LDS), so a launch takes
+// ceil(tiles / CUs) rounds of a fixed part (latency, the sum over the waves, the epilogue) and a
+// part in K (what the second-level cache delivers to a CU per code of its tile).  Both were
+// measured for every tile (us, and us per 1024 codes, cold weights); the cheapest product wins.
+struct TileCost {
+  int mt, nt;
+  float fixed, per_1024;
+};
+constexpr TileCost kCost16[] = {{1, 1, 0.8f, 1.5f}, {1, 2, 1.3f, 2.0f}, {1, 3, 1.7f, 2.5f},
+                                {2, 1, 0.7f, 2.0f}, {2, 2, 2.4f, 2.6f}, {2, 3, 2.2f, 3.6f}};
+constexpr TileCost kCostSplit[] = {{1, 1, 0.2f, 2.45f}, {1, 2, 0.4f, 2.9f}, {1, 3, 0.9f, 3.4f},
+                                   {2, 1, 0.2f, 3.5f}, {2, 2, 1.0f, 4.5f}};
+constexpr TileCost kCost32[] = {{1, 1, 0.8f, 1.75f}, {1, 2, 1.3f, 2.3f}, {1, 3, 1.7f, 2.9f},
+                                {2, 1, 0.7f, 2.75f}, {2, 2, 2.2f, 3.3f}};
+
+template <int XKIND, int STEPS>
+int32_t pick_tile(krm_ctx* ctx, const SliceCall& c) {
+  const TileCost* table = XKIND == kX16 ? kCost16 : XKIND == kXSplit ? kCostSplit : kCost32;
+  const int count = XKIND == kX16 ? 6 : 5;
+  const uint64_t cus = (uint64_t)ctx->num_cus, rows = c.row_end - c.row_begin;
+  int best = 0;
+  float best_cost = 0.f;
+  for (int i = 0; i < count; ++i) {
+    const TileCost& t = table[i];
+    // (below groups of 128 codes the wide tiles' LDS goes to scales; groups of 16 take 32 x 32)
+    if ((STEPS < 8 && t.nt > 2) || (STEPS < 8 && t.mt * t.nt > 2 && XKIND != kX16) ||
+        (STEPS == 1 && t.mt * t.nt > 1))
+      continue;
+    const uint64_t tiles = ((rows + 32 * t.mt - 1) / (32 * t.mt)) * (((uint64_t)c.n + 32 * t.nt - 1) / (32 * t.nt));
+    const float cost = (float)((tiles + cus - 1) / cus) * (t.fixed + t.per_1024 * (float)c.k * (1.0f / 1024));
+    if (i == 0 || cost < best_cost) {
+      best = i;
+      best_cost = cost;
+    }
+  }
+  const int tile = table[best].mt * 10 + table[best].nt;
+  if constexpr (STEPS == 8 && XKIND == kX16) {
+    if (tile == 23) return launch_slices<XKIND, 2, 3, STEPS>(ctx, c);
+  }
+  if constexpr (STEPS == 8) {
+    if (tile == 13) return launch_slices<XKIND, 1, 3, STEPS>(ctx, c);
+  }
+  if constexpr (STEPS == 8 || (STEPS > 1 && XKIND == kX16)) {
+    if (tile == 22) return launch_slices<XKIND, 2, 2, STEPS>(ctx, c);
+  }
+  if constexpr (STEPS > 1) {
+    if (tile == 12) return launch_slices<XKIND, 1, 2, STEPS>(ctx, c);
+    if (tile == 21) return launch_slices<XKIND, 2, 1, STEPS>(ctx, c);
+  }
+  return launch_slices<XKIND, 1, 1, STEPS>(ctx, c);
+}
+
+template <int XKIND>
+int32_t pick_steps(krm_ctx* ctx, const SliceCall& c) {
+  if (c.group_shift >= 7) return pick_tile<XKIND, 8>(ctx, c);
+  if (c.group_shift == 6) return pick_tile<XKIND, 4>(ctx, c);
+  if (c.group_shift == 5) return pick_tile<XKIND, 2>(ctx, c);
+  return pick_tile<XKIND, 1>(ctx, c);
+}
+
+}  // namespace
+
+namespace krm {
+
+// Any shape with K a multiple of 32 (at least 64), any group size of the format and 16-byte
+// aligned rows.  *handled = false (nothing launched) otherwise.
+int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
+                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
+                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
+                              const RowsFusion& fuse, bool* handled, int32_t x_dtype) {
+  *handled = false;
+  const bool half_x = x_dtype == KRM_F16 && io_dtype == KRM_F32;  // fp16 x, f32 bias / out
+  if (x_dtype != io_dtype && !(half_x && compute == KRM_COMPUTE_F16)) return KRM_OK;
+  const bool split = compute == KRM_COMPUTE_F32 && io_dtype == KRM_F32;
+  if (k % 32 != 0 || k < 64 || !aligned(w, 16) || !aligned(x, 16)) return KRM_OK;
+  if ((uint64_t)m * k > 0xffffffffull || (uint64_t)n * (k >> 1) > 0xffffffffull) return KRM_OK;
+  if ((uint64_t)((m + 31) / 32) * ((n + 31) / 32) > 0x7fffffffull) return KRM_OK;
+  SliceCall c{};
+  c.x = ptr<const void>(x);
+  c.w = ptr<const void>(w);
+  c.scales = ptr<const void>(scales);
+  c.row_end = c.m = m;
+  c.n = n;
+  c.k = k;
+  while ((1u << c.group_shift) < group) ++c.group_shift;
+  c.scale_f16 = scale_dtype == KRM_F16;
+  c.io_f16 = io_dtype == KRM_F16;
+  c.tail.bias = ptr<const void>(bias);
+  c.tail.out = ptr<void>(out);
+  c.tail.fuse = fuse;
+  if (!split) {
+    *handled = true;
+    return x_dtype == KRM_F16 ? pick_steps<kX16>(ctx, c) : pick_steps<kX32>(ctx, c);
+  }
+  // hi and lo of as many rows as the context's scratch holds at a time
+  const uint64_t scratch = (uint64_t)2 * ctx->num_cus * kGemmPartialBytes, row_bytes = (uint64_t)k * 4;
+  const uint64_t fit = scratch / row_bytes / 32 * 32;
+  if (m > kMaxSplitRows || fit == 0) return KRM_OK;
+  // (groups below 64 codes have a form without scratch, which a side branch may record)
+  if (group < 64 && ctx->stream != ctx->main_stream) return KRM_OK;
+  KRM_TRY(needs_serial_scratch(ctx, "the f32-class few-row GEMM"));
+  *handled = true;
+  c.tail.row_scale = ctx->row_scales;
+  for (uint64_t first = 0; first < m; first += fit) {
+    const uint32_t rows = (uint32_t)(m - first < fit ? m - first : fit);
+    split_rows_kernel<<<dim3(rows), dim3(512), 0, ctx->stream>>>(
+        ptr<const float>(x) + first * k, reinterpret_cast<uint4*>(ctx->gemm_partials),
+        ctx->row_scales + 2 * first, k);
+    KRM_TRY(launched(ctx, "split_rows_kernel"));
+    c.x = reinterpret_cast<const uint8_t*>(ctx->gemm_partials);
+    c.row_begin = (uint32_t)first;
+    c.row_end = (uint32_t)first + rows;
+    KRM_TRY(pick_steps<kXSplit>(ctx, c));
+  }
+  return KRM_OK;
+}
+
+}  // namespace krm

@@ -1139,7 +1139,7 @@ int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
                              bool* handled);
-int32_t linear_i4_gemm_rows(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
+int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                             krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                             int32_t io_dtype, int32_t scale_dtype, int32_t compute,
                             const RowsFusion& fuse, bool* handled, int32_t x_dtype);
@@ -1173,23 +1173,11 @@ int32_t krm_linear_i4(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_bu
   if (m <= 16)
     return linear_i4_gemv(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype);
   bool handled = false;
-  // Both MFMA forms compute the same arithmetic class.  The 32-row tiles win while their
-  // workgroups make at most three rounds over the CUs (measured: 128 x 11264 x 2048 28.5 us
-  // against 34.2 us, 512 x 2560 x 2048 29.2 against 33.9; 256 x 11264 x 2048 53.7 against 37.7).
-  {
-    uint64_t workgroups = (uint64_t)((m + 31) / 32) * ((n + 31) / 32);
-    if (workgroups > (uint64_t)ctx->num_cus) workgroups = (workgroups + 1) / 2;
-    if (workgroups <= 3ull * (uint64_t)ctx->num_cus) {
-      KRM_TRY(linear_i4_gemm_rows(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
-                                  scale_dtype, compute, RowsFusion{}, &handled, io_dtype));
-      if (handled) return KRM_OK;
-    }
-  }
   KRM_TRY(linear_i4_gemm_exact(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
                                scale_dtype, compute, &handled));
   if (handled) return KRM_OK;
-  KRM_TRY(linear_i4_gemm_rows(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
-                              compute, RowsFusion{}, &handled, io_dtype));
+  KRM_TRY(linear_i4_gemm_slices(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
+                                compute, RowsFusion{}, &handled, io_dtype));
   if (handled) return KRM_OK;
   if (compute == KRM_COMPUTE_F16)
     return linear_i4_gemm_f16(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
@@ -1319,8 +1307,9 @@ int32_t krm_linear_i4_rows(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, k
   fuse.residual = ptr<const void>(residual);
   fuse.mode = epilogue == KRM_EPILOGUE_SILU_PAIRS ? 1 : 0;
   bool handled = false;
-  KRM_TRY(linear_i4_gemm_rows(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
-                              compute, fuse, &handled, x_dtype));
+  if (group >= 64)
+    KRM_TRY(linear_i4_gemm_slices(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
+                                  compute, fuse, &handled, x_dtype));
   if (handled) return KRM_OK;
   return fail(ctx, KRM_ERR_VALIDATION,
               "krm_linear_i4_rows: covers group_size >= 64, k %% 32 == 0, 16-byte aligned x and w, "
@@ -1375,8 +1364,9 @@ int32_t krm_prefill_qkv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_
   fuse.table_rows = table_rows;
   const uint32_t n = (heads + 2 * kv_heads) * depth;
   bool handled = false;
-  KRM_TRY(linear_i4_gemm_rows(ctx, x, w, scales, bias, q_out, m, n, k, group, io_dtype, scale_dtype,
-                              compute, fuse, &handled, x_dtype));
+  if (group >= 64)
+    KRM_TRY(linear_i4_gemm_slices(ctx, x, w, scales, bias, q_out, m, n, k, group, io_dtype,
+                                  scale_dtype, compute, fuse, &handled, x_dtype));
   if (handled) return KRM_OK;
   return fail(ctx, KRM_ERR_VALIDATION,
               "krm_prefill_qkv: covers group_size >= 64, k %% 32 == 0, 16-byte aligned x and w, "

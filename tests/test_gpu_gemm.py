@@ -358,3 +358,36 @@ def test_few_row_results_do_not_depend_on_the_batch(gpu_ctx, compute):
     for rows in ([5], [0, 5, 77], list(range(40, 73))):   # 1, 3 and 33 rows: 32-column tiles
         part = run_rows(gpu_ctx, x[rows], packed, scale, bias, n, k, g, compute)
         assert np.array_equal(part.view(np.uint32), whole[rows].view(np.uint32)), rows
+
+
+# (m, n, k, group): one tile of 32 x 32 / its neighbours, K of one unit, of an odd half unit (ends
+# on 32 of 64 codes), fewer blocks than waves, slices of unequal length, every tile size of the
+# dispatch on 256 CUs (32 x 32, 32 x 64, 32 x 96, 64 x 32, 64 x 64, 64 x 96), the smallest groups
+SLICES_SHAPES = [(17, 31, 64, 16), (32, 33, 96, 16), (33, 64, 96, 32), (77, 300, 2080, 32),
+                 (65, 2049, 160, 32), (64, 129, 1056, 16), (129, 1600, 192, 64), (40, 97, 2624, 64),
+                 (100, 2500, 640, 128), (200, 2500, 1024, 128), (64, 8100, 384, 128),
+                 (512, 2044, 512, 128), (200, 5003, 1024, 256)]
+
+
+@pytest.mark.parametrize("m,n,k,g", SLICES_SHAPES)
+@pytest.mark.parametrize("mode", ["f32", "f16 on f32", "f16"])
+def test_k_slices_kernel_at_the_edges_of_its_tiles(gpu_ctx, m, n, k, g, mode):
+    """krm_linear_i4 for M > 16 at every group size, ragged tiles and K tails, f32 and fp16
+    scales, against the oracle at the gate of the exact-operand kernels."""
+    rng = np.random.default_rng(m + n * 3 + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    scale = scale.astype(np.float32 if (m + k) % 3 else np.float16)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[m // 2] *= 1e3
+    bias = rng.normal(size=n).astype(np.float32)
+    seen = x if mode == "f32" else x.astype(np.float16).astype(np.float32)
+    if mode == "f16":
+        x, bias = x.astype(np.float16), bias.astype(np.float16)
+    compute = ka.COMPUTE_F32 if mode == "f32" else ka.COMPUTE_F16
+    got = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g, compute=compute)
+    want = oracle.linear_i4(seen, packed, scale.astype(np.float32), bias.astype(np.float32), n, k, g)
+    err = np.abs(got.astype(np.float64) - want)
+    bound = row_gate(seen) + 1e-5 * np.abs(want)
+    if mode == "f16":
+        bound = bound + 2.0 ** -11 * np.abs(want) + 1e-7
+    assert np.all(err <= bound), float(np.max(err / bound))
