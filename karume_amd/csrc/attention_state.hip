@@ -518,6 +518,47 @@ __device__ inline float group_sum(float v) {
   return v;
 }
 
+// Halves (x = 32) or neighbouring rows (x = 16) of a wave trade places in one instruction: {a of
+// the lanes whose bit x is clear | b of the same lanes, x further on} and the same of the lanes
+// whose bit is set.
+struct Exchanged {
+  float clear, set;
+};
+__device__ inline Exchanged exchange(float a, float b, int x) {
+  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+  const auto s = x == 32 ? __builtin_amdgcn_permlane32_swap(ua, ub, false, false)
+                         : __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+  return {__uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+__device__ inline float exchange_max(float v, int x) {
+  const Exchanged s = exchange(v, v, x);
+  return fmaxf(s.clear, s.set);
+}
+// Sums of N values (a power of two) over the four 16-lane rows of a wave, each lane left with its
+// share of them: returns the index of the first and leaves max(1, N / 4) totals in v[0..].  A
+// value's tree is the same for every N.
+template <int N>
+__device__ inline int sum_rows(float (&v)[N], int lane) {
+  int n = N, first = 0;
+#pragma unroll
+  for (int x = 32; x >= 16; x >>= 1) {
+    if (n > 1) {
+      n >>= 1;
+#pragma unroll
+      for (int i = 0; i < N / 2; ++i) {
+        if (i >= n) continue;
+        const Exchanged s = exchange(v[i], v[i + n], x);
+        v[i] = s.clear + s.set;
+      }
+      first += (lane & x) ? n : 0;
+    } else {
+      const Exchanged s = exchange(v[0], v[0], x);
+      v[0] = s.clear + s.set;
+    }
+  }
+  return first;
+}
+
 template <typename ST>
 struct RowChunk;  // 16 bytes of a K/V row
 template <>
@@ -603,13 +644,20 @@ constexpr int kMergeChunk = 32;  // split partials merged per pass (all requeste
 // Workgroup = (split, kv head, batch | -): 256 threads = G groups of LPR lanes; a group owns
 // one K/V row per iteration, a lane 16 bytes of it.  Every group keeps its own running
 // (max, sum, weighted V) over the rows it sees — no workgroup barrier inside the column walk —
-// and the G group states are merged once at the end, in ascending group order.  Scores live
-// in the base-2 domain (q carries scale^2 * log2 e), so exponentials are single v_exp_f32.
+// and the group states (where the scores run on the matrix cores: four wave states) are merged
+// once at the end, in ascending order.  Scores live in the base-2 domain (q carries
+// scale^2 * log2 e), so exponentials are single v_exp_f32.
 // With several splits every workgroup publishes its merged partial; the one that arrives last
 // at the (sequence, kv head) counter merges the partials of its r heads in ascending split
 // order — the result does not depend on which workgroup that is.
+// What bounds a long launch is the chain of one workgroup (addresses, rows, scores, P * V, merge,
+// publish: half of a wave's time is waiting) against how many of them a CU holds.  fp16, r = 4,
+// D = 128, sixteen ragged sequences of 4096 columns at most: held to two waves a SIMD and with
+// every head's exponentials in every lane 178 us for four layers (3.1 TB/s); at three waves a SIMD
+// 158; with a wave's softmax shared by its lanes and its groups summed in registers 151
+// (3.7 TB/s).  Forced to four waves it spills: 168.
 template <typename XT, typename ST, int R, int LPR, bool RAGGED>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 2)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 4)))
 void attention_decode_kernel(
     const XT* __restrict__ q, const XT* __restrict__ ins_k, const XT* __restrict__ ins_v,
     const ST* __restrict__ slot_k, const ST* __restrict__ slot_v, XT* __restrict__ out,
@@ -620,10 +668,11 @@ void attention_decode_kernel(
   constexpr int kChunkCols = kDecodeIter * G;
   // fp16 queries and fp16 rows of 128 dims: the scores run on the matrix cores
   constexpr bool kMfma = sizeof(XT) == 2 && sizeof(ST) == 2 && LPR == 16 && kDecodeIter == 8;
+  constexpr int kParts = kMfma ? kThreads / kWave : G;  // states merged through LDS
   constexpr int kOuts = (R * D + kThreads - 1) / kThreads;
-  __shared__ float s_m[G][R];
-  __shared__ float s_l[G][R];
-  __shared__ float s_acc[G][R][D];
+  __shared__ float s_m[kParts][R];
+  __shared__ float s_l[kParts][R];
+  __shared__ __align__(16) float s_acc[kParts][R * D];
   __shared__ float s_w[R][kMergeChunk];
   __shared__ float s_wl[R][kMergeChunk];
   __shared__ uint32_t s_ticket;
@@ -708,19 +757,35 @@ void attention_decode_kernel(
   uint32_t seq, split, nsplit, first_split;
   uint32_t past, row_base;
   if constexpr (RAGGED) {
-    // binary search: last sequence whose first split is <= blockIdx.x
-    uint32_t lo_i = 0, hi_i = a.nseq;
-    while (hi_i - lo_i > 1) {
-      const uint32_t mid = (lo_i + hi_i) >> 1;
-      if ((uint32_t)a.split_prefix[mid] <= blockIdx.x) lo_i = mid; else hi_i = mid;
+    // The last sequence whose first split is <= blockIdx.x, 64 sequences at a time: every lane
+    // asks for one sequence's entries at once, so the tables cost one round trip (a binary search
+    // cost log2(nseq) of them in a row, 0.6 us each, in front of the first row's address).
+    uint32_t first_of = 0, next_of = 0, row_of = 0, row_end_of = 0;
+    seq = 0;
+    for (uint32_t base = 0;; base += kWave) {
+      const uint32_t i = min(base + (uint32_t)lane, a.nseq - 1u);
+      first_of = (uint32_t)a.split_prefix[i];
+      next_of = (uint32_t)a.split_prefix[i + 1];
+      row_of = (uint32_t)a.cu_rows[i];
+      row_end_of = (uint32_t)a.cu_rows[i + 1];
+      const uint64_t mine = __ballot(base + (uint32_t)lane < a.nseq && first_of <= blockIdx.x &&
+                                     blockIdx.x < next_of);
+      if (mine) {
+        const int owner = __builtin_ctzll(mine);
+        seq = base + owner;
+        first_of = __builtin_amdgcn_readlane(first_of, owner);
+        next_of = __builtin_amdgcn_readlane(next_of, owner);
+        row_of = __builtin_amdgcn_readlane(row_of, owner);
+        row_end_of = __builtin_amdgcn_readlane(row_end_of, owner);
+        break;
+      }
+      if (base + kWave >= a.nseq) return;  // a grid sized for the most splits the batch may need
     }
-    seq = lo_i;
-    first_split = (uint32_t)a.split_prefix[seq];
-    nsplit = (uint32_t)a.split_prefix[seq + 1] - first_split;
+    first_split = first_of;
+    nsplit = next_of - first_of;
     split = blockIdx.x - first_split;
-    if (split >= nsplit) return;  // a grid sized for the most splits the batch may need
-    row_base = (uint32_t)a.cu_rows[seq];
-    past = (uint32_t)a.cu_rows[seq + 1] - row_base;
+    row_base = row_of;
+    past = row_end_of - row_of;
   } else {
     seq = blockIdx.z;
     uint32_t p32 = a.past, q32 = 1;
@@ -751,30 +816,37 @@ void attention_decode_kernel(
   const ST* kslot = slot_k + slot_base;
   const ST* vslot = slot_v + slot_base;
 
-  // this step's own row and the query heads (valid addresses for every lane)
   const bool own = last && group == 0;  // the lanes that also take this step's own column
-  float kx[E], vx[E];
-  {
-    const size_t ins_base = ((size_t)seq * a.kv_heads + hk) * D + sub * E;
+  // This step's own row and the query heads (valid addresses for every lane)
+  const size_t ins_base = ((size_t)seq * a.kv_heads + hk) * D;
+  float kx[kMfma ? 1 : E], vx[kMfma ? 1 : E], qf[kMfma ? 1 : R][E];
+  if constexpr (!kMfma) {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      kx[e] = ld_f32<XT>(ins_k, ins_base + e);
-      vx[e] = ld_f32<XT>(ins_v, ins_base + e);
+      kx[e] = ld_f32<XT>(ins_k, ins_base + sub * E + e);
+      vx[e] = ld_f32<XT>(ins_v, ins_base + sub * E + e);
     }
-  }
-  float qf[R][E];
 #pragma unroll
-  for (int h = 0; h < R; ++h) {
-    const size_t q_base = ((size_t)seq * a.heads + head0 + h) * D + sub * E;
+    for (int h = 0; h < R; ++h) {
+      const size_t q_base = ((size_t)seq * a.heads + head0 + h) * D + sub * E;
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-      qf[h][e] = ((ld_f32<XT>(q, q_base + e) * a.scale) * a.scale) * kLog2e;
+      for (int e = 0; e < E; ++e)
+        qf[h][e] = ((ld_f32<XT>(q, q_base + e) * a.scale) * a.scale) * kLog2e;
+    }
   }
 
   // B operand of the score MFMAs: lane (n = lane % 16, g = lane / 16) holds head n's query at
   // dims 32t + 8g.. as raw fp16 (exact products; the scale is applied to the f32 score)
   half8_t qb[kMfma ? 4 : 1];
+  // ... and the A operand whose 16 rows are all this step's own K row: its products are the own
+  // column's scores, head n's in every register of lane n.
+  half8_t own_k[kMfma ? 4 : 1];
+  uint4 own_v;
   if constexpr (kMfma) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      own_k[t] = *reinterpret_cast<const half8_t*>(ins_k + ins_base + 32 * t + 8 * frag_g);
+    own_v = *reinterpret_cast<const uint4*>(ins_v + ins_base + sub * E);
     const int n = tid & 15, g = (tid & 63) >> 4;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -786,14 +858,20 @@ void attention_decode_kernel(
     }
   }
 
-  float run_m[R], run_l[R], acc[R][E];
+  // Running state.  Where the scores run on the matrix cores, lane n of every 16-lane row keeps
+  // head n's maximum (one for the whole wave) and its own groups' sum, so a chunk costs a lane
+  // eight exponentials whatever the number of heads; elsewhere a group keeps every head's.
+  constexpr int kStates = kMfma ? 1 : R;
+  float run_m[kStates], run_l[kStates], acc[R][E];
 #pragma unroll
-  for (int h = 0; h < R; ++h) {
+  for (int h = 0; h < kStates; ++h) {
     run_m[h] = -INFINITY;
     run_l[h] = 0.f;
+  }
+#pragma unroll
+  for (int h = 0; h < R; ++h)
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[h][e] = 0.f;
-  }
 
   auto chunk_begin = [&](uint32_t chunk) { return c_first + chunk * kChunkCols; };
   auto chunk_end = [&](uint32_t c_begin) {  // c_begin < past: no overflow
@@ -808,10 +886,10 @@ void attention_decode_kernel(
     bool valid[kDecodeIter];
 #pragma unroll
     for (int it = 0; it < kDecodeIter; ++it) valid[it] = column_of(it) < width;
-    float sc[kDecodeIter][R];
-    float cm[R];
+    float sc[kDecodeIter][kStates];  // score, then probability
+    float cm[kStates];
 #pragma unroll
-    for (int h = 0; h < R; ++h) cm[h] = -INFINITY;
+    for (int h = 0; h < kStates; ++h) cm[h] = -INFINITY;
     if constexpr (kMfma) {
       // Scores on the matrix cores: the query heads are the B operand (one column per head);
       // lane (h, g) receives the scores of columns 4g..4g+3 of a tile for head h, and lane
@@ -829,13 +907,11 @@ void attention_decode_kernel(
       const float qscale = (a.scale * a.scale) * kLog2e;
 #pragma unroll
       for (int it = 0; it < kDecodeIter; ++it) {
-        const float mine = scores[it / 4][it & 3] * qscale;  // (column of `it`, head lane % 16)
-#pragma unroll
-        for (int h = 0; h < R; ++h) {
-          sc[it][h] = valid[it] ? row_broadcast(mine, h) : -INFINITY;
-          cm[h] = fmaxf(cm[h], sc[it][h]);
-        }
+        // (column of `it`, head lane % 16)
+        sc[it][0] = valid[it] ? scores[it / 4][it & 3] * qscale : -INFINITY;
+        cm[0] = fmaxf(cm[0], sc[it][0]);
       }
+      cm[0] = exchange_max(exchange_max(cm[0], 32), 16);
     } else {
 #pragma unroll
       for (int it = 0; it < kDecodeIter; ++it) {
@@ -852,16 +928,29 @@ void attention_decode_kernel(
         }
       }
     }
-    float keep[R], ref[R];
+    float keep[kStates];
 #pragma unroll
-    for (int h = 0; h < R; ++h) {
+    for (int h = 0; h < kStates; ++h) {
       const float m_new = fmaxf(run_m[h], cm[h]);
-      ref[h] = m_new == -INFINITY ? 0.f : m_new;      // nothing seen yet: 2^(-inf - 0) = 0
-      keep[h] = __builtin_amdgcn_exp2f(run_m[h] - ref[h]);
+      const float ref = m_new == -INFINITY ? 0.f : m_new;  // nothing seen yet: 2^(-inf - 0) = 0
+      keep[h] = __builtin_amdgcn_exp2f(run_m[h] - ref);
       run_m[h] = m_new;
       run_l[h] *= keep[h];
 #pragma unroll
-      for (int e = 0; e < E; ++e) acc[h][e] *= keep[h];
+      for (int it = 0; it < kDecodeIter; ++it) {
+        sc[it][h] = __builtin_amdgcn_exp2f(sc[it][h] - ref);  // 0 outside the chunk
+        run_l[h] += sc[it][h];
+      }
+    }
+    auto of_head = [&](const float (&v)[kStates], int h) {
+      if constexpr (kMfma) return row_broadcast(v[0], h);
+      else return v[h];
+    };
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+      const float scale = of_head(keep, h);
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc[h][e] *= scale;
     }
 #pragma unroll
     for (int it = 0; it < kDecodeIter; ++it) {
@@ -872,8 +961,7 @@ void attention_decode_kernel(
       RowChunk<ST>::unpack(raw, vf);
 #pragma unroll
       for (int h = 0; h < R; ++h) {
-        const float p = __builtin_amdgcn_exp2f(sc[it][h] - ref[h]);  // 0 outside the chunk
-        run_l[h] += p;
+        const float p = of_head(sc[it], h);
 #pragma unroll
         for (int e = 0; e < E; ++e) acc[h][e] = fmaf(p, vf[e], acc[h][e]);
       }
@@ -885,6 +973,16 @@ void attention_decode_kernel(
   // their uses in one branch: a branch between a load and its use makes the compiler wait
   // inside it.
   if (!early) load_chunk(0, rows0);  // harmless when the split has no column at all
+  // The own column's scores, as soon as every row is asked for: the operand's registers go.
+  float own_dot = 0.f;
+  if constexpr (kMfma) {
+    __builtin_amdgcn_sched_barrier(0);
+    float4_t dots = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      dots = __builtin_amdgcn_mfma_f32_16x16x32_f16(own_k[t], qb[t], dots, 0, 0, 0);
+    own_dot = dots[0] * ((a.scale * a.scale) * kLog2e);
+  }
   bool walked = false;
   if constexpr (R == 1) {
     if (nsplit == 1 && total_chunks == 2) {
@@ -933,33 +1031,72 @@ void attention_decode_kernel(
   // this step's own column: one more row for group 0 of the last split (for every other lane
   // the update below is the identity, so the other splits skip it)
   if (last) {
+    float s_own[kStates], vo[E];
+    if constexpr (kMfma) {
+      s_own[0] = wave == 0 ? own_dot : -INFINITY;
+      RowChunk<ST>::unpack(own_v, vo);
+    } else {
+#pragma unroll
+      for (int h = 0; h < R; ++h) {
+        float part = 0.f;
+#pragma unroll
+        for (int e = 0; e < E; ++e) part = fmaf(qf[h][e], kx[e], part);
+        part = group_sum<LPR>(part);
+        s_own[h] = own ? part : -INFINITY;
+      }
+#pragma unroll
+      for (int e = 0; e < E; ++e) vo[e] = vx[e];
+    }
+    float keep[kStates], p_own[kStates];
+#pragma unroll
+    for (int h = 0; h < kStates; ++h) {
+      const float m_new = fmaxf(run_m[h], s_own[h]);
+      const float ref = m_new == -INFINITY ? 0.f : m_new;
+      keep[h] = __builtin_amdgcn_exp2f(run_m[h] - ref);
+      p_own[h] = own ? __builtin_amdgcn_exp2f(s_own[h] - ref) : 0.f;
+      run_m[h] = m_new;
+      run_l[h] = run_l[h] * keep[h] + p_own[h];
+    }
 #pragma unroll
     for (int h = 0; h < R; ++h) {
-      float part = 0.f;
-#pragma unroll
-      for (int e = 0; e < E; ++e) part = fmaf(qf[h][e], kx[e], part);
-      part = group_sum<LPR>(part);
-      const float s_own = own ? part : -INFINITY;
-      const float m_new = fmaxf(run_m[h], s_own);
-      const float ref = m_new == -INFINITY ? 0.f : m_new;
-      const float keep = __builtin_amdgcn_exp2f(run_m[h] - ref);
-      const float p = __builtin_amdgcn_exp2f(s_own - ref);
-      run_m[h] = m_new;
-      run_l[h] = run_l[h] * keep + p;
+      float k = keep[kMfma ? 0 : h], p = p_own[kMfma ? 0 : h];
+      if constexpr (kMfma) {
+        k = row_broadcast(k, h);
+        p = row_broadcast(p, h);
+      }
 #pragma unroll
       for (int e = 0; e < E; ++e)
-        acc[h][e] = fmaf(p, own ? vx[e] : 0.f, acc[h][e] * keep);  // 0 * NaN must not leak
+        acc[h][e] = fmaf(p, own ? vo[e] : 0.f, acc[h][e] * k);  // 0 * NaN must not leak
     }
   }
 
-  // merge of the G group states, ascending group order
+  // The states are merged in ascending order.  A wave that keeps one maximum for its groups sums
+  // them in registers first, a quarter of the outputs left to each lane (sixteen group states
+  // through LDS cost 32 KB and every output sixteen exponentials).
+  if constexpr (kMfma) {
+    constexpr int kHeld = R * E / 4;  // consecutive dims of one head
+    float flat[R * E];
 #pragma unroll
-  for (int h = 0; h < R; ++h) {
+    for (int i = 0; i < R * E; ++i) flat[i] = acc[i / E][i % E];
+    const int first = sum_rows(flat, lane);
+    float* mine = &s_acc[wave][(first / E) * D + sub * E + first % E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) s_acc[group][h][sub * E + e] = acc[h][e];
-    if (sub == 0) {
-      s_m[group][h] = run_m[h];
-      s_l[group][h] = run_l[h];
+    for (int i = 0; i < kHeld; i += 2)
+      *reinterpret_cast<float2*>(mine + i) = make_float2(flat[i], flat[i + 1]);
+    sum_rows(run_l, lane);
+    if (lane < R) {
+      s_m[wave][lane] = run_m[0];
+      s_l[wave][lane] = run_l[0];
+    }
+  } else {
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) s_acc[group][h * D + sub * E + e] = acc[h][e];
+      if (sub == 0) {
+        s_m[group][h] = run_m[h];
+        s_l[group][h] = run_l[h];
+      }
     }
   }
   __syncthreads();
@@ -974,13 +1111,13 @@ void attention_decode_kernel(
     const int h = o / D, d = o - h * D;
     float m = s_m[0][h];
 #pragma unroll
-    for (int g = 1; g < G; ++g) m = fmaxf(m, s_m[g][h]);  // finite: the split holds a column
+    for (int w = 1; w < kParts; ++w) m = fmaxf(m, s_m[w][h]);  // finite: the split holds a column
     float total = 0.f, l = 0.f;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const float wgt = __builtin_amdgcn_exp2f(s_m[g][h] - m);
-      total = fmaf(wgt, s_acc[g][h][d], total);
-      l = fmaf(wgt, s_l[g][h], l);
+    for (int w = 0; w < kParts; ++w) {
+      const float wgt = __builtin_amdgcn_exp2f(s_m[w][h] - m);
+      total = fmaf(wgt, s_acc[w][o], total);
+      l = fmaf(wgt, s_l[w][h], l);
     }
     part_o[i] = total;
     part_l[i] = l;
@@ -1111,10 +1248,6 @@ int32_t decode_by_repeat(krm_ctx* ctx, const DecodeLaunch& L, uint32_t per_block
     case 1: return launch_decode<XT, ST, 1, LPR, RAGGED>(ctx, L);
     case 2: return launch_decode<XT, ST, 2, LPR, RAGGED>(ctx, L);
     case 4: return launch_decode<XT, ST, 4, LPR, RAGGED>(ctx, L);
-    case 8:
-      // (rows that span a whole wave: eight heads' state does not fit the registers)
-      if constexpr (LPR < 64) return launch_decode<XT, ST, 8, LPR, RAGGED>(ctx, L);
-      [[fallthrough]];
     default: return fail(ctx, KRM_ERR_VALIDATION, "decode attention: %u heads per block", per_block);
   }
 }
@@ -1134,12 +1267,15 @@ int32_t decode_by_depth(krm_ctx* ctx, const DecodeLaunch& L, uint32_t per_block,
 // Few (split, kv head) pairs leave most of the chip idle while each workgroup walks its
 // columns once per query head; the query heads of a kv head are then spread over several
 // workgroups (each re-reads the K/V rows, which the L2 serves) until the grid covers the CUs.
+// Four heads at most: the state of eight takes a SIMD's registers to one wave or two, and sixteen
+// sequences of eight heads of D = 256 then took 198 us where two groups of four take 133
+// (D = 64: 134 and 105).
 template <bool RAGGED>
 int32_t decode_dispatch(krm_ctx* ctx, DecodeLaunch& L, uint32_t repeat, uint32_t lpr,
                         int32_t io_dtype, int32_t kv_dtype) {
   uint32_t per_block = repeat;
   uint64_t blocks = (uint64_t)L.grid_x * L.grid_z * L.args.kv_heads;
-  while (per_block > 1 && (blocks < 2ull * (uint64_t)ctx->num_cus || (lpr == 64 && per_block > 4))) {
+  while (per_block > 4 || (per_block > 1 && blocks < 2ull * (uint64_t)ctx->num_cus)) {
     per_block >>= 1;
     blocks <<= 1;
   }

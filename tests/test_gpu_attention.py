@@ -106,6 +106,27 @@ def test_decode_split_k(gpu_ctx, case, io, kv):
         assert np.all(err <= ulp), float(np.max(err))
 
 
+@pytest.mark.parametrize("depth", [32, 64, 128, 256])
+@pytest.mark.parametrize("repeat,past", [(8, 0), (4, 1), (8, 65), (2, 129), (1, 127), (4, 600)])
+@pytest.mark.parametrize("io,kv", [(np.float32, np.float32), (np.float16, np.float16),
+                                   (np.float32, np.float16)])
+def test_decode_wave_states_with_several_heads_a_workgroup(gpu_ctx, depth, repeat, past, io, kv):
+    """Enough sequences that a workgroup carries up to four heads of a kv head: waves without a
+    column, one row past a wave's share, the own column alone, several splits; every head dim
+    (groups of 4 to 64 lanes)."""
+    batch = 520 if past < 600 else 64
+    case = StateCase("", batch, repeat, 1, 1, depth, past + 8, 0, past, 1)
+    x = random_state_inputs(case, seed=past + depth + repeat, f16_values=True)
+    want = oracle_state_attention(case, x)
+    got = run_attention(gpu_ctx, case, x, io=io, kv=kv)
+    if io == np.float32:
+        ok, fails, max_abs, worst = oracle.allclose(got, want, atol=STATE_ATOL, rtol=0)
+        assert ok, (fails, max_abs, worst)
+    else:
+        ulp = np.spacing(np.abs(want.astype(np.float16))).astype(np.float32)
+        assert np.all(np.abs(got.astype(np.float32) - want.astype(np.float16)) <= ulp + STATE_ATOL)
+
+
 ROWS_CASES = [
     # chunks of rows with D = 64 / 128: the matrix-core form (16 query rows a workgroup, key
     # blocks of 32 dealt to the waves: eight for D = 64, four for D = 128)
