@@ -19,6 +19,7 @@
 #include "krm_internal.h"
 
 #include <cmath>
+#include <type_traits>
 
 using namespace krm;
 
@@ -189,12 +190,19 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 //                  exchange between the four lane groups;
 //   O^T += V^T P^T the scores a lane holds are exactly a B operand if MFMA step (t, i) is
 //                  given the keys 16 t + 4 g + i, so the probabilities never move; V^T is the A
-//                  operand, read from the parked V block with the same key per step.  The
-//                  result again has the query row in lane % 16 (dims 16 dt + 4 g + 0..3).
-// K and V blocks are parked in the wave's own LDS area (coalesced 16-byte loads; a block may
-// straddle the state slot and this step's rows).  The waves' (max, sum, O) are merged in LDS
-// at the end; rows >= query are written as +0.  Sixteen rows a workgroup (not 32) so that a
-// 128-row chunk of 32 heads is 256 workgroups, one per CU.
+//                  operand with the same key per step: 16 lanes take that key's row 16 bytes each
+//                  and keep it in registers (a piece's four dims feed four output tiles), so V
+//                  needs no LDS at all.
+// The K block is parked in the wave's own LDS area (coalesced 16-byte loads; a block may straddle
+// the state slot and this step's rows): read as an operand from memory it came in half lines,
+// half as fast.  D = 64: the next block's rows are asked for as soon as this one's are used.  The
+// waves' (max, sum, O) are merged in LDS at the end; rows >= query are written as +0.  Sixteen
+// rows a workgroup (not 32) so that a 128-row chunk of 32 heads is 256 workgroups, one per CU.
+// What bounds it is the f32 matrix rate with two waves a SIMD to cover softmax and waits (D = 64,
+// r = 8, 128 rows behind 1024: 8 us of MFMA).  With V parked as well, rows looked up one by one
+// (two element types: a wait at each), expf and no requests ahead, us before / now: that case
+// 22.7 / 19.2; fp16, D = 128, r = 4: 49.2 / 33.9; f32 over fp16 slots 105.6 / 36.2; D = 256, r = 8
+// (two waves then, four now that LDS holds K alone): 162 / 70.
 typedef float float4v_t __attribute__((ext_vector_type(4)));
 
 template <typename T>
@@ -210,6 +218,43 @@ __device__ inline float4 load4_f32<__half>(const __half* p) {
   return make_float4(__low2float(a), __high2float(a), __low2float(b), __high2float(b));
 }
 
+// Halves (x = 32) or neighbouring rows (x = 16) of a wave trade places in one instruction: {a of
+// the lanes whose bit x is clear | b of the same lanes, x further on} and the same of the lanes
+// whose bit is set.
+struct Exchanged {
+  float clear, set;
+};
+__device__ inline Exchanged exchange(float a, float b, int x) {
+  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+  const auto s = x == 32 ? __builtin_amdgcn_permlane32_swap(ua, ub, false, false)
+                         : __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+  return {__uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+__device__ inline float exchange_max(float v, int x) {
+  const Exchanged s = exchange(v, v, x);
+  return fmaxf(s.clear, s.set);
+}
+// A 4-element piece of a row as it arrives: 16 bytes of f32 or 8 of fp16.
+template <typename T>
+__device__ inline uint4 load4_raw(const T* p) {
+  if constexpr (sizeof(T) == 4) {
+    return *reinterpret_cast<const uint4*>(p);
+  } else {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    return make_uint4(v.x, v.y, 0u, 0u);
+  }
+}
+template <typename T>
+__device__ inline float4 raw4_f32(const uint4& v) {
+  if constexpr (sizeof(T) == 4) {
+    return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z),
+                       __uint_as_float(v.w));
+  } else {
+    const __half2 a = __builtin_bit_cast(__half2, v.x), b = __builtin_bit_cast(__half2, v.y);
+    return make_float4(__low2float(a), __high2float(a), __low2float(b), __high2float(b));
+  }
+}
+
 template <typename XT, typename ST, int D, int WAVES, int RB>
 __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     const XT* __restrict__ q, const XT* __restrict__ ins_k, const XT* __restrict__ ins_v,
@@ -220,11 +265,11 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   constexpr int kRow = D + 4;                 // floats of a parked row
   constexpr int DT = D / 16;                  // output tiles of 16 dims
   constexpr int kQuarter = D / 4;             // dims a lane group walks
+  constexpr int kVPieces = D / 64;            // 16-byte pieces of a V row a lane takes
   constexpr int kPieces = D / 4;              // 4-element pieces of a row
   constexpr int kRowsPerLoad = 64 / kPieces;
   constexpr int kLoads = 32 / kRowsPerLoad;
   __shared__ __align__(16) float s_k[WAVES][32 * kRow];
-  __shared__ __align__(16) float s_v[WAVES][32 * kRow];
   __shared__ float s_m[WAVES][kRows], s_l[WAVES][kRows];
 
   const uint32_t z = blockIdx.x, row0 = blockIdx.y * (uint32_t)kRows;
@@ -242,24 +287,6 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     }
     return ((size_t)z * a.chunk_rows + row) * D + d;
   };
-  // The chunk's own K / V rows of this block go to the state slots here when asked for (the
-  // first query head of each kv plane does it).  Without a window no reader of this launch
-  // touches them: slot rows are read for columns < past only, these are rows past + row.
-  if ((flags & KRM_CHUNK_APPEND) && z % (a.heads / a.kv_heads) == 0) {
-    const uint32_t plane = z / (a.heads / a.kv_heads);
-    for (uint32_t i = tid; i < (uint32_t)kRows * kPieces; i += kBlock) {
-      const uint32_t rr = i / kPieces, piece = i - rr * kPieces;
-      const uint32_t row = row0 + rr;
-      if (row >= query) continue;
-      const size_t src = ((size_t)plane * a.chunk_rows + row) * D + 4 * piece;
-      const size_t dst = ((size_t)plane * a.capacity + past + row) * D + 4 * piece;
-      const float4 kv = load4_f32<XT>(ins_k + src), vv = load4_f32<XT>(ins_v + src);
-      st_f32<ST>(slot_k, dst, kv.x); st_f32<ST>(slot_k, dst + 1, kv.y);
-      st_f32<ST>(slot_k, dst + 2, kv.z); st_f32<ST>(slot_k, dst + 3, kv.w);
-      st_f32<ST>(slot_v, dst, vv.x); st_f32<ST>(slot_v, dst + 1, vv.y);
-      st_f32<ST>(slot_v, dst + 2, vv.z); st_f32<ST>(slot_v, dst + 3, vv.w);
-    }
-  }
   if (row0 >= query) {  // a block of pad rows: exact zeros, nothing is read
     for (uint32_t i = tid; i < (uint32_t)kRows * D; i += kBlock) {
       const uint32_t row = row0 + i / D;
@@ -273,25 +300,15 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   }
   const uint32_t kv_plane = z / (a.heads / a.kv_heads);
 
-  // Q block -> LDS (scaled), then each lane's B operands: Q[r][g * D/4 + s]
-  for (uint32_t i = tid; i < (uint32_t)kRows * kPieces; i += kBlock) {
-    const uint32_t rr = i / kPieces, piece = i - rr * kPieces;
-    const uint32_t row = min(row0 + rr, a.chunk_rows - 1);
-    float4 v = load4_f32<XT>(q + ((size_t)z * a.chunk_rows + row) * D + 4 * piece);
-    v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
-    *reinterpret_cast<float4*>(&s_k[0][rr * kRow + 4 * piece]) = v;
+  // Q block: asked for first, parked (scaled) behind the request of the wave's first key block
+  constexpr int kQUnits = kRows * kPieces, kQPer = (kQUnits + (int)kBlock - 1) / (int)kBlock;
+  uint4 qraw[kQPer];
+#pragma unroll
+  for (int j = 0; j < kQPer; ++j) {
+    const uint32_t i = min((uint32_t)tid + j * kBlock, (uint32_t)kQUnits - 1u);
+    const uint32_t row = min(row0 + i / kPieces, a.chunk_rows - 1);
+    qraw[j] = load4_raw<XT>(q + ((size_t)z * a.chunk_rows + row) * D + 4 * (i % kPieces));
   }
-  __syncthreads();
-  float qf[RB][kQuarter];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int i = 0; i < kQuarter / 4; ++i) {
-      const float4 v = *reinterpret_cast<const float4*>(
-          &s_k[0][(16 * rb + r) * kRow + g * kQuarter + 4 * i]);
-      qf[rb][4 * i] = v.x; qf[rb][4 * i + 1] = v.y; qf[rb][4 * i + 2] = v.z; qf[rb][4 * i + 3] = v.w;
-    }
-  __syncthreads();
 
   // columns the block's rows can see: [c_lo, limit_hi]
   const uint32_t last_row = min(row0 + (uint32_t)kRows - 1u, query - 1u);
@@ -306,12 +323,114 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   }
 
   float* mk = s_k[wave];
-  float* mv = s_v[wave];
   auto wave_sync = [] {  // the areas are the wave's own: its LDS queue orders them
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
+
+  // Requests only: the K rows of key block kb (whole rows, parked in LDS later) and its V rows (in
+  // the operand layout: step j of lane group g carries the key 16 (j / 4) + 4 g + j % 4, and 16
+  // lanes take that row 16 bytes each).  Columns below `past` are slot rows, the rest this step's;
+  // a column beyond the last one is the last one again, masked when used.  A block on one side of
+  // `past` whose slot rows do not wrap is 32-bit offsets from one base; only the others look every
+  // row up.
+  const uint32_t load_key = lane / kPieces, load_piece = 4u * (lane % kPieces);
+  const size_t slot_plane = (size_t)kv_plane * a.capacity * D;
+  const size_t ins_plane = (size_t)kv_plane * a.chunk_rows * D;
+  auto slot_columns = [&](uint64_t c0) -> uint32_t {  // of the block's 32
+    return c0 >= past ? 0u : (uint32_t)(past - c0 < 32u ? past - c0 : 32u);
+  };
+  // `keys` lane rows, row i the block's key key_of(i), `pieces` pieces of 4 elements 64 apart
+  auto request = [&](uint32_t kb, const ST* slot, const XT* ins, auto keys, auto key_of,
+                     uint32_t lane_dim, auto pieces, uint4* raw) {
+    constexpr int kKeys = decltype(keys)::value, kPer = decltype(pieces)::value;
+    const uint64_t c0 = c_lo + (uint64_t)kb * 32u;
+    const uint32_t slots = slot_columns(c0);
+    const uint32_t first = a.window ? (uint32_t)c0 % a.window : (uint32_t)c0;
+    if (slots == 32u && (a.window == 0 || first + 32u <= a.window)) {
+      const ST* base = slot + slot_plane + (size_t)first * D;
+#pragma unroll
+      for (int i = 0; i < kKeys; ++i)
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+          raw[i * kPer + j] = load4_raw<ST>(base + (key_of(i) * D + lane_dim + 64 * j));
+    } else if (slots == 0u) {
+      const XT* base = ins + ins_plane + (size_t)(c0 - past) * D;
+      const uint32_t most = limit_hi - c0 < 31u ? (uint32_t)(limit_hi - c0) : 31u;
+#pragma unroll
+      for (int i = 0; i < kKeys; ++i)
+#pragma unroll
+        for (int j = 0; j < kPer; ++j)
+          raw[i * kPer + j] = load4_raw<XT>(base + (min(key_of(i), most) * D + lane_dim + 64 * j));
+    } else {
+#pragma unroll
+      for (int i = 0; i < kKeys; ++i) {
+        const uint32_t key = min(key_of(i), (uint32_t)(limit_hi - c0 < 31u ? limit_hi - c0 : 31u));
+        const bool in_slot = key < slots;
+        uint32_t at = first + key;  // (a block of 32 wraps once, unless the window is shorter)
+        if (a.window && at >= a.window) at = a.window >= 32u ? at - a.window : at % a.window;
+        const size_t row = lane_dim + (in_slot ? slot_plane + (size_t)at * D
+                                               : ins_plane + (size_t)(c0 + key - past) * D);
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+          if constexpr (sizeof(ST) == sizeof(XT))
+            raw[i * kPer + j] = load4_raw<XT>((in_slot ? reinterpret_cast<const XT*>(slot) : ins) + row + 64 * j);
+          else
+            raw[i * kPer + j] = in_slot ? load4_raw<ST>(slot + row + 64 * j) : load4_raw<XT>(ins + row + 64 * j);
+        }
+      }
+    }
+  };
+  auto v_key = [&](int j) -> uint32_t { return (uint32_t)(16 * (j / 4) + 4 * g + j % 4); };
+  uint4 kraw[kLoads], vraw[8 * kVPieces];
+  auto request_k = [&](uint32_t kb) {
+    request(kb, slot_k, ins_k, std::integral_constant<int, kLoads>{},
+            [&](int i) { return (uint32_t)(i * kRowsPerLoad) + load_key; }, load_piece,
+            std::integral_constant<int, 1>{}, kraw);
+  };
+  auto request_v = [&](uint32_t kb) {
+    request(kb, slot_v, ins_v, std::integral_constant<int, 8>{}, v_key, 4u * r,
+            std::integral_constant<int, kVPieces>{}, vraw);
+  };
+  // f32 of what arrived
+  auto element4 = [&](const uint4& v, uint32_t key, uint32_t slots) {
+    if constexpr (sizeof(ST) == sizeof(XT)) {
+      return raw4_f32<XT>(v);
+    } else {
+      const float4 s4 = raw4_f32<ST>(v), x4 = raw4_f32<XT>(v);
+      const bool in_slot = key < slots;
+      return make_float4(in_slot ? s4.x : x4.x, in_slot ? s4.y : x4.y, in_slot ? s4.z : x4.z,
+                         in_slot ? s4.w : x4.w);
+    }
+  };
+  // (longer rows: the next block's beside this one's would take the registers of the state)
+  constexpr bool kAhead = D * sizeof(XT) * sizeof(ST) <= 64 * 16;
+  if (kAhead && (uint32_t)wave < blocks) {
+    request_k((uint32_t)wave);
+    request_v((uint32_t)wave);
+  }
+
+  // each lane's B operands: Q[r][g * D/4 + s]
+#pragma unroll
+  for (int j = 0; j < kQPer; ++j) {
+    const uint32_t i = (uint32_t)tid + j * kBlock;
+    float4 v = raw4_f32<XT>(qraw[j]);
+    v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
+    if (i < (uint32_t)kQUnits)
+      *reinterpret_cast<float4*>(&s_k[0][(i / kPieces) * kRow + 4 * (i % kPieces)]) = v;
+  }
+  __syncthreads();
+  float qf[RB][kQuarter];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int i = 0; i < kQuarter / 4; ++i) {
+      const float4 v = *reinterpret_cast<const float4*>(
+          &s_k[0][(16 * rb + r) * kRow + g * kQuarter + 4 * i]);
+      qf[rb][4 * i] = v.x; qf[rb][4 * i + 1] = v.y; qf[rb][4 * i + 2] = v.z; qf[rb][4 * i + 3] = v.w;
+    }
+  __syncthreads();
 
   float run_m[RB], run_l[RB];
   float4v_t acc[RB][DT];
@@ -327,32 +446,19 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 
   for (uint32_t kb = (uint32_t)wave; kb < blocks; kb += (uint32_t)WAVES) {
     const uint64_t c0 = c_lo + (uint64_t)kb * 32u;
-    // park the K (scaled) and V rows of the block
-    float4 kraw[kLoads], vraw[kLoads];
+    // park the K rows of the block (scaled), then ask for the next one's
+    const bool more = kb + (uint32_t)WAVES < blocks;
+    if constexpr (!kAhead) request_k(kb);
+    const uint32_t slots = slot_columns(c0);
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      const uint32_t key = j * kRowsPerLoad + lane / kPieces, piece = lane % kPieces;
-      uint64_t c = c0 + key;
-      c = c < limit_hi ? c : limit_hi;  // beyond the last column: any valid row, masked below
-      if (c < past) {
-        const uint32_t prow = a.window ? (uint32_t)c % a.window : (uint32_t)c;  // c < past: a u32
-        const size_t at = ((size_t)kv_plane * a.capacity + prow) * D + 4 * piece;
-        kraw[j] = load4_f32<ST>(slot_k + at);
-        vraw[j] = load4_f32<ST>(slot_v + at);
-      } else {
-        const size_t at = ((size_t)kv_plane * a.chunk_rows + (size_t)(c - past)) * D + 4 * piece;
-        kraw[j] = load4_f32<XT>(ins_k + at);
-        vraw[j] = load4_f32<XT>(ins_v + at);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kLoads; ++j) {
-      const uint32_t key = j * kRowsPerLoad + lane / kPieces, piece = lane % kPieces;
-      float4 kv = kraw[j];
+      const uint32_t key = j * kRowsPerLoad + load_key;
+      float4 kv = element4(kraw[j], key, slots);
       kv.x *= a.scale; kv.y *= a.scale; kv.z *= a.scale; kv.w *= a.scale;
-      *reinterpret_cast<float4*>(&mk[key * kRow + 4 * piece]) = kv;
-      *reinterpret_cast<float4*>(&mv[key * kRow + 4 * piece]) = vraw[j];
+      *reinterpret_cast<float4*>(&mk[key * kRow + load_piece]) = kv;
     }
+    if constexpr (!kAhead) request_v(kb);
+    if (kAhead && more) request_k(kb + (uint32_t)WAVES);
     wave_sync();
 
 #pragma unroll
@@ -361,86 +467,128 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       // rows see further)
       if (c0 > (uint64_t)past + row0 + (uint32_t)(16 * rb + 15)) continue;
       // S^T[key][query row], tile t = keys 16 t ..: A = K[16 t + r][g * D/4 + s], B = Q^T
+      // (the two tiles, and below the dims, in turn: neighbouring MFMAs do not wait for each other)
       float4v_t st[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) st[t][i] = 0.f;
-#pragma unroll
-        for (int i = 0; i < kQuarter / 4; ++i) {
-          const float4 kf =
-              *reinterpret_cast<const float4*>(&mk[(16 * t + r) * kRow + g * kQuarter + 4 * i]);
-          st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf[rb][4 * i], st[t], 0, 0, 0);
-          st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf[rb][4 * i + 1], st[t], 0, 0, 0);
-          st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf[rb][4 * i + 2], st[t], 0, 0, 0);
-          st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf[rb][4 * i + 3], st[t], 0, 0, 0);
-        }
-      }
-      // this lane: query row 16 rb + r, keys 16 t + 4 g + i
-      float block_max = -INFINITY;
-      bool valid[2][4];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint64_t c = c0 + (uint32_t)(16 * t + 4 * g + i);
-          valid[t][i] = c <= my_limit[rb] && c >= my_low[rb];
-          block_max = fmaxf(block_max, valid[t][i] ? st[t][i] : -INFINITY);
-        }
-      block_max = fmaxf(block_max, __shfl_xor(block_max, 16, kWave));
-      block_max = fmaxf(block_max, __shfl_xor(block_max, 32, kWave));
+        for (int i = 0; i < 4; ++i) st[t][i] = 0.f;
+#pragma unroll
+      for (int i = 0; i < kQuarter / 4; ++i) {
+        float kf[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          *reinterpret_cast<float4*>(kf[t]) =
+              *reinterpret_cast<const float4*>(&mk[(16 * t + r) * kRow + g * kQuarter + 4 * i]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][j], qf[rb][4 * i + j], st[t], 0, 0, 0);
+      }
+      // this lane: query row 16 rb + r, keys 16 t + 4 g + i
+      // (uniform: a block that every one of these rows sees whole needs no mask)
+      const uint64_t first_limit = (uint64_t)past + row0 + 16u * (uint32_t)rb;
+      if (c0 + 31u > first_limit || window_low(a.window, first_limit + 15u) > c0) {
+        const int last_key = my_limit[rb] < c0 ? -1 : (int)(my_limit[rb] - c0 < 32u ? my_limit[rb] - c0 : 32u);
+        const int first_key = my_low[rb] <= c0 ? 0 : (int)(my_low[rb] - c0 < 32u ? my_low[rb] - c0 : 32u);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int key = 16 * t + 4 * g + i;
+            if (key > last_key || key < first_key) st[t][i] = -INFINITY;
+          }
+      }
+      float block_max = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) block_max = fmaxf(block_max, st[t][i]);
+      block_max = exchange_max(exchange_max(block_max, 16), 32);
       const float new_m = fmaxf(run_m[rb], block_max);
       const float ref = new_m == -INFINITY ? 0.f : new_m;  // nothing seen yet: exp(-inf - 0) = 0
-      const float alpha = expf(run_m[rb] - ref);
+      // (the difference first, then its product with log2 e: one v_exp_f32, within an ulp of expf on
+      // what it is added to; expf's own range handling was a quarter of the loop's instructions)
+      const float alpha = __builtin_amdgcn_exp2f((run_m[rb] - ref) * 1.4426950408889634f);
       float p[2][4], sum = 0.f;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          p[t][i] = valid[t][i] ? expf(st[t][i] - ref) : 0.f;
+          p[t][i] = __builtin_amdgcn_exp2f((st[t][i] - ref) * 1.4426950408889634f);  // 0 where masked
           sum += p[t][i];
         }
       run_l[rb] = run_l[rb] * alpha + sum;
       run_m[rb] = new_m;
       // O^T[d][query row] = alpha * O^T + V^T P^T: step (t, i) carries the keys 16 t + 4 g + i
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= alpha;
+      // (tile dt = 4 i + e holds the dims 64 i + 4 r + e: a 16-byte piece feeds four tiles)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+      for (int j = 0; j < 8; ++j) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float vf = mv[(16 * t + 4 * g + i) * kRow + 16 * dt + r];
-            acc[rb][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf, p[t][i], acc[rb][dt], 0, 0, 0);
-          }
+        for (int i = 0; i < kVPieces; ++i) {
+          const float4 v4 = element4(vraw[j * kVPieces + i], v_key(j), slots);
+          const float vf[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[rb][4 * i + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[e], p[j / 4][j % 4],
+                                                                     acc[rb][4 * i + e], 0, 0, 0);
+        }
       }
     }
+    if (kAhead && more) request_v(kb + (uint32_t)WAVES);
     wave_sync();  // the block's rows have been read: the next block may be parked
+  }
+
+  // The chunk's own K / V rows of this block go to the state slots when asked for (the first query
+  // head of each kv plane does it; asked for here, stored behind the merge).  Without a window no
+  // reader of this launch touches them: slot rows are read for columns < past only, these are
+  // rows past + row.
+  const bool append = (flags & KRM_CHUNK_APPEND) && z % (a.heads / a.kv_heads) == 0;
+  uint4 own_k[kQPer], own_v[kQPer];
+#pragma unroll
+  for (int j = 0; j < kQPer; ++j) {
+    const uint32_t i = min((uint32_t)tid + j * kBlock, (uint32_t)kQUnits - 1u);
+    const uint32_t row = min(row0 + i / kPieces, query - 1u);
+    const size_t src = ((size_t)kv_plane * a.chunk_rows + row) * D + 4 * (i % kPieces);
+    if (append) {
+      own_k[j] = load4_raw<XT>(ins_k + src);
+      own_v[j] = load4_raw<XT>(ins_v + src);
+    }
   }
 
   // the wave's state: (max, sum) per query row and O[row][d] in its own area
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
-    run_l[rb] += __shfl_xor(run_l[rb], 16, kWave);
-    run_l[rb] += __shfl_xor(run_l[rb], 32, kWave);
+    for (int x = 16; x <= 32; x <<= 1) {
+      const Exchanged both = exchange(run_l[rb], run_l[rb], x);
+      run_l[rb] = both.clear + both.set;
+    }
     if (g == 0) {
       s_m[wave][16 * rb + r] = run_m[rb];
       s_l[wave][16 * rb + r] = run_l[rb];
     }
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)  // registers 0..3: dims 16 dt + 4 g + 0..3
-      *reinterpret_cast<float4*>(&mk[(16 * rb + r) * kRow + 16 * dt + 4 * g]) =
-          make_float4(acc[rb][dt][0], acc[rb][dt][1], acc[rb][dt][2], acc[rb][dt][3]);
+    for (int i = 0; i < kVPieces; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)  // register j of tiles 4 i + 0..3: dims 64 i + 16 g + 4 j + 0..3
+        *reinterpret_cast<float4*>(&mk[(16 * rb + r) * kRow + 64 * i + 16 * g + 4 * j]) =
+            make_float4(acc[rb][4 * i][j], acc[rb][4 * i + 1][j], acc[rb][4 * i + 2][j],
+                        acc[rb][4 * i + 3][j]);
   }
   __syncthreads();
 
-  // merge of the waves, wave order; 16 threads a row (256 row-part units, dealt over the
-  // workgroup's threads: a workgroup of two waves takes two rounds)
-  for (uint32_t unit = tid; unit < 256u; unit += kBlock) {
+  // merge of the waves, wave order: a row's dims dealt over the threads of its block of 16 rows (a
+  // workgroup of two waves takes two rounds)
+  constexpr uint32_t kUnits = kBlock < 256u ? 256u : kBlock;
+  for (uint32_t unit = tid; unit < kUnits; unit += kBlock) {
    for (uint32_t rb = 0; rb < (uint32_t)RB; ++rb) {
-    constexpr int kPer = D / 16;
-    const uint32_t rr = 16u * rb + (unit >> 4), d0 = (unit & 15u) * kPer;
+    constexpr int kPer = 16 * D / (int)kUnits, kParts = D / kPer;
+    const uint32_t rr = 16u * rb + unit / kParts, d0 = (unit % kParts) * kPer;
     const uint32_t row = row0 + rr;
     float top = s_m[0][rr];
 #pragma unroll
@@ -467,6 +615,19 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       }
     }
    }
+  }
+  if (append) {
+#pragma unroll
+    for (int j = 0; j < kQPer; ++j) {
+      const uint32_t i = (uint32_t)tid + j * kBlock, row = row0 + i / kPieces;
+      if (i >= (uint32_t)kQUnits || row >= query) continue;
+      const size_t dst = ((size_t)kv_plane * a.capacity + past + row) * D + 4 * (i % kPieces);
+      const float4 kv = raw4_f32<XT>(own_k[j]), vv = raw4_f32<XT>(own_v[j]);
+      st_f32<ST>(slot_k, dst, kv.x); st_f32<ST>(slot_k, dst + 1, kv.y);
+      st_f32<ST>(slot_k, dst + 2, kv.z); st_f32<ST>(slot_k, dst + 3, kv.w);
+      st_f32<ST>(slot_v, dst, vv.x); st_f32<ST>(slot_v, dst + 1, vv.y);
+      st_f32<ST>(slot_v, dst + 2, vv.z); st_f32<ST>(slot_v, dst + 3, vv.w);
+    }
   }
 }
 
@@ -518,22 +679,6 @@ __device__ inline float group_sum(float v) {
   return v;
 }
 
-// Halves (x = 32) or neighbouring rows (x = 16) of a wave trade places in one instruction: {a of
-// the lanes whose bit x is clear | b of the same lanes, x further on} and the same of the lanes
-// whose bit is set.
-struct Exchanged {
-  float clear, set;
-};
-__device__ inline Exchanged exchange(float a, float b, int x) {
-  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
-  const auto s = x == 32 ? __builtin_amdgcn_permlane32_swap(ua, ub, false, false)
-                         : __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
-  return {__uint_as_float(s[0]), __uint_as_float(s[1])};
-}
-__device__ inline float exchange_max(float v, int x) {
-  const Exchanged s = exchange(v, v, x);
-  return fmaxf(s.clear, s.set);
-}
 // Sums of N values (a power of two) over the four 16-lane rows of a wave, each lane left with its
 // share of them: returns the index of the first and leaves max(1, N / 4) totals in v[0..].  A
 // value's tree is the same for every N.
@@ -1326,16 +1471,16 @@ template <typename XT, typename ST>
 int32_t launch_rows(krm_ctx* ctx, krm_buf q, krm_buf ins_k, krm_buf ins_v, krm_buf slot_k,
                     krm_buf slot_v, krm_buf out, uint32_t batch, const GenericArgs& a,
                     uint32_t flags) {
-  // D = 64: eight waves, two a SIMD, so that one wave's softmax and LDS traffic run under the
-  // other's MFMAs; the parked blocks of eight waves of D = 128 would not fit the LDS.  A
-  // workgroup takes one block of 16 query rows, or two (the parked K / V blocks then serve
-  // both) once that still leaves two workgroups per CU.  A row's arithmetic is the same in
-  // both forms and the wave count depends on D only, so its bits depend neither on the chunk
-  // length, the batch, the past or the capacity nor on the lengths form.
+  // Eight waves, two a SIMD, so that one wave's softmax and LDS traffic run under the other's
+  // MFMAs; D = 256: four (the state of a wave takes a SIMD's registers).  A workgroup takes one
+  // block of 16 query rows; with D = 64, whose second block fits the registers, two (the K / V
+  // blocks then serve both) once that still leaves two workgroups per CU.  A row's arithmetic is
+  // the same in both forms and the wave count depends on D only, so its bits depend neither on the
+  // chunk length, the batch, the past or the capacity nor on the lengths form.
   const uint32_t row_blocks = (a.chunk_rows + 15) / 16;
   // (with a window the key blocks start at the first row's lower bound, which a second row
   // block would not share: one block a workgroup there)
-  const bool two = a.window == 0 && a.depth != 256 &&
+  const bool two = a.window == 0 && a.depth == 64 &&
                    (uint64_t)batch * a.heads * ((row_blocks + 1) / 2) >= 2ull * ctx->num_cus;
   const dim3 grid(batch * a.heads, two ? (row_blocks + 1) / 2 : row_blocks);
 #define KRM_ROWS_ATTENTION(DEPTH, WAVES, RB)                                                   \
@@ -1343,12 +1488,11 @@ int32_t launch_rows(krm_ctx* ctx, krm_buf q, krm_buf ins_k, krm_buf ins_v, krm_b
       ptr<const XT>(q), ptr<const XT>(ins_k), ptr<const XT>(ins_v), ptr<ST>(slot_k),           \
       ptr<ST>(slot_v), ptr<XT>(out), a, flags)
   if (a.depth == 256) {
-    // two waves: a parked block of 32 rows of 256 floats is 33 KB for K and as much for V
-    KRM_ROWS_ATTENTION(256, 2, 1);
+    KRM_ROWS_ATTENTION(256, 4, 1);
   } else if (a.depth == 64) {
     if (two) KRM_ROWS_ATTENTION(64, 8, 2); else KRM_ROWS_ATTENTION(64, 8, 1);
   } else {
-    if (two) KRM_ROWS_ATTENTION(128, 4, 2); else KRM_ROWS_ATTENTION(128, 4, 1);
+    KRM_ROWS_ATTENTION(128, 8, 1);
   }
 #undef KRM_ROWS_ATTENTION
   return launched(ctx, "attention_rows_kernel");

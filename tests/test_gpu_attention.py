@@ -171,6 +171,32 @@ def test_chunks_of_rows_on_the_matrix_cores(gpu_ctx, case, io, kv):
         assert np.all(err <= ulp + STATE_ATOL), float(np.max(err - ulp))
 
 
+@pytest.mark.parametrize("case", [
+    StateCase("D128 more blocks than waves", 1, 4, 2, 40, 128, 800, 0, 700, 37),
+    StateCase("D256 more blocks than waves", 1, 4, 1, 20, 256, 400, 0, 290, 20),
+    StateCase("D256 straddle at the first key", 1, 2, 1, 33, 256, 64, 0, 1, 31),
+    StateCase("D128 window wraps inside a block", 1, 4, 2, 24, 128, 90, 90, 155, 24),
+    StateCase("D256 window below a block", 1, 2, 1, 18, 256, 20, 20, 70, 18),
+    StateCase("D64 window whole blocks", 1, 4, 2, 17, 64, 512, 512, 999, 17),
+], ids=lambda c: c.name)
+@pytest.mark.parametrize("io,kv", [(np.float32, np.float32), (np.float16, np.float16),
+                                   (np.float32, np.float16)])
+def test_chunk_key_blocks_from_slot_and_step(gpu_ctx, case, io, kv):
+    """Key blocks wholly in the slot, wholly in this step's rows, straddling both, and wrapping in
+    the window, for every head dim's wave count."""
+    x = random_state_inputs(case, seed=case.past + case.depth, f16_values=True)
+    x["ins_k"][:, :, case.query:] = 9.0
+    x["ins_v"][:, :, case.query:] = 400.0
+    want = oracle_state_attention(case, x)
+    got = run_attention(gpu_ctx, case, x, io=io, kv=kv).astype(np.float32)
+    if io == np.float32:
+        ok, fails, max_abs, worst = oracle.allclose(got, want, atol=STATE_ATOL, rtol=0)
+        assert ok, (fails, max_abs, worst)
+    else:
+        ulp = np.spacing(np.abs(want.astype(np.float16))).astype(np.float32)
+        assert np.all(np.abs(got - want.astype(np.float16)) <= ulp + STATE_ATOL)
+
+
 def test_chunk_rows_do_not_depend_on_the_batch(gpu_ctx):
     """A large grid puts two blocks of 16 query rows into one workgroup (the parked K / V blocks
     serve both); a row's arithmetic is the same, so one sequence alone and the same sequence as
