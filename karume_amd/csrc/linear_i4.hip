@@ -476,6 +476,133 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_kernel(
 }
 
 
+// More tiles of 16 weight rows than CUs, K of up to 256 KW CHUNKS codes: a workgroup a CU walks the
+// tiles blockIdx.x, + gridDim.x, ..., two tiles' weights on their way, and a wave keeps its whole
+// share of x in registers (32 a chunk, read through one LDS strip).  One tile a workgroup fetched
+// and parked all of x (16 K fp16: four times the tile's weights) for every tile, one workgroup a CU
+// at a time (its strips filled the LDS).  Same sums in the same order.  What bounds it now is the
+// weights' stream behind the first round trip.
+template <typename ST, int CHUNKS, bool EVEN, int KW>
+__global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_tiles_kernel(
+    const __half* __restrict__ x, const uint32_t* __restrict__ w, const ST* __restrict__ scales,
+    const __half* __restrict__ bias, __half* __restrict__ out, uint32_t m, uint32_t n, uint32_t k,
+    uint32_t group_shift) {
+  constexpr int kChunk = 256;
+  constexpr int kRowBytes = kChunk * 2 + 16;
+  __shared__ float s_part[2][KW][4][kWave];  // [tile parity][wave][register][lane]
+  __shared__ __attribute__((aligned(16))) unsigned char s_x[KW][16 * kRowBytes];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x >> 6;
+  const int r16 = lane & 15, g = lane >> 4;
+  // this wave's share of K: the chunks dealt to the waves in order, the first ones one more
+  const uint32_t total_chunks = k / kChunk, base = total_chunks / KW, extra = total_chunks % KW;
+  const uint32_t chunks = base + ((uint32_t)wave < extra ? 1u : 0u);
+  const uint32_t k_first = (wave * base + ((uint32_t)wave < extra ? (uint32_t)wave : extra)) * kChunk;
+  // (a share is CHUNKS or, unless EVEN, CHUNKS - 1 chunks: the last one is then the one before it
+  // again, requested and not used — a branch around requests would wait inside)
+  auto mine = [&](int c) { return EVEN || c + 1 < CHUNKS || chunks == (uint32_t)CHUNKS; };
+  auto chunk_k0 = [&](int c) { return k_first + (mine(c) || c == 0 ? c : c - 1) * 256u; };
+
+  const uint32_t tiles = (n + 15) / 16;
+  struct Tile {
+    uint4 words[CHUNKS][2];  // pieces g and 4 + g of the row's 32 words
+    ST scale[CHUNKS][2];     // (as loaded: a conversion here would wait inside the branch)
+  };
+  auto fetch_tile = [&](uint32_t tile, Tile& t) {
+    const uint32_t row = min(tile * 16 + r16, n - 1);  // rows past N re-read the last row, unused
+    const uint32_t* wrow = w + (size_t)row * (k >> 3) + 4 * g;
+    const ST* srow = scales + (size_t)row * (k >> group_shift);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const uint32_t at = chunk_k0(c);
+      t.words[c][0] = *reinterpret_cast<const uint4*>(wrow + (at >> 3));
+      t.words[c][1] = *reinterpret_cast<const uint4*>(wrow + (at >> 3) + 16);
+      t.scale[c][0] = srow[at >> group_shift];
+      t.scale[c][1] = srow[(at + 128) >> group_shift];
+    }
+  };
+
+  // The activations first: they come from the cache and loads return in order, so they are parked
+  // while the first tiles' weights are still on their way.
+  uint4 xa[CHUNKS][8];  // pieces as loaded: rows 2j + lane / 32, piece lane % 32
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t row = min((uint32_t)(2 * j + (lane >> 5)), m - 1);
+      xa[c][j] = *reinterpret_cast<const uint4*>(x + (size_t)row * k + chunk_k0(c) + 8 * (lane & 31));
+    }
+  Tile even, odd;  // (in turn: a copy between them would wait for what is on its way)
+  fetch_tile(blockIdx.x, even);
+  if (blockIdx.x + gridDim.x < tiles) fetch_tile(blockIdx.x + gridDim.x, odd);
+  __builtin_amdgcn_sched_barrier(0);
+  half8_t fx[CHUNKS][8];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      half2_t p[4];
+      pair_activations(xa[c][j], p);
+      *reinterpret_cast<uint4*>(&s_x[wave][(2 * j + (lane >> 5)) * kRowBytes + 16 * (lane & 31)]) =
+          make_uint4(__builtin_bit_cast(uint32_t, p[0]), __builtin_bit_cast(uint32_t, p[1]),
+                     __builtin_bit_cast(uint32_t, p[2]), __builtin_bit_cast(uint32_t, p[3]));
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      fx[c][s] = *reinterpret_cast<const half8_t*>(
+          &s_x[wave][r16 * kRowBytes + 16 * ((s < 4 ? 4 * g + s : 16 + 4 * g + (s - 4)))]);
+  }
+
+  // multiplies the tile in `own` and asks for the one after the next in its place
+  auto step = [&](uint32_t tile, int parity, Tile& own) {
+    float4_t total = {0.f, 0.f, 0.f, 0.f};  // out[m = 4g + i][n = lane % 16] over this share of K
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+      if (mine(c)) {
+        float4_t half_sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          const uint32_t word = (&own.words[c][s >> 2].x)[s & 3];
+          half2_t q[4];
+          codes_to_half2(word, q);
+          const half8_t b = {q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+          half_sum[s >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fx[c][s], b, half_sum[s >> 2], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          total[i] = fmaf(half_sum[0][i], (float)own.scale[c][0], total[i]);
+          total[i] = fmaf(half_sum[1][i], (float)own.scale[c][1], total[i]);
+        }
+      }
+    if (tile + 2u * gridDim.x < tiles) fetch_tile(tile + 2u * gridDim.x, own);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_part[parity][wave][i][lane] = total[i];
+    // (one barrier a tile: the wave that adds a tile passes the next barrier after its reads, and
+    // this parity's area is written again behind that)
+    __syncthreads();
+    if (wave == (int)(tile / gridDim.x) % KW) {
+      const uint32_t col = tile * 16 + r16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v = s_part[parity][0][i][lane];
+#pragma unroll
+        for (int q = 1; q < KW; ++q) v += s_part[parity][q][i][lane];
+        const uint32_t row = 4 * g + i;
+        if (row < m && col < n) {
+          if (bias) v += __half2float(bias[col]);
+          out[(size_t)row * n + col] = __float2half_rn(v);
+        }
+      }
+    }
+  };
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += 2u * gridDim.x) {
+    step(tile, 0, even);
+    if (tile + gridDim.x >= tiles) break;
+    step(tile + gridDim.x, 1, odd);
+  }
+}
+
+
 template <typename T>
 __device__ inline float to_f32(T v);
 template <>
@@ -1089,7 +1216,27 @@ static int32_t gemv_dispatch(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
         aligned(scales, 4)) {
       uint32_t group_shift = 0;
       while ((1u << group_shift) < group) ++group_shift;
-      const uint32_t blocks = (n + 15) / 16;
+      const uint32_t blocks = (n + 15) / 16, share = (k / 256 + 7) / 8;
+      // (measured, 16 rows, us before / now: N = 11008, K = 4096 13.7 / 10.2; N = 32000, K = 2048
+      // 15.4 / 11.5; N = 9000, K = 5632 17 / 12.5.  Up to a tile a CU, or four chunks a wave and more: the kernel above.)
+      if (k >= 2048 && share <= 3 && blocks > (uint32_t)ctx->num_cus) {
+#define KRM_MFMA_TILES(ST, CH, EVEN)                                                           \
+  gemv_i4_mfma_tiles_kernel<ST, CH, EVEN, 8><<<dim3(ctx->num_cus), dim3(512), 0, ctx->stream>>>( \
+      ptr<const __half>(x), ptr<const uint32_t>(w), ptr<const ST>(scales),                     \
+      ptr<const __half>(bias), ptr<__half>(out), m, n, k, group_shift)
+        auto launch = [&](auto scale_tag) {
+          using ST = decltype(scale_tag);
+          const bool even = k % 2048 == 0;
+          if (share == 1) KRM_MFMA_TILES(ST, 1, true);
+          else if (share == 2 && even) KRM_MFMA_TILES(ST, 2, true);
+          else if (share == 2) KRM_MFMA_TILES(ST, 2, false);
+          else if (even) KRM_MFMA_TILES(ST, 3, true);
+          else KRM_MFMA_TILES(ST, 3, false);
+        };
+        if (scale_dtype == KRM_F16) launch(__half{}); else launch(float{});
+#undef KRM_MFMA_TILES
+        return launched(ctx, "gemv_i4_mfma_tiles_kernel");
+      }
 #define KRM_MFMA_GEMV(ST, CH, KW)                                                              \
   gemv_i4_mfma_kernel<ST, CH, KW><<<dim3(blocks), dim3(KW * 64), 0, ctx->stream>>>(            \
       ptr<const __half>(x), ptr<const uint32_t>(w), ptr<const ST>(scales),                     \

@@ -176,6 +176,29 @@ def test_batched_fp16_rows_on_matrix_cores_match_oracle(gpu_ctx, m, n, k, g, sca
     assert np.all(err <= 2.0 ** -10 * np.abs(want) + 4e-5), float(err.max())
 
 
+@pytest.mark.parametrize("m,n,k,g,scale_f16,with_bias", [
+    (2, 4097, 2048, 128, True, True), (16, 4128, 2304, 128, False, False),
+    (5, 8193, 4096, 256, False, True), (16, 8300, 5632, 128, True, False),
+    (9, 12400, 6144, 128, True, True)])
+def test_batched_fp16_rows_with_more_tiles_than_cus(gpu_ctx, m, n, k, g, scale_f16, with_bias):
+    """A workgroup walks several tiles of 16 weight rows (two, three and four rounds, the last one
+    ragged), even and uneven shares of K: the oracle's gate, and the bits of the narrow form."""
+    rng = np.random.default_rng(m + n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g, scale_f16=scale_f16)
+    x = rng.normal(size=(m, k)).astype(np.float16)
+    bias = rng.normal(size=n).astype(np.float16) if with_bias else None
+    got = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g)
+    few = 64
+    first = n - few  # the last rows, the ragged tile among them
+    codes = np.ascontiguousarray(packed.reshape(-1).view(np.uint8).reshape(n, k // 2)[first:])
+    narrow = run_linear(gpu_ctx, x, codes, scale[first:], bias[first:] if with_bias else None, few, k, g)
+    assert np.ascontiguousarray(got[:, first:]).tobytes() == narrow.tobytes()
+    want = oracle.linear_i4(x.astype(np.float32), packed, scale.astype(np.float32),
+                            (bias if with_bias else np.zeros(n)).astype(np.float32), n, k, g)
+    err = np.abs(got.astype(np.float32) - want)
+    assert np.all(err <= 2.0 ** -10 * np.abs(want) + 4e-5), float(err.max())
+
+
 @pytest.mark.parametrize("shape", [(1, 256, 2048, 128), (3, 2048, 5632, 128), (1, 100, 11008, 128),
                                    (7, 33, 96, 32), (2, 5, 64, 16), (16, 32000, 2048, 128)])
 def test_linear_shapes_of_the_decoder(gpu_ctx, shape):
