@@ -666,7 +666,7 @@ __device__ inline void slot_store(void* slot, int32_t is_f16, size_t i, float v)
 //  weight requests are out.
 template <typename XT, int MB, int NSTEP>
 constexpr bool share_x_in_lds() {
-  return MB == 1 && NSTEP > 0 && NSTEP <= 4;
+  return MB == 1 && NSTEP > 0;
 }
 
 // NORM and DECODE_ROW are compile-time so that the plain kernel carries neither their branches
@@ -1100,6 +1100,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
   }
 }
 
+// steps of 2048 codes up to which the rms_norm and the decode row have a form that is requested whole
+constexpr int kFusedSteps = 3;
+
 template <typename XT, typename ST, int MB, int ROWS, int VEC, int NSTEP>
 int32_t launch_gemv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                     krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group_shift,
@@ -1113,14 +1116,18 @@ int32_t launch_gemv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf 
                                                     ptr<const ST>(scales), fuse.norm_weight,   \
                                                     ptr<XT>(out), n, k, group_shift, m,         \
                                                     ptr<const XT>(bias), fuse)
-  if constexpr (MB == 1 && ROWS % 2 == 0) {
+  if constexpr (MB == 1 && ROWS % 2 == 0 && NSTEP <= kFusedSteps) {
     if (fuse.positions) {
       if (fuse.norm_weight) KRM_GEMV_LAUNCH(true, true); else KRM_GEMV_LAUNCH(false, true);
       return launched(ctx, "gemv_i4_kernel");
     }
   }
   if (fuse.positions) return fail(ctx, KRM_ERR_VALIDATION, "decode row: one row, even row count");
-  if (fuse.norm_weight) KRM_GEMV_LAUNCH(true, false); else KRM_GEMV_LAUNCH(false, false);
+  if constexpr (NSTEP <= kFusedSteps) {
+    if (fuse.norm_weight) KRM_GEMV_LAUNCH(true, false); else KRM_GEMV_LAUNCH(false, false);
+  } else {  // (pick_steps)
+    KRM_GEMV_LAUNCH(false, false);
+  }
 #undef KRM_GEMV_LAUNCH
   return launched(ctx, "gemv_i4_kernel");
 }
@@ -1139,6 +1146,22 @@ int32_t pick_steps(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf b
     if constexpr (ROWS <= 2)
       if (steps == 3)
         return launch_gemv<XT, ST, MB, ROWS, VEC, 3>(ctx, x, w, scales, bias, out, m, n, k, group_shift, fuse);
+    // (up to eight steps a wave's words still fit the registers and x the LDS.  Walked step by step
+    // every wave read all of x itself, and waited at each step for the next one's registers; us
+    // before / now: 4096 x 11008 fp16 8.5 / 7.2, f32 13.1 / 8.0; 32000 x 6400 f32 57 / 26.5)
+    if constexpr (ROWS <= 2)
+      if (steps <= 8 && !fuse.norm_weight && !fuse.positions) {
+#define KRM_GEMV_STEPS(COUNT)                                                                  \
+  if (steps == COUNT)                                                                          \
+    return launch_gemv<XT, ST, MB, ROWS, VEC, COUNT>(ctx, x, w, scales, bias, out, m, n, k,    \
+                                                     group_shift, fuse)
+        KRM_GEMV_STEPS(4);
+        KRM_GEMV_STEPS(5);
+        KRM_GEMV_STEPS(6);
+        KRM_GEMV_STEPS(7);
+        KRM_GEMV_STEPS(8);
+#undef KRM_GEMV_STEPS
+      }
   }
   return launch_gemv<XT, ST, MB, ROWS, VEC, 0>(ctx, x, w, scales, bias, out, m, n, k, group_shift, fuse);
 }

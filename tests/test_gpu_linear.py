@@ -231,6 +231,24 @@ def test_row_bits_do_not_depend_on_rows_per_wave(gpu_ctx, k, io, many):
     assert wide[:, :few].tobytes() == narrow.tobytes()
 
 
+@pytest.mark.parametrize("n,k", [(3, 6272), (1031, 8192), (2100, 10272), (17, 12320), (2049, 14368),
+                                 (5, 16384), (7, 16416)])
+@pytest.mark.parametrize("io", [np.float32, np.float16])
+def test_single_row_of_a_long_k_is_requested_whole(gpu_ctx, n, k, io):
+    """4 to 8 steps of 2048 codes (the last one full, or a single group), one and two rows a wave,
+    and the first K that is walked step by step again."""
+    g = 32
+    rng = np.random.default_rng(n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    x = rng.normal(size=(1, k)).astype(np.float16).astype(io)
+    bias = rng.normal(size=n).astype(np.float16).astype(io)
+    want = oracle.linear_i4(x.astype(np.float32), packed, scale.astype(np.float32),
+                            bias.astype(np.float32), n, k, g)
+    got = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g).astype(np.float32)
+    rel = 1e-5 if io == np.float32 else 2.0 ** -10
+    assert np.all(np.abs(got - want) <= rel * np.abs(want) + 5e-5), float(np.abs(got - want).max())
+
+
 def test_linear_rejections(gpu_ctx):
     """Unsupported combinations fail before launch (never approximated)."""
     buf = gpu_ctx.zeros(4096)
