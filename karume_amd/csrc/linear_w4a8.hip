@@ -662,27 +662,28 @@ void linear_w4a8_tile_kernel(
   }
 }
 
-// The same staging with a 128 x 256 workgroup tile, wave = 64 x 64, for groups of 64 or 128
+// The same staging with a 128 x 256 workgroup tile, wave = 64 x 64 (or 64 x 128 and 64 x 32, four
+// waves), for groups of 64 or 128
 // codes.  Four 32 x 32 tiles per wave would need 64 int32 and 64 f32 accumulators at once, more
 // than two waves per SIMD leave room for, so the work is ordered by group: the group's weight
 // words are expanded once (both column tiles, all MFMA steps of the group), then each row tile
 // in turn runs its two MFMA chains over the group and is fused into its f32 accumulators — 32
 // int32 accumulators live at a time, and the expansion is shared by the two row tiles.
-template <typename ST, int GSH>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <typename ST, int GSH, int WM, int NW, int WN>
+__global__ __launch_bounds__(64 * WM * NW) __attribute__((amdgpu_waves_per_eu(2, WN == 2 ? 2 : 4)))
 void linear_w4a8_tall_kernel(
     const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w,
     const ST* __restrict__ scales, const float* __restrict__ bias, float* __restrict__ out,
     uint32_t m, uint32_t n, uint32_t k, uint32_t m_blocks, uint32_t n_blocks) {
   static_assert(GSH == 6 || GSH == 7, "groups of 64 or 128 codes");
-  constexpr int MT = 2, WN = 2;
-  constexpr int BM = 128, BN = 256;
+  constexpr int T = 64 * WM * NW, MT = 2;
+  constexpr int BM = 64 * WM, BN = 32 * WN * NW;
   constexpr int kStage = 128;                          // codes per LDS stage
   constexpr int kRowA = kStage + 16, kRowB = kStage / 2 + 16;
   constexpr int kGroupsPerStage = kStage >> GSH;       // 2 or 1
   constexpr int kStepsPerGroup = 1 << (GSH - 5);       // MFMA steps of 32 codes: 2 or 4
-  constexpr int kAUnits = BM * (kStage / 16) / 512;    // 16-byte units of xq per thread: 2
-  constexpr int kBUnits = BN * (kStage / 32) / 512;    // and of packed weights: 2
+  constexpr int kAUnits = BM * (kStage / 16) / T;      // 16-byte units of xq per thread
+  constexpr int kBUnits = BN * (kStage / 32) / T;      // and of packed weights
   __shared__ __align__(16) uint8_t s_a[2][BM * kRowA];
   __shared__ __align__(16) uint8_t s_b[2][BN * kRowB];
   __shared__ __align__(16) float s_s[2][BN][2];
@@ -691,7 +692,7 @@ void linear_w4a8_tall_kernel(
   const uint32_t mb = slot % m_blocks, nb = (slot / m_blocks) * 8u + xcd;
   if (nb >= n_blocks) return;  // the whole workgroup leaves before any barrier
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave / NW, wn = wave % NW;
   const int frag_row = lane & 31, frag_h = lane >> 5;
   const uint32_t m0 = mb * BM, n0 = nb * BN;
   const uint32_t groups = k >> GSH;
@@ -702,7 +703,7 @@ void linear_w4a8_tall_kernel(
   // (rows tid / 4 + 128 i)
   const uint32_t arow0 = tid >> 3, aunit = (tid & 7u) * 16u;
   const uint32_t brow0 = tid >> 2, bunit = (tid & 3u) * 16u;
-  const ST* ssrc = scales + (size_t)min(n0 + (uint32_t)(tid & 255), n - 1) * groups;
+  const ST* ssrc = scales + (size_t)min(n0 + (uint32_t)(tid < BN ? tid : 0), n - 1) * groups;
 
   struct Staged {
     uint4 a[kAUnits];
@@ -715,11 +716,11 @@ void linear_w4a8_tall_kernel(
 #pragma unroll
     for (int i = 0; i < kAUnits; ++i)
       d.a[i] = *reinterpret_cast<const uint4*>(
-          xq + (size_t)min(m0 + arow0 + 64u * i, m - 1) * k + a_off);
+          xq + (size_t)min(m0 + arow0 + (T / 8) * i, m - 1) * k + a_off);
 #pragma unroll
     for (int i = 0; i < kBUnits; ++i)
       d.b[i] = *reinterpret_cast<const uint4*>(
-          w + (size_t)min(n0 + brow0 + 128u * i, n - 1) * (k >> 1) + b_off);
+          w + (size_t)min(n0 + brow0 + (T / 4) * i, n - 1) * (k >> 1) + b_off);
 #pragma unroll
     for (int j = 0; j < kGroupsPerStage; ++j) {
       const uint32_t code = stage * kStage + (j << GSH);
@@ -735,12 +736,12 @@ void linear_w4a8_tall_kernel(
       v.y = __builtin_amdgcn_perm(d.a[i].y, d.a[i].x, 0x07050301u) & keep;
       v.z = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x06040200u) & keep;
       v.w = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x07050301u) & keep;
-      *reinterpret_cast<uint4*>(&s_a[buf][(arow0 + 64u * i) * kRowA + aunit]) = v;
+      *reinterpret_cast<uint4*>(&s_a[buf][(arow0 + (T / 8) * i) * kRowA + aunit]) = v;
     }
 #pragma unroll
     for (int i = 0; i < kBUnits; ++i)
-      *reinterpret_cast<uint4*>(&s_b[buf][(brow0 + 128u * i) * kRowB + bunit]) = d.b[i];
-    if (tid < 256) {
+      *reinterpret_cast<uint4*>(&s_b[buf][(brow0 + (T / 4) * i) * kRowB + bunit]) = d.b[i];
+    if (tid < BN) {
 #pragma unroll
       for (int j = 0; j < kGroupsPerStage; ++j) s_s[buf][tid][j] = scale_f32<ST>(&d.s[j], 0);
     }
@@ -761,7 +762,7 @@ void linear_w4a8_tall_kernel(
   __syncthreads();
 
   const uint32_t a_base = (uint32_t)((wm * 64 + frag_row) * kRowA + 32 * frag_h);
-  const uint32_t b_base = (uint32_t)((wn * 64 + frag_row) * kRowB + 16 * frag_h);
+  const uint32_t b_base = (uint32_t)((wn * 32 * WN + frag_row) * kRowB + 16 * frag_h);
   auto run_stage = [&](uint32_t stage, int buf) {
     load_stage(stage + 1, staged);
     __builtin_amdgcn_sched_barrier(0);  // the requests stay a stage ahead of their use
@@ -790,7 +791,7 @@ void linear_w4a8_tall_kernel(
             bexp[nt][2 * cc + s] = b;
           }
         }
-        const float ws = s_s[buf][wn * 64 + nt * 32 + frag_row][gi];
+        const float ws = s_s[buf][wn * 32 * WN + nt * 32 + frag_row][gi];
         // an fp16 scale / 16 is exact in f32; an f32 scale may not be (subnormal quotient):
         // then the sums are shifted instead (below)
         mult[nt] = valid ? ws : 0.f;  // past K: accf + 0 * 0
@@ -829,7 +830,7 @@ void linear_w4a8_tall_kernel(
 
 #pragma unroll
   for (int nt = 0; nt < WN; ++nt) {
-    const uint32_t col = n0 + wn * 64 + nt * 32 + frag_row;
+    const uint32_t col = n0 + wn * 32 * WN + nt * 32 + frag_row;
     const float b = (bias && col < n) ? bias[col] : 0.f;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -870,20 +871,31 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
   }
   if (m > 8 && group >= 64 && group <= kMaxGroupTimes16 && aligned(xq, 16) && aligned(w, 16)) {
     const uint32_t n_blocks = (n + 255) / 256;
-    // 128-row tiles for groups of 64 / 128 when they still cover most of the chip
-    const uint32_t tall_blocks = (m + 127) / 128;
-    if ((shift == 6 || shift == 7) &&
-        (uint64_t)tall_blocks * n_blocks * 5 >= (uint64_t)ctx->num_cus * 3) {
-      const uint64_t blocks = (uint64_t)((n_blocks + 7) / 8) * 8u * tall_blocks;
+    // 128 x 256 tiles for groups of 64 / 128 when they still cover most of the chip, or 64 x 128 ones
+    // of four waves, several to a CU, when their finer grain makes fewer rounds of a CU's work: a
+    // quarter of a tall tile each, at 1.15 of its time per output (less is shared).  us before / now:
+    // 512 x 11008 x 4096 59.5 / 56, in groups of 64 70 / 60; 400 x 9000 x 3072 49.5 / 35; 200 x 20000
+    // x 4096 55.4 / 48; 300 x 14000 x 2048 in groups of 64 42 / 34.5; where the tall ones fill whole
+    // rounds (2048 x 11008 x 4096, 256 x 32000 x 2048) these take 2 % longer.
+    const uint64_t cus = (uint64_t)ctx->num_cus;
+    const uint64_t tall_tiles = (uint64_t)((m + 127) / 128) * n_blocks;
+    if ((shift == 6 || shift == 7) && tall_tiles * 5 >= cus * 3) {
+      const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
+      const uint64_t small_rounds = ((uint64_t)small_m * small_n + cus - 1) / cus;
+      const bool small = small_rounds * 115 < (tall_tiles + cus - 1) / cus * 400;
+      const uint32_t mb = small ? small_m : (m + 127) / 128, nb = small ? small_n : n_blocks;
+      const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * mb;
       if (blocks <= 0x7fffffffull) {
-        if (shift == 6)
-          hipLaunchKernelGGL((linear_w4a8_tall_kernel<ST, 6>), dim3((uint32_t)blocks), dim3(512),
-                             0, ctx->stream, ptr<const uint8_t>(xq), pxs, ptr<const uint8_t>(w),
-                             ps, pb, po, m, n, k, tall_blocks, n_blocks);
-        else
-          hipLaunchKernelGGL((linear_w4a8_tall_kernel<ST, 7>), dim3((uint32_t)blocks), dim3(512),
-                             0, ctx->stream, ptr<const uint8_t>(xq), pxs, ptr<const uint8_t>(w),
-                             ps, pb, po, m, n, k, tall_blocks, n_blocks);
+#define KRM_W4A8_TALL(GSH, WM, WN)                                                             \
+  hipLaunchKernelGGL((linear_w4a8_tall_kernel<ST, GSH, WM, 4, WN>), dim3((uint32_t)blocks),    \
+                     dim3(256 * WM), 0, ctx->stream, ptr<const uint8_t>(xq), pxs,              \
+                     ptr<const uint8_t>(w), ps, pb, po, m, n, k, mb, nb)
+        if (small) {
+          if (shift == 6) KRM_W4A8_TALL(6, 1, 1); else KRM_W4A8_TALL(7, 1, 1);
+        } else {
+          if (shift == 6) KRM_W4A8_TALL(6, 2, 2); else KRM_W4A8_TALL(7, 2, 2);
+        }
+#undef KRM_W4A8_TALL
         return launched(ctx, "linear_w4a8_tall_kernel");
       }
     }

@@ -211,6 +211,21 @@ def test_w4a8_random_shapes_bit_exact(gpu_ctx, m, n, k, group, scale_f16, with_b
     assert_exact(got, want, (m, n, k, group))
 
 
+@pytest.mark.parametrize("m, n, k, group, scale_f16", [
+    (129, 20033, 256, 128, True), (400, 9000, 384, 128, False), (200, 20000, 192, 64, True),
+    (300, 14001, 64, 64, False), (257, 16500, 320, 64, True)])
+def test_w4a8_small_tiles_of_a_chip_that_tall_ones_leave_idle(gpu_ctx, m, n, k, group, scale_f16):
+    """Several 64 x 128 tiles a CU where 128 x 256 ones would not fill a round: ragged M, N and a K
+    that ends inside a stage."""
+    rng = np.random.default_rng(m + n)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, group, scale_f16=scale_f16)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    bias = rng.normal(size=n).astype(np.float32)
+    got = run_w4a8(gpu_ctx, x, packed, scale, bias, n, k, group)
+    want = oracle.linear_w4a8(x, packed, np.asarray(scale, dtype=np.float32), bias, n, k, group)
+    assert_exact(got, want, (m, n, k))
+
+
 def test_w4a8_rows_do_not_depend_on_the_batch(gpu_ctx):
     rng = np.random.default_rng(3)
     n, k, group = 512, 4096, 128
