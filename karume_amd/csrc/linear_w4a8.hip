@@ -663,7 +663,7 @@ void linear_w4a8_tile_kernel(
 }
 
 // The same staging with a 128 x 256 workgroup tile, wave = 64 x 64 (or 64 x 128 and 64 x 32, four
-// waves), for groups of 64 or 128
+// waves), for groups of 32, 64 or 128
 // codes.  Four 32 x 32 tiles per wave would need 64 int32 and 64 f32 accumulators at once, more
 // than two waves per SIMD leave room for, so the work is ordered by group: the group's weight
 // words are expanded once (both column tiles, all MFMA steps of the group), then each row tile
@@ -675,18 +675,18 @@ void linear_w4a8_tall_kernel(
     const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w,
     const ST* __restrict__ scales, const float* __restrict__ bias, float* __restrict__ out,
     uint32_t m, uint32_t n, uint32_t k, uint32_t m_blocks, uint32_t n_blocks) {
-  static_assert(GSH == 6 || GSH == 7, "groups of 64 or 128 codes");
+  static_assert(GSH >= 5 && GSH <= 7, "groups of 32, 64 or 128 codes");
   constexpr int T = 64 * WM * NW, MT = 2;
   constexpr int BM = 64 * WM, BN = 32 * WN * NW;
   constexpr int kStage = 128;                          // codes per LDS stage
   constexpr int kRowA = kStage + 16, kRowB = kStage / 2 + 16;
-  constexpr int kGroupsPerStage = kStage >> GSH;       // 2 or 1
-  constexpr int kStepsPerGroup = 1 << (GSH - 5);       // MFMA steps of 32 codes: 2 or 4
+  constexpr int kGroupsPerStage = kStage >> GSH;       // 4, 2 or 1
+  constexpr int kStepsPerGroup = 1 << (GSH - 5);       // MFMA steps of 32 codes: 1, 2 or 4
   constexpr int kAUnits = BM * (kStage / 16) / T;      // 16-byte units of xq per thread
   constexpr int kBUnits = BN * (kStage / 32) / T;      // and of packed weights
   __shared__ __align__(16) uint8_t s_a[2][BM * kRowA];
   __shared__ __align__(16) uint8_t s_b[2][BN * kRowB];
-  __shared__ __align__(16) float s_s[2][BN][2];
+  __shared__ __align__(16) float s_s[2][BN][kGroupsPerStage];
 
   const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
   const uint32_t mb = slot % m_blocks, nb = (slot / m_blocks) * 8u + xcd;
@@ -697,6 +697,9 @@ void linear_w4a8_tall_kernel(
   const uint32_t m0 = mb * BM, n0 = nb * BN;
   const uint32_t groups = k >> GSH;
   const uint32_t chunks_total = k >> 6;
+  // bytes of a step's codes that a half of the wave takes: a step of a 64-code chunk is 16 codes of
+  // each half of it, of a group of 32 the two halves of the group
+  constexpr int kHalfA = GSH == 5 ? 16 : 32, kHalfB = GSH == 5 ? 8 : 16;
   const uint32_t stages = (k + kStage - 1) / kStage;
 
   // staging roles: xq rows in 8 units of 16 bytes (rows tid / 8 + 64 i), weight rows in 4
@@ -761,8 +764,8 @@ void linear_w4a8_tall_kernel(
   park_stage(0, 0, staged);
   __syncthreads();
 
-  const uint32_t a_base = (uint32_t)((wm * 64 + frag_row) * kRowA + 32 * frag_h);
-  const uint32_t b_base = (uint32_t)((wn * 32 * WN + frag_row) * kRowB + 16 * frag_h);
+  const uint32_t a_base = (uint32_t)((wm * 64 + frag_row) * kRowA + kHalfA * frag_h);
+  const uint32_t b_base = (uint32_t)((wn * 32 * WN + frag_row) * kRowB + kHalfB * frag_h);
   auto run_stage = [&](uint32_t stage, int buf) {
     load_stage(stage + 1, staged);
     __builtin_amdgcn_sched_barrier(0);  // the requests stay a stage ahead of their use
@@ -771,7 +774,8 @@ void linear_w4a8_tall_kernel(
       // codes 0 .. (1 << GSH) - 1 of the group = MFMA steps 0 .. kStepsPerGroup - 1;
       // step st lies in chunk (gi << GSH) / 64 + st / 2, half st % 2
       const int first_chunk_in_stage = (gi << GSH) >> 6;
-      const bool valid = stage * 2u + first_chunk_in_stage < chunks_total;
+      const bool valid = GSH == 5 ? stage * 4u + gi < groups
+                                  : stage * 2u + first_chunk_in_stage < chunks_total;
       v4i_t bexp[WN][kStepsPerGroup];
       float mult[WN];
 #pragma unroll
@@ -791,6 +795,14 @@ void linear_w4a8_tall_kernel(
             bexp[nt][2 * cc + s] = b;
           }
         }
+        if constexpr (GSH == 5) {
+          const uint2 words = *reinterpret_cast<const uint2*>(
+              &s_b[buf][b_base + nt * 32 * kRowB + 16 * gi]);
+          bexp[nt][0][0] = (int)(((words.x << 4) ^ 0x80808080u) & 0xF0F0F0F0u);
+          bexp[nt][0][1] = (int)((words.x ^ 0x88888888u) & 0xF0F0F0F0u);
+          bexp[nt][0][2] = (int)(((words.y << 4) ^ 0x80808080u) & 0xF0F0F0F0u);
+          bexp[nt][0][3] = (int)((words.y ^ 0x88888888u) & 0xF0F0F0F0u);
+        }
         const float ws = s_s[buf][wn * 32 * WN + nt * 32 + frag_row][gi];
         // an fp16 scale / 16 is exact in f32; an f32 scale may not be (subnormal quotient):
         // then the sums are shifted instead (below)
@@ -802,8 +814,9 @@ void linear_w4a8_tall_kernel(
 #pragma unroll
         for (int st = 0; st < kStepsPerGroup; ++st) {
           const v4i_t a = *reinterpret_cast<const v4i_t*>(
-              &s_a[buf][a_base + mt * 32 * kRowA + 64 * (first_chunk_in_stage + st / 2) +
-                        16 * (st & 1)]);
+              &s_a[buf][a_base + mt * 32 * kRowA +
+                        (GSH == 5 ? 32 * gi
+                                  : 64 * (first_chunk_in_stage + st / 2) + 16 * (st & 1))]);
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt)
             acc[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bexp[nt][st],
@@ -869,7 +882,7 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
                          pxs, pw, ps, pb, po, m, n, k, shift);
     return launched(ctx, "linear_w4a8_rows_kernel");
   }
-  if (m > 8 && group >= 64 && group <= kMaxGroupTimes16 && aligned(xq, 16) && aligned(w, 16)) {
+  if (m > 8 && group >= 32 && group <= kMaxGroupTimes16 && aligned(xq, 16) && aligned(w, 16)) {
     const uint32_t n_blocks = (n + 255) / 256;
     // 128 x 256 tiles for groups of 64 / 128 when they still cover most of the chip, or 64 x 128 ones
     // of four waves, several to a CU, when their finer grain makes fewer rounds of a CU's work: a
@@ -877,9 +890,12 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
     // 512 x 11008 x 4096 59.5 / 56, in groups of 64 70 / 60; 400 x 9000 x 3072 49.5 / 35; 200 x 20000
     // x 4096 55.4 / 48; 300 x 14000 x 2048 in groups of 64 42 / 34.5; where the tall ones fill whole
     // rounds (2048 x 11008 x 4096, 256 x 32000 x 2048) these take 2 % longer.
+    // Groups of 32 always come here, the generic kernel re-reads both operands for every output: 512 x
+    // 11008 x 4096 50785 / 111, 197 x 1655 x 9600 7716 / 120, 20 x 20000 x 1024 914 / 19, 9 x 300 x
+    // 512 11.7 / 11.8.
     const uint64_t cus = (uint64_t)ctx->num_cus;
     const uint64_t tall_tiles = (uint64_t)((m + 127) / 128) * n_blocks;
-    if ((shift == 6 || shift == 7) && tall_tiles * 5 >= cus * 3) {
+    if (shift == 5 || ((shift == 6 || shift == 7) && tall_tiles * 5 >= cus * 3)) {
       const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
       const uint64_t small_rounds = ((uint64_t)small_m * small_n + cus - 1) / cus;
       const bool small = small_rounds * 115 < (tall_tiles + cus - 1) / cus * 400;
@@ -891,9 +907,11 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
                      dim3(256 * WM), 0, ctx->stream, ptr<const uint8_t>(xq), pxs,              \
                      ptr<const uint8_t>(w), ps, pb, po, m, n, k, mb, nb)
         if (small) {
-          if (shift == 6) KRM_W4A8_TALL(6, 1, 1); else KRM_W4A8_TALL(7, 1, 1);
+          if (shift == 5) KRM_W4A8_TALL(5, 1, 1);
+          else if (shift == 6) KRM_W4A8_TALL(6, 1, 1); else KRM_W4A8_TALL(7, 1, 1);
         } else {
-          if (shift == 6) KRM_W4A8_TALL(6, 2, 2); else KRM_W4A8_TALL(7, 2, 2);
+          if (shift == 5) KRM_W4A8_TALL(5, 2, 2);
+          else if (shift == 6) KRM_W4A8_TALL(6, 2, 2); else KRM_W4A8_TALL(7, 2, 2);
         }
 #undef KRM_W4A8_TALL
         return launched(ctx, "linear_w4a8_tall_kernel");
@@ -904,7 +922,7 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
     const bool narrow = (uint64_t)m_blocks * n_blocks * 4 < (uint64_t)ctx->num_cus * 3;
     const uint32_t nb = narrow ? (n + 127) / 128 : n_blocks;
     const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * m_blocks;
-    if (blocks <= 0x7fffffffull) {
+    if (shift > 5 && blocks <= 0x7fffffffull) {
 #define KRM_W4A8_TILE(GSH, WN)                                                                 \
   hipLaunchKernelGGL((linear_w4a8_tile_kernel<ST, GSH, 1, WN>), dim3((uint32_t)blocks),        \
                      dim3(512), 0, ctx->stream, ptr<const uint8_t>(xq), pxs,                  \

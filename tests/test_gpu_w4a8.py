@@ -312,6 +312,18 @@ def test_w4a8_fused_call_equals_the_two_steps(gpu_ctx, m, n, k, group, scale_f16
             run_w4a8_fused(gpu_ctx, x, packed, scale, bias, n, k, group, work=False)
 
 
+@pytest.mark.parametrize("m, n, k, scale_f16, with_bias", [
+    (9, 1, 32, True, False), (64, 128, 96, False, True), (65, 129, 160, True, True),
+    (197, 333, 1056, True, False), (600, 8200, 64, False, False)])
+def test_w4a8_many_rows_in_groups_of_32(gpu_ctx, m, n, k, scale_f16, with_bias):
+    rng = np.random.default_rng(m + n + k)
+    packed, q, scale = helpers.synthetic_int4(rng, n, k, 32, scale_f16)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    bias = rng.normal(size=n).astype(np.float32) if with_bias else None
+    want = oracle.linear_w4a8(x, packed, np.asarray(scale, dtype=np.float32), bias, n, k, 32)
+    assert_exact(run_w4a8(gpu_ctx, x, packed, scale, bias, n, k, 32), want, (m, n, k))
+
+
 def test_w4a8_fused_call_special_rows_and_ties(gpu_ctx):
     """A NaN row, a row of zeros, a row with an infinity and quotients on rounding ties."""
     rng = np.random.default_rng(11)
