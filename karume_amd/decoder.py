@@ -16,6 +16,7 @@ Every tensor operation is a call into libkarume_hip.so; this module only sequenc
 """
 from __future__ import annotations
 
+import weakref
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional
 
@@ -286,6 +287,10 @@ class LlamaDecoderSession:
                 self.buf[f"qkv{li}"] = a((sp["hd"] + 2 * sp["kvd"]) * eb)
         self.workspace: Optional[DeviceBuffer] = None
         self._workspace_uses = 0        # recorded steps hold the workspace's address
+        # Recorded steps hold this session's weights, tables and buffers: they are kept with the
+        # memory they run on, under the session that recorded them, and go with either.
+        self._steps = object()
+        self._recorded_on = weakref.WeakSet()   # memories that hold steps of this session
         self._spare_memory: List[ContextMemory] = []   # of the last retired context, at most one
         self._closed = False
         self.logits_shape = (1, c.vocab)
@@ -295,6 +300,8 @@ class LlamaDecoderSession:
         self._closed = True
         while self._spare_memory:
             self._spare_memory.pop().free()
+        for memory in list(self._recorded_on):   # also those of contexts still in use
+            memory.drop_graphs(self._steps)
         for entry in self.layers:
             for value in entry.values():
                 if isinstance(value, _DeviceLinear):
@@ -639,7 +646,7 @@ class LlamaDecoderSession:
         return max(512, 1 << past.bit_length()) - 1
 
     def _graph_key(self, kind: str, past: int) -> tuple:
-        return (kind, self._past_bucket(past), self._workspace_uses)
+        return (self._steps, kind, self._past_bucket(past), self._workspace_uses)
 
     def _recorded(self, memory: ContextMemory, kind: str, past: int) -> bool:
         return self._graph_key(kind, past) in memory.graphs
@@ -653,8 +660,7 @@ class LlamaDecoderSession:
         graph = memory.graphs.get(key)
         if graph is not None:
             return graph
-        for old in [k for k in memory.graphs if k[0] == kind]:   # outgrown
-            memory.graphs.pop(old).destroy()
+        memory.drop_graphs(self._steps, kind)   # outgrown
         g, c, b = self.gpu, self.config, self.buf
         step = memory.step
         self._replay_last_past = self._past_bucket(past)
@@ -674,6 +680,7 @@ class LlamaDecoderSession:
             b["pos"], b["token"] = saved_pos, saved_token
             self._replay_last_past = None
         memory.graphs[key] = rec.graph
+        self._recorded_on.add(memory)
         return rec.graph
 
     def _replay_step(self, context: GenerationContext, ids, pos, past: int, want_logits: bool):

@@ -843,3 +843,36 @@ def test_recorded_one_row_runs_equal_plain_ones_and_survive_context_reuse(gpu_ct
         ref.dispose()
     session.close()
     plain.close()
+
+
+def test_sessions_that_take_turns_on_one_context_equal_plain_launches(gpu_ctx):
+    """A session may run on a context of another session of its geometry: each replays the step
+    it recorded itself, so alternating runs equal the launches of sessions that never replay, bit
+    for bit, and so do the tokens of their replayed loops."""
+    config = LlamaConfig(layers=2, d_model=256, ffn=384, heads=4, kv_heads=2, head_dim=64,
+                         vocab=512, group_size=128, max_position=64)
+    sessions = [LlamaDecoderSession(gpu_ctx, random_weights(config, seed=s), chunk_length=8)
+                for s in (21, 22)]
+    shared = [s.create_generation_context(capacity=64, chunk_length=8) for s in sessions][0]
+    ref = sessions[0].create_generation_context(capacity=64, chunk_length=8)
+    memory, ref.memory = ref.memory, None     # a context without memory never replays
+    ids, positions = np.arange(3, 11, dtype=np.int32)[None], np.arange(8, dtype=np.int32)[None]
+    for context in (shared, ref):
+        tok = int(sessions[0].run(ids, positions, 7, context=context, query_length=8)[0, 0, 0])
+    for turn in range(8):
+        session = sessions[turn % 2]
+        row = np.array([[tok]], dtype=np.int32), np.array([[8 + turn]], dtype=np.int32)
+        got = session.run(*row, 0, context=shared, query_length=1, want_logits=True)
+        want = session.run(*row, 0, context=ref, query_length=1, want_logits=True)
+        assert np.array_equal(got[1].view(np.uint32), want[1].view(np.uint32)), turn
+        assert np.array_equal(got[0], want[0])
+        tok = int(got[0][0, 0, 0])
+    for session in sessions + sessions:
+        tokens = session.decode_tokens(shared, tok, 3)
+        assert tokens == session.decode_tokens(ref, tok, 3)
+        tok = tokens[-1]
+    ref.memory = memory
+    for context in (shared, ref):
+        context.dispose()
+    for session in sessions:
+        session.close()

@@ -1,0 +1,49 @@
+"""What a decoder session launches, seen through a stand-in for the device (no GPU)."""
+import numpy as np
+import pytest
+
+from karume_amd.decoder import LlamaConfig, LlamaDecoderSession, random_weights
+from stand_in_gpu import StandInGpu
+
+CONFIG = LlamaConfig(layers=2, d_model=128, ffn=256, heads=2, kv_heads=1, head_dim=64, vocab=64,
+                     group_size=64, max_position=256)
+
+
+def make_session(gpu, seed, config=CONFIG):
+    return LlamaDecoderSession(gpu, random_weights(config, seed=seed), chunk_length=8)
+
+
+def one_row(session, context, past):
+    return session.run(np.array([[1]], dtype=np.int32), np.array([[past]], dtype=np.int32), 0,
+                       context=context, query_length=1)
+
+
+# ---- recorded steps belong to the session that recorded them -----------------------------------
+
+@pytest.mark.parametrize("through", ["run", "decode_tokens"])
+def test_a_session_on_another_sessions_context_launches_its_own_weights(through):
+    gpu = StandInGpu()
+    a, b = make_session(gpu, 1), make_session(gpu, 2)
+    context = a.create_generation_context(capacity=64, chunk_length=8)
+    b.create_generation_context(capacity=64, chunk_length=8)
+
+    def step(session, past):
+        if through == "run":
+            one_row(session, context, past)
+        else:
+            session.decode_tokens(context, 1, 1)
+            context.past = past + 1   # (the stand-in's lengths read back as zeros)
+    for past, (session, other) in enumerate([(a, b), (a, b), (b, a), (b, a), (a, b), (b, a)]):
+        gpu.clear()
+        step(session, past)
+        for name in ("q", "o", "down"):
+            assert not gpu.mentions(other.layers[0][name].w), (past, name)
+        assert gpu.mentions(session.layers[1]["down"].w)
+        assert gpu.mentions(session.lm_head.w) and not gpu.mentions(other.lm_head.w)
+        assert gpu.mentions(session.buf["logits"]) and not gpu.mentions(other.buf["logits"])
+    assert gpu.open_graphs() == 2     # each session's step is kept, not recorded at every turn
+    b.close()
+    assert gpu.open_graphs() == 1
+    context.dispose()
+    a.close()
+    assert gpu.open_graphs() == 0
