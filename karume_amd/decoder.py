@@ -318,8 +318,13 @@ class LlamaDecoderSession:
             self.workspace = None
         self.layers, self.buf = [], {}
 
+    def _assert_open(self) -> None:
+        if self._closed:   # its buffers are freed: nothing may be launched over them
+            raise ExecutionError("the session is closed")
+
     # -- GreedySession surface ---------------------------------------------------------------
     def create_generation_context(self, *, capacity: int, chunk_length: int) -> GenerationContext:
+        self._assert_open()
         if chunk_length != self.chunk_length:
             raise ExecutionError(f"chunkLength {chunk_length} differs from the session's "
                                  f"{self.chunk_length}")
@@ -373,6 +378,7 @@ class LlamaDecoderSession:
         With `last_row=None` the session returns what the reference graph itself returns
         (tools/export-recipes/minicpm5/export_decode.py:14-22): the argmax of every row,
         [1, M, 1] (and logits [1, M, V]); rows past `query_length` are unspecified."""
+        self._assert_open()
         ids = np.ascontiguousarray(input_ids, dtype=np.int32)
         pos = np.ascontiguousarray(position_ids, dtype=np.int32)
         if ids.ndim != 2 or ids.shape[0] != 1 or pos.shape != ids.shape:
@@ -776,6 +782,7 @@ class LlamaDecoderSession:
         stay on the device and the tokens are read back once at the end."""
         if count < 1:
             return []
+        self._assert_open()
         if context.window == 0 and context.past + count > context.capacity:
             raise ExecutionError(f"pastLength {context.past} + {count} steps exceeds capacity "
                                  f"{context.capacity}")

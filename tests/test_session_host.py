@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from karume_amd.decoder import LlamaConfig, LlamaDecoderSession, random_weights
+from karume_amd.runtime import ExecutionError
 from stand_in_gpu import StandInGpu
 
 CONFIG = LlamaConfig(layers=2, d_model=128, ffn=256, heads=2, kv_heads=1, head_dim=64, vocab=64,
@@ -47,3 +48,27 @@ def test_a_session_on_another_sessions_context_launches_its_own_weights(through)
     context.dispose()
     a.close()
     assert gpu.open_graphs() == 0
+
+
+def test_a_closed_session_refuses_every_call_and_launches_nothing():
+    gpu = StandInGpu()
+    session = make_session(gpu, 3)
+    context = session.create_generation_context(capacity=64, chunk_length=8)
+    for past in range(3):
+        one_row(session, context, past)      # the second and third replay a recorded step
+    session.decode_tokens(context, 1, 2)
+    context.past = 5
+    session.close()
+    assert gpu.open_graphs() == 0
+    gpu.clear()
+    calls = [lambda: one_row(session, context, 5), lambda: session.decode_tokens(context, 1, 1),
+             lambda: session.run(np.zeros((1, 8), np.int32), np.zeros((1, 8), np.int32), 7,
+                                 context=context, query_length=8),
+             lambda: session.create_generation_context(capacity=64, chunk_length=8)]
+    for call in calls:
+        with pytest.raises(ExecutionError, match="closed"):
+            call()
+    assert gpu.log == [] and not context.poisoned and context.past == 5
+    context.dispose()                        # what is left is the context's own memory
+    session.close()
+    assert gpu.live == {}
