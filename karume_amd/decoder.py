@@ -287,10 +287,10 @@ class LlamaDecoderSession:
                 self.buf[f"qkv{li}"] = a((sp["hd"] + 2 * sp["kvd"]) * eb)
         self.workspace: Optional[DeviceBuffer] = None
         self._workspace_uses = 0        # recorded steps hold the workspace's address
-        # Recorded steps hold this session's weights, tables and buffers: they are kept with the
-        # memory they run on, under the session that recorded them, and go with either.
-        self._steps = object()
-        self._recorded_on = weakref.WeakSet()   # memories that hold steps of this session
+        # Recorded steps hold this session's weights, tables and buffers.  They are kept with the
+        # memory of its own contexts, whose stream, sizes and workspace they rely on, and go with
+        # either; a context of another session runs by plain launches.
+        self._recorded_on = weakref.WeakSet()   # memories that hold steps
         self._spare_memory: List[ContextMemory] = []   # of the last retired context, at most one
         self._closed = False
         self.logits_shape = (1, c.vocab)
@@ -301,7 +301,7 @@ class LlamaDecoderSession:
         while self._spare_memory:
             self._spare_memory.pop().free()
         for memory in list(self._recorded_on):   # also those of contexts still in use
-            memory.drop_graphs(self._steps)
+            memory.drop_graphs()
         for entry in self.layers:
             for value in entry.values():
                 if isinstance(value, _DeviceLinear):
@@ -362,7 +362,7 @@ class LlamaDecoderSession:
         if memory is not None and memory.slot_bytes != tuple(slot_bytes):
             memory.free()
             memory = None
-        return memory or ContextMemory(self.gpu, slot_bytes, history_len)
+        return memory or ContextMemory(self.gpu, slot_bytes, history_len, owner=self)
 
     def _give_memory(self, memory: ContextMemory, reusable: bool) -> None:
         if reusable and not self._closed and not self._spare_memory:
@@ -390,7 +390,7 @@ class LlamaDecoderSession:
         if not all_rows and not 0 <= last_row < query_length:
             raise ExecutionError(f"last_row {last_row} is outside the {query_length} valid rows")
         try:
-            if m == 1 and self.fuse_decode and context.memory is not None:
+            if m == 1 and self._records_on(context):
                 context.one_row_runs += 1
                 if context.one_row_runs > 1 or self._recorded(context.memory, "step", past):
                     token, logits = self._replay_step(context, ids, pos, past, want_logits)
@@ -652,7 +652,11 @@ class LlamaDecoderSession:
         return max(512, 1 << past.bit_length()) - 1
 
     def _graph_key(self, kind: str, past: int) -> tuple:
-        return (self._steps, kind, self._past_bucket(past), self._workspace_uses)
+        return (kind, self._past_bucket(past), self._workspace_uses)
+
+    def _records_on(self, context: GenerationContext) -> bool:
+        return (self.fuse_decode and context.memory is not None
+                and context.memory.owner is self)
 
     def _recorded(self, memory: ContextMemory, kind: str, past: int) -> bool:
         return self._graph_key(kind, past) in memory.graphs
@@ -666,7 +670,7 @@ class LlamaDecoderSession:
         graph = memory.graphs.get(key)
         if graph is not None:
             return graph
-        memory.drop_graphs(self._steps, kind)   # outgrown
+        memory.drop_graphs(kind)   # outgrown
         g, c, b = self.gpu, self.config, self.buf
         step = memory.step
         self._replay_last_past = self._past_bucket(past)
@@ -790,7 +794,7 @@ class LlamaDecoderSession:
             raise ExecutionError("the decode would run past the RoPE table")
         g, b = self.gpu, self.buf
         context.begin_run(1, 1)
-        cached = self.fuse_decode and context.memory is not None
+        cached = self._records_on(context)
         history = context.memory.history if cached else g.zeros(count * 4)
         graph = None
         try:

@@ -48,14 +48,15 @@ def plan_prefill_chunks(prompt_length: int, chunk_length: int) -> List[PrefillCh
 class ContextMemory:
     """The device memory of one generation context in a single allocation: zeroed state slots,
     the lengths, and the words of a recorded one-row step.  A session keeps the memory of one
-    retired context for its next one, together with the steps recorded on it: `graphs`, by
-    (recording session's key, kind of step, ...).  Any session may run on a context, so the steps
-    of several may stand side by side; a session drops its own when it closes."""
+    retired context for its next one, together with the steps recorded on it (`graphs`, by (kind of
+    step, ...)).  `owner` is that session: any session may run on a context, but only its owner
+    records steps there."""
 
     STEP_BYTES = 64    # ids[4], positions[4], lengths[4], token[4]
 
-    def __init__(self, gpu: GpuContext, slot_bytes: Sequence[int], history_len: int):
+    def __init__(self, gpu: GpuContext, slot_bytes: Sequence[int], history_len: int, owner=None):
         self.gpu = gpu
+        self.owner = owner
         self.slot_bytes = tuple(slot_bytes)
         self.history_len = history_len
         ends, at = [], 0
@@ -71,10 +72,10 @@ class ContextMemory:
         self.history = view(count + 2, 4 * history_len)
         self.graphs: dict = {}
 
-    def drop_graphs(self, *key) -> None:
-        """Destroy the recorded steps whose key starts with `key` (all of them without one)."""
-        for full in [k for k in self.graphs if k[:len(key)] == key]:
-            self.graphs.pop(full).destroy()
+    def drop_graphs(self, kind: Optional[str] = None) -> None:
+        """Destroy the recorded steps of a kind (None: all of them)."""
+        for key in [k for k in self.graphs if kind in (None, k[0])]:
+            self.graphs.pop(key).destroy()
 
     def free(self) -> None:
         self.drop_graphs()

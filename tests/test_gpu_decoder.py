@@ -846,9 +846,9 @@ def test_recorded_one_row_runs_equal_plain_ones_and_survive_context_reuse(gpu_ct
 
 
 def test_sessions_that_take_turns_on_one_context_equal_plain_launches(gpu_ctx):
-    """A session may run on a context of another session of its geometry: each replays the step
-    it recorded itself, so alternating runs equal the launches of sessions that never replay, bit
-    for bit, and so do the tokens of their replayed loops."""
+    """A session may run on a context of another session of its geometry.  The context's own
+    session replays its recorded step, the other one launches: alternating runs equal those of
+    sessions that never replay, bit for bit, and so do the tokens of their replayed loops."""
     config = LlamaConfig(layers=2, d_model=256, ffn=384, heads=4, kv_heads=2, head_dim=64,
                          vocab=512, group_size=128, max_position=64)
     sessions = [LlamaDecoderSession(gpu_ctx, random_weights(config, seed=s), chunk_length=8)

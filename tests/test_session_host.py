@@ -1,4 +1,6 @@
 """What a decoder session launches, seen through a stand-in for the device (no GPU)."""
+from dataclasses import replace
+
 import numpy as np
 import pytest
 
@@ -42,7 +44,8 @@ def test_a_session_on_another_sessions_context_launches_its_own_weights(through)
         assert gpu.mentions(session.layers[1]["down"].w)
         assert gpu.mentions(session.lm_head.w) and not gpu.mentions(other.lm_head.w)
         assert gpu.mentions(session.buf["logits"]) and not gpu.mentions(other.buf["logits"])
-    assert gpu.open_graphs() == 2     # each session's step is kept, not recorded at every turn
+    # the context's own session keeps its step; the other runs by plain launches
+    assert gpu.open_graphs() == 1
     b.close()
     assert gpu.open_graphs() == 1
     context.dispose()
@@ -72,3 +75,46 @@ def test_a_closed_session_refuses_every_call_and_launches_nothing():
     context.dispose()                        # what is left is the context's own memory
     session.close()
     assert gpu.live == {}
+
+
+# ---- contexts that are not the session's own ---------------------------------------------------
+
+def test_a_context_on_another_stream_is_not_stepped_through_a_recorded_step():
+    """The words of a recorded step travel on the stream of the context's own memory; a session
+    whose launches go to another stream must not replay between them."""
+    mine, other = StandInGpu(), StandInGpu()
+    a, b = make_session(other, 4), make_session(mine, 5)
+    context = a.create_generation_context(capacity=64, chunk_length=8)
+    b.create_generation_context(capacity=64, chunk_length=8)
+    for past in range(4):
+        other.clear()
+        one_row(b, context, past)
+        assert other.log == [], past     # ids and positions went up on b's own stream
+    assert mine.open_graphs() == other.open_graphs() == 0
+    mine.clear()
+    b.decode_tokens(context, 1, 3)
+    assert [name for name, _ in other.log] == ["krm_buf_download"]    # the lengths, at the end
+    assert mine.open_graphs() == 0
+
+
+def test_a_replayed_decode_longer_than_the_contexts_own_history():
+    gpu = StandInGpu()
+    short = make_session(gpu, 6, replace(CONFIG, max_position=16))
+    long = make_session(gpu, 7)
+    context = short.create_generation_context(capacity=64, chunk_length=8)
+    long.create_generation_context(capacity=64, chunk_length=8)
+    assert context.memory.history_len == 16
+    assert len(long.decode_tokens(context, 1, 40)) == 40
+
+
+def test_a_context_larger_than_the_sessions_own_needs_no_workspace_ahead():
+    """A session that never made a context of this capacity has no workspace, or a smaller one: a
+    run is sized for its own columns, not for those that a recorded step would be kept for."""
+    gpu = StandInGpu()
+    a, b = make_session(gpu, 8), make_session(gpu, 9)
+    context = a.create_generation_context(capacity=200, chunk_length=8)
+    for past in range(3):
+        gpu.clear()
+        one_row(b, context, past)
+        assert [args[14] for name, args in gpu.log if name == "krm_attention_state"] == [past] * 2
+        assert not any(name == "krm_attention_state_lengths" for name, _ in gpu.log)
