@@ -16,6 +16,7 @@ Every tensor operation is a call into libkarume_hip.so; this module only sequenc
 """
 from __future__ import annotations
 
+import threading
 import weakref
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional
@@ -26,6 +27,11 @@ from .format_i4 import pack_int4
 from .generation import ContextMemory, GenerationContext
 from .runtime import (COMPUTE_F16, COMPUTE_F32, F16, F32, DeviceBuffer, ExecutionError,
                       GpuContext, KarumeError)
+
+
+# A retired context's memory is kept up to this size (the default decoder's state is 23 MB in f32):
+# what a long context held goes back to the other users of the card when it is disposed.
+MAX_SPARE_BYTES = 1 << 30
 
 
 @dataclass(frozen=True)
@@ -291,15 +297,17 @@ class LlamaDecoderSession:
         # memory of its own contexts, whose stream, sizes and workspace they rely on, and go with
         # either; a context of another session runs by plain launches.
         self._recorded_on = weakref.WeakSet()   # memories that hold steps
-        self._spare_memory: List[ContextMemory] = []   # of the last retired context, at most one
+        self._spare_memory: Optional[ContextMemory] = None   # of a retired context
+        self._memory_lock = threading.Lock()    # contexts may be disposed on any thread
         self._closed = False
+        gpu.spare_holders.add(self)
         self.logits_shape = (1, c.vocab)
 
     def close(self) -> None:
         """Free every device buffer of the session (weights, tables, scratch activations)."""
-        self._closed = True
-        while self._spare_memory:
-            self._spare_memory.pop().free()
+        with self._memory_lock:
+            self._closed = True
+        self.release_spare_memory()
         for memory in list(self._recorded_on):   # also those of contexts still in use
             memory.drop_graphs()
         for entry in self.layers:
@@ -354,20 +362,27 @@ class LlamaDecoderSession:
     def _take_memory(self, slot_bytes: List[int]) -> ContextMemory:
         """Memory of a new context: the retired context's when it has the same slots (44
         allocations and 44 fills took 1.0 ms for the default decoder, one fill takes 0.05)."""
-        history_len = self.config.max_position
-        try:
-            memory = self._spare_memory.pop()
-        except IndexError:
-            memory = None
+        with self._memory_lock:
+            memory, self._spare_memory = self._spare_memory, None
         if memory is not None and memory.slot_bytes != tuple(slot_bytes):
             memory.free()
             memory = None
-        return memory or ContextMemory(self.gpu, slot_bytes, history_len, owner=self)
+        return memory or ContextMemory(self.gpu, slot_bytes, self.config.max_position, owner=self)
 
     def _give_memory(self, memory: ContextMemory, reusable: bool) -> None:
-        if reusable and not self._closed and not self._spare_memory:
-            self._spare_memory.append(memory)
-        else:
+        with self._memory_lock:
+            if (reusable and not self._closed and self._spare_memory is None
+                    and memory.buffer.nbytes <= MAX_SPARE_BYTES):
+                self._spare_memory = memory
+                return
+        memory.free()
+
+    def release_spare_memory(self) -> None:
+        """Free the device memory kept from the last retired context for the next one.  An
+        allocation of this GpuContext that finds no room does so by itself."""
+        with self._memory_lock:
+            memory, self._spare_memory = self._spare_memory, None
+        if memory is not None:
             memory.free()
 
     def run(self, input_ids: np.ndarray, position_ids: np.ndarray, last_row: Optional[int], *,

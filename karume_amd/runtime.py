@@ -8,6 +8,7 @@ around the C ABI: no arithmetic happens in Python.
 from __future__ import annotations
 
 import ctypes as C
+import weakref
 from typing import Optional, Sequence, Union
 
 import numpy as np
@@ -190,6 +191,8 @@ class GpuContext:
         self._handle = handle
         self.device = device
         self._buffers: set[DeviceBuffer] = set()
+        # objects that keep memory they could do without (release_spare_memory())
+        self.spare_holders: weakref.WeakSet = weakref.WeakSet()
 
     # -- lifecycle -------------------------------------------------------------------------
     def destroy(self) -> None:
@@ -224,7 +227,12 @@ class GpuContext:
     # -- buffers ---------------------------------------------------------------------------
     def alloc(self, nbytes: int) -> DeviceBuffer:
         address = C.c_uint64()
-        self._check(self._lib.krm_buf_alloc(self._handle, nbytes, C.byref(address)))
+        try:
+            self._check(self._lib.krm_buf_alloc(self._handle, nbytes, C.byref(address)))
+        except GpuOutOfMemoryError:
+            for holder in list(self.spare_holders):
+                holder.release_spare_memory()
+            self._check(self._lib.krm_buf_alloc(self._handle, nbytes, C.byref(address)))
         buf = DeviceBuffer(self, address.value, nbytes, owned=True)
         self._buffers.add(buf)
         return buf

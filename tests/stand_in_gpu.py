@@ -6,6 +6,7 @@ library behind it is replaced.  Addresses come from one counter and are never re
 argument of a logged call names its buffer for good; `live` holds the ranges not freed yet.
 """
 import ctypes as C
+import weakref
 
 from karume_amd import _ffi
 from karume_amd.runtime import GpuContext
@@ -32,10 +33,15 @@ class _Library:
 
     def _krm_buf_alloc(self, _handle, nbytes, out):
         global _next_address
+        if sum(self._gpu.live.values()) + nbytes > self._gpu.memory:
+            return -2
         out._obj.value = _next_address
         self._gpu.live[_next_address] = nbytes
         _next_address += (nbytes + 511) // 256 * 256
         return 0
+
+    def _krm_last_error(self, _handle):
+        return b"out of memory"
 
     def _krm_buf_free(self, _handle, address):
         del self._gpu.live[int(address)]
@@ -73,6 +79,8 @@ class StandInGpu(GpuContext):
         self._handle = C.c_void_p(1)
         self.device = 0
         self._buffers = set()
+        self.spare_holders = weakref.WeakSet()
+        self.memory = 1 << 40
         self.live, self.graphs = {}, []
         self.log, self.recording = [], None
 

@@ -4,8 +4,9 @@ from dataclasses import replace
 import numpy as np
 import pytest
 
+from karume_amd import decoder
 from karume_amd.decoder import LlamaConfig, LlamaDecoderSession, random_weights
-from karume_amd.runtime import ExecutionError
+from karume_amd.runtime import ExecutionError, GpuOutOfMemoryError
 from stand_in_gpu import StandInGpu
 
 CONFIG = LlamaConfig(layers=2, d_model=128, ffn=256, heads=2, kv_heads=1, head_dim=64, vocab=64,
@@ -118,3 +119,42 @@ def test_a_context_larger_than_the_sessions_own_needs_no_workspace_ahead():
         one_row(b, context, past)
         assert [args[14] for name, args in gpu.log if name == "krm_attention_state"] == [past] * 2
         assert not any(name == "krm_attention_state_lengths" for name, _ in gpu.log)
+
+
+# ---- memory kept from a retired context ---------------------------------------------------------
+
+def used(gpu):
+    return sum(gpu.live.values())
+
+
+def test_a_session_keeps_one_retired_contexts_memory_and_gives_it_back(monkeypatch):
+    gpu = StandInGpu()
+    session = make_session(gpu, 10)
+    make = lambda: session.create_generation_context(capacity=64, chunk_length=8)  # noqa: E731
+    make().dispose()
+    with_one, one = used(gpu), session._spare_memory.buffer.nbytes
+    first, second = make(), make()
+    one_row(session, first, 0), one_row(session, first, 1)
+    assert used(gpu) == with_one + one and gpu.open_graphs() == 1
+    second.dispose(), first.dispose()              # the second one finds the place taken
+    assert used(gpu) == with_one and gpu.open_graphs() == 0
+    session.release_spare_memory()
+    assert used(gpu) == with_one - one
+    session.release_spare_memory()
+    monkeypatch.setattr(decoder, "MAX_SPARE_BYTES", one - 1)
+    make().dispose()                               # larger than what is worth keeping
+    assert used(gpu) == with_one - one
+
+
+def test_an_allocation_without_room_takes_the_kept_memory_back():
+    gpu = StandInGpu()
+    session = make_session(gpu, 11)
+    make = lambda: session.create_generation_context(capacity=64, chunk_length=8)  # noqa: E731
+    make().dispose()
+    one = session._spare_memory.buffer.nbytes
+    gpu.memory = used(gpu) + one - 1
+    buffer = gpu.alloc(one)
+    assert session._spare_memory is None
+    with pytest.raises(GpuOutOfMemoryError):
+        gpu.alloc(one)
+    buffer.free()
