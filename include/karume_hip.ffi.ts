@@ -17,6 +17,7 @@ export const KARUME_HIP_SYMBOLS = {
   krm_buf_alloc: { parameters: ["pointer", "usize", "buffer"], result: "i32" },
   krm_buf_free: { parameters: ["pointer", "u64"], result: "i32" },
   krm_buf_upload: { parameters: ["pointer", "u64", "usize", "buffer", "usize"], result: "i32" },
+  krm_buf_write: { parameters: ["pointer", "u64", "usize", "buffer", "usize"], result: "i32" },
   krm_buf_download: { parameters: ["pointer", "u64", "usize", "buffer", "usize"], result: "i32" },
   krm_buf_zero: { parameters: ["pointer", "u64", "usize", "usize"], result: "i32" },
   krm_buf_copy: { parameters: ["pointer", "u64", "u64", "usize"], result: "i32" },

@@ -15,7 +15,8 @@
  *  - `krm_buf` is a raw device address (uint64).  Offsets are applied by the caller
  *    (address + bytes).  The caller owns every buffer; the library owns its context, its
  *    stream and whatever scratch it allocated itself.
- *  - launches are asynchronous on the context's stream; krm_buf_download and krm_sync fence.
+ *  - launches are asynchronous on the context's stream; krm_buf_upload, krm_buf_download and
+ *    krm_sync fence.
  *  - host pointers are only read/written during the call.
  *  - one context = one stream, externally serialised (the reference serialises runs per
  *    Session, packages/runtime/src/runtime/generation-context.ts:103-106).  The device is set
@@ -90,8 +91,14 @@ const char* krm_version(void);
  *      packages/runtime/src/runtime/executor.ts:870-896,1272) ------------------------------ */
 int32_t krm_buf_alloc(krm_ctx* ctx, size_t bytes, krm_buf* out);
 int32_t krm_buf_free(krm_ctx* ctx, krm_buf buf);
+/* Waits for the copy: any context or stream may read the buffer once the call has returned. */
 int32_t krm_buf_upload(krm_ctx* ctx, krm_buf dst, size_t dst_offset, const void* host,
                        size_t bytes);
+/* The same bytes in the order of the context's stream (queue.writeBuffer): work queued on this
+ * context later sees them, other contexts and streams only behind krm_sync or another fence.
+ * Does not wait for up to 1024 bytes in whole words at a 4-byte aligned address. */
+int32_t krm_buf_write(krm_ctx* ctx, krm_buf dst, size_t dst_offset, const void* host,
+                      size_t bytes);
 int32_t krm_buf_download(krm_ctx* ctx, krm_buf src, size_t src_offset, void* host, size_t bytes);
 /* State slots are zero-initialised at creation
  * (packages/runtime/tests/gpu_state_execution_test.ts:159-164). */
@@ -111,7 +118,7 @@ int32_t krm_event_destroy(krm_ctx* ctx, krm_event* ev);
  * Between krm_graph_begin and krm_graph_end the op entry points record instead of running
  * (HIP stream capture); krm_graph_launch replays the recorded sequence on the context's
  * stream with the pointers and scalars it was recorded with.  Calls that must wait for the
- * device (upload, download, free, sync, krm_attention_varlen) are rejected while recording. */
+ * device (upload, write, download, free, sync, krm_attention_varlen) are rejected while recording. */
 typedef struct krm_graph krm_graph;
 int32_t krm_graph_begin(krm_ctx* ctx);
 /* While recording: the ops that follow go to parallel branch `branch` (0 = the main branch,

@@ -29,6 +29,7 @@ PROTOTYPES = {
     "krm_buf_alloc": (i32, [c_ctx, size_t, C.POINTER(c_buf)]),
     "krm_buf_free": (i32, [c_ctx, c_buf]),
     "krm_buf_upload": (i32, [c_ctx, c_buf, size_t, C.c_void_p, size_t]),
+    "krm_buf_write": (i32, [c_ctx, c_buf, size_t, C.c_void_p, size_t]),
     "krm_buf_download": (i32, [c_ctx, c_buf, size_t, C.c_void_p, size_t]),
     "krm_buf_zero": (i32, [c_ctx, c_buf, size_t, size_t]),
     "krm_buf_copy": (i32, [c_ctx, c_buf, c_buf, size_t]),

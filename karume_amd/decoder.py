@@ -413,8 +413,8 @@ class LlamaDecoderSession:
                         logits = logits.reshape(1, 1, self.config.vocab)
                     context.advance(past, query_length)
                     return (token, logits) if want_logits else token
-            self.buf["ids"].upload(ids)
-            self.buf["pos"].upload(pos)
+            self.buf["ids"].write(ids)
+            self.buf["pos"].write(pos)
             if all_rows and m > 1:
                 self._forward(context, m, past, query_length, None, lengths=None)
                 token = self.buf["tokens_all"].download(np.int32, (1, m, 1))
@@ -710,13 +710,13 @@ class LlamaDecoderSession:
 
     def _replay_step(self, context: GenerationContext, ids, pos, past: int, want_logits: bool):
         """One row through the recorded step: the id, the position and the lengths in one small
-        upload, one graph launch, one read-back (112 launches from Python took 0.60 ms of host
+        write, one graph launch, one read-back (112 launches from Python took 0.60 ms of host
         time a token, the device needs 0.45)."""
         graph = self._recorded_step(context, "step", past)
         words = np.zeros(12, dtype=np.int32)
         words[0], words[4], words[8], words[9] = ids[0, 0], pos[0, 0], past, 1
         step = context.memory.step
-        step.upload(words)
+        step.write(words)
         graph.launch()
         token = step.download(np.int32, (1, 1, 1), byte_offset=48)
         logits = self.buf["logits"].download(self.io_np, self.logits_shape) if want_logits else None
@@ -815,7 +815,7 @@ class LlamaDecoderSession:
         try:
             # the token buffer doubles as the id input: argmax writes it, the next replay's
             # embedding reads it
-            b["token"].upload(np.array([first_token, 0, 0, 0], dtype=np.int32))
+            b["token"].write(np.array([first_token, 0, 0, 0], dtype=np.int32))
             g.lengths_set(context.lengths, context.past, 1)
             g.lengths_positions(context.lengths, b["pos"], 1)
             if self.fuse_decode:

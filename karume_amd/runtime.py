@@ -78,10 +78,18 @@ class DeviceBuffer:
         return self.address + byte_offset
 
     def upload(self, array: np.ndarray, byte_offset: int = 0) -> None:
+        """Copy `array` and wait for it: any context or stream may read the buffer now."""
+        self._copy_in("krm_buf_upload", array, byte_offset)
+
+    def write(self, array: np.ndarray, byte_offset: int = 0) -> None:
+        """Copy `array` in the order of this context's stream; a few words do not wait."""
+        self._copy_in("krm_buf_write", array, byte_offset)
+
+    def _copy_in(self, entry: str, array: np.ndarray, byte_offset: int) -> None:
         data = np.ascontiguousarray(array)
         if byte_offset + data.nbytes > self.nbytes:
             raise GpuValidationError("upload past the end of the buffer")
-        self.ctx._check(self.ctx._lib.krm_buf_upload(
+        self.ctx._check(getattr(self.ctx._lib, entry)(
             self.ctx._handle, self.address, byte_offset, data.ctypes.data, data.nbytes))
 
     def download(self, dtype, shape: Sequence[int], byte_offset: int = 0) -> np.ndarray:
