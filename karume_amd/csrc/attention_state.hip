@@ -1116,7 +1116,11 @@ void attention_decode_kernel(
   // chunks are requested together (a chunk costs 0.95 us when each waits for its own round
   // trip; 3 x 32 registers of rows fit beside one head's state).  Each case holds its loads and
   // their uses in one branch: a branch between a load and its use makes the compiler wait
-  // inside it.
+  // inside it.  Two chunks where three would pass 256 registers, i.e. one workgroup a CU for
+  // launches of many splits: the variant that scores on the matrix cores, and ragged batches whose
+  // f32 queries meet fp16 rows (178 registers, 263 with three; 24 sequences up to 3000 columns of 16
+  // heads, D = 64, two layers: 77.6 us, 110.6 with three).
+  constexpr bool kThreeChunks = !kMfma && !(RAGGED && sizeof(XT) > sizeof(ST));
   if (!early) load_chunk(0, rows0);  // harmless when the split has no column at all
   // The own column's scores, as soon as every row is asked for: the operand's registers go.
   float own_dot = 0.f;
@@ -1137,11 +1141,9 @@ void attention_decode_kernel(
       consume_chunk(1, rows1);
       walked = true;
     } else if (nsplit == 1 && total_chunks > 2) {
-      // (the variant that scores on the matrix cores holds more state: two chunks at once keep
-      // it within 256 registers, i.e. two workgroups a CU for its many-split launches)
       ChunkRows rows1;
       load_chunk(1, rows1);
-      if constexpr (!kMfma) {
+      if constexpr (kThreeChunks) {
         ChunkRows rows2;
         load_chunk(2, rows2);
         consume_chunk(0, rows0);
@@ -1151,7 +1153,7 @@ void attention_decode_kernel(
         consume_chunk(0, rows0);
         consume_chunk(1, rows1);
       }
-      for (uint32_t chunk = kMfma ? 2 : 3; chunk < total_chunks; ++chunk) {
+      for (uint32_t chunk = kThreeChunks ? 3 : 2; chunk < total_chunks; ++chunk) {
         load_chunk(chunk, rows0);
         consume_chunk(chunk, rows0);
       }

@@ -1,0 +1,31 @@
+"""Registers and scratch of the built kernels: figures that decide how many waves a SIMD holds, and
+that a change of a kernel can move without any result showing it.  Read from the library; no GPU."""
+import os
+import re
+
+import pytest
+
+import kernel_resources
+from karume_amd import _ffi
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    if not os.path.exists(_ffi.LIB_PATH):
+        pytest.skip("the library has not been built")
+    found = kernel_resources.kernels()
+    assert len(found) > 500
+    return found
+
+
+def arguments(name):
+    return [a.strip() for a in re.search(r"<(.*)>", name).group(1).split(",")]
+
+
+def test_one_head_decode_attention_leaves_room_for_two_waves_a_simd(kernels):
+    checked = 0
+    for name, kernel in kernels.items():
+        if name.startswith("attention_decode_kernel<") and arguments(name)[2] == "1":
+            assert kernel_resources.registers(kernel) <= 256, name
+            checked += 1
+    assert checked == 4 * 5 * 2    # element types, lanes a row, single and ragged
