@@ -669,6 +669,7 @@ void linear_w4a8_tile_kernel(
 // words are expanded once (both column tiles, all MFMA steps of the group), then each row tile
 // in turn runs its two MFMA chains over the group and is fused into its f32 accumulators — 32
 // int32 accumulators live at a time, and the expansion is shared by the two row tiles.
+// (Groups of 32 in the smaller tile only, see the dispatch.)
 template <typename ST, int GSH, int WM, int NW, int WN>
 __global__ __launch_bounds__(64 * WM * NW) __attribute__((amdgpu_waves_per_eu(2, WN == 2 ? 2 : 4)))
 void linear_w4a8_tall_kernel(
@@ -676,6 +677,7 @@ void linear_w4a8_tall_kernel(
     const ST* __restrict__ scales, const float* __restrict__ bias, float* __restrict__ out,
     uint32_t m, uint32_t n, uint32_t k, uint32_t m_blocks, uint32_t n_blocks) {
   static_assert(GSH >= 5 && GSH <= 7, "groups of 32, 64 or 128 codes");
+  static_assert(GSH > 5 || WN == 1, "two column tiles of groups of 32 spill");
   constexpr int T = 64 * WM * NW, MT = 2;
   constexpr int BM = 64 * WM, BN = 32 * WN * NW;
   constexpr int kStage = 128;                          // codes per LDS stage
@@ -890,15 +892,18 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
     // 512 x 11008 x 4096 59.5 / 56, in groups of 64 70 / 60; 400 x 9000 x 3072 49.5 / 35; 200 x 20000
     // x 4096 55.4 / 48; 300 x 14000 x 2048 in groups of 64 42 / 34.5; where the tall ones fill whole
     // rounds (2048 x 11008 x 4096, 256 x 32000 x 2048) these take 2 % longer.
-    // Groups of 32 always come here, the generic kernel re-reads both operands for every output: 512 x
-    // 11008 x 4096 50785 / 111, 197 x 1655 x 9600 7716 / 120, 20 x 20000 x 1024 914 / 19, 9 x 300 x
-    // 512 11.7 / 11.8.
+    // Groups of 32 always come here and always take the 64 x 128 tiles: the generic kernel re-reads both
+    // operands for every output (512 x 11008 x 4096 50785 / 116 us, 197 x 1655 x 9600 7716 / 120, 20 x
+    // 20000 x 1024 914 / 19, 9 x 300 x 512 11.7 / 11.8), and a 128 x 256 tile of four groups a stage does
+    // not fit the registers (206 spilled: 2048 x 11008 x 4096 1907 us, 352 in 64 x 128 tiles; 2048 x 4096
+    // x 4096 709 and 130).
     const uint64_t cus = (uint64_t)ctx->num_cus;
     const uint64_t tall_tiles = (uint64_t)((m + 127) / 128) * n_blocks;
     if (shift == 5 || ((shift == 6 || shift == 7) && tall_tiles * 5 >= cus * 3)) {
       const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
       const uint64_t small_rounds = ((uint64_t)small_m * small_n + cus - 1) / cus;
-      const bool small = small_rounds * 115 < (tall_tiles + cus - 1) / cus * 400;
+      const bool small =
+          shift == 5 || small_rounds * 115 < (tall_tiles + cus - 1) / cus * 400;
       const uint32_t mb = small ? small_m : (m + 127) / 128, nb = small ? small_n : n_blocks;
       const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * mb;
       if (blocks <= 0x7fffffffull) {
@@ -910,8 +915,7 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
           if (shift == 5) KRM_W4A8_TALL(5, 1, 1);
           else if (shift == 6) KRM_W4A8_TALL(6, 1, 1); else KRM_W4A8_TALL(7, 1, 1);
         } else {
-          if (shift == 5) KRM_W4A8_TALL(5, 2, 2);
-          else if (shift == 6) KRM_W4A8_TALL(6, 2, 2); else KRM_W4A8_TALL(7, 2, 2);
+          if (shift == 6) KRM_W4A8_TALL(6, 2, 2); else KRM_W4A8_TALL(7, 2, 2);
         }
 #undef KRM_W4A8_TALL
         return launched(ctx, "linear_w4a8_tall_kernel");

@@ -314,7 +314,7 @@ def test_w4a8_fused_call_equals_the_two_steps(gpu_ctx, m, n, k, group, scale_f16
 
 @pytest.mark.parametrize("m, n, k, scale_f16, with_bias", [
     (9, 1, 32, True, False), (64, 128, 96, False, True), (65, 129, 160, True, True),
-    (197, 333, 1056, True, False), (600, 8200, 64, False, False)])
+    (197, 333, 1056, True, False), (600, 8200, 64, False, False), (1024, 8192, 96, True, True)])
 def test_w4a8_many_rows_in_groups_of_32(gpu_ctx, m, n, k, scale_f16, with_bias):
     rng = np.random.default_rng(m + n + k)
     packed, q, scale = helpers.synthetic_int4(rng, n, k, 32, scale_f16)

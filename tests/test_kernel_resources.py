@@ -29,3 +29,10 @@ def test_one_head_decode_attention_leaves_room_for_two_waves_a_simd(kernels):
             assert kernel_resources.registers(kernel) <= 256, name
             checked += 1
     assert checked == 4 * 5 * 2    # element types, lanes a row, single and ragged
+
+
+def test_tiles_of_w4a8_groups_up_to_128_keep_their_state_in_registers(kernels):
+    tiles = {n: k for n, k in kernels.items() if n.startswith("linear_w4a8_tall_kernel<")}
+    assert {arguments(n)[1] for n in tiles} == {"5", "6", "7"}
+    for name, kernel in tiles.items():
+        assert kernel_resources.scratch(kernel) == 0, name
