@@ -273,7 +273,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   __shared__ float s_m[WAVES][kRows], s_l[WAVES][kRows];
 
   const uint32_t z = blockIdx.x, row0 = blockIdx.y * (uint32_t)kRows;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // key blocks are a wave's: scalar
   const int r = lane & 15, g = lane >> 4;
   uint32_t past = a.past, query = a.query;
   if (!device_lengths(a.lengths, a.chunk_rows, a.capacity, a.window, past, query)) return;
@@ -336,14 +337,23 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   // `past` whose slot rows do not wrap is 32-bit offsets from one base; only the others look every
   // row up.
   const uint32_t load_key = lane / kPieces, load_piece = 4u * (lane % kPieces);
+  // A lane's key numbers inside a block, formed anew for every block where two element types meet:
+  // there every row of a block keeps a number of its own, and kept over the walk these took the
+  // state's registers to spilling.
+  auto lane_key_of = [](uint32_t key) {
+    if constexpr (sizeof(ST) != sizeof(XT)) asm volatile("" : "+v"(key));
+    return key;
+  };
   const size_t slot_plane = (size_t)kv_plane * a.capacity * D;
   const size_t ins_plane = (size_t)kv_plane * a.chunk_rows * D;
   auto slot_columns = [&](uint64_t c0) -> uint32_t {  // of the block's 32
     return c0 >= past ? 0u : (uint32_t)(past - c0 < 32u ? past - c0 : 32u);
   };
-  // `keys` lane rows, row i the block's key key_of(i), `pieces` pieces of 4 elements 64 apart
-  auto request = [&](uint32_t kb, const ST* slot, const XT* ins, auto keys, auto key_of,
-                     uint32_t lane_dim, auto pieces, uint4* raw) {
+  // `keys` lane rows, row i the block's key lane_key + step_of(i), `pieces` pieces of 4 elements 64
+  // apart
+  auto request = [&](uint32_t kb, const ST* slot, const XT* ins, auto keys, uint32_t lane_key,
+                     auto step_of, uint32_t lane_dim, auto pieces, uint4* raw) {
+    lane_key = lane_key_of(lane_key);
     constexpr int kKeys = decltype(keys)::value, kPer = decltype(pieces)::value;
     const uint64_t c0 = c_lo + (uint64_t)kb * 32u;
     const uint32_t slots = slot_columns(c0);
@@ -354,7 +364,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       for (int i = 0; i < kKeys; ++i)
 #pragma unroll
         for (int j = 0; j < kPer; ++j)
-          raw[i * kPer + j] = load4_raw<ST>(base + (key_of(i) * D + lane_dim + 64 * j));
+          raw[i * kPer + j] = load4_raw<ST>(base + ((lane_key + step_of(i)) * D + lane_dim + 64 * j));
     } else if (slots == 0u) {
       const XT* base = ins + ins_plane + (size_t)(c0 - past) * D;
       const uint32_t most = limit_hi - c0 < 31u ? (uint32_t)(limit_hi - c0) : 31u;
@@ -362,11 +372,12 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       for (int i = 0; i < kKeys; ++i)
 #pragma unroll
         for (int j = 0; j < kPer; ++j)
-          raw[i * kPer + j] = load4_raw<XT>(base + (min(key_of(i), most) * D + lane_dim + 64 * j));
+          raw[i * kPer + j] = load4_raw<XT>(
+              base + (min(lane_key + step_of(i), most) * D + lane_dim + 64 * j));
     } else {
 #pragma unroll
       for (int i = 0; i < kKeys; ++i) {
-        const uint32_t key = min(key_of(i), (uint32_t)(limit_hi - c0 < 31u ? limit_hi - c0 : 31u));
+        const uint32_t key = min(lane_key + step_of(i), (uint32_t)(limit_hi - c0 < 31u ? limit_hi - c0 : 31u));
         const bool in_slot = key < slots;
         uint32_t at = first + key;  // (a block of 32 wraps once, unless the window is shorter)
         if (a.window && at >= a.window) at = a.window >= 32u ? at - a.window : at % a.window;
@@ -382,15 +393,15 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       }
     }
   };
-  auto v_key = [&](int j) -> uint32_t { return (uint32_t)(16 * (j / 4) + 4 * g + j % 4); };
+  auto v_step = [](int j) -> uint32_t { return (uint32_t)(16 * (j / 4) + j % 4); };
   uint4 kraw[kLoads], vraw[8 * kVPieces];
   auto request_k = [&](uint32_t kb) {
-    request(kb, slot_k, ins_k, std::integral_constant<int, kLoads>{},
-            [&](int i) { return (uint32_t)(i * kRowsPerLoad) + load_key; }, load_piece,
+    request(kb, slot_k, ins_k, std::integral_constant<int, kLoads>{}, load_key,
+            [](int i) { return (uint32_t)(i * kRowsPerLoad); }, load_piece,
             std::integral_constant<int, 1>{}, kraw);
   };
   auto request_v = [&](uint32_t kb) {
-    request(kb, slot_v, ins_v, std::integral_constant<int, 8>{}, v_key, 4u * r,
+    request(kb, slot_v, ins_v, std::integral_constant<int, 8>{}, 4u * g, v_step, 4u * r,
             std::integral_constant<int, kVPieces>{}, vraw);
   };
   // f32 of what arrived
@@ -450,9 +461,10 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     const bool more = kb + (uint32_t)WAVES < blocks;
     if constexpr (!kAhead) request_k(kb);
     const uint32_t slots = slot_columns(c0);
+    const uint32_t parked_key = lane_key_of(load_key);
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      const uint32_t key = j * kRowsPerLoad + load_key;
+      const uint32_t key = j * kRowsPerLoad + parked_key;
       float4 kv = element4(kraw[j], key, slots);
       kv.x *= a.scale; kv.y *= a.scale; kv.z *= a.scale; kv.w *= a.scale;
       *reinterpret_cast<float4*>(&mk[key * kRow + load_piece]) = kv;
@@ -527,11 +539,12 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= alpha;
       // (tile dt = 4 i + e holds the dims 64 i + 4 r + e: a 16-byte piece feeds four tiles)
+      const uint32_t pv_key = lane_key_of(4u * g);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
 #pragma unroll
         for (int i = 0; i < kVPieces; ++i) {
-          const float4 v4 = element4(vraw[j * kVPieces + i], v_key(j), slots);
+          const float4 v4 = element4(vraw[j * kVPieces + i], pv_key + v_step(j), slots);
           const float vf[4] = {v4.x, v4.y, v4.z, v4.w};
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -1476,7 +1489,9 @@ int32_t launch_rows(krm_ctx* ctx, krm_buf q, krm_buf ins_k, krm_buf ins_v, krm_b
   // Eight waves, two a SIMD, so that one wave's softmax and LDS traffic run under the other's
   // MFMAs; D = 256: four (the state of a wave takes a SIMD's registers).  A workgroup takes one
   // block of 16 query rows; with D = 64, whose second block fits the registers, two (the K / V
-  // blocks then serve both) once that still leaves two workgroups per CU.  A row's arithmetic is
+  // blocks then serve both) once that still leaves two workgroups per CU.  (D = 128 in two blocks
+  // had to park V as well: 512 rows behind 2048, r = 4, in f32 303 us, 233 in single blocks; 585
+  // and 261 in f32 over fp16 slots.)  A row's arithmetic is
   // the same in both forms and the wave count depends on D only, so its bits depend neither on the
   // chunk length, the batch, the past or the capacity nor on the lengths form.
   const uint32_t row_blocks = (a.chunk_rows + 15) / 16;
