@@ -201,8 +201,8 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // What bounds it is the f32 matrix rate with two waves a SIMD to cover softmax and waits (D = 64,
 // r = 8, 128 rows behind 1024: 8 us of MFMA).  With V parked as well, rows looked up one by one
 // (two element types: a wait at each), expf and no requests ahead, us before / now: that case
-// 22.7 / 19.2; fp16, D = 128, r = 4: 49.2 / 33.9; f32 over fp16 slots 105.6 / 36.2; D = 256, r = 8
-// (two waves then, four now that LDS holds K alone): 162 / 70.
+// 22.7 / 19.3; fp16, D = 128, r = 4: 49.4 / 32.6; f32 over fp16 slots 106.5 / 36.8; D = 256, r = 8
+// (two waves then, four now that LDS holds K alone): 172 / 71.
 typedef float float4v_t __attribute__((ext_vector_type(4)));
 
 template <typename T>
@@ -255,6 +255,20 @@ __device__ inline float4 raw4_f32(const uint4& v) {
   }
 }
 
+// e^d for d <= 0 (or -inf: 0) with one v_exp_f32.  2^t with t = d log2 e rounded alone is off by up
+// to |d| 2^-24 of itself; e^d = 2^t e^r with r = d - t ln 2, and r is so small that 1 + r is its
+// exponential.  ln 2 in two parts, the first of 24 bits: the first difference is exact.  (The bounds
+// hold r finite where 2^t is 0 anyway.)  2^t alone took 1 to 2 % less of a long chunk (512 rows behind
+// 2048, D = 128, f32: 233 us, 237 so).
+__device__ inline float exp_of_difference(float d) {
+  const float t = d * 1.4426950408889634f;
+  const float high = 0.69314718055994531f;
+  const float low = (float)(0.693147180559945309417 - (double)0.69314718055994531f);
+  const float r = __builtin_amdgcn_fmed3f(fmaf(-t, low, fmaf(-t, high, d)), -1.0f, 1.0f);
+  const float p = __builtin_amdgcn_exp2f(t);
+  return fmaf(p, r, p);
+}
+
 template <typename XT, typename ST, int D, int WAVES, int RB>
 __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     const XT* __restrict__ q, const XT* __restrict__ ins_k, const XT* __restrict__ ins_v,
@@ -299,7 +313,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     }
     return;
   }
-  const uint32_t kv_plane = z / (a.heads / a.kv_heads);
+  // (scalar, which the compiler's division is not: the planes' addresses take no vector registers)
+  const uint32_t kv_plane = __builtin_amdgcn_readfirstlane(z / (a.heads / a.kv_heads));
 
   // Q block: asked for first, parked (scaled) behind the request of the wave's first key block
   constexpr int kQUnits = kRows * kPieces, kQPer = (kQUnits + (int)kBlock - 1) / (int)kBlock;
@@ -337,12 +352,12 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   // `past` whose slot rows do not wrap is 32-bit offsets from one base; only the others look every
   // row up.
   const uint32_t load_key = lane / kPieces, load_piece = 4u * (lane % kPieces);
-  // A lane's key numbers inside a block, formed anew for every block where two element types meet:
-  // there every row of a block keeps a number of its own, and kept over the walk these took the
-  // state's registers to spilling.
-  auto lane_key_of = [](uint32_t key) {
-    if constexpr (sizeof(ST) != sizeof(XT)) asm volatile("" : "+v"(key));
-    return key;
+  // A lane's key number inside a block, from which its rows' numbers are formed anew for every block
+  // where two element types meet: there every row keeps one of its own, and held over the walk these
+  // took the state's registers to spilling.
+  auto lane_number = [](uint32_t number) {
+    if constexpr (sizeof(ST) != sizeof(XT)) asm volatile("" : "+v"(number));
+    return number;
   };
   const size_t slot_plane = (size_t)kv_plane * a.capacity * D;
   const size_t ins_plane = (size_t)kv_plane * a.chunk_rows * D;
@@ -353,7 +368,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   // apart
   auto request = [&](uint32_t kb, const ST* slot, const XT* ins, auto keys, uint32_t lane_key,
                      auto step_of, uint32_t lane_dim, auto pieces, uint4* raw) {
-    lane_key = lane_key_of(lane_key);
+    lane_key = lane_number(lane_key);
     constexpr int kKeys = decltype(keys)::value, kPer = decltype(pieces)::value;
     const uint64_t c0 = c_lo + (uint64_t)kb * 32u;
     const uint32_t slots = slot_columns(c0);
@@ -461,7 +476,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     const bool more = kb + (uint32_t)WAVES < blocks;
     if constexpr (!kAhead) request_k(kb);
     const uint32_t slots = slot_columns(c0);
-    const uint32_t parked_key = lane_key_of(load_key);
+    const uint32_t parked_key = lane_number(load_key);
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const uint32_t key = j * kRowsPerLoad + parked_key;
@@ -520,15 +535,14 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       block_max = exchange_max(exchange_max(block_max, 16), 32);
       const float new_m = fmaxf(run_m[rb], block_max);
       const float ref = new_m == -INFINITY ? 0.f : new_m;  // nothing seen yet: exp(-inf - 0) = 0
-      // (the difference first, then its product with log2 e: one v_exp_f32, within an ulp of expf on
-      // what it is added to; expf's own range handling was a quarter of the loop's instructions)
-      const float alpha = __builtin_amdgcn_exp2f((run_m[rb] - ref) * 1.4426950408889634f);
+      // (expf's own range handling was a quarter of the loop's instructions)
+      const float alpha = exp_of_difference(run_m[rb] - ref);
       float p[2][4], sum = 0.f;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          p[t][i] = __builtin_amdgcn_exp2f((st[t][i] - ref) * 1.4426950408889634f);  // 0 where masked
+          p[t][i] = exp_of_difference(st[t][i] - ref);  // 0 where masked
           sum += p[t][i];
         }
       run_l[rb] = run_l[rb] * alpha + sum;
@@ -539,7 +553,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= alpha;
       // (tile dt = 4 i + e holds the dims 64 i + 4 r + e: a 16-byte piece feeds four tiles)
-      const uint32_t pv_key = lane_key_of(4u * g);
+      const uint32_t pv_key = lane_number(4u * g);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
 #pragma unroll

@@ -822,3 +822,58 @@ def test_head_dim_256_forms(gpu_ctx, case, io, kv):
         assert np.all(np.abs(got.astype(np.float32) - ref) <= np.abs(ref) * 2.0 ** -10 + 1e-6)
     pad = got[:, :, case.query:, :]
     assert not pad.size or (np.all(pad == 0) and not np.any(np.signbit(pad)))
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+def test_chunk_probabilities_far_below_the_maximum_are_exact_exponentials(gpu_ctx, depth):
+    """Row r of a chunk sees column 0 at a score d_r and its own columns at 0; only column 0 has a
+    value, large enough to show its probability e^d_r.  The scores are exact (one product with 1), so
+    the output's relative error is that of the exponential (2 ulp), the value's product, the sum's
+    reciprocal and the last product: 2^-22 + 3 * 2^-24."""
+    rng = np.random.default_rng(depth)
+    m = 40
+    d = -rng.uniform(0.5, 84.0, size=m).astype(np.float32)
+    d[:3] = -83.7, -84.0, -0.5
+    q = np.zeros((1, 1, m, depth), dtype=np.float32)
+    q[0, 0, :, 0] = d                 # against k = (1, 0, ..): the score is d_r itself
+    ins = np.zeros((1, 1, m, depth), dtype=np.float32)
+    slot_k = np.zeros((1, 1, 64, depth), dtype=np.float32)
+    slot_v = np.zeros((1, 1, 64, depth), dtype=np.float32)
+    slot_k[0, 0, 0, 0] = 1.0
+    slot_v[0, 0, 0, :] = 1e30
+    bufs = [gpu_ctx.upload(a) for a in (q, ins, ins, slot_k, slot_v)]
+    out = gpu_ctx.alloc(q.nbytes)
+    gpu_ctx.attention_chunk(*bufs, out, batch=1, heads=1, kv_heads=1, chunk_rows=m, depth=depth,
+                            capacity=64, window=0, half_scale=1.0, past=1, query=m)
+    got = out.download(np.float32, (m, depth)).astype(np.float64)
+    p = np.exp(d.astype(np.float64))
+    want = (p * np.float32(1e30) / (p + np.arange(1, m + 1)))[:, None]
+    error = np.abs(got / want - 1.0).max(axis=1)
+    assert error.max() <= 2.0 ** -22 + 3 * 2.0 ** -24, (float(error.max()), float(d[error.argmax()]))
+    for b in bufs + [out]:
+        b.free()
+
+
+def test_chunk_scores_that_are_not_finite(gpu_ctx):
+    """A NaN among a row's scores makes that row NaN, one at -inf counts as nothing, and rows whose
+    differences overflow f32 keep the maximum's value alone."""
+    m, depth = 20, 64
+    rng = np.random.default_rng(5)
+    q = np.zeros((1, 1, m, depth), dtype=np.float32)
+    q[0, 0, :, 0] = 1.0
+    ins_k = np.zeros((1, 1, m, depth), dtype=np.float32)
+    ins_v = rng.normal(size=ins_k.shape).astype(np.float32)
+    ins_k[0, 0, 0, 0] = 3e38
+    ins_k[0, 0, 1, 0] = -3e38         # a difference of -6e38: -inf
+    ins_k[0, 0, 2, 0] = -np.inf
+    ins_k[0, 0, 10, 0] = np.nan
+    slots = [np.zeros((1, 1, 32, depth), dtype=np.float32) for _ in range(2)]
+    bufs = [gpu_ctx.upload(a) for a in (q, ins_k, ins_v, *slots)]
+    out = gpu_ctx.alloc(q.nbytes)
+    gpu_ctx.attention_chunk(*bufs, out, batch=1, heads=1, kv_heads=1, chunk_rows=m, depth=depth,
+                            capacity=32, window=0, half_scale=1.0, past=0, query=m)
+    got = out.download(np.float32, (m, depth))
+    assert np.array_equal(got[:10], np.repeat(ins_v[0, 0, :1], 10, axis=0))
+    assert np.isnan(got[10:]).all()
+    for b in bufs + [out]:
+        b.free()
