@@ -1007,6 +1007,14 @@ void attention_decode_kernel(
     }
   }
 
+  // (this step's rows may start at any element: 16 bytes at once, but not 16-byte aligned)
+  struct __attribute__((packed, aligned(2))) ElementAligned {
+    uint32_t x, y, z, w;
+  };
+  auto load_own = [](const XT* p) {
+    const ElementAligned v = *reinterpret_cast<const ElementAligned*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+  };
   // B operand of the score MFMAs: lane (n = lane % 16, g = lane / 16) holds head n's query at
   // dims 32t + 8g.. as raw fp16 (exact products; the scale is applied to the f32 score)
   half8_t qb[kMfma ? 4 : 1];
@@ -1017,8 +1025,8 @@ void attention_decode_kernel(
   if constexpr (kMfma) {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
-      own_k[t] = *reinterpret_cast<const half8_t*>(ins_k + ins_base + 32 * t + 8 * frag_g);
-    own_v = *reinterpret_cast<const uint4*>(ins_v + ins_base + sub * E);
+      own_k[t] = __builtin_bit_cast(half8_t, load_own(ins_k + ins_base + 32 * t + 8 * frag_g));
+    own_v = load_own(ins_v + ins_base + sub * E);
     const int n = tid & 15, g = (tid & 63) >> 4;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {

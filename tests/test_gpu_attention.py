@@ -877,3 +877,39 @@ def test_chunk_scores_that_are_not_finite(gpu_ctx):
     assert np.isnan(got[10:]).all()
     for b in bufs + [out]:
         b.free()
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3, 7])
+@pytest.mark.parametrize("past", [3, 300])
+def test_decode_takes_this_steps_rows_at_any_element(gpu_ctx, shift, past):
+    """ins_k and ins_v need the alignment of an element only: rows that start `shift` elements into
+    their buffers give the bits of aligned ones, in both the single and the ragged form."""
+    heads, kv_heads, depth, cap = 8, 2, 128, 320
+    rng = np.random.default_rng(shift + past)
+    half = lambda *s: rng.normal(size=s).astype(np.float16)  # noqa: E731
+    q, slot_k, slot_v = half(heads, depth), half(kv_heads, cap, depth), half(kv_heads, cap, depth)
+    ins = [half(kv_heads, depth), half(kv_heads, depth)]
+    pad = lambda a: np.concatenate([np.full(shift, np.nan, np.float16), a.reshape(-1)])  # noqa: E731
+    dq, dk, dv = (gpu_ctx.upload(a) for a in (q, slot_k, slot_v))
+    plain = [gpu_ctx.upload(a) for a in ins]
+    moved = [gpu_ctx.upload(pad(a)) for a in ins]
+    out = gpu_ctx.alloc(q.nbytes)
+    ws = gpu_ctx.alloc(max(gpu_ctx.attention_varlen_workspace(1, heads, kv_heads, depth, cap),
+                           gpu_ctx.attention_state_workspace(1, heads, kv_heads, 1, depth, 0, cap)))
+    scale = oracle.half_scale(depth)
+    results = []
+    for k, v in (plain, [b.offset(2 * shift) for b in moved]):
+        gpu_ctx.attention_state(dq, k, v, dk, dv, out, batch=1, heads=heads, kv_heads=kv_heads,
+                                chunk_rows=1, depth=depth, capacity=cap, window=0,
+                                half_scale=scale, past=past, query=1, io_dtype=ka.F16,
+                                kv_dtype=ka.F16, workspace=ws)
+        results.append(out.download(np.uint16, (heads, depth)))
+        gpu_ctx.attention_varlen(dq, k, v, dk, dv, out, np.array([0, past], np.int32), heads=heads,
+                                 kv_heads=kv_heads, depth=depth, total_rows=cap, half_scale=scale,
+                                 io_dtype=ka.F16, kv_dtype=ka.F16, workspace=ws)
+        results.append(out.download(np.uint16, (heads, depth)))
+    assert np.isfinite(results[0].view(np.float16)).all()
+    for other in results[1:]:
+        assert np.array_equal(results[0], other)
+    for b in [dq, dk, dv, out, ws] + plain + moved:
+        b.free()
