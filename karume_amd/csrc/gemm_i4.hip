@@ -1268,7 +1268,7 @@ void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ 
   }
 }
 
-// The deal of the 64 x 512 tiles: one workgroup per CU, every workgroup at least two stages.
+// The deal of the 64 x 512 tiles: one workgroup per CU, every workgroup at least twelve stages.
 bool plan_exact_deal(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, bool split, uint32_t& grid,
                      UnitDeal& deal) {
   const uint64_t cus = (uint64_t)ctx->num_cus;
@@ -1281,6 +1281,12 @@ bool plan_exact_deal(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, bool spli
   // there, 138 us here; 512 x 11008 x 4096: 138 and 126 us).
   if (tiles > kTicketSlots || units > 0x7fffffffull || units < 12 * cus) return false;
   if (split && k > n) return false;
+  // Up to six 32 x 32 tiles of output a CU stay with the tiles that split K inside a workgroup, which
+  // need no scratch with fp16 operands (a side branch of a graph may hold them) and give a row the
+  // same bits whatever M is.  fp16, us there / here: 128 x 12288 x 8192 41.9 / 52.2, 256 x 4096 x 12288
+  // 39.8 / 48.2, 96 x 8192 x 16384 55.9 / 60.3, 192 x 8192 x 8192 48.8 / 47.7, but 384 x 4096 x 16384
+  // 98 / 78.
+  if ((uint64_t)((m + 31) / 32) * ((n + 31) / 32) <= 6 * cus) return false;
   if (tiles * 8 < cus) return false;  // a tile shared by more than eight workgroups
   if (!ctx->gemm_partials) return false;
   grid = (uint32_t)cus;

@@ -92,3 +92,32 @@ def test_scratch_users_are_rejected_on_a_side_branch(gpu_ctx):
     rec.graph.destroy()
     for b in list(bufs.values()) + [out, ws, dx, dw, ds, dout]:
         b.free()
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 12288, 8192), (64, 16400, 12288)])
+def test_long_products_of_few_tiles_need_no_scratch_and_no_batch(gpu_ctx, m, n, k):
+    """fp16 products of at most six 32 x 32 output tiles a CU, K long enough for the unit-dealt form:
+    a side branch takes them, and a row has the same bits in the whole batch, in a part of it and
+    in the replayed graph."""
+    ctx, g = gpu_ctx, 128
+    rng = np.random.default_rng(n)
+    packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    scale = rng.uniform(0.01, 0.03, size=(n, k // g)).astype(np.float16)
+    x = rng.normal(size=(m, k)).astype(np.float16)
+    dx, dw, ds, out = ctx.upload(x), ctx.upload(packed), ctx.upload(scale), ctx.alloc(m * n * 2)
+    call = lambda rows: ctx.linear_i4(dx, dw, ds, None, out, rows, n, k, g, ka.F16, ka.F16)  # noqa: E731
+    call(m)
+    whole = out.download(np.uint16, (m, n))
+    assert np.isfinite(whole.view(np.float16)).all() and whole.any()
+    call(17)
+    assert np.array_equal(out.download(np.uint16, (17, n)), whole[:17])
+    with ctx.record() as rec:
+        rec.branch(1)
+        call(m)
+    for _ in range(3):
+        out.zero()
+        rec.graph.launch()
+        assert np.array_equal(out.download(np.uint16, (m, n)), whole)
+    rec.graph.destroy()
+    for b in (dx, dw, ds, out):
+        b.free()
