@@ -52,20 +52,21 @@ typedef struct krm_event krm_event;
 /* `linear` arithmetic, the reference's SessionOptions.linearCompute
  * (packages/runtime/src/runtime/session-types.ts:127-195).  M <= 16 always runs the
  * bandwidth-bound GEMV (exact products, f32 accumulation).  For M > 16:
- *   KRM_COMPUTE_F32  — f32-class results for every M (the reference default).  f32 activations
- *                      on large shapes run on the matrix cores: x * 2^e = hi + lo (two fp16,
- *                      22 bits, e per row), weights as the exact integers (u - 8), products
- *                      exact, f32 sums, the group scale applied to the f32 sum of each group;
- *                      gated at the GEMV's tolerance.  fp16 activations need no split.  Other
- *                      shapes take the GEMV over blocks of 16 rows.
- *   KRM_COMPUTE_F16  — f32 activations are rounded to fp16 once.  Large shapes (the (tile,
- *                      stage) units of 64 x 512 tiles cover every CU at least twice, group >= 64,
- *                      k % 32 == 0): exact integer weights as above, so with fp16 activations
- *                      the result is of f32 class.  Smaller shapes: every weight rounded once
- *                      to fp16((u - 8) * scale), which bounds an output's error by about
- *                      2^-11 * sqrt(k) * rms(x * w).  (The reference rejects f16 compute with
- *                      i4 weights, packages/runtime/src/kernels/gemm.ts:1204-1209: no
- *                      same-numerics counterpart there.) */
+ *   KRM_COMPUTE_F32  — f32-class results for every M (the reference default).  With K a multiple of
+ *                      32 the products run on the matrix cores: weights as the exact integers
+ *                      (u - 8), products exact, f32 sums, the group scale applied to the f32 sum
+ *                      of each group; gated at the GEMV's tolerance.  f32 activations enter in
+ *                      groups of 64 and more as x * 2^e = hi + lo (two fp16, 22 bits, e per
+ *                      row: entries below 2^-15 of their row's largest keep fewer), in groups of
+ *                      16 and 32 with all their bits (three bf16); fp16 activations need no
+ *                      split.  Other shapes take the GEMV over blocks of 16 rows.
+ *   KRM_COMPUTE_F16  — f32 activations are rounded to fp16 once.  With K a multiple of 32: exact
+ *                      integer weights as above, so with fp16 activations the result is of f32
+ *                      class.  Other shapes: every weight rounded once to fp16((u - 8) * scale),
+ *                      which bounds an output's error by about 2^-11 * sqrt(k) * rms(x * w).
+ *                      (The reference rejects f16 compute with i4 weights,
+ *                      packages/runtime/src/kernels/gemm.ts:1204-1209: no same-numerics
+ *                      counterpart there.) */
 #define KRM_COMPUTE_F32 0
 #define KRM_COMPUTE_F16 1
 
@@ -132,7 +133,8 @@ int32_t krm_graph_begin(krm_ctx* ctx);
  * main branch; while a side branch is selected they fail with KRM_ERR_VALIDATION and record
  * nothing: the decode attention when it splits the columns (more than four chunks),
  * krm_attention_varlen / _planned, the unit-dealt MFMA GEMMs of krm_linear_i4 (never with up to six
- * 32 x 32 tiles of output a CU) and every f32-class (KRM_COMPUTE_F32 with f32 x) MFMA product.  GEMVs (m <= 16), the fp16-operand
+ * 32 x 32 tiles of output a CU) and every f32-class (KRM_COMPUTE_F32 with f32 x) MFMA product in
+ * groups of 64 and more.  GEMVs (m <= 16), the fp16-operand
  * few-row products, krm_attention_state_noalloc (its own scratch: still one call at a time per
  * GPU) and the glue ops carry no such state. */
 int32_t krm_graph_branch(krm_ctx* ctx, uint32_t branch);

@@ -4,11 +4,14 @@
 // (packages/runtime/src/kernels/linear.ts:34-64, packages/runtime/src/kernels/gemm.ts:1187-1237).
 // The weights enter the matrix cores as the exact integers (u - 8) in fp16, products are exact,
 // sums are f32 (v_mfma_f32_32x32x16_f16) and the group scale multiplies the f32 sum of each scale
-// group.  Three forms of x:
+// group.  Four forms of x:
 //   kX16     fp16 activations as they are;
 //   kX32     f32 activations, each rounded to fp16 once where it is read from LDS;
 //   kXSplit  f32 activations as x * 2^e = hi + lo (both fp16, e per row), written once per call
-//            by split_rows_kernel below: two matrix instructions a step, 22 bits of x.
+//            by split_rows_kernel below: two matrix instructions a step, 22 bits of x;
+//   kXThree  f32 activations with all their bits, groups of 16 and 32: x = t1 + t2 + t3, each the
+//            next 8 bits as a bf16, taken where x is read from LDS: three matrix instructions a
+//            step, no scratch, no pass ahead and no exponent that a row's entries would share.
 //
 // A workgroup owns a tile of 32 MT rows x 32 NT columns; its eight waves take an eighth of K each
 // and run on their own: a wave streams its slice of x and of the packed weights from memory
@@ -27,8 +30,15 @@
 // Measured on cold weights, fp16 x (f32 class in brackets), against the kernel that loaded through
 // registers, one 32 x 32 or 32 x 64 tile a workgroup: 128 x 2560 x 2048 6.6 us, 9.6 before (11.8,
 // 14.5); 128 x 2048 x 2048 5.4, 7.0 (10.1, 12.5); 128 x 11264 x 2048 15.1, 27.0 (25.9, 38.6); 128 x
-// 2048 x 5632 10.6, 13.0 (19.7, 26.2); 77 x 3000 x 2080 with groups of 32 in the f32 class 13.8 us,
-// 221 before (sixteen rows at a time through the GEMV).
+// 2048 x 5632 10.6, 13.0 (19.7, 26.2).
+//
+// kXThree is bounded by the vector ALUs (11 operations a pair of x, 14 a word of weights, both at
+// every step).  Groups of 32, against the GEMV over blocks of 16 rows (in brackets: hi + lo planes,
+// which lost the small entries of a row beside a large one): 77 x 3000 x 2080 14.6 us, 210 (14.1); 17
+// rows of it 10.2, 45.5 (10.2); 128 x 2048 x 2048 11.3, 156 (12.0); 512 x 4096 x 4096 92, 1969 (81);
+// 512 x 11008 x 4096 255, 5594 (213); in groups of 16 380, 2427 (330).  Error against 64 bits (2-norm,
+// normal x): 77 x 3000 x 2080 in groups of 32 9.5e-8, the GEMV 1.24e-7; 40 x 1000 x 4096 in groups of
+// 16 1.04e-7 and 1.05e-7; 300 x 512 x 11008 in groups of 32 1.21e-7 and 1.33e-7.
 #include "krm_internal.h"
 
 #include <type_traits>
@@ -39,9 +49,10 @@ namespace {
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kX16 = 0, kXSplit = 1, kX32 = 2;
+constexpr int kX16 = 0, kXSplit = 1, kX32 = 2, kXThree = 3;
 constexpr int kWaves = 8;
 
 template <typename T>
@@ -97,6 +108,61 @@ __device__ inline half8_t ints_natural(uint32_t word) {
     q[i] = __builtin_elementwise_fma(
         __builtin_bit_cast(half2_t, and_or(twice[i], 0x00F0000Fu, magic)), factor, offset);
   return half8_t{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+}
+
+// The high halves of two f32 as a pair of bf16.
+__device__ inline uint32_t high_pair(uint32_t even, uint32_t odd) {
+  return __builtin_amdgcn_perm(odd, even, 0x07060302u);
+}
+// 8 codes of a word -> 8 bf16 (u - 8) / 16, exact, natural order (a 4-bit integer with its sign is
+// what v_cvt_off_f32_i4 takes; the sum over K is multiplied by 16 at the end).
+__device__ inline half8_t sixteenths(uint32_t word) {
+  const uint32_t even = word ^ 0x88888888u, odd = even >> 4;
+  uint32_t v[8];  // (a byte of a register is an operand: no shift of its own)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[2 * i] = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((int)((even >> (8 * i)) & 0xffu)));
+    v[2 * i + 1] = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((int)((odd >> (8 * i)) & 0xffu)));
+  }
+  return __builtin_bit_cast(half8_t, make_uint4(high_pair(v[0], v[1]), high_pair(v[2], v[3]),
+                                                high_pair(v[4], v[5]), high_pair(v[6], v[7])));
+}
+// 8 f32 -> three times 8 bf16 whose sum they are, every part the leading 8 bits of what is left.
+// (Cut off, not rounded: the first part of the largest f32 stays finite.)  An infinity is its own
+// first part; the rest of it would be inf - inf.
+__device__ inline void three_parts(const float (&x)[8], half8_t (&part)[3]) {
+  uint32_t bits[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) bits[i] = __float_as_uint(x[i]);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    part[p] = __builtin_bit_cast(
+        half8_t, make_uint4(high_pair(bits[0], bits[1]), high_pair(bits[2], bits[3]),
+                            high_pair(bits[4], bits[5]), high_pair(bits[6], bits[7])));
+    if (p == 2) break;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      bits[i] = __float_as_uint(__uint_as_float(bits[i]) - __uint_as_float(bits[i] & 0xffff0000u));
+    if (p == 0) {
+      float top = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) top = fmaxf(top, fabsf(x[i]));
+      if (__any(top == INFINITY)) {
+        asm volatile("");  // (a branch that is hardly ever taken, not selects in every step)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (fabsf(x[i]) == INFINITY) bits[i] = 0u;
+      }
+    }
+  }
+}
+template <int XKIND>
+__device__ inline float16_t product(const half8_t& a, const half8_t& b, const float16_t& sum) {
+  if constexpr (XKIND == kXThree)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), sum, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, sum, 0, 0, 0);
 }
 
 // ------------------------------------------------------------------- memory -> LDS, counted waits
@@ -278,7 +344,10 @@ struct SliceTail {         // what the end of the kernel needs
 // groups of 128 and more), or 4, 2, 1 (blocks of 64 codes, groups of 64, 32, 16).
 template <int XKIND, int MT, int NT, int STEPS>
 struct SliceGeometry {
-  static constexpr int kPlanes = XKIND == kXSplit ? 2 : 1;
+  static constexpr int kPlanes = XKIND == kXThree ? 3 : XKIND == kXSplit ? 2 : 1;
+  // Two running totals, groups in turn, where x keeps its bits: a sum's rounding then acts on half as
+  // much, and the error against 64 bits is not above that of the GEMV over blocks of 16 rows.
+  static constexpr int kTotals = XKIND == kXThree ? 2 : 1;
   static constexpr int kArea = 20 * 1024;            // a wave's share of the LDS
   // An x stage holds whole 128-byte lines where the LDS has room: what the second-level cache
   // delivers counts lines and half lines alike (127 GB/s a CU in 128-byte segments, 80 in 64-byte,
@@ -315,7 +384,7 @@ template <int XKIND, int MT, int NT, int STEPS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_i4_slices_kernel(
     // (the leading 14 dwords of the arguments arrive in scalar registers with the wave)
-    const uint8_t* __restrict__ x,  // kX16 / kX32: [m][k]; kXSplit: [m][k / 32][hi, lo][32] fp16
+    const uint8_t* __restrict__ x,  // [m][k], but kXSplit: [m][k / 32][hi, lo][32] fp16
     const uint8_t* __restrict__ w, const uint8_t* __restrict__ scales, uint32_t row_begin,
     uint32_t row_end, uint32_t n, uint32_t k, uint32_t group_shift, uint32_t m_blocks, uint32_t tiles, uint32_t scale_f16_arg,
     uint32_t io_f16, uint32_t m, SliceTail tail) {
@@ -439,14 +508,18 @@ void gemm_i4_slices_kernel(
     }
   };
 
-  float16_t total[MT][NT], acc[MT][NT];
+  float16_t total[G::kTotals][MT][NT], acc[MT][NT];
   float16_t zero16;
 #pragma unroll
   for (int r = 0; r < 16; ++r) zero16[r] = 0.f;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) total[mt][nt] = acc[mt][nt] = zero16;
+    for (int nt = 0; nt < NT; ++nt) {
+      acc[mt][nt] = zero16;
+#pragma unroll
+      for (int i = 0; i < G::kTotals; ++i) total[i][mt][nt] = zero16;
+    }
 
   // fragment addresses inside a stage / a unit.  Step j of 32 codes covers the 8-code pieces
   // 2 h + j (one 8-byte read of weights); groups of 16 need the two pieces of a step next to each
@@ -457,7 +530,8 @@ void gemm_i4_slices_kernel(
       area + DX * G::kXBytes + frag_row * (16 * kPieces) + (STEPS == 1 ? 4u : 8u) * frag_h;
   const uint32_t w_turn = w_turn_of(frag_row);
 
-  auto flush = [&](uint32_t unit_slot, int e) {
+  auto flush = [&](uint32_t unit_slot, int e, int turn) {
+    auto& to = total[turn % G::kTotals];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       uint32_t bits;
@@ -472,13 +546,14 @@ void gemm_i4_slices_kernel(
       for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          total[mt][nt][r] = fmaf(acc[mt][nt][r], s, total[mt][nt][r]);
+          to[mt][nt][r] = fmaf(acc[mt][nt][r], s, to[mt][nt][r]);
     }
   };
   // 32 codes: quarter `wq` of the weight unit in slot `unit_slot`, half `xq` of the stage in slot
   // `slot`; `opens`: the first step starts a scale group (its sums start from zero); `e`: the
-  // unit's scale entry (half of 64 codes) for groups below 64
-  auto half = [&](uint32_t unit_slot, uint32_t wq, uint32_t slot, int xq, bool opens, int e) {
+  // unit's scale entry (half of 64 codes) for groups below 64, added to the totals of `turn`
+  auto half = [&](uint32_t unit_slot, uint32_t wq, uint32_t slot, int xq, bool opens, int e,
+                  int turn) {
     const uint8_t* xs = x_frag + slot * G::kXBytes;
     const uint8_t* ws = w_frag + unit_slot * G::kWBytes + ((wq ^ w_turn) * 16u);
     uint2 words[NT];
@@ -499,11 +574,19 @@ void gemm_i4_slices_kernel(
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         const uint8_t* row = xs + mt * (32 * kRowBytes);
-        if constexpr (XKIND == kX32) {
+        if constexpr (XKIND == kX32 || XKIND == kXThree) {
           const float4 lo = *reinterpret_cast<const float4*>(row + (((2u * piece) ^ x_turn) * 16u));
           const float4 hi = *reinterpret_cast<const float4*>(row + (((2u * piece + 1u) ^ x_turn) * 16u));
-          a[0][mt] = half8_t{(_Float16)lo.x, (_Float16)lo.y, (_Float16)lo.z, (_Float16)lo.w,
-                             (_Float16)hi.x, (_Float16)hi.y, (_Float16)hi.z, (_Float16)hi.w};
+          if constexpr (XKIND == kXThree) {
+            const float eight[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            half8_t part[3];
+            three_parts(eight, part);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) a[p][mt] = part[p];
+          } else {
+            a[0][mt] = half8_t{(_Float16)lo.x, (_Float16)lo.y, (_Float16)lo.z, (_Float16)lo.w,
+                               (_Float16)hi.x, (_Float16)hi.y, (_Float16)hi.z, (_Float16)hi.w};
+          }
         } else {
 #pragma unroll
           for (int p = 0; p < kPlanes; ++p)
@@ -514,19 +597,19 @@ void gemm_i4_slices_kernel(
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const uint32_t word = j == 0 ? words[nt].x : words[nt].y;
-        const half8_t b = XKIND == kXSplit ? ints_paired(word) : ints_natural(word);
+        const half8_t b = XKIND == kXThree ? sixteenths(word)
+                          : XKIND == kXSplit ? ints_paired(word) : ints_natural(word);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int p = 0; p < kPlanes; ++p) {
             const bool zero = p == 0 && (STEPS == 1 || (j == 0 && opens));
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                a[p][mt], b, zero ? zero16 : acc[mt][nt], 0, 0, 0);
+            acc[mt][nt] = product<XKIND>(a[p][mt], b, zero ? zero16 : acc[mt][nt]);
           }
       }
-      if constexpr (STEPS == 1) flush(unit_slot, 2 * e + j);
+      if constexpr (STEPS == 1) flush(unit_slot, 2 * e + j, j);
     }
-    if constexpr (STEPS == 2) flush(unit_slot, e);
+    if constexpr (STEPS == 2) flush(unit_slot, e, turn);
   };
   constexpr int kRegScales = STEPS == 8 ? NT : 0;  // loads of a block's scales
 
@@ -573,13 +656,13 @@ void gemm_i4_slices_kernel(
           const uint32_t unit_slot = g / R % DW, slot = g % DX, wq = (g % R) * (kStage / 32);
           if constexpr (kStage == 64) {
             const bool early = ends_early && g + 1 == stages;
-            if (!early) half(unit_slot, wq, slot, 0, i == 0, 0);
-            half(unit_slot, wq + 1, slot, 1, STEPS <= 2, 1);
+            if (!early) half(unit_slot, wq, slot, 0, i == 0, 0, 0);
+            half(unit_slot, wq + 1, slot, 1, STEPS <= 2, 1, 1);
           } else {
             const bool early = ends_early && g + 1 == stages;  // the last 64 codes: second half
-            half(unit_slot, early ? 1u : wq, slot, 0, STEPS <= 2 || i == 0, early ? 1 : i % 2);
+            half(unit_slot, early ? 1u : wq, slot, 0, STEPS <= 2 || i == 0, early ? 1 : i % 2, i);
           }
-          if constexpr (STEPS == 4) { if (i == kStages - 1) flush(unit_slot, 0); }
+          if constexpr (STEPS == 4) { if (i == kStages - 1) flush(unit_slot, 0, 0); }
           // the reads of a slot are over before it is filled again
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
@@ -592,7 +675,7 @@ void gemm_i4_slices_kernel(
         }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(scale_raw[nt])::"memory");
-        flush(0, 0);
+        flush(0, 0, 0);
       }
     }
   }
@@ -614,7 +697,8 @@ void gemm_i4_slices_kernel(
 #pragma unroll
           for (int r = 0; r < 16; ++r)
             sums[(mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4)) * kCols + t * 32 + frag_row] =
-                total[mt][t0 + t][r];
+                G::kTotals == 2 ? total[0][mt][t0 + t][r] + total[G::kTotals - 1][mt][t0 + t][r]
+                                : total[0][mt][t0 + t][r];
       }
     __syncthreads();
     auto finish = [&](auto type_tag) {
@@ -626,17 +710,30 @@ void gemm_i4_slices_kernel(
         const int local = p / quads, c4 = p % quads;
         const uint32_t row = m0 + local, col = n0 + 32u * t0 + 4u * c4;
         if ((work % 512 == 0 || p < work) && row < row_end && col < n) {
-          float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+          float4 part[kWaves];
 #pragma unroll
-          for (int wv = 0; wv < kWaves; ++wv) {
-            const float4 part =
+          for (int wv = 0; wv < kWaves; ++wv)
+            part[wv] =
                 *reinterpret_cast<const float4*>(s_area[wv] + (size_t)(local * kCols + 4 * c4) * 4);
-            v.x += part.x; v.y += part.y; v.z += part.z; v.w += part.w;
+          auto add = [](float4& to, const float4& v) {
+            to.x += v.x; to.y += v.y; to.z += v.z; to.w += v.w;
+          };
+          float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+          if constexpr (XKIND == kXThree) {  // in pairs: three roundings of a whole sum, not seven
+#pragma unroll
+            for (int step = 1; step < kWaves; step *= 2)
+#pragma unroll
+              for (int wv = 0; wv < kWaves; wv += 2 * step) add(part[wv], part[wv + step]);
+            v = part[0];
+          } else {
+#pragma unroll
+            for (int wv = 0; wv < kWaves; ++wv) add(v, part[wv]);
           }
           if constexpr (XKIND == kXSplit) {  // exact: a power of two
             const float inv = tail.row_scale[2 * (size_t)row + 1];
             v.x *= inv; v.y *= inv; v.z *= inv; v.w *= inv;
           }
+          if constexpr (XKIND == kXThree) { v.x *= 16.f; v.y *= 16.f; v.z *= 16.f; v.w *= 16.f; }
           finish_pair<T>(v.x, v.y, row, col, m, n, static_cast<const T*>(tail.bias),
                          static_cast<T*>(tail.out), tail.fuse);
           if (col + 2 < n)
@@ -679,13 +776,15 @@ constexpr TileCost kCost16[] = {{1, 1, 0.8f, 1.5f}, {1, 2, 1.3f, 2.0f}, {1, 3, 1
                                 {2, 1, 0.7f, 2.0f}, {2, 2, 2.4f, 2.6f}, {2, 3, 2.2f, 3.6f}};
 constexpr TileCost kCostSplit[] = {{1, 1, 0.2f, 2.45f}, {1, 2, 0.4f, 2.9f}, {1, 3, 0.9f, 3.4f},
                                    {2, 1, 0.2f, 3.5f}, {2, 2, 1.0f, 4.5f}};
+constexpr TileCost kCostThree[] = {{1, 1, 3.2f, 3.35f}, {1, 2, 4.8f, 4.65f}, {2, 1, 4.6f, 4.97f}};
 constexpr TileCost kCost32[] = {{1, 1, 0.8f, 1.75f}, {1, 2, 1.3f, 2.3f}, {1, 3, 1.7f, 2.9f},
                                 {2, 1, 0.7f, 2.75f}, {2, 2, 2.2f, 3.3f}};
 
 template <int XKIND, int STEPS>
 int32_t pick_tile(krm_ctx* ctx, const SliceCall& c) {
-  const TileCost* table = XKIND == kX16 ? kCost16 : XKIND == kXSplit ? kCostSplit : kCost32;
-  const int count = XKIND == kX16 ? 6 : 5;
+  const TileCost* table = XKIND == kX16 ? kCost16 : XKIND == kXSplit ? kCostSplit
+                          : XKIND == kXThree ? kCostThree : kCost32;
+  const int count = XKIND == kX16 ? 6 : XKIND == kXThree ? 3 : 5;
   const uint64_t cus = (uint64_t)ctx->num_cus, rows = c.row_end - c.row_begin;
   int best = 0;
   float best_cost = 0.f;
@@ -721,10 +820,14 @@ int32_t pick_tile(krm_ctx* ctx, const SliceCall& c) {
 
 template <int XKIND>
 int32_t pick_steps(krm_ctx* ctx, const SliceCall& c) {
-  if (c.group_shift >= 7) return pick_tile<XKIND, 8>(ctx, c);
-  if (c.group_shift == 6) return pick_tile<XKIND, 4>(ctx, c);
-  if (c.group_shift == 5) return pick_tile<XKIND, 2>(ctx, c);
-  return pick_tile<XKIND, 1>(ctx, c);
+  if constexpr (XKIND != kXThree) {
+    if (c.group_shift >= 7) return pick_tile<XKIND, 8>(ctx, c);
+    if (c.group_shift == 6) return pick_tile<XKIND, 4>(ctx, c);
+  }
+  if constexpr (XKIND == kXSplit)
+    return fail(ctx, KRM_ERR_VALIDATION, "linear: hi + lo planes need groups of 64 and more");
+  else
+    return c.group_shift == 5 ? pick_tile<XKIND, 2>(ctx, c) : pick_tile<XKIND, 1>(ctx, c);
 }
 
 }  // namespace
@@ -761,12 +864,14 @@ int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales
     *handled = true;
     return x_dtype == KRM_F16 ? pick_steps<kX16>(ctx, c) : pick_steps<kX32>(ctx, c);
   }
+  if (group < 64) {
+    *handled = true;
+    return pick_steps<kXThree>(ctx, c);
+  }
   // hi and lo of as many rows as the context's scratch holds at a time
   const uint64_t scratch = (uint64_t)2 * ctx->num_cus * kGemmPartialBytes, row_bytes = (uint64_t)k * 4;
   const uint64_t fit = scratch / row_bytes / 32 * 32;
   if (m > kMaxSplitRows || fit == 0) return KRM_OK;
-  // (groups below 64 codes have a form without scratch, which a side branch may record)
-  if (group < 64 && ctx->stream != ctx->main_stream) return KRM_OK;
   KRM_TRY(needs_serial_scratch(ctx, "the f32-class few-row GEMM"));
   *handled = true;
   c.tail.row_scale = ctx->row_scales;

@@ -391,3 +391,77 @@ def test_k_slices_kernel_at_the_edges_of_its_tiles(gpu_ctx, m, n, k, g, mode):
     if mode == "f16":
         bound = bound + 2.0 ** -11 * np.abs(want) + 1e-7
     assert np.all(err <= bound), float(np.max(err / bound))
+
+
+SMALL_GROUP_SHAPES = [(17, 33, 96, 32), (77, 300, 2080, 32), (100, 200, 2048, 16), (300, 2500, 512, 32)]
+
+
+@pytest.mark.parametrize("m,n,k,g", SMALL_GROUP_SHAPES)
+def test_small_groups_keep_entries_beside_an_outlier(gpu_ctx, m, n, k, g):
+    """The f32 class in groups of 16 and 32 takes every bit of x: entries of 1e-3 count in full
+    beside entries of 1e6 that meet a zero code.  The bound grows with what is summed, not with the
+    row's maximum: at most 64 roundings of 2^-24 act on a part of sum |x w| each (a wave's flushes,
+    the steps of a group, the waves' sums)."""
+    rng = np.random.default_rng(m + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    packed = packed.reshape(n, k // 2).copy()
+    at = np.arange(5, k, 3 * g)
+    packed[:, at // 2] = (packed[:, at // 2] & 0x0F) | 0x80     # odd columns: the high nibble, code 0
+    x = (rng.normal(size=(m, k)) * 1e-3).astype(np.float32)
+    x[:, at] = 1e6
+    got = run_linear(gpu_ctx, x, packed, scale, None, n, k, g)
+    codes = np.stack([packed & 15, packed >> 4], axis=-1).reshape(n, k).astype(np.float64) - 8.0
+    w = codes * np.repeat(scale.astype(np.float64).reshape(n, k // g), g, axis=1)
+    want, size = x.astype(np.float64) @ w.T, np.abs(x).astype(np.float64) @ np.abs(w).T
+    assert np.all(np.abs(got - want) <= 64 * 2.0 ** -24 * size), \
+        float(np.max(np.abs(got - want) / size))
+
+
+@pytest.mark.parametrize("m,n,k,g", SMALL_GROUP_SHAPES)
+def test_small_groups_give_what_the_gemv_gives_for_values_that_are_not_finite(gpu_ctx, m, n, k, g):
+    """Infinities (against codes of either sign and zero codes), two that cancel, a NaN whose payload
+    lies in its low bits, 1e37 (the largest f32 overflows the GEMV's sums), subnormals (whose parts
+    may count as zeros): the same rows, 16 at a time, run the GEMV."""
+    rng = np.random.default_rng(n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[0, 3] = np.inf
+    x[1, k - 1] = -np.inf
+    x[2, [1, k // 2]] = np.inf, -np.inf
+    x[3, 7] = np.array([0x7F800001], dtype=np.uint32).view(np.float32)[0]
+    x[4, 9] = 1e37
+    x[5] = 1e-42
+    got = run_linear(gpu_ctx, x, packed, scale, None, n, k, g)
+    want = run_linear(gpu_ctx, x[:16], packed, scale, None, n, k, g)
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(kind(got[:16]), kind(want)), kind.__name__
+    assert np.isfinite(got[16:]).all() and np.isfinite(got[4]).all()
+    finite = np.isfinite(want)
+    err = np.abs(got[:16].astype(np.float64) - want)[finite]
+    size = np.broadcast_to(np.abs(np.where(np.isfinite(x[:16]), x[:16], 0)).sum(1, keepdims=True)
+                           * 8.0 * float(np.abs(scale).max()), want.shape)[finite]
+    assert np.all(err <= 64 * 2.0 ** -24 * size + 1e-37)
+    if m > 22:     # a row's bits do not depend on the others
+        assert np.array_equal(got[6:], run_linear(gpu_ctx, x[6:], packed, scale, None, n, k, g))
+
+
+def test_small_groups_need_no_scratch(gpu_ctx):
+    """A side branch of a graph takes the f32 class in groups of 32, as it took the GEMV."""
+    ctx, (m, n, k, g) = gpu_ctx, SMALL_GROUP_SHAPES[1]
+    rng = np.random.default_rng(3)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    want = run_linear(ctx, x, packed, scale, None, n, k, g)
+    dx, dw, ds = ctx.upload(x), ctx.upload(packed), ctx.upload(np.ascontiguousarray(scale))
+    out = ctx.alloc(m * n * 4)
+    with ctx.record() as rec:
+        rec.branch(1)
+        ctx.linear_i4(dx, dw, ds, None, out, m, n, k, g, ka.F32, ka.dtype_code(scale.dtype),
+                      ka.COMPUTE_F32)
+    for _ in range(3):
+        out.zero()
+        rec.graph.launch()
+        assert np.array_equal(out.download(np.float32, (m, n)), want)
+    rec.graph.destroy()
+    for b in (dx, dw, ds, out):
+        b.free()
