@@ -132,9 +132,10 @@ int32_t krm_graph_begin(krm_ctx* ctx);
  * Ops that use the context's own scratch share it in launch order and therefore belong on the
  * main branch; while a side branch is selected they fail with KRM_ERR_VALIDATION and record
  * nothing: the decode attention when it splits the columns (more than four chunks),
- * krm_attention_varlen / _planned, the unit-dealt MFMA GEMMs of krm_linear_i4 (never with up to six
- * 32 x 32 tiles of output a CU) and every f32-class (KRM_COMPUTE_F32 with f32 x) MFMA product in
- * groups of 64 and more.  GEMVs (m <= 16), the fp16-operand
+ * krm_attention_varlen / _planned and every f32-class (KRM_COMPUTE_F32 with f32 x) MFMA product in
+ * groups of 64 and more.  krm_linear_i4 of fp16 operands whose large products share tiles through
+ * that scratch on the main branch takes the form without it on a side branch: the same class of
+ * result, other bits for more than six 32 x 32 tiles of output a CU.  GEMVs (m <= 16), the fp16-operand
  * few-row products, krm_attention_state_noalloc (its own scratch: still one call at a time per
  * GPU) and the glue ops carry no such state. */
 int32_t krm_graph_branch(krm_ctx* ctx, uint32_t branch);

@@ -1268,19 +1268,35 @@ void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ 
   }
 }
 
-// The deal of the 64 x 512 tiles: one workgroup per CU, every workgroup at least twelve stages.
-bool plan_exact_deal(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, bool split, uint32_t& grid,
-                     UnitDeal& deal) {
+// The deal of the 64 x 512 tiles: one workgroup per CU, every workgroup at least two stages.
+bool plan_exact_deal(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group, bool half_x,
+                     bool split, uint32_t& grid, UnitDeal& deal) {
   const uint64_t cus = (uint64_t)ctx->num_cus;
   const uint64_t tiles = (uint64_t)((m + 63) / 64) * ((n + 511) / 512);
   const uint32_t spt = (k + 127) / 128;
   const uint64_t units = tiles * spt;
-  // At least twelve stages a workgroup: below, the K-splitting tiles of gemm_i4_slices.hip win (256 x
-  // 11264 x 2048, 5.5 stages: 24.5 us there, 31.1 us here; 512 x 11008 x 4096, 21.5 stages: 81 us
-  // there, 64.6 us here).  In the split form the two meet for a long K (512 x 4096 x 11008: 122 us
-  // there, 138 us here; 512 x 11008 x 4096: 138 and 126 us).
-  if (tiles > kTicketSlots || units > 0x7fffffffull || units < 12 * cus) return false;
-  if (split && k > n) return false;
+  if (tiles > kTicketSlots || units > 0x7fffffffull || units < 2 * cus) return false;
+  if (units < 12 * cus) {
+    // Fewer than twelve stages a workgroup: the K-splitting tiles of gemm_i4_slices.hip, unless
+    // their estimate is clearly above this form's, {fixed, a stage} in us, fitted over 16 to 21 shapes
+    // (rms 6 to 8 %).  Over 100 shapes of 65 to 512 rows the choice is 1 % behind the better of the two
+    // and 4 % at worst behind the tiles alone.  us there / here: fp16 406 x 24848 x 512 in groups of 64 61 / 27, 198 x 26342 x 768 35 / 24, 237 x
+    // 7285 x 2688 in groups of 64 26 / 31; f32 rounded to fp16 399 x 26833 x 896 in groups of 64 115 /
+    // 57, 169 x 8597 x 1664 19 / 33; f32 class 470 x 23723 x 512 81 / 63, 190 x 11922 x 1920 30 / 55.
+    struct Fit {
+      float fixed, stage;
+    };
+    const bool wide_groups = group >= 128;
+    const Fit f = half_x ? (wide_groups ? Fit{14.1f, 2.45f} : Fit{14.7f, 2.6f})
+                  : split ? (wide_groups ? Fit{36.3f, 4.0f} : Fit{37.3f, 4.0f})
+                          : (wide_groups ? Fit{19.8f, 2.7f} : Fit{20.6f, 3.1f});
+    const float here = f.fixed + f.stage * ((float)units / (float)cus);
+    if (here > 0.88f * slices_estimate_us(ctx, m, n, k, group, half_x, split)) return false;
+  } else if (split && k > n) {
+    // In the f32 class the two meet for a long K (512 x 4096 x 11008: 122 us there, 138 us here; 512 x
+    // 11008 x 4096: 138 and 126 us).
+    return false;
+  }
   // Up to six 32 x 32 tiles of output a CU stay with the tiles that split K inside a workgroup, which
   // need no scratch with fp16 operands (a side branch of a graph may hold them) and give a row the
   // same bits whatever M is.  fp16, us there / here: 128 x 12288 x 8192 41.9 / 52.2, 256 x 4096 x 12288
@@ -1448,7 +1464,10 @@ int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
   if (split && (m > kMaxSplitRows || !ctx->row_scales)) return KRM_OK;
   uint32_t grid = 0;
   UnitDeal deal{};
-  if (!plan_exact_deal(ctx, m, n, k, split, grid, deal)) return KRM_OK;
+  // (a side branch of a graph has no scratch: there the K-splitting tiles, which need none with fp16
+  // operands, take these shapes too)
+  if (!split && ctx->stream != ctx->main_stream) return KRM_OK;
+  if (!plan_exact_deal(ctx, m, n, k, group, io_dtype == KRM_F16, split, grid, deal)) return KRM_OK;
   uint32_t group_shift = 0;
   while ((1u << group_shift) < group) ++group_shift;
   *handled = true;

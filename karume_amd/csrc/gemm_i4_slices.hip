@@ -780,12 +780,13 @@ constexpr TileCost kCostThree[] = {{1, 1, 3.2f, 3.35f}, {1, 2, 4.8f, 4.65f}, {2,
 constexpr TileCost kCost32[] = {{1, 1, 0.8f, 1.75f}, {1, 2, 1.3f, 2.3f}, {1, 3, 1.7f, 2.9f},
                                 {2, 1, 0.7f, 2.75f}, {2, 2, 2.2f, 3.3f}};
 
+// The cheapest tile of a shape, and its rounds over the CUs.
 template <int XKIND, int STEPS>
-int32_t pick_tile(krm_ctx* ctx, const SliceCall& c) {
+TileCost cheapest_tile(const krm_ctx* ctx, uint64_t rows, uint32_t n, uint32_t k, uint64_t* rounds) {
   const TileCost* table = XKIND == kX16 ? kCost16 : XKIND == kXSplit ? kCostSplit
                           : XKIND == kXThree ? kCostThree : kCost32;
   const int count = XKIND == kX16 ? 6 : XKIND == kXThree ? 3 : 5;
-  const uint64_t cus = (uint64_t)ctx->num_cus, rows = c.row_end - c.row_begin;
+  const uint64_t cus = (uint64_t)ctx->num_cus;
   int best = 0;
   float best_cost = 0.f;
   for (int i = 0; i < count; ++i) {
@@ -794,14 +795,23 @@ int32_t pick_tile(krm_ctx* ctx, const SliceCall& c) {
     if ((STEPS < 8 && t.nt > 2) || (STEPS < 8 && t.mt * t.nt > 2 && XKIND != kX16) ||
         (STEPS == 1 && t.mt * t.nt > 1))
       continue;
-    const uint64_t tiles = ((rows + 32 * t.mt - 1) / (32 * t.mt)) * (((uint64_t)c.n + 32 * t.nt - 1) / (32 * t.nt));
-    const float cost = (float)((tiles + cus - 1) / cus) * (t.fixed + t.per_1024 * (float)c.k * (1.0f / 1024));
+    const uint64_t tiles = ((rows + 32 * t.mt - 1) / (32 * t.mt)) * (((uint64_t)n + 32 * t.nt - 1) / (32 * t.nt));
+    const uint64_t turns = (tiles + cus - 1) / cus;
+    const float cost = (float)turns * (t.fixed + t.per_1024 * (float)k * (1.0f / 1024));
     if (i == 0 || cost < best_cost) {
       best = i;
       best_cost = cost;
+      *rounds = turns;
     }
   }
-  const int tile = table[best].mt * 10 + table[best].nt;
+  return table[best];
+}
+
+template <int XKIND, int STEPS>
+int32_t pick_tile(krm_ctx* ctx, const SliceCall& c) {
+  uint64_t rounds = 0;
+  const TileCost best = cheapest_tile<XKIND, STEPS>(ctx, c.row_end - c.row_begin, c.n, c.k, &rounds);
+  const int tile = best.mt * 10 + best.nt;
   if constexpr (STEPS == 8 && XKIND == kX16) {
     if (tile == 23) return launch_slices<XKIND, 2, 3, STEPS>(ctx, c);
   }
@@ -833,6 +843,32 @@ int32_t pick_steps(krm_ctx* ctx, const SliceCall& c) {
 }  // namespace
 
 namespace krm {
+
+// Microseconds of a call over more rounds than one, for the choice against the unit-dealt form of
+// gemm_i4.hip (groups of 64 and more).  The costs above choose between tiles; a round's absolute time
+// is {per call, more per round, factor of the part in K}, fitted over 17 to 33 shapes of 65 to 512
+// rows each (rms 6 to 10 %).
+float slices_estimate_us(const krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
+                         bool half_x, bool split) {
+  struct Fit {
+    float call, round, factor;
+  };
+  uint64_t rounds = 0;
+  TileCost t;
+  Fit f;
+  if (group >= 128) {
+    t = half_x ? cheapest_tile<kX16, 8>(ctx, m, n, k, &rounds)
+        : split ? cheapest_tile<kXSplit, 8>(ctx, m, n, k, &rounds)
+                : cheapest_tile<kX32, 8>(ctx, m, n, k, &rounds);
+    f = half_x ? Fit{0.4f, 2.0f, 1.0f} : split ? Fit{5.1f, 2.0f, 0.93f} : Fit{0.5f, 1.25f, 1.15f};
+  } else {
+    t = half_x ? cheapest_tile<kX16, 4>(ctx, m, n, k, &rounds)
+        : split ? cheapest_tile<kXSplit, 4>(ctx, m, n, k, &rounds)
+                : cheapest_tile<kX32, 4>(ctx, m, n, k, &rounds);
+    f = half_x ? Fit{1.2f, 0.7f, 1.26f} : split ? Fit{7.9f, 1.4f, 0.95f} : Fit{2.9f, 1.0f, 1.25f};
+  }
+  return f.call + (float)rounds * (t.fixed + f.round + f.factor * t.per_1024 * (float)k * (1.0f / 1024));
+}
 
 // Any shape with K a multiple of 32 (at least 64), any group size of the format and 16-byte
 // aligned rows.  *handled = false (nothing launched) otherwise.

@@ -113,6 +113,10 @@ inline T* ptr(krm_buf address) {
   return reinterpret_cast<T*>(static_cast<uintptr_t>(address));
 }
 
+// What a product of the K-splitting tiles takes (gemm_i4_slices.hip).
+float slices_estimate_us(const krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
+                         bool half_x, bool split);
+
 // What the few-row MFMA GEMM (gemm_i4.hip) does with a finished sum besides storing it.
 struct RowsFusion {
   const void* residual = nullptr;  // [m, n_out] added to the result (the activation type)

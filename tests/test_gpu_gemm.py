@@ -465,3 +465,44 @@ def test_small_groups_need_no_scratch(gpu_ctx):
     rec.graph.destroy()
     for b in (dx, dw, ds, out):
         b.free()
+
+
+@pytest.mark.parametrize("m,n,k,g", [(330, 11300, 448, 64), (400, 20011, 512, 128), (65, 31000, 704, 64)])
+@pytest.mark.parametrize("mode", ["f32", "f16 on f32", "f16"])
+def test_wide_short_products_on_either_form(gpu_ctx, m, n, k, g, mode):
+    """Two to twelve stages a workgroup of the unit-dealt form: whichever form the estimates pick, and
+    the one without scratch that a side branch takes, meet the gate of the exact-operand kernels."""
+    ctx = gpu_ctx
+    rng = np.random.default_rng(m + n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    if mode == "f16":
+        x = x.astype(np.float16)
+    compute = ka.COMPUTE_F32 if mode == "f32" else ka.COMPUTE_F16
+    seen = x if mode == "f32" else x.astype(np.float16).astype(np.float32)
+    dx, dw, ds = ctx.upload(x), ctx.upload(packed), ctx.upload(np.ascontiguousarray(scale))
+    out = ctx.alloc(m * n * x.itemsize)
+    call = lambda: ctx.linear_i4(dx, dw, ds, None, out, m, n, k, g, ka.dtype_code(x.dtype),  # noqa: E731
+                                 ka.dtype_code(scale.dtype), compute)
+    call()
+    results = [out.download(x.dtype, (m, n))]
+    if mode != "f32":      # (hi and lo planes need scratch)
+        with ctx.record() as rec:
+            rec.branch(1)
+            call()
+        for _ in range(2):
+            out.zero()
+            rec.graph.launch()
+            results.append(out.download(x.dtype, (m, n)))
+        rec.graph.destroy()
+        assert np.array_equal(results[1], results[2])
+    cols = np.unique(np.concatenate([rng.choice(n, size=96), [0, 1, 511, 512, n - 2, n - 1]]))
+    want = sampled_oracle(seen, packed, scale.astype(np.float32), np.zeros(n, np.float32), n, k, g, cols)
+    bound = row_gate(seen) + 1e-5 * np.abs(want)
+    if mode == "f16":
+        bound = bound + 2.0 ** -11 * np.abs(want) + 1e-7
+    for got in results:
+        err = np.abs(got[:, cols].astype(np.float64) - want)
+        assert np.all(err <= bound), float(np.max(err / bound))
+    for b in (dx, dw, ds, out):
+        b.free()
