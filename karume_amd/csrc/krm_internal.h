@@ -117,7 +117,7 @@ inline T* ptr(krm_buf address) {
 float slices_estimate_us(const krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                          bool half_x, bool split);
 
-// What the few-row MFMA GEMM (gemm_i4.hip) does with a finished sum besides storing it.
+// What the K-splitting MFMA GEMM (gemm_i4_slices.hip) does with a finished sum besides storing it.
 struct RowsFusion {
   const void* residual = nullptr;  // [m, n_out] added to the result (the activation type)
   // 0: plain; 1: columns (2i, 2i+1) = (gate_i, up_i), out[., i] = silu(gate) * up;

@@ -1148,7 +1148,7 @@ int32_t pick_steps(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf b
         return launch_gemv<XT, ST, MB, ROWS, VEC, 3>(ctx, x, w, scales, bias, out, m, n, k, group_shift, fuse);
     // (up to eight steps a wave's words still fit the registers and x the LDS.  Walked step by step
     // every wave read all of x itself, and waited at each step for the next one's registers; us
-    // before / now: 4096 x 11008 fp16 8.5 / 7.2, f32 13.1 / 8.0; 32000 x 6400 f32 57 / 26.5)
+    // before / now: 4096 x 11008 fp16 7.8 / 6.4, f32 13.3 / 8.3; 32000 x 6400 f32 57 / 26)
     if constexpr (ROWS <= 2)
       if (steps <= 8 && !fuse.norm_weight && !fuse.positions) {
 #define KRM_GEMV_STEPS(COUNT)                                                                  \
@@ -1240,8 +1240,8 @@ static int32_t gemv_dispatch(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
       uint32_t group_shift = 0;
       while ((1u << group_shift) < group) ++group_shift;
       const uint32_t blocks = (n + 15) / 16, share = (k / 256 + 7) / 8;
-      // (measured, 16 rows, us before / now: N = 11008, K = 4096 13.7 / 10.2; N = 32000, K = 2048
-      // 15.4 / 11.5; N = 9000, K = 5632 17 / 12.5.  Up to a tile a CU, or four chunks a wave and more: the kernel above.)
+      // (measured, 16 rows, us before / now: N = 11008, K = 4096 13.7 / 10.0; N = 32000, K = 2048
+      // 15.2 / 11.5; N = 9000, K = 5632 16.3 / 12.2.  Up to a tile a CU, or four chunks a wave and more: the kernel above.)
       if (k >= 2048 && share <= 3 && blocks > (uint32_t)ctx->num_cus) {
 #define KRM_MFMA_TILES(ST, CH, EVEN)                                                           \
   gemv_i4_mfma_tiles_kernel<ST, CH, EVEN, 8><<<dim3(ctx->num_cus), dim3(512), 0, ctx->stream>>>( \
@@ -1304,7 +1304,8 @@ int32_t linear_i4_gemv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_b
                        GemvFusion{});
 }
 
-// MFMA GEMMs for M > 16 (gemm_i4.hip): exact integer weights (large shapes), fp16 weights.
+// MFMA GEMMs for M > 16: exact integer weights dealt by units (gemm_i4.hip) or with K split inside a
+// workgroup (gemm_i4_slices.hip); fp16 weights (gemm_i4.hip).
 int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,

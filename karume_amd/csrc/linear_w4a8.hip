@@ -888,10 +888,10 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
     const uint32_t n_blocks = (n + 255) / 256;
     // 128 x 256 tiles for groups of 64 / 128 when they still cover most of the chip, or 64 x 128 ones
     // of four waves, several to a CU, when their finer grain makes fewer rounds of a CU's work: a
-    // quarter of a tall tile each, at 1.15 of its time per output (less is shared).  us before / now:
-    // 512 x 11008 x 4096 59.5 / 56, in groups of 64 70 / 60; 400 x 9000 x 3072 49.5 / 35; 200 x 20000
-    // x 4096 55.4 / 48; 300 x 14000 x 2048 in groups of 64 42 / 34.5; where the tall ones fill whole
-    // rounds (2048 x 11008 x 4096, 256 x 32000 x 2048) these take 2 % longer.
+    // quarter of a tall tile each, at 1.15 of its time per output (less is shared).  us before / now,
+    // the quantiser's launch included: 512 x 11008 x 4096 57.3 / 51, in groups of 64 72 / 62; 200 x
+    // 20000 x 4096 59 / 54; 300 x 14000 x 2048 in groups of 64 42 / 33; where the tall ones fill whole
+    // rounds (2048 x 11008 x 4096 181, 256 x 32000 x 2048 41) they stay.
     // Groups of 32 always come here and always take the 64 x 128 tiles: the generic kernel re-reads both
     // operands for every output (512 x 11008 x 4096 50785 / 116 us, 197 x 1655 x 9600 7716 / 120, 20 x
     // 20000 x 1024 914 / 19, 9 x 300 x 512 11.7 / 11.8), and a 128 x 256 tile of four groups a stage does

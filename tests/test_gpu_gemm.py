@@ -1,11 +1,12 @@
 """GPU parity of the MFMA GEMM paths of `linear` (M > 16) against the CPU oracle.
 
 Two numerics classes (stated in the kernels):
-* exact-operand kernel (large shapes; KRM_COMPUTE_F16, and KRM_COMPUTE_F32 with the f32
-  activations split into fp16 hi + lo): weights enter as exact integers, the group scale
-  multiplies f32 group sums — gated at the GEMV's tolerance (`row_gate`: atol 3e-5 times the
-  row's largest |x|, rtol 1e-5).
-* fp16-weight kernels (smaller shapes under KRM_COMPUTE_F16): x rounded to fp16, each weight
+* exact-operand kernels (K a multiple of 32; KRM_COMPUTE_F16, and KRM_COMPUTE_F32 with the f32
+  activations split into fp16 hi + lo, in groups of 16 and 32 into three bf16): weights enter as
+  exact integers, the group scale multiplies f32 group sums — gated at the GEMV's tolerance
+  (`row_gate`: atol 3e-5 times the row's largest |x|, rtol 1e-5); the small groups, which keep every
+  bit of x, also at a bound that grows with what is summed.
+* fp16-weight kernels (other shapes under KRM_COMPUTE_F16): x rounded to fp16, each weight
   dequantised to fp16 as fp16((u-8) * scale) — one fp16 rounding, relative error <= 2^-11 — and
   products accumulated in f32.  With K terms of typical size t the error of an output behaves
   like sqrt(K) * t * 2^-11 / sqrt(3); those tests scale their tolerance with the RMS of the
@@ -437,7 +438,7 @@ def test_small_groups_give_what_the_gemv_gives_for_values_that_are_not_finite(gp
         assert np.array_equal(kind(got[:16]), kind(want)), kind.__name__
     assert np.isfinite(got[16:]).all() and np.isfinite(got[4]).all()
     finite = np.isfinite(want)
-    err = np.abs(got[:16].astype(np.float64) - want)[finite]
+    err = np.abs(got[:16][finite].astype(np.float64) - want[finite])
     size = np.broadcast_to(np.abs(np.where(np.isfinite(x[:16]), x[:16], 0)).sum(1, keepdims=True)
                            * 8.0 * float(np.abs(scale).max()), want.shape)[finite]
     assert np.all(err <= 64 * 2.0 ** -24 * size + 1e-37)

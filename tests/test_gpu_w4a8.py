@@ -213,7 +213,7 @@ def test_w4a8_random_shapes_bit_exact(gpu_ctx, m, n, k, group, scale_f16, with_b
 
 @pytest.mark.parametrize("m, n, k, group, scale_f16", [
     (129, 20033, 256, 128, True), (400, 9000, 384, 128, False), (200, 20000, 192, 64, True),
-    (300, 14001, 64, 64, False), (257, 16500, 320, 64, True)])
+    (300, 14001, 64, 64, False), (257, 16500, 320, 64, True), (400, 10300, 384, 128, True)])
 def test_w4a8_small_tiles_of_a_chip_that_tall_ones_leave_idle(gpu_ctx, m, n, k, group, scale_f16):
     """Several 64 x 128 tiles a CU where 128 x 256 ones would not fill a round: ragged M, N and a K
     that ends inside a stage."""
