@@ -214,7 +214,8 @@ int32_t krm_linear_i4_rows(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, k
  * matrix is never materialised.
  *   q      [B, H,   M, D]  io_dtype
  *   ins_k  [B, Hkv, M, D]  io_dtype   this step's keys   (valid rows: first `query`)
- *   ins_v  [B, Hkv, M, D]  io_dtype   this step's values
+ *   ins_v  [B, Hkv, M, D]  io_dtype   this step's values (one-row calls take both at any element;
+ *                                     16-byte aligned chunks of rows run on the matrix cores)
  *   slot_k [B, Hkv, C, D]  kv_dtype   past keys   (logical column c < past lives in physical
  *   slot_v [B, Hkv, C, D]  kv_dtype   past values  row c, or c % window when window > 0)
  *   out    [B, H,   M, D]  io_dtype   rows >= query are written as exact +0
