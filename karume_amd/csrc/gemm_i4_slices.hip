@@ -32,11 +32,12 @@
 // 14.5); 128 x 2048 x 2048 5.4, 7.0 (10.1, 12.5); 128 x 11264 x 2048 15.1, 27.0 (25.9, 38.6); 128 x
 // 2048 x 5632 10.6, 13.0 (19.7, 26.2).
 //
-// kXThree is bounded by the vector ALUs (11 operations a pair of x, 14 a word of weights, both at
-// every step).  Groups of 32, against the GEMV over blocks of 16 rows (in brackets: hi + lo planes,
-// which lost the small entries of a row beside a large one): 77 x 3000 x 2080 14.6 us, 210 (14.1); 17
-// rows of it 10.2, 45.5 (10.2); 128 x 2048 x 2048 11.3, 156 (12.0); 512 x 4096 x 4096 92, 1969 (81);
-// 512 x 11008 x 4096 255, 5594 (213); in groups of 16 380, 2427 (330).  Error against 64 bits (2-norm,
+// kXThree is bounded by the vector ALUs (11 operations a pair of x, 10 a word of weights, both at
+// every step; tiles of up to four columns share x).  Groups of 32, against the GEMV over blocks of 16
+// rows (in brackets: hi + lo planes, which lost the small entries of a row beside a large one): 77 x
+// 3000 x 2080 13.8 us, 210 (13.8); 17 rows of it 10.1, 45.5 (10.2); 128 x 2048 x 2048 11.2, 156 (12.0);
+// 32 x 4096 x 8192 29, - (25); 512 x 4096 x 4096 77, 1969 (81); 512 x 11008 x 4096 215, 5594 (214); in
+// groups of 16 277, 2427 (332).  Error against 64 bits (2-norm,
 // normal x): 77 x 3000 x 2080 in groups of 32 9.5e-8, the GEMV 1.24e-7; 40 x 1000 x 4096 in groups of
 // 16 1.04e-7 and 1.05e-7; 300 x 512 x 11008 in groups of 32 1.21e-7 and 1.33e-7.
 #include "krm_internal.h"
@@ -118,12 +119,15 @@ __device__ inline uint32_t high_pair(uint32_t even, uint32_t odd) {
 // what v_cvt_off_f32_i4 takes; the sum over K is multiplied by 16 at the end).
 __device__ inline half8_t sixteenths(uint32_t word) {
   const uint32_t even = word ^ 0x88888888u, odd = even >> 4;
-  uint32_t v[8];  // (a byte of a register is an operand: no shift of its own)
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    v[2 * i] = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((int)((even >> (8 * i)) & 0xffu)));
-    v[2 * i + 1] = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((int)((odd >> (8 * i)) & 0xffu)));
-  }
+  uint32_t v[8];  // (a byte of a register is an operand; the compiler shifts most of them down first)
+#define KRM_SIXTEENTH(TO, FROM, BYTE)                                                          \
+  asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #BYTE  \
+      : "=v"(TO) : "v"(FROM))
+  KRM_SIXTEENTH(v[0], even, 0); KRM_SIXTEENTH(v[1], odd, 0);
+  KRM_SIXTEENTH(v[2], even, 1); KRM_SIXTEENTH(v[3], odd, 1);
+  KRM_SIXTEENTH(v[4], even, 2); KRM_SIXTEENTH(v[5], odd, 2);
+  KRM_SIXTEENTH(v[6], even, 3); KRM_SIXTEENTH(v[7], odd, 3);
+#undef KRM_SIXTEENTH
   return __builtin_bit_cast(half8_t, make_uint4(high_pair(v[0], v[1]), high_pair(v[2], v[3]),
                                                 high_pair(v[4], v[5]), high_pair(v[6], v[7])));
 }
@@ -776,7 +780,7 @@ constexpr TileCost kCost16[] = {{1, 1, 0.8f, 1.5f}, {1, 2, 1.3f, 2.0f}, {1, 3, 1
                                 {2, 1, 0.7f, 2.0f}, {2, 2, 2.4f, 2.6f}, {2, 3, 2.2f, 3.6f}};
 constexpr TileCost kCostSplit[] = {{1, 1, 0.2f, 2.45f}, {1, 2, 0.4f, 2.9f}, {1, 3, 0.9f, 3.4f},
                                    {2, 1, 0.2f, 3.5f}, {2, 2, 1.0f, 4.5f}};
-constexpr TileCost kCostThree[] = {{1, 1, 3.2f, 3.35f}, {1, 2, 4.8f, 4.65f}, {2, 1, 4.6f, 4.97f}};
+constexpr TileCost kCostThree[] = {{1, 1, 3.2f, 3.35f}, {1, 2, 4.8f, 4.5f}, {1, 3, 6.4f, 5.7f}, {1, 4, 8.5f, 6.85f}, {2, 1, 4.6f, 4.8f}};
 constexpr TileCost kCost32[] = {{1, 1, 0.8f, 1.75f}, {1, 2, 1.3f, 2.3f}, {1, 3, 1.7f, 2.9f},
                                 {2, 1, 0.7f, 2.75f}, {2, 2, 2.2f, 3.3f}};
 
@@ -785,15 +789,16 @@ template <int XKIND, int STEPS>
 TileCost cheapest_tile(const krm_ctx* ctx, uint64_t rows, uint32_t n, uint32_t k, uint64_t* rounds) {
   const TileCost* table = XKIND == kX16 ? kCost16 : XKIND == kXSplit ? kCostSplit
                           : XKIND == kXThree ? kCostThree : kCost32;
-  const int count = XKIND == kX16 ? 6 : XKIND == kXThree ? 3 : 5;
+  const int count = XKIND == kX16 ? 6 : 5;
   const uint64_t cus = (uint64_t)ctx->num_cus;
   int best = 0;
   float best_cost = 0.f;
   for (int i = 0; i < count; ++i) {
     const TileCost& t = table[i];
-    // (below groups of 128 codes the wide tiles' LDS goes to scales; groups of 16 take 32 x 32)
-    if ((STEPS < 8 && t.nt > 2) || (STEPS < 8 && t.mt * t.nt > 2 && XKIND != kX16) ||
-        (STEPS == 1 && t.mt * t.nt > 1))
+    // (below groups of 128 codes the wide tiles' LDS goes to scales; groups of 16 take 32 x 32.  Three
+    // parts of f32 x: wide tiles share the conversion, 32 x 128 in groups of 16 would spill)
+    if ((STEPS < 8 && t.nt > 2 && XKIND != kXThree) || (STEPS < 8 && t.mt * t.nt > 2 && XKIND != kX16 && XKIND != kXThree) ||
+        (STEPS == 1 && (XKIND == kXThree ? t.mt > 1 || t.nt > 3 : t.mt * t.nt > 1)))
       continue;
     const uint64_t tiles = ((rows + 32 * t.mt - 1) / (32 * t.mt)) * (((uint64_t)n + 32 * t.nt - 1) / (32 * t.nt));
     const uint64_t turns = (tiles + cus - 1) / cus;
@@ -815,14 +820,19 @@ int32_t pick_tile(krm_ctx* ctx, const SliceCall& c) {
   if constexpr (STEPS == 8 && XKIND == kX16) {
     if (tile == 23) return launch_slices<XKIND, 2, 3, STEPS>(ctx, c);
   }
-  if constexpr (STEPS == 8) {
+  if constexpr (STEPS == 2 && XKIND == kXThree) {
+    if (tile == 14) return launch_slices<XKIND, 1, 4, STEPS>(ctx, c);
+  }
+  if constexpr (STEPS == 8 || XKIND == kXThree) {
     if (tile == 13) return launch_slices<XKIND, 1, 3, STEPS>(ctx, c);
   }
   if constexpr (STEPS == 8 || (STEPS > 1 && XKIND == kX16)) {
     if (tile == 22) return launch_slices<XKIND, 2, 2, STEPS>(ctx, c);
   }
-  if constexpr (STEPS > 1) {
+  if constexpr (STEPS > 1 || XKIND == kXThree) {
     if (tile == 12) return launch_slices<XKIND, 1, 2, STEPS>(ctx, c);
+  }
+  if constexpr (STEPS > 1) {
     if (tile == 21) return launch_slices<XKIND, 2, 1, STEPS>(ctx, c);
   }
   return launch_slices<XKIND, 1, 1, STEPS>(ctx, c);

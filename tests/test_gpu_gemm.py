@@ -394,7 +394,11 @@ def test_k_slices_kernel_at_the_edges_of_its_tiles(gpu_ctx, m, n, k, g, mode):
     assert np.all(err <= bound), float(np.max(err / bound))
 
 
-SMALL_GROUP_SHAPES = [(17, 33, 96, 32), (77, 300, 2080, 32), (100, 200, 2048, 16), (300, 2500, 512, 32)]
+# (one to four column tiles of 32 a workgroup in groups of 32, one to three in groups of 16, two row
+# tiles, on 256 CUs)
+SMALL_GROUP_SHAPES = [(17, 33, 96, 32), (77, 300, 2080, 32), (100, 200, 2048, 16), (300, 2500, 512, 32),
+                      (77, 3001, 96, 16), (100, 9001, 96, 16), (100, 9001, 96, 32),
+                      (512, 11003, 160, 32), (512, 2050, 96, 32)]
 
 
 @pytest.mark.parametrize("m,n,k,g", SMALL_GROUP_SHAPES)
