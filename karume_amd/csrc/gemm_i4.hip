@@ -22,7 +22,7 @@
 // value before it is parked, so the waits are counted) -> LDS -> fragments.  Pipelined form:
 // two LDS copies (distinct objects, so fragment reads may pass the parking writes), the
 // dequantisation of chunk c + 1 interleaved with the MFMAs of chunk c, one barrier a chunk.
-#include "krm_internal.h"
+#include "gemm_i4_deal.h"
 
 using namespace krm;
 
@@ -636,38 +636,6 @@ void gemm_i4_f16_packed_kernel(const XT* __restrict__ x, const uint8_t* __restri
 // the stores, and takes a ticket on the tile's counter; the workgroup that arrives last adds
 // the partials in ascending K order — its own from registers — so the bits do not depend on
 // who arrives last.  No workgroup ever waits for another.
-struct UnitDeal {
-  uint32_t stages_per_tile;
-  uint32_t units_lo, extra;  // workgroup v owns units_lo + (v < extra) units from deal_begin(v)
-  float* partials;           // [2 * workgroups] slots of 128 x 256 floats
-  uint32_t* tickets;         // one counter per tile, kTicketStride words apart, zero at rest
-};
-__host__ __device__ inline uint32_t deal_begin(const UnitDeal& d, uint32_t v) {
-  return v * d.units_lo + (v < d.extra ? v : d.extra);
-}
-__device__ inline uint32_t deal_owner(const UnitDeal& d, uint32_t unit) {
-  const uint32_t big = d.extra * (d.units_lo + 1u);
-  return unit < big ? unit / (d.units_lo + 1u) : d.extra + (unit - big) / d.units_lo;
-}
-constexpr uint32_t kPartialFloats = 128u * 256u;
-
-typedef float float4_t __attribute__((ext_vector_type(4)));
-// 16 bytes written through to / read from memory that every XCD sees (device scope).
-__device__ inline void publish4(float4_t* p, float4_t v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
-}
-__device__ inline float4_t observe4(const float4_t* p) {
-  float4_t v;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
-  return v;
-}
-// The eight requests above have landed; the values pass through so that no use moves ahead.
-__device__ inline void landed(float4_t (&p)[8]) {
-  asm volatile("s_waitcnt vmcnt(0)"
-               : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]),
-                 "+v"(p[7])::"memory");
-}
-
 // WM = 2 (the one in use): eight waves, wave = 64 x 64, two waves a SIMD, as above.  WM = 1: four
 // waves, wave = 128 x 64, every weight word dequantised once for four MFMAs instead of twice for
 // two — measured 101 us against 78 us on the 512 x 11008 x 4096 product: the single wave of a
@@ -910,14 +878,9 @@ void gemm_i4_f16_dealt_kernel(const XT* __restrict__ x, const uint8_t* __restric
 // ------------------------------------------------ exact integer operands, 64 x 512 tiles
 //
 // The weights enter the matrix cores as the exact integers (u - 8) in fp16 and the group scale
-// multiplies the f32 sum of a group afterwards — the arithmetic of the GEMV, on MFMA.  Two
-// activation forms:
-//   kOperandF16  x is rounded to fp16 once (exact when it already is fp16): one MFMA a step;
-//   kOperandSplit  f32 x is split as x * 2^e = hi + lo, both fp16, |x * 2^e - (hi + lo)| <=
-//                2^-23 |x * 2^e| (e per row, chosen so that the row's largest magnitude lands in
-//                [2^13, 2^14): no overflow, and small entries keep an absolute resolution of
-//                2^-38 of the row's maximum): two MFMAs a step, products exact, f32 sums —
-//                the class of the reference's default f32 `linear`, on the matrix cores.
+// multiplies the f32 sum of a group afterwards — the arithmetic of the GEMV, on MFMA.  x is rounded to
+// fp16 once (exact when it already is fp16): one MFMA a step.  (f32 x as hi + lo, and fp16 x where the
+// ranges are long: gemm_i4_exact.hip, which also holds what was measured of both.)
 // Tile 64 x 512, eight waves side by side (wave = 64 rows x 64 columns = 2 x 2 MFMA tiles), so
 // every weight word is turned into integers exactly once per workgroup (in the 128 x 256 tile
 // above the two waves of a column strip each do it).  Per MFMA step the wave holds the sums of
@@ -925,8 +888,6 @@ void gemm_i4_f16_dealt_kernel(const XT* __restrict__ x, const uint8_t* __restric
 // (the C layout keeps the column in lane % 32, so the scale is one value per lane and column
 // tile).  Stages, LDS layout, the (tile, stage) deal over the CUs and the ordered merge of the
 // partials are those of the kernel above.
-constexpr int kOperandF16 = 0, kOperandSplit = 1;
-
 // 8 codes of a word -> 8 fp16 integers (u - 8), order (c0,c4,c1,c5,c2,c6,c3,c7).
 __device__ inline uint4 ints_word(uint32_t word) {
   const uint32_t magic = 0x64006400u;  // (1024, 1024)
@@ -944,82 +905,23 @@ __device__ inline uint4 ints_word(uint32_t word) {
                     __builtin_bit_cast(uint32_t, q2), __builtin_bit_cast(uint32_t, q3));
 }
 
-// x * scale = hi + lo for eight f32 activations, both halves in the paired order.
-__device__ inline void split_paired(const uint4& a, const uint4& b, float scale, uint4& hi,
-                                    uint4& lo) {
-  const float v[8] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z),
-                      __uint_as_float(a.w), __uint_as_float(b.x), __uint_as_float(b.y),
-                      __uint_as_float(b.z), __uint_as_float(b.w)};
-  _Float16 h[8], l[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float xs = v[i] * scale;             // exact: a power of two
-    h[i] = (_Float16)xs;                       // round to nearest even
-    l[i] = (_Float16)(xs - (float)h[i]);       // the difference is exact in f32
-  }
-  auto pack = [](_Float16 p, _Float16 q) {
-    const half2_t t = {p, q};
-    return __builtin_bit_cast(uint32_t, t);
-  };
-  hi = make_uint4(pack(h[0], h[4]), pack(h[1], h[5]), pack(h[2], h[6]), pack(h[3], h[7]));
-  lo = make_uint4(pack(l[0], l[4]), pack(l[1], l[5]), pack(l[2], l[6]), pack(l[3], l[7]));
-}
-
-// Row scales of the split form: scale[2r] = 2^e with max|x[r, :]| * 2^e in [2^13, 2^14),
-// scale[2r + 1] = 2^-e.  A row of zeros (or whose maximum is not finite) gets 1 / 1: what is
-// not finite stays so through the product.
-__global__ __launch_bounds__(256) void row_scale_kernel(const float* __restrict__ x,
-                                                        float* __restrict__ row_scale, uint32_t k) {
-  __shared__ uint32_t s_max[4];
-  const float* row = x + (size_t)blockIdx.x * k;
-  uint32_t top = 0;  // largest |x| as raw bits (monotonic for non-negative floats; NaN on top)
-  const uint32_t pieces = k >> 2;
-  for (uint32_t i = threadIdx.x; i < pieces; i += 256) {
-    const uint4 v = reinterpret_cast<const uint4*>(row)[i];
-    top = max(max(top, v.x & 0x7fffffffu), max(v.y & 0x7fffffffu, max(v.z & 0x7fffffffu, v.w & 0x7fffffffu)));
-  }
-  for (uint32_t i = (pieces << 2) + threadIdx.x; i < k; i += 256)
-    top = max(top, __float_as_uint(row[i]) & 0x7fffffffu);
-  for (int off = 32; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off, kWave));
-  if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = top;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    top = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
-    const uint32_t biased = top >> 23;  // exponent of the maximum
-    uint32_t up = 127u, down = 127u;    // 2^0
-    if (top != 0 && biased != 255u) {
-      // e = 13 - (biased - 127), kept inside the normal range of both 2^e and 2^-e
-      int e = 13 - ((int)biased - 127);
-      e = e > 126 ? 126 : (e < -126 ? -126 : e);
-      up = (uint32_t)(127 + e);
-      down = (uint32_t)(127 - e);
-    }
-    row_scale[2 * (size_t)blockIdx.x] = __uint_as_float(up << 23);
-    row_scale[2 * (size_t)blockIdx.x + 1] = __uint_as_float(down << 23);
-  }
-}
-
-template <typename XT, typename ST, int OPERAND>
+template <typename XT, typename ST>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ w,
+void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ w,
                           const ST* __restrict__ scales, const XT* __restrict__ bias,
                           XT* __restrict__ out, uint32_t m, uint32_t n, uint32_t k,
-                          uint32_t group_shift, uint32_t m_blocks, UnitDeal deal,
-                          const float* __restrict__ row_scale) {
+                          uint32_t group_shift, uint32_t m_blocks, UnitDeal deal) {
   constexpr int MT = 2, WN = 2, T = 512;
   constexpr int BM = 64, BN = 512;
-  constexpr int NA = OPERAND == kOperandSplit ? 2 : 1;  // copies of the x tile (hi, lo)
   constexpr int kStage = 128;
   constexpr int kRowA = kStage * 2 + 16;
   constexpr int kRowB = kStage / 2 + 16;
   constexpr int kAUnits = BM * (kStage / 8) / T;   // 2
   constexpr int kBUnits = BN * (kStage / 32) / T;  // 4
   static_assert((size_t)BM * BN == kPartialFloats, "the partial slots hold one tile");
-  static_assert(OPERAND == kOperandF16 || sizeof(XT) == 4, "only f32 activations are split");
-  __shared__ __align__(16) uint8_t s_a[2][NA][BM * kRowA];
+  __shared__ __align__(16) uint8_t s_a[2][BM * kRowA];
   __shared__ __align__(16) uint8_t s_b[2][BN * kRowB];
   __shared__ float s_s[2][BN][2];
-  __shared__ float s_inv[BM];
   __shared__ uint32_t s_ticket;
 
   const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
@@ -1039,63 +941,49 @@ void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ 
 
   while (left > 0) {
     const uint32_t range_end = my_begin + left;
-    const uint32_t tile = (range_end - 1u) / spt;
+    const uint32_t tile = __builtin_amdgcn_readfirstlane((range_end - 1u) / spt);
     const uint32_t tile_first = tile * spt;
     const uint32_t s0 = my_begin > tile_first ? my_begin - tile_first : 0u;
     const uint32_t s1 = range_end - tile_first;
-    const uint32_t nb = tile / m_blocks, mb = tile - nb * m_blocks;
+    const uint32_t nb = __builtin_amdgcn_readfirstlane(tile / m_blocks), mb = tile - nb * m_blocks;
     const uint32_t m0 = mb * BM, n0 = nb * BN;
-    const ST* ssrc = scales + (size_t)min(n0 + (uint32_t)tid, n - 1) * groups;
-
-    float rs[kAUnits];  // 2^e of the rows this thread stages
-#pragma unroll
-    for (int i = 0; i < kAUnits; ++i) rs[i] = 1.0f;
-    if constexpr (OPERAND == kOperandSplit) {
-#pragma unroll
-      for (int i = 0; i < kAUnits; ++i)
-        rs[i] = row_scale[2 * (size_t)min(m0 + arow0 + 32u * i, m - 1)];
-      if (tid < BM) s_inv[tid] = row_scale[2 * (size_t)min(m0 + (uint32_t)tid, m - 1) + 1];
-    }
-
+    const ST* const s_tile = scales + (size_t)n0 * groups;
+    const uint32_t s_row = min((uint32_t)tid, n - 1 - n0) * groups;
+    // the tile's rows: one base each and 32-bit offsets (plan_staged bounds K)
+    const uint8_t* const x_tile = reinterpret_cast<const uint8_t*>(x) + (size_t)m0 * k * sizeof(XT);
+    const uint8_t* const w_tile = w + (size_t)n0 * (k >> 1);
     struct Staged {
       Acts8<XT> a[kAUnits];
       uint4 b[kBUnits];
     };
     auto load_stage = [&](uint32_t stage, Staged& d) {
       const uint32_t a_at = stage * kStage + aunit, b_at = stage * (kStage / 2) + bunit;
+      // (opaque, so that the rows' offsets are formed here and hold no registers between stages)
+      uint32_t a_last = m - 1 - m0, b_last = n - 1 - n0;
+      asm volatile("" : "+s"(a_last), "+s"(b_last));
       const uint32_t a_off = a_at < k ? a_at : 0u, b_off = b_at < (k >> 1) ? b_at : 0u;
 #pragma unroll
       for (int i = 0; i < kAUnits; ++i)
-        d.a[i].load(x + (size_t)min(m0 + arow0 + 32u * i, m - 1) * k + a_off);
+        d.a[i].load(reinterpret_cast<const XT*>(x_tile + (min(arow0 + 32u * i, a_last) * k + a_off) * (uint32_t)sizeof(XT)));
 #pragma unroll
       for (int i = 0; i < kBUnits; ++i)
-        d.b[i] = *reinterpret_cast<const uint4*>(
-            w + (size_t)min(n0 + brow0 + 128u * i, n - 1) * (k >> 1) + b_off);
+        d.b[i] = *reinterpret_cast<const uint4*>(w_tile + (min(brow0 + 128u * i, b_last) * (k >> 1) + b_off));
     };
     auto park_stage = [&](uint32_t stage, int buf, Staged& d) {
       const uint32_t keep = stage * kStage + aunit < k ? 0xFFFFFFFFu : 0u;
 #pragma unroll
       for (int i = 0; i < kAUnits; ++i) {
         const uint32_t at = (arow0 + 32u * i) * kRowA + aunit * 2u;
-        if constexpr (OPERAND == kOperandSplit) {
-          uint4 hi, lo;
-          split_paired(d.a[i].a, d.a[i].b, rs[i], hi, lo);
-          hi.x &= keep; hi.y &= keep; hi.z &= keep; hi.w &= keep;  // past K: zeros
-          lo.x &= keep; lo.y &= keep; lo.z &= keep; lo.w &= keep;
-          *reinterpret_cast<uint4*>(&s_a[buf][0][at]) = hi;
-          *reinterpret_cast<uint4*>(&s_a[buf][NA - 1][at]) = lo;
-        } else {
-          uint4 pv = d.a[i].paired();
-          pv.x &= keep; pv.y &= keep; pv.z &= keep; pv.w &= keep;
-          *reinterpret_cast<uint4*>(&s_a[buf][0][at]) = pv;
-        }
+        uint4 pv = d.a[i].paired();
+        pv.x &= keep; pv.y &= keep; pv.z &= keep; pv.w &= keep;  // past K: zeros
+        *reinterpret_cast<uint4*>(&s_a[buf][at]) = pv;
       }
 #pragma unroll
       for (int i = 0; i < kBUnits; ++i)
         *reinterpret_cast<uint4*>(&s_b[buf][(brow0 + 128u * i) * kRowB + bunit]) = d.b[i];
       const uint32_t c0 = stage * kStage, c1 = stage * kStage + 64u;
-      s_s[buf][tid][0] = load_scale_f32<ST>(ssrc, (c0 < k ? c0 : 0u) >> group_shift);
-      s_s[buf][tid][1] = load_scale_f32<ST>(ssrc, (c1 < k ? c1 : 0u) >> group_shift);
+      s_s[buf][tid][0] = load_scale_f32<ST>(s_tile, s_row + ((c0 < k ? c0 : 0u) >> group_shift));
+      s_s[buf][tid][1] = load_scale_f32<ST>(s_tile, s_row + ((c1 < k ? c1 : 0u) >> group_shift));
     };
 
     float16_t total[MT][WN], acc[MT][WN];
@@ -1128,13 +1016,10 @@ void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ 
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          half8_t a[NA][MT];
+          half8_t a[MT];
 #pragma unroll
-          for (int copy = 0; copy < NA; ++copy)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-              a[copy][mt] = *reinterpret_cast<const half8_t*>(
-                  &s_a[buf][copy][a_base + mt * 32 * kRowA + 128 * c + 16 * j]);
+          for (int mt = 0; mt < MT; ++mt)
+            a[mt] = *reinterpret_cast<const half8_t*>(&s_a[buf][a_base + mt * 32 * kRowA + 128 * c + 16 * j]);
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt) {
             const uint32_t word = j == 0 ? braw[nt].x : j == 1 ? braw[nt].y : j == 2 ? braw[nt].z
@@ -1143,14 +1028,10 @@ void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ 
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-              for (int copy = 0; copy < NA; ++copy) {
-                // the first product of a scale group starts from zero (an inline constant of
-                // the instruction: the sums are not cleared by VALU moves)
-                const bool opens = copy == 0 && j == 0 && (c == 0 || half_stage_groups);
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                    a[copy][mt], b, opens ? zero16 : acc[mt][nt], 0, 0, 0);
-              }
+              // the first product of a scale group starts from zero (an inline constant of the
+              // instruction: the sums are not cleared by VALU moves)
+              const bool opens = j == 0 && (c == 0 || half_stage_groups);
+              acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt], b, opens ? zero16 : acc[mt][nt], 0, 0, 0);
             }
             __builtin_amdgcn_s_setprio(0);
           }
@@ -1180,9 +1061,7 @@ void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ 
       for (int r = 0; r < 16; ++r) {
         const uint32_t local = mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4);
         const uint32_t row = m0 + local;
-        float value = sum[r];
-        if constexpr (OPERAND == kOperandSplit) value *= s_inv[local];  // exact: a power of two
-        if (row < m && col < n) store_out<XT>(out, (size_t)row * n + col, value + b);
+        if (row < m && col < n) store_out<XT>(out, (size_t)row * n + col, sum[r] + b);
       }
     };
 
@@ -1263,39 +1142,35 @@ void gemm_i4_exact_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ 
           __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-    __syncthreads();  // s_inv and the LDS tiles are rewritten by the next tile of the range
+    __syncthreads();  // the LDS tiles are rewritten by the next tile of the range
     left -= s1 - s0;
   }
 }
 
 // The deal of the 64 x 512 tiles: one workgroup per CU, every workgroup at least two stages.
-bool plan_exact_deal(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group, bool half_x,
-                     bool split, uint32_t& grid, UnitDeal& deal) {
+bool plan_staged(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group, bool half_x,
+                     uint32_t& grid, UnitDeal& deal) {
   const uint64_t cus = (uint64_t)ctx->num_cus;
   const uint64_t tiles = (uint64_t)((m + 63) / 64) * ((n + 511) / 512);
   const uint32_t spt = (k + 127) / 128;
   const uint64_t units = tiles * spt;
   if (tiles > kTicketSlots || units > 0x7fffffffull || units < 2 * cus) return false;
+  if (k > 1u << 24) return false;  // 32-bit offsets inside a tile's rows
   if (units < 12 * cus) {
     // Fewer than twelve stages a workgroup: the K-splitting tiles of gemm_i4_slices.hip, unless
     // their estimate is clearly above this form's, {fixed, a stage} in us, fitted over 16 to 21 shapes
     // (rms 6 to 8 %).  Over 100 shapes of 65 to 512 rows the choice is 1 % behind the better of the two
     // and 4 % at worst behind the tiles alone.  us there / here: fp16 406 x 24848 x 512 in groups of 64 61 / 27, 198 x 26342 x 768 35 / 24, 237 x
     // 7285 x 2688 in groups of 64 26 / 31; f32 rounded to fp16 399 x 26833 x 896 in groups of 64 115 /
-    // 57, 169 x 8597 x 1664 19 / 33; f32 class 470 x 23723 x 512 81 / 63, 190 x 11922 x 1920 30 / 55.
+    // 57, 169 x 8597 x 1664 19 / 33.
     struct Fit {
       float fixed, stage;
     };
     const bool wide_groups = group >= 128;
     const Fit f = half_x ? (wide_groups ? Fit{14.1f, 2.45f} : Fit{14.7f, 2.6f})
-                  : split ? (wide_groups ? Fit{36.3f, 4.0f} : Fit{37.3f, 4.0f})
-                          : (wide_groups ? Fit{19.8f, 2.7f} : Fit{20.6f, 3.1f});
+                         : (wide_groups ? Fit{19.8f, 2.7f} : Fit{20.6f, 3.1f});
     const float here = f.fixed + f.stage * ((float)units / (float)cus);
-    if (here > 0.88f * slices_estimate_us(ctx, m, n, k, group, half_x, split)) return false;
-  } else if (split && k > n) {
-    // In the f32 class the two meet for a long K (512 x 4096 x 11008: 122 us there, 138 us here; 512 x
-    // 11008 x 4096: 138 and 126 us).
-    return false;
+    if (here > 0.88f * slices_estimate_us(ctx, m, n, k, group, half_x, false)) return false;
   }
   // Up to six 32 x 32 tiles of output a CU stay with the tiles that split K inside a workgroup, which
   // need no scratch with fp16 operands (a side branch of a graph may hold them) and give a row the
@@ -1433,57 +1308,48 @@ int32_t pick_tile(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bi
   return launch<XT, ST, 1, 1, 64, 1, 1>(ctx, x, w, scales, bias, out, m, n, k, group_shift);
 }
 
-template <typename XT, typename ST, int OPERAND>
-int32_t launch_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias, krm_buf out,
+template <typename XT, typename ST>
+int32_t launch_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias, krm_buf out,
                      uint32_t m, uint32_t n, uint32_t k, uint32_t group_shift, uint32_t grid,
                      const UnitDeal& deal) {
   KRM_TRY(needs_serial_scratch(ctx, "the unit-dealt GEMM"));
-  if constexpr (OPERAND == kOperandSplit) {
-    row_scale_kernel<<<dim3(m), dim3(256), 0, ctx->stream>>>(ptr<const float>(x), ctx->row_scales, k);
-    KRM_TRY(launched(ctx, "row_scale_kernel"));
-  }
-  gemm_i4_exact_kernel<XT, ST, OPERAND><<<dim3(grid), dim3(512), 0, ctx->stream>>>(
+  gemm_i4_staged_kernel<XT, ST><<<dim3(grid), dim3(512), 0, ctx->stream>>>(
       ptr<const XT>(x), ptr<const uint8_t>(w), ptr<const ST>(scales), ptr<const XT>(bias),
-      ptr<XT>(out), m, n, k, group_shift, (m + 63) / 64, deal, ctx->row_scales);
-  return launched(ctx, "gemm_i4_exact_kernel");
+      ptr<XT>(out), m, n, k, group_shift, (m + 63) / 64, deal);
+  return launched(ctx, "gemm_i4_staged_kernel");
 }
 
 }  // namespace
 
 namespace krm {
 
-// The exact-integer-operand GEMM for shapes whose (tile, stage) units cover the chip; sets
+// The exact-integer GEMM with x in fp16 for shapes whose (tile, stage) units cover the chip; sets
 // *handled = false (and launches nothing) for every other shape.
-int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
+int32_t linear_i4_gemm_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
                              bool* handled) {
   *handled = false;
-  const bool split = compute == KRM_COMPUTE_F32 && io_dtype == KRM_F32;
+  if (compute == KRM_COMPUTE_F32 && io_dtype == KRM_F32) return KRM_OK;
   if (group < 64 || k % 32 != 0 || !aligned(w, 16) || !aligned(x, 16)) return KRM_OK;
-  if (split && (m > kMaxSplitRows || !ctx->row_scales)) return KRM_OK;
   uint32_t grid = 0;
   UnitDeal deal{};
   // (a side branch of a graph has no scratch: there the K-splitting tiles, which need none with fp16
   // operands, take these shapes too)
-  if (!split && ctx->stream != ctx->main_stream) return KRM_OK;
-  if (!plan_exact_deal(ctx, m, n, k, group, io_dtype == KRM_F16, split, grid, deal)) return KRM_OK;
+  if (ctx->stream != ctx->main_stream) return KRM_OK;
+  if (!plan_staged(ctx, m, n, k, group, io_dtype == KRM_F16, grid, deal)) return KRM_OK;
   uint32_t group_shift = 0;
   while ((1u << group_shift) < group) ++group_shift;
   *handled = true;
-#define KRM_EXACT(XT, ST, OP) \
-  return launch_exact<XT, ST, OP>(ctx, x, w, scales, bias, out, m, n, k, group_shift, grid, deal)
+#define KRM_STAGED(XT, ST) \
+  return launch_staged<XT, ST>(ctx, x, w, scales, bias, out, m, n, k, group_shift, grid, deal)
   if (io_dtype == KRM_F16) {
-    if (scale_dtype == KRM_F16) KRM_EXACT(__half, __half, kOperandF16);
-    KRM_EXACT(__half, float, kOperandF16);
+    if (scale_dtype == KRM_F16) KRM_STAGED(__half, __half);
+    KRM_STAGED(__half, float);
   }
-  if (split) {
-    if (scale_dtype == KRM_F16) KRM_EXACT(float, __half, kOperandSplit);
-    KRM_EXACT(float, float, kOperandSplit);
-  }
-  if (scale_dtype == KRM_F16) KRM_EXACT(float, __half, kOperandF16);
-  KRM_EXACT(float, float, kOperandF16);
-#undef KRM_EXACT
+  if (scale_dtype == KRM_F16) KRM_STAGED(float, __half);
+  KRM_STAGED(float, float);
+#undef KRM_STAGED
 }
 
 int32_t linear_i4_gemm_f16(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,

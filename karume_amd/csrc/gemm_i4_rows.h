@@ -1,0 +1,250 @@
+// What the exact-integer MFMA products share (gemm_i4_slices.hip, gemm_i4_exact.hip): packed codes to
+// fp16 integers, loads from memory into LDS with counted waits, f32 x as two fp16 planes, and what
+// happens to a finished pair of columns.
+#pragma once
+
+#include "krm_internal.h"
+
+namespace krm {
+namespace {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+template <typename T>
+__device__ inline float to_f32(T v);
+template <>
+__device__ inline float to_f32<float>(float v) { return v; }
+template <>
+__device__ inline float to_f32<__half>(__half v) { return __half2float(v); }
+template <typename T>
+__device__ inline T from_f32(float v);
+template <>
+__device__ inline float from_f32<float>(float v) { return v; }
+template <>
+__device__ inline __half from_f32<__half>(float v) { return __float2half_rn(v); }
+
+// (a & mask) | bits in one VALU op (the compiler emits two when both constants are literals).
+__device__ inline uint32_t and_or(uint32_t a, uint32_t mask, uint32_t bits) {
+  uint32_t d;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(mask), "v"(bits));
+  return d;
+}
+
+// 8 codes of a word -> 8 fp16 integers (u - 8).  1024 + u (or 1024 + 16 u) is built in the fp16
+// mantissa, one packed op removes the offset.
+// Order (c0,c4,c1,c5,c2,c6,c3,c7): two ops a pair, for activations stored in the same order.
+__device__ inline half8_t ints_paired(uint32_t word) {
+  const uint32_t magic = 0x64006400u;  // (1024, 1024)
+  const half2_t off_lo = {(_Float16)1032.0f, (_Float16)1032.0f};
+  const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
+  const half2_t off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
+  const uint32_t upper = word >> 8;
+  const half2_t q0 = __builtin_bit_cast(half2_t, and_or(word, 0x000F000Fu, magic)) - off_lo;
+  const half2_t q1 = __builtin_elementwise_fma(
+      __builtin_bit_cast(half2_t, and_or(word, 0x00F000F0u, magic)), sixteenth, off_hi);
+  const half2_t q2 = __builtin_bit_cast(half2_t, and_or(upper, 0x000F000Fu, magic)) - off_lo;
+  const half2_t q3 = __builtin_elementwise_fma(
+      __builtin_bit_cast(half2_t, and_or(upper, 0x00F000F0u, magic)), sixteenth, off_hi);
+  return half8_t{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
+}
+// Natural order c0..c7: a byte of the word is copied to both halves, the even code is read from
+// its low nibble and the odd one from its high nibble (three ops a pair).
+__device__ inline half8_t ints_natural(uint32_t word) {
+  const uint32_t magic = 0x64006400u;
+  const half2_t factor = {(_Float16)1.0f, (_Float16)0.0625f};
+  const half2_t offset = {(_Float16)-1032.0f, (_Float16)-72.0f};
+  half2_t q[4];
+  const uint32_t twice[4] = {__builtin_amdgcn_perm(word, word, 0x0c000c00u),
+                             __builtin_amdgcn_perm(word, word, 0x0c010c01u),
+                             __builtin_amdgcn_perm(word, word, 0x0c020c02u),
+                             __builtin_amdgcn_perm(word, word, 0x0c030c03u)};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    q[i] = __builtin_elementwise_fma(
+        __builtin_bit_cast(half2_t, and_or(twice[i], 0x00F0000Fu, magic)), factor, offset);
+  return half8_t{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+}
+
+// ------------------------------------------------------------------- memory -> LDS, counted waits
+//
+// The loads below do not pass through registers and the compiler does not see them; the waits are
+// counted by hand (vector memory operations of a wave complete in order).  Nothing else of the K
+// loop loads from memory through the compiler.
+
+// 16 bytes a lane from base + offset to LDS at lds + 16 * lane.
+__device__ inline void stream_to_lds(uint32_t lds, uint32_t offset, const void* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds),
+               "v"(offset), "s"(base)
+               : "memory");
+}
+// The same for a dword or a zero-extended ushort a lane, to LDS at lds + 4 * lane.
+__device__ inline void stream_word_to_lds(uint32_t lds, uint32_t offset, const void* base, bool half) {
+  if (half)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" ::"s"(lds),
+                 "v"(offset), "s"(base)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds),
+                 "v"(offset), "s"(base)
+                 : "memory");
+}
+template <int N>
+__device__ inline void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// Columns (col, col + 1) of output row `row`, summed: bias, then what the call asked for.
+template <typename T>
+__device__ inline void finish_pair(float v0, float v1, uint32_t row, uint32_t col, uint32_t m,
+                                   uint32_t n, const T* __restrict__ bias, T* __restrict__ out,
+                                   const RowsFusion& fuse) {
+  const T* residual = static_cast<const T*>(fuse.residual);
+  const bool two = col + 1 < n;
+  if (bias) {
+    v0 += to_f32<T>(bias[col]);
+    if (two) v1 += to_f32<T>(bias[col + 1]);
+  }
+  if (fuse.mode == 1) {
+    // (gate, up) -> silu(gate) * up, the roundings of the decode row's epilogue
+    const float t = __builtin_amdgcn_exp2f(-fabsf(v0) * 1.4426950408889634f);
+    const float r = __builtin_amdgcn_rcpf(1.0f + t);
+    const float sig = v0 < 0.f ? t * r : r;
+    float value = __fmul_rn(__fmul_rn(v0, sig), v1);
+    const size_t at = (size_t)row * (n >> 1) + (col >> 1);
+    if (residual) value += to_f32<T>(residual[at]);
+    out[at] = from_f32<T>(value);
+  } else if (fuse.mode == 2) {
+    // what a separate linear would have stored, then the rotation of krm_rope_half
+    const float x0 = to_f32<T>(from_f32<T>(v0)), x1 = to_f32<T>(from_f32<T>(v1));
+    const uint32_t half = fuse.depth >> 1, pair = col >> 1;
+    const uint32_t rope_pairs = (fuse.heads + fuse.kv_heads) * half;
+    if (pair < rope_pairs) {
+      const uint32_t head = pair / half, j = pair - head * half;
+      const int32_t pos = fuse.positions[row];
+      float o0 = NAN, o1 = NAN;  // a position outside the table is never a valid rotation
+      if (pos >= 0 && (uint32_t)pos < fuse.table_rows) {
+        const size_t t = (size_t)pos * fuse.depth + j;
+        o0 = __fadd_rn(__fmul_rn(x0, fuse.cos_table[t]), __fmul_rn(-x1, fuse.sin_table[t]));
+        o1 = __fadd_rn(__fmul_rn(x1, fuse.cos_table[t + half]),
+                       __fmul_rn(x0, fuse.sin_table[t + half]));
+      }
+      T* dst = head < fuse.heads
+                   ? static_cast<T*>(fuse.q_out) + ((size_t)head * m + row) * fuse.depth
+                   : static_cast<T*>(fuse.k_out) + ((size_t)(head - fuse.heads) * m + row) * fuse.depth;
+      dst[j] = from_f32<T>(o0);
+      dst[j + half] = from_f32<T>(o1);
+    } else {
+      const uint32_t e = (pair - rope_pairs) * 2u;  // the v section keeps its natural order
+      const uint32_t plane = e / fuse.depth, d = e - plane * fuse.depth;
+      T* dst = static_cast<T*>(fuse.v_out) + ((size_t)plane * m + row) * fuse.depth;
+      dst[d] = from_f32<T>(x0);
+      dst[d + 1] = from_f32<T>(x1);
+    }
+  } else {
+    const size_t at = (size_t)row * n + col;
+    if (residual) {
+      v0 += to_f32<T>(residual[at]);
+      if (two) v1 += to_f32<T>(residual[at + 1]);
+    }
+    out[at] = from_f32<T>(v0);
+    if (two) out[at + 1] = from_f32<T>(v1);
+  }
+}
+
+template <typename T>
+struct type_tag { using type = T; };
+
+struct SliceTail {         // what the end of the kernel needs
+  const void* bias;
+  void* out;
+  const float* row_scale;  // kXSplit
+  RowsFusion fuse;
+};
+
+// ------------------------------------------------------------------------------- x = hi + lo
+//
+// Row r of the split form: for every 32 codes, 64 bytes of hi and 64 bytes of lo (one line), eight
+// codes at a time in the order (x0,x4,x1,x5,x2,x6,x3,x7); scale[2r] = 2^e with max|x[r, :]| * 2^e in [2^13, 2^14) (no
+// overflow, small entries keep a resolution of 2^-38 of the row's maximum), scale[2r + 1] = 2^-e.
+// A row of zeros, or whose maximum is not finite, gets 1 / 1: what is not finite stays so.
+// One trip over memory up to 16384 codes a row (kept in registers between the maximum and the
+// split), two beyond.  A row takes `padded` codes in the planes, zeros past k.
+__global__ __launch_bounds__(512) void split_rows_kernel(const float* __restrict__ x,
+                                                         uint4* __restrict__ planes,
+                                                         float* __restrict__ scale, uint32_t k,
+                                                         uint32_t padded) {
+  constexpr uint32_t kHeld = 4;
+  __shared__ uint32_t s_max[8];
+  const uint4* row = reinterpret_cast<const uint4*>(x + (size_t)blockIdx.x * k);
+  const uint32_t pieces = k >> 3;
+  uint4 a[kHeld], b[kHeld];
+#pragma unroll
+  for (uint32_t i = 0; i < kHeld; ++i) {
+    const uint32_t p = threadIdx.x + 512u * i;
+    const uint32_t at = p < pieces ? p : 0u;
+    a[i] = row[2 * at];
+    b[i] = row[2 * at + 1];
+  }
+  auto larger = [](uint32_t top, const uint4& v) {
+    return max(max(top, v.x & 0x7fffffffu),
+               max(v.y & 0x7fffffffu, max(v.z & 0x7fffffffu, v.w & 0x7fffffffu)));
+  };
+  uint32_t top = 0;  // largest |x| as raw bits (monotonic for non-negative floats; NaN on top)
+#pragma unroll
+  for (uint32_t i = 0; i < kHeld; ++i) top = larger(larger(top, a[i]), b[i]);
+  for (uint32_t p = threadIdx.x + 512u * kHeld; p < pieces; p += 512u)
+    top = larger(larger(top, row[2 * p]), row[2 * p + 1]);
+  for (int off = 32; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off, kWave));
+  if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = top;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 8; ++i) top = max(top, s_max[i]);
+  const uint32_t biased = top >> 23;  // exponent of the maximum
+  uint32_t up = 127u, down = 127u;    // 2^0
+  if (top != 0 && biased != 255u) {
+    // e = 13 - (biased - 127), kept inside the normal range of both 2^e and 2^-e
+    int e = 13 - ((int)biased - 127);
+    e = e > 126 ? 126 : (e < -126 ? -126 : e);
+    up = (uint32_t)(127 + e);
+    down = (uint32_t)(127 - e);
+  }
+  const float factor = __uint_as_float(up << 23);
+  if (threadIdx.x == 0) {
+    scale[2 * (size_t)blockIdx.x] = factor;
+    scale[2 * (size_t)blockIdx.x + 1] = __uint_as_float(down << 23);
+  }
+  uint4* dst = planes + (size_t)blockIdx.x * (padded >> 2);
+  auto split = [&](uint32_t p, const uint4& va, const uint4& vb) {
+    const uint32_t raw[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
+    _Float16 h[8], l[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float xs = __uint_as_float(raw[i]) * factor;  // exact: a power of two
+      h[i] = (_Float16)xs;                                // round to nearest even
+      l[i] = (_Float16)(xs - (float)h[i]);                // the difference is exact in f32
+    }
+    auto pack = [](_Float16 p0, _Float16 p1) {
+      const half2_t t = {p0, p1};
+      return __builtin_bit_cast(uint32_t, t);
+    };
+    const uint32_t at = (p >> 2) * 8u + (p & 3u);
+    dst[at] = make_uint4(pack(h[0], h[4]), pack(h[1], h[5]), pack(h[2], h[6]), pack(h[3], h[7]));
+    dst[at + 4] =
+        make_uint4(pack(l[0], l[4]), pack(l[1], l[5]), pack(l[2], l[6]), pack(l[3], l[7]));
+  };
+#pragma unroll
+  for (uint32_t i = 0; i < kHeld; ++i) {
+    const uint32_t p = threadIdx.x + 512u * i;
+    if (p < pieces) split(p, a[i], b[i]);
+  }
+  for (uint32_t p = threadIdx.x + 512u * kHeld; p < pieces; p += 512u)
+    split(p, row[2 * p], row[2 * p + 1]);
+  for (uint32_t p = pieces + threadIdx.x; p < padded >> 3; p += 512u) {
+    const uint32_t at = (p >> 2) * 8u + (p & 3u);
+    dst[at] = dst[at + 4] = make_uint4(0u, 0u, 0u, 0u);
+  }
+}
+
+}  // namespace
+}  // namespace krm

@@ -29,6 +29,8 @@ struct krm_ctx {
   // Per-row scales {2^e, 2^-e} of the f32-class prefill GEMM (kMaxSplitRows rows), written by
   // a pre-pass of every such launch.
   float* row_scales = nullptr;
+  // fp16 planes of f32 activations, written by a pre-pass of every unit-dealt GEMM (kPlaneBytes).
+  void* x_planes = nullptr;
   bool recording = false;  // between krm_graph_begin and krm_graph_end
   // Parallel branches of a recording (krm_graph_branch): `stream` is the stream launches go
   // to, which is `main_stream` except while a side branch is selected.  Side streams are
@@ -61,6 +63,7 @@ constexpr uint32_t kTicketSlots = 1u << 16;
 constexpr uint32_t kTicketStride = 32;
 constexpr size_t kGemmPartialBytes = 128u * 256u * sizeof(float);
 constexpr uint32_t kMaxSplitRows = 1u << 16;
+constexpr size_t kPlaneBytes = (size_t)64 << 20;
 
 // Records the message on the context (or on the context-less slot) and returns `code`.
 int32_t fail(krm_ctx* ctx, int32_t code, const char* fmt, ...);

@@ -1304,12 +1304,17 @@ int32_t linear_i4_gemv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_b
                        GemvFusion{});
 }
 
-// MFMA GEMMs for M > 16: exact integer weights dealt by units (gemm_i4.hip) or with K split inside a
-// workgroup (gemm_i4_slices.hip); fp16 weights (gemm_i4.hip).
+// MFMA GEMMs for M > 16: exact integer weights dealt by units (gemm_i4_exact.hip; short ranges of
+// products with fp16 x and f32 x rounded to fp16: gemm_i4.hip) or with K split inside a workgroup
+// (gemm_i4_slices.hip); fp16 weights (gemm_i4.hip).
 int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
                              bool* handled);
+int32_t linear_i4_gemm_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
+                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
+                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
+                              bool* handled);
 int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                             krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                             int32_t io_dtype, int32_t scale_dtype, int32_t compute,
@@ -1346,6 +1351,9 @@ int32_t krm_linear_i4(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_bu
   bool handled = false;
   KRM_TRY(linear_i4_gemm_exact(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
                                scale_dtype, compute, &handled));
+  if (handled) return KRM_OK;
+  KRM_TRY(linear_i4_gemm_staged(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
+                                scale_dtype, compute, &handled));
   if (handled) return KRM_OK;
   KRM_TRY(linear_i4_gemm_slices(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
                                 compute, RowsFusion{}, &handled, io_dtype));

@@ -222,8 +222,10 @@ int32_t krm_ctx_create_on_stream(int32_t device, void* hip_stream, krm_ctx** out
   if (st == hipSuccess)
     st = hipMalloc(reinterpret_cast<void**>(&ctx->row_scales),
                    (size_t)kMaxSplitRows * 2 * sizeof(float));
+  if (st == hipSuccess) st = hipMalloc(&ctx->x_planes, kPlaneBytes);
   if (st == hipSuccess) st = hipDeviceSynchronize();
   if (st != hipSuccess) {
+    if (ctx->x_planes) (void)hipFree(ctx->x_planes);
     if (ctx->row_scales) (void)hipFree(ctx->row_scales);
     if (ctx->gemm_partials) (void)hipFree(ctx->gemm_partials);
     if (ctx->tickets) (void)hipFree(ctx->tickets);
@@ -245,6 +247,7 @@ int32_t krm_ctx_create(int32_t device, krm_ctx** out) {
   // Default priority on purpose: mixed stream priorities are not used anywhere.
   hipError_t st = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
   if (st != hipSuccess) {
+    (void)hipFree(ctx->x_planes);
     (void)hipFree(ctx->row_scales);
     (void)hipFree(ctx->gemm_partials);
     (void)hipFree(ctx->tickets);
@@ -273,6 +276,7 @@ int32_t krm_ctx_destroy(krm_ctx* ctx) {
   if (ctx->tickets) (void)hipFree(ctx->tickets);
   if (ctx->gemm_partials) (void)hipFree(ctx->gemm_partials);
   if (ctx->row_scales) (void)hipFree(ctx->row_scales);
+  if (ctx->x_planes) (void)hipFree(ctx->x_planes);
   delete ctx;
   return KRM_OK;
 }

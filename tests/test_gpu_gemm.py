@@ -511,3 +511,35 @@ def test_wide_short_products_on_either_form(gpu_ctx, m, n, k, g, mode):
         assert np.all(err <= bound), float(np.max(err / bound))
     for b in (dx, dw, ds, out):
         b.free()
+
+
+# (fp16: 128 x 256 tiles with a K that ends half-way through a stage; 64 x 512 tiles of M = 64; the f32
+# class: 64 x 512 tiles at ranges of a few stages and, with K of 16384, rows in two blocks because the hi
+# and lo planes of all do not fit their scratch, the second block overlapping the first)
+@pytest.mark.parametrize("m,n,k,g,mode", [(330, 20011, 1344, 64, "f16"), (257, 24577, 1408, 128, "f16"),
+                                          (64, 25001, 8128, 64, "f16"), (330, 11300, 448, 64, "f32"),
+                                          (257, 7001, 2048, 128, "f32"), (129, 16300, 1344, 64, "f32"),
+                                          (1100, 1601, 16384, 256, "f32")])
+def test_unit_dealt_products_at_the_edges_of_their_tiles(gpu_ctx, m, n, k, g, mode):
+    """Ragged tiles, shared tiles and K tails of the unit-dealt forms, f32 and fp16 scales, with bias, at
+    the gate of the exact-operand kernels; the same bits from every run."""
+    rng = np.random.default_rng(m + n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    scale = scale.astype(np.float32 if m % 2 else np.float16)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[m // 2] *= 1e3 if mode == "f32" else 10
+    bias = rng.normal(size=n).astype(np.float32)
+    if mode == "f16":
+        x, bias = x.astype(np.float16), bias.astype(np.float16)
+    seen = x.astype(np.float32)
+    compute = ka.COMPUTE_F32 if mode == "f32" else ka.COMPUTE_F16
+    got = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g, compute=compute)
+    again = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g, compute=compute)
+    assert np.array_equal(got.view(np.uint8), again.view(np.uint8))
+    cols = np.unique(np.concatenate([rng.choice(n, size=64), [0, 255, 256, 511, 512, n - 2, n - 1]]))
+    want = sampled_oracle(seen, packed, scale.astype(np.float32), bias.astype(np.float32), n, k, g, cols)
+    bound = row_gate(seen) + 1e-5 * np.abs(want)
+    if mode == "f16":
+        bound = bound + 2.0 ** -11 * np.abs(want) + 1e-7
+    err = np.abs(got[:, cols].astype(np.float64) - want)
+    assert np.all(err <= bound), float(np.max(err / bound))
