@@ -94,6 +94,14 @@ template <int N>
 __device__ inline void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// silu(gate) * up with the roundings of the decode row's epilogue
+__device__ inline float silu_times(float gate, float up) {
+  const float t = __builtin_amdgcn_exp2f(-fabsf(gate) * 1.4426950408889634f);
+  const float r = __builtin_amdgcn_rcpf(1.0f + t);
+  const float sig = gate < 0.f ? t * r : r;
+  return __fmul_rn(__fmul_rn(gate, sig), up);
+}
+
 // Columns (col, col + 1) of output row `row`, summed: bias, then what the call asked for.
 template <typename T>
 __device__ inline void finish_pair(float v0, float v1, uint32_t row, uint32_t col, uint32_t m,
@@ -106,11 +114,7 @@ __device__ inline void finish_pair(float v0, float v1, uint32_t row, uint32_t co
     if (two) v1 += to_f32<T>(bias[col + 1]);
   }
   if (fuse.mode == 1) {
-    // (gate, up) -> silu(gate) * up, the roundings of the decode row's epilogue
-    const float t = __builtin_amdgcn_exp2f(-fabsf(v0) * 1.4426950408889634f);
-    const float r = __builtin_amdgcn_rcpf(1.0f + t);
-    const float sig = v0 < 0.f ? t * r : r;
-    float value = __fmul_rn(__fmul_rn(v0, sig), v1);
+    float value = silu_times(v0, v1);
     const size_t at = (size_t)row * (n >> 1) + (col >> 1);
     if (residual) value += to_f32<T>(residual[at]);
     out[at] = from_f32<T>(value);
@@ -152,6 +156,124 @@ __device__ inline void finish_pair(float v0, float v1, uint32_t row, uint32_t co
   }
 }
 
+// Four elements next to each other, as wide as they are aligned (`quads_aligned` below).
+template <typename T>
+__device__ inline float4 load_quad(const T* p) {
+  if constexpr (sizeof(T) == 4) {
+    return *reinterpret_cast<const float4*>(p);
+  } else {
+    const uint2 raw = *reinterpret_cast<const uint2*>(p);
+    const half2_t a = __builtin_bit_cast(half2_t, raw.x), b = __builtin_bit_cast(half2_t, raw.y);
+    return make_float4((float)a.x, (float)a.y, (float)b.x, (float)b.y);
+  }
+}
+template <typename T>
+__device__ inline void store_pair(T* p, float v0, float v1) {
+  if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<float2*>(p) = make_float2(v0, v1);
+  } else {
+    *reinterpret_cast<uint32_t*>(p) =
+        __builtin_bit_cast(uint32_t, half2_t{(_Float16)v0, (_Float16)v1});
+  }
+}
+template <typename T>
+__device__ inline void store_quad(T* p, float v0, float v1, float v2, float v3) {
+  if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<float4*>(p) = make_float4(v0, v1, v2, v3);
+  } else {
+    *reinterpret_cast<uint2*>(p) =
+        make_uint2(__builtin_bit_cast(uint32_t, half2_t{(_Float16)v0, (_Float16)v1}),
+                   __builtin_bit_cast(uint32_t, half2_t{(_Float16)v2, (_Float16)v3}));
+  }
+}
+// Columns col .. col + 3 (a multiple of 4, all below n) of a row at once: what the end of the
+// product reads from memory, asked for while the sums are still on their way through LDS, and the
+// same arithmetic as finish_pair behind them.
+struct QuadAhead {
+  float4 bias, residual;
+  float2 cos[2], sin[2];  // mode 2: of dims j, j + 1 and of j + D/2, j + 1 + D/2
+};
+template <typename T>
+__device__ inline void fetch_quad(QuadAhead& q, uint32_t row, uint32_t col, uint32_t n, int32_t pos,
+                                  const T* bias, const RowsFusion& fuse) {
+  if (bias) q.bias = load_quad<T>(bias + col);
+  const T* residual = static_cast<const T*>(fuse.residual);
+  if (fuse.mode == 2) {
+    const uint32_t half = fuse.depth >> 1, pair = col >> 1;
+    if (pair < (fuse.heads + fuse.kv_heads) * half && pos >= 0 && (uint32_t)pos < fuse.table_rows) {
+      const size_t t = (size_t)pos * fuse.depth + pair % half;
+      q.cos[0] = *reinterpret_cast<const float2*>(fuse.cos_table + t);
+      q.sin[0] = *reinterpret_cast<const float2*>(fuse.sin_table + t);
+      q.cos[1] = *reinterpret_cast<const float2*>(fuse.cos_table + t + half);
+      q.sin[1] = *reinterpret_cast<const float2*>(fuse.sin_table + t + half);
+    }
+  } else if (residual && fuse.mode == 0) {
+    q.residual = load_quad<T>(residual + (size_t)row * n + col);
+  } else if (residual) {
+    const size_t at = (size_t)row * (n >> 1) + (col >> 1);
+    q.residual.x = to_f32<T>(residual[at]);
+    q.residual.y = to_f32<T>(residual[at + 1]);
+  }
+}
+template <typename T>
+__device__ inline void finish_quad(float4 v, const QuadAhead& q, uint32_t row, uint32_t col,
+                                   uint32_t m, uint32_t n, int32_t pos, bool bias, T* out,
+                                   const RowsFusion& fuse) {
+  if (bias) {
+    v.x += q.bias.x; v.y += q.bias.y; v.z += q.bias.z; v.w += q.bias.w;
+  }
+  if (fuse.mode == 0) {
+    if (fuse.residual) {
+      v.x += q.residual.x; v.y += q.residual.y; v.z += q.residual.z; v.w += q.residual.w;
+    }
+    store_quad<T>(out + (size_t)row * n + col, v.x, v.y, v.z, v.w);
+  } else if (fuse.mode == 1) {
+    float a = silu_times(v.x, v.y), b = silu_times(v.z, v.w);
+    if (fuse.residual) { a += q.residual.x; b += q.residual.y; }
+    store_pair<T>(out + (size_t)row * (n >> 1) + (col >> 1), a, b);
+  } else {
+    // what a separate linear would have stored, then the rotation
+    auto stored = [](float x) { return to_f32<T>(from_f32<T>(x)); };
+    const float x[2][2] = {{stored(v.x), stored(v.y)}, {stored(v.z), stored(v.w)}};
+    const uint32_t half = fuse.depth >> 1, pair = col >> 1;
+    const uint32_t rope_pairs = (fuse.heads + fuse.kv_heads) * half;
+    if (pair < rope_pairs) {
+      const uint32_t head = pair / half, j = pair - head * half;
+      float lo[2] = {NAN, NAN}, hi[2] = {NAN, NAN};  // outside the table: never a valid rotation
+      if (pos >= 0 && (uint32_t)pos < fuse.table_rows) {
+        const float c0[2] = {q.cos[0].x, q.cos[0].y}, s0[2] = {q.sin[0].x, q.sin[0].y};
+        const float c1[2] = {q.cos[1].x, q.cos[1].y}, s1[2] = {q.sin[1].x, q.sin[1].y};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          lo[i] = __fadd_rn(__fmul_rn(x[i][0], c0[i]), __fmul_rn(-x[i][1], s0[i]));
+          hi[i] = __fadd_rn(__fmul_rn(x[i][1], c1[i]), __fmul_rn(x[i][0], s1[i]));
+        }
+      }
+      T* dst = head < fuse.heads
+                   ? static_cast<T*>(fuse.q_out) + ((size_t)head * m + row) * fuse.depth
+                   : static_cast<T*>(fuse.k_out) + ((size_t)(head - fuse.heads) * m + row) * fuse.depth;
+      store_pair<T>(dst + j, lo[0], lo[1]);
+      store_pair<T>(dst + j + half, hi[0], hi[1]);
+    } else {
+      const uint32_t e = (pair - rope_pairs) * 2u;
+      const uint32_t plane = e / fuse.depth, d = e - plane * fuse.depth;
+      store_quad<T>(static_cast<T*>(fuse.v_out) + ((size_t)plane * m + row) * fuse.depth + d, x[0][0],
+                    x[0][1], x[1][0], x[1][1]);
+    }
+  }
+}
+// Whether quads of columns may be read and written at once: n in whole quads, rows and buffers
+// aligned to them (a rope table to the pairs it is read in).
+inline bool quads_aligned(const void* bias, const void* out, uint32_t n, size_t eb,
+                          const RowsFusion& fuse) {
+  auto at = [](const void* p, size_t bytes) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; };
+  if (n % 4 != 0 || !at(bias, 4 * eb)) return false;
+  if (fuse.mode == 2)
+    return fuse.depth % 4 == 0 && at(fuse.cos_table, 8) && at(fuse.sin_table, 8) &&
+           at(fuse.q_out, 2 * eb) && at(fuse.k_out, 2 * eb) && at(fuse.v_out, 4 * eb);
+  return fuse.mode == 0 ? at(out, 4 * eb) && at(fuse.residual, 4 * eb) : at(out, 2 * eb);
+}
+
 template <typename T>
 struct type_tag { using type = T; };
 
@@ -159,6 +281,7 @@ struct SliceTail {         // what the end of the kernel needs
   const void* bias;
   void* out;
   const float* row_scale;  // kXSplit
+  uint32_t quads;          // quads_aligned
   RowsFusion fuse;
 };
 

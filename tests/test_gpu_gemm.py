@@ -543,3 +543,77 @@ def test_unit_dealt_products_at_the_edges_of_their_tiles(gpu_ctx, m, n, k, g, mo
         bound = bound + 2.0 ** -11 * np.abs(want) + 1e-7
     err = np.abs(got[:, cols].astype(np.float64) - want)
     assert np.all(err <= bound), float(np.max(err / bound))
+
+
+@pytest.mark.parametrize("io", [ka.F16, ka.F32])
+@pytest.mark.parametrize("compute", [ka.COMPUTE_F16, ka.COMPUTE_F32])
+@pytest.mark.parametrize("m,n,k,silu", [(17, 4, 64, False), (33, 64, 128, True), (50, 96, 576, False),
+                                        (128, 2048, 2048, False), (128, 11264, 256, True),
+                                        (300, 260, 1152, True)])
+def test_quads_and_pairs_of_columns_are_finished_alike(gpu_ctx, io, compute, m, n, k, silu):
+    """A finished sum is stored four columns at a time where rows and buffers are aligned to that, two
+    at a time elsewhere: the same bits, with a bias and (in place) a residual, for one tile of a few
+    columns, tiles that are cut off and waves that own no codes (k of 64 and 128)."""
+    rng = np.random.default_rng(m + n + k)
+    group = 64
+    io_np = np.float32 if io == ka.F32 else np.float16
+    eb, n_out = np.dtype(io_np).itemsize, n // 2 if silu else n
+    packed, _codes, scales = helpers.synthetic_int4(rng, n, k, group)
+    x = rng.normal(size=(m, k)).astype(io_np)
+    bias, residual = rng.normal(size=n).astype(io_np), rng.normal(size=m * n_out).astype(io_np)
+    dx, dw, ds = map(gpu_ctx.upload, (x, packed, scales))
+    got = []
+    for shift in (0, 1):     # in elements
+        pad = np.zeros(shift, dtype=io_np)
+        db = gpu_ctx.upload(np.concatenate([pad, bias]))
+        out = gpu_ctx.upload(np.concatenate([pad, residual]))
+        at = out.offset(shift * eb)
+        gpu_ctx.linear_i4_rows(dx, dw, ds, at, m, n, k, group, bias=db.offset(shift * eb), residual=at,
+                               io_dtype=io, scale_dtype=ka.F16, compute=compute,
+                               epilogue=ka.EPILOGUE_SILU_PAIRS if silu else ka.EPILOGUE_NONE)
+        got.append(out.download(io_np, (shift + m * n_out,))[shift:].reshape(m, n_out))
+    bits = np.uint32 if io == ka.F32 else np.uint16
+    assert np.isfinite(got[0]).all()
+    assert np.array_equal(got[0].view(bits), got[1].view(bits))
+    if not silu:
+        want = oracle.linear_i4(x.astype(np.float32), packed, scales.astype(np.float32),
+                                bias.astype(np.float32), n, k, group) + residual.reshape(m, n)
+        # (f32 sums of exact products; x rounded to fp16 in that class, and the fp16 result)
+        half = io == ka.F16 or compute == ka.COMPUTE_F16
+        err, rms = np.abs(got[0] - want), float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+        assert float(np.max(err - (2e-3 if half else 3e-5) * (np.abs(want) + rms))) <= 0.0
+
+
+@pytest.mark.parametrize("io", [ka.F16, ka.F32])
+@pytest.mark.parametrize("m,heads,kv_heads,d", [(17, 1, 1, 4), (40, 3, 1, 12), (128, 32, 4, 64),
+                                                (130, 4, 2, 6)])
+def test_rope_of_a_fused_projection_by_quads_and_by_pairs(gpu_ctx, io, m, heads, kv_heads, d):
+    """The rotation reads its table rows two dims at a time where the tables are aligned to that:
+    the bits of one dim at a time (tables a float off; a head dim of 6 has no quads at all)."""
+    rng = np.random.default_rng(m + d)
+    n, k, group, table = (heads + 2 * kv_heads) * d, 256, 64, 50
+    io_np = np.float32 if io == ka.F32 else np.float16
+    eb = np.dtype(io_np).itemsize
+    packed, _codes, scales = helpers.synthetic_int4(rng, n, k, group)
+    x = rng.normal(size=(m, k)).astype(io_np)
+    bias = rng.normal(size=n).astype(io_np)
+    ang = rng.normal(size=table * d)
+    pos = rng.integers(0, table, size=m).astype(np.int32)
+    pos[m // 2] = table                           # outside the table: NaN in q and k
+    dx, dw, ds, db, dp = map(gpu_ctx.upload, (x, packed, scales, bias, pos))
+    got = []
+    for shift in (0, 1):
+        pad = np.zeros(shift, dtype=np.float32)
+        cos, sin = (gpu_ctx.upload(np.concatenate([pad, f(ang).astype(np.float32)]))
+                    for f in (np.cos, np.sin))
+        q, kk, v = (gpu_ctx.zeros(m * planes * d * eb) for planes in (heads, kv_heads, kv_heads))
+        gpu_ctx.prefill_qkv(dx, dw, ds, dp, cos.offset(4 * shift), sin.offset(4 * shift), q, kk, v,
+                            bias=db, m=m, heads=heads, kv_heads=kv_heads, depth=d, k=k, group=group,
+                            table_rows=table, io_dtype=io, scale_dtype=ka.F16, compute=ka.COMPUTE_F32)
+        got.append([b.download(io_np, (planes, m, d)) for b, planes in
+                    ((q, heads), (kk, kv_heads), (v, kv_heads))])
+    bits = np.uint32 if io == ka.F32 else np.uint16
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(bits), b.view(bits))
+    assert np.isnan(got[0][0][:, m // 2]).all() and np.isfinite(got[0][2]).all()
+    assert np.isfinite(np.delete(got[0][0], m // 2, 1)).all()
