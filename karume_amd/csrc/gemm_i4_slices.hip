@@ -26,7 +26,7 @@
 // over all banks.
 //
 // What bounds it: what the second-level cache delivers to a CU (tiles of 64 x 96: 2 * 64 + 96 / 2
-// bytes a code), then the conversion of the weights on the vector ALUs (12 operations a word).
+// bytes a code), then the conversion of the weights on the vector ALUs (10 operations a word, 9 beside hi + lo planes).
 // Measured on cold weights, fp16 x (f32 class in brackets), against the kernel that loaded through
 // registers, one 32 x 32 or 32 x 64 tile a workgroup: 128 x 2560 x 2048 6.6 us, 9.6 before (11.8,
 // 14.5); 128 x 2048 x 2048 5.4, 7.0 (10.1, 12.5); 128 x 11264 x 2048 15.1, 27.0 (25.9, 38.6); 128 x
@@ -551,7 +551,10 @@ void gemm_i4_slices_kernel(
         if constexpr (XKIND == kXSplit) {  // exact: a power of two
           v.x *= inv[i]; v.y *= inv[i]; v.z *= inv[i]; v.w *= inv[i];
         }
-        if constexpr (XKIND == kXThree) { v.x *= 16.f; v.y *= 16.f; v.z *= 16.f; v.w *= 16.f; }
+        if constexpr (XKIND != kXSplit) {  // the weights went in as sixteenths or 1024ths
+          constexpr float kWhole = XKIND == kXThree ? 16.f : 1024.f;
+          v.x *= kWhole; v.y *= kWhole; v.z *= kWhole; v.w *= kWhole;
+        }
         if (tail.quads) {
           finish_quad<T>(v, ahead[i], row, col, m, n, pos[i], bias != nullptr, out, tail.fuse);
         } else {
