@@ -180,9 +180,16 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 //
 // A chunk of M > 1 rows with D = 64 or 128 (a prefill step): workgroup = (plane z, 16 query
 // rows), WAVES waves; the key columns the 16 rows can see are walked in blocks of 32 and wave w
-// takes blocks w, w + WAVES, ...  All arithmetic is f32 (v_mfma_f32_16x16x4_f32: f32 products,
-// f32 sums), the operand roundings are the generic kernel's: q * scale and k * scale are
-// rounded before the product.  With g = lane / 16:
+// takes blocks w, w + WAVES, ...  Products and sums are f32's.  Rows of f32 (the state's, or this step's
+// beside an fp16 state) run on v_mfma_f32_16x16x4_f32 with the generic kernel's operand roundings: q *
+// scale and k * scale are rounded before the product.  Blocks of fp16 rows run on
+// v_mfma_f32_16x16x32_f16, sixteen times that rate, with no fewer bits: K and V are fp16 as they are, q is
+// fp16 or three fp16 parts of the row times a power of two (33 bits), a probability two parts of p 2^15
+// (22 bits of p, 2^-39 where it is small), products are exact, sums f32, scale^2 multiplies the f32 sum.
+// Error against 64 bits (2-norm, f32 queries, normal values; f32 operands before): D = 64 behind 1024
+// 2.4e-7 (3.7e-7), D = 128 2.8e-7 (4.7e-7), D = 256 3.5e-7 (6.2e-7).  A part of zero beside an infinity
+// of the state is a NaN that the value itself would not give: a wave whose walk leaves a NaN walks again
+// with f32 operands.  With g = lane / 16:
 //   S^T = K Q^T    two tiles of 16 keys; A = the K tile (row = key, lane group g walks dims
 //                  g D/4 ..), B = Q^T (column = query row): a lane ends up with the scores of
 //                  ONE query row (lane % 16) against keys 16 t + 4 g + i (t < 2, i < 4), so the
@@ -192,18 +199,24 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 //                  given the keys 16 t + 4 g + i, so the probabilities never move; V^T is the A
 //                  operand with the same key per step: 16 lanes take that key's row 16 bytes each
 //                  and keep it in registers (a piece's four dims feed four output tiles), so V
-//                  needs no LDS at all.
+//                  needs no LDS at all (fp16: the eight keys of a dim, two to a register, are one
+//                  operand of 32 keys).
 // The K block is parked in the wave's own LDS area (coalesced 16-byte loads; a block may straddle
 // the state slot and this step's rows): read as an operand from memory it came in half lines,
 // half as fast.  D = 64: the next block's rows are asked for as soon as this one's are used.  The
 // waves' (max, sum, O) are merged in LDS at the end; rows >= query are written as +0.  Sixteen
 // rows a workgroup (not 32) so that a 128-row chunk of 32 heads is 256 workgroups, one per CU.
-// What bounds it is the f32 matrix rate with two waves a SIMD to cover softmax and waits (D = 64,
-// r = 8, 128 rows behind 1024: 8 us of MFMA).  With V parked as well, rows looked up one by one
-// (two element types: a wait at each), expf and no requests ahead, us before / now: that case
+// What bounds f32 rows is their matrix rate with two waves a SIMD to cover softmax and waits (D = 64,
+// r = 8, 128 rows behind 1024: 8 us of MFMA), fp16 rows the vector instructions of softmax and operands.
+// us with f32 operands / with fp16 ones, 128 rows behind 1024 and 512 behind 2048: fp16 D = 64 19.6 /
+// 10.1, 120 / 50; D = 128, r = 4 34.7 / 17.5, 236 / 102; D = 256 72 / 33, 148 / 64; f32 queries D = 64
+// 21.6 / 15.3, 132 / 75; D = 128 38.5 / 22.1, 267 / 140; D = 256 77 / 46, 161 / 97.  Before those f32
+// forms, with V parked as well, rows looked up one by one (two element types: a wait at each), expf and no
+// requests ahead, us before / with f32 operands: the case of 8 us of MFMA
 // 22.7 / 19.3; fp16, D = 128, r = 4: 49.4 / 32.6; f32 over fp16 slots 106.5 / 36.8; D = 256, r = 8
 // (two waves then, four now that LDS holds K alone): 172 / 71.
 typedef float float4v_t __attribute__((ext_vector_type(4)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
 template <typename T>
 __device__ inline float4 load4_f32(const T* p);
@@ -283,7 +296,16 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   constexpr int kPieces = D / 4;              // 4-element pieces of a row
   constexpr int kRowsPerLoad = 64 / kPieces;
   constexpr int kLoads = 32 / kRowsPerLoad;
+  // State rows of fp16 are products of fp16 operands: see `half_block` below.
+  constexpr bool kHalf = sizeof(ST) == 2;
+  constexpr int kHalfRow = D + 8;             // halves of a parked row
+  constexpr int kPParts = 2;
+  constexpr float kPScale = 32768.0f;
+  constexpr int kQParts = sizeof(XT) == 2 ? 1 : 3, kSteps = D / 32;
   __shared__ __align__(16) float s_k[WAVES][32 * kRow];
+  constexpr bool kSplitQ = kHalf && sizeof(XT) == 4;
+  __shared__ __align__(16) __half s_q[kSplitQ ? kQParts * kRows * kHalfRow : 8];  // the parts of Q
+  __shared__ float s_factor[kSplitQ ? kRows : 1];                                // scale^2 2^-e of a row
   __shared__ float s_m[WAVES][kRows], s_l[WAVES][kRows];
 
   const uint32_t z = blockIdx.x, row0 = blockIdx.y * (uint32_t)kRows;
@@ -317,10 +339,22 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   const uint32_t kv_plane = __builtin_amdgcn_readfirstlane(z / (a.heads / a.kv_heads));
 
   // Q block: asked for first, parked (scaled) behind the request of the wave's first key block
+  // (fp16 beside fp16 state rows: each lane's operand pieces instead, which never see the LDS)
   constexpr int kQUnits = kRows * kPieces, kQPer = (kQUnits + (int)kBlock - 1) / (int)kBlock;
+  constexpr bool kQDirect = kHalf && sizeof(XT) == 2;
+  half8_t qh[kQDirect ? RB : 1][kQDirect ? kSteps : 1];
+  if constexpr (kQDirect) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const uint32_t row = min(row0 + 16u * rb + r, a.chunk_rows - 1);
+#pragma unroll
+      for (int i = 0; i < kSteps; ++i)
+        qh[rb][i] = *reinterpret_cast<const half8_t*>(q + ((size_t)z * a.chunk_rows + row) * D + 32 * i + 8 * g);
+    }
+  }
   uint4 qraw[kQPer];
 #pragma unroll
-  for (int j = 0; j < kQPer; ++j) {
+  for (int j = 0; j < kQPer && !kQDirect; ++j) {
     const uint32_t i = min((uint32_t)tid + j * kBlock, (uint32_t)kQUnits - 1u);
     const uint32_t row = min(row0 + i / kPieces, a.chunk_rows - 1);
     qraw[j] = load4_raw<XT>(q + ((size_t)z * a.chunk_rows + row) * D + 4 * (i % kPieces));
@@ -367,7 +401,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   // `keys` lane rows, row i the block's key lane_key + step_of(i), `pieces` pieces of 4 elements 64
   // apart
   auto request = [&](uint32_t kb, const ST* slot, const XT* ins, auto keys, uint32_t lane_key,
-                     auto step_of, uint32_t lane_dim, auto pieces, uint4* raw) {
+                     auto step_of, uint32_t lane_dim, auto pieces, auto& raw) __attribute__((always_inline)) {
     lane_key = lane_number(lane_key);
     constexpr int kKeys = decltype(keys)::value, kPer = decltype(pieces)::value;
     const uint64_t c0 = c_lo + (uint64_t)kb * 32u;
@@ -410,12 +444,12 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   };
   auto v_step = [](int j) -> uint32_t { return (uint32_t)(16 * (j / 4) + j % 4); };
   uint4 kraw[kLoads], vraw[8 * kVPieces];
-  auto request_k = [&](uint32_t kb) {
+  auto request_k = [&](uint32_t kb) __attribute__((always_inline)) {
     request(kb, slot_k, ins_k, std::integral_constant<int, kLoads>{}, load_key,
             [](int i) { return (uint32_t)(i * kRowsPerLoad); }, load_piece,
             std::integral_constant<int, 1>{}, kraw);
   };
-  auto request_v = [&](uint32_t kb) {
+  auto request_v = [&](uint32_t kb) __attribute__((always_inline)) {
     request(kb, slot_v, ins_v, std::integral_constant<int, 8>{}, 4u * g, v_step, 4u * r,
             std::integral_constant<int, kVPieces>{}, vraw);
   };
@@ -430,36 +464,74 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
                          in_slot ? s4.w : x4.w);
     }
   };
-  // (longer rows: the next block's beside this one's would take the registers of the state)
-  constexpr bool kAhead = D * sizeof(XT) * sizeof(ST) <= 64 * 16;
+  // (longer rows: the next block's beside this one's would take the registers of the state; f32 queries
+  // beside fp16 rows of 128 spill with it, 128 rows behind 1024 24.7 us, 22.1 without)
+  constexpr bool kAhead = D * sizeof(XT) * sizeof(ST) <= 64 * 16 && !(kSplitQ && D > 64);
   if (kAhead && (uint32_t)wave < blocks) {
     request_k((uint32_t)wave);
     request_v((uint32_t)wave);
   }
 
   // each lane's B operands: Q[r][g * D/4 + s]
+  float qf[RB][kQDirect ? 1 : kQuarter];
+  if constexpr (!kQDirect) {
+    const bool split = kSplitQ && slot_columns(c_lo) == 32u;  // (no fp16 block, nothing to split)
 #pragma unroll
-  for (int j = 0; j < kQPer; ++j) {
-    const uint32_t i = (uint32_t)tid + j * kBlock;
-    float4 v = raw4_f32<XT>(qraw[j]);
-    v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
-    if (i < (uint32_t)kQUnits)
-      *reinterpret_cast<float4*>(&s_k[0][(i / kPieces) * kRow + 4 * (i % kPieces)]) = v;
-  }
-  __syncthreads();
-  float qf[RB][kQuarter];
+    for (int j = 0; j < kQPer; ++j) {
+      const uint32_t i = (uint32_t)tid + j * kBlock;
+      float4 v = raw4_f32<XT>(qraw[j]);
+      if (split) {
+        // The row times 2^e, its largest magnitude in [2^13, 2^14), as three fp16 parts (33 bits).  A
+        // row lies in kPieces neighbouring lanes.
+        float top = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
+        for (int off = 1; off < kPieces; off <<= 1) top = fmaxf(top, __shfl_xor(top, off, kWave));
+        const int biased = (int)(__float_as_uint(top) >> 23);
+        float up = 1.f, down = 1.f;
+        if (top != 0.f && biased != 255) {
+          int power = 13 - (biased - 127);
+          power = power > 100 ? 100 : power < -100 ? -100 : power;  // (2^-e scale^2 stays normal)
+          up = __uint_as_float((uint32_t)(127 + power) << 23);
+          down = __uint_as_float((uint32_t)(127 - power) << 23);
+        }
+        float left[4] = {v.x * up, v.y * up, v.z * up, v.w * up};  // exact: a power of two
+        if (i < (uint32_t)kQUnits) {
+          if (i % kPieces == 0) s_factor[i / kPieces] = a.scale * a.scale * down;
 #pragma unroll
-    for (int i = 0; i < kQuarter / 4; ++i) {
-      const float4 v = *reinterpret_cast<const float4*>(
-          &s_k[0][(16 * rb + r) * kRow + g * kQuarter + 4 * i]);
-      qf[rb][4 * i] = v.x; qf[rb][4 * i + 1] = v.y; qf[rb][4 * i + 2] = v.z; qf[rb][4 * i + 3] = v.w;
+          for (int p = 0; p < kQParts; ++p) {
+            __half* to = s_q + (p * kRows + i / kPieces) * kHalfRow + 4 * (i % kPieces);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const __half part = __float2half_rn(left[e]);
+              to[e] = part;
+              left[e] -= __half2float(part);
+            }
+          }
+        }
+      }
+      v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
+      if (i < (uint32_t)kQUnits)
+        *reinterpret_cast<float4*>(&s_k[0][(i / kPieces) * kRow + 4 * (i % kPieces)]) = v;
     }
-  __syncthreads();
+    __syncthreads();
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int i = 0; i < kQuarter / 4; ++i) {
+        const float4 v = *reinterpret_cast<const float4*>(
+            &s_k[0][(16 * rb + r) * kRow + g * kQuarter + 4 * i]);
+        qf[rb][4 * i] = v.x; qf[rb][4 * i + 1] = v.y; qf[rb][4 * i + 2] = v.z; qf[rb][4 * i + 3] = v.w;
+      }
+    __syncthreads();
+  }
 
   float run_m[RB], run_l[RB];
   float4v_t acc[RB][DT];
+  // One walk over the wave's key blocks: kNever, kAlways or (f32 queries: this step's own rows are f32)
+  // kSlotBlocks with fp16 operands.
+  enum { kNever, kAlways, kSlotBlocks };
+  auto walk = [&](auto mode_tag) __attribute__((always_inline)) {
+    constexpr int kMode = decltype(mode_tag)::value;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     run_m[rb] = -INFINITY;
@@ -477,6 +549,16 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     if constexpr (!kAhead) request_k(kb);
     const uint32_t slots = slot_columns(c0);
     const uint32_t parked_key = lane_number(load_key);
+    // Every key of the block is fp16 as it lies in memory: it is parked so, and K Q^T and V^T P^T run
+    // on v_mfma_f32_16x16x32_f16, sixteen times the rate of f32 operands.
+    const bool half_block = kMode == kAlways || (kMode == kSlotBlocks && slots == 32u);
+    if (half_block) {
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j)
+        *reinterpret_cast<uint2*>(reinterpret_cast<__half*>(mk) +
+                                  (j * kRowsPerLoad + parked_key) * kHalfRow + load_piece) =
+            make_uint2(kraw[j].x, kraw[j].y);
+    } else
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const uint32_t key = j * kRowsPerLoad + parked_key;
@@ -500,8 +582,41 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) st[t][i] = 0.f;
+      if (half_block) {
+        const __half* keys = reinterpret_cast<const __half*>(mk) + r * kHalfRow + 8 * g;
+        const float factor = kQDirect ? a.scale * a.scale : s_factor[kSplitQ ? 16 * rb + r : 0];
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) {
+          half8_t qs[kQParts];
+#pragma unroll
+          for (int p = 0; p < kQParts; ++p)
+            qs[p] = kQDirect ? qh[kQDirect ? rb : 0][kQDirect ? i : 0]
+                             : *reinterpret_cast<const half8_t*>(
+                                   s_q + (p * kRows + 16 * rb + r) * kHalfRow + 32 * i + 8 * g);
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const half8_t kh = *reinterpret_cast<const half8_t*>(keys + 16 * t * kHalfRow + 32 * i);
+#pragma unroll
+            for (int p = kQParts - 1; p >= 0; --p)
+              st[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qs[p], st[t], 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[t][i] *= factor;
+      } else
 #pragma unroll
       for (int i = 0; i < kQuarter / 4; ++i) {
+        float qs[4];
+        if constexpr (kQDirect) {  // (the walk behind a NaN)
+          const uint32_t row = min(row0 + (uint32_t)(16 * rb + r), a.chunk_rows - 1);
+          const float4 v = load4_f32<XT>(q + ((size_t)z * a.chunk_rows + row) * D + g * kQuarter + 4 * i);
+          qs[0] = v.x * a.scale; qs[1] = v.y * a.scale; qs[2] = v.z * a.scale; qs[3] = v.w * a.scale;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) qs[j] = qf[rb][4 * i + j];
+        }
         float kf[2][4];
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -511,7 +626,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int t = 0; t < 2; ++t)
-            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][j], qf[rb][4 * i + j], st[t], 0, 0, 0);
+            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][j], qs[j], st[t], 0, 0, 0);
       }
       // this lane: query row 16 rb + r, keys 16 t + 4 g + i
       // (uniform: a block that every one of these rows sees whole needs no mask)
@@ -554,6 +669,43 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
         for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= alpha;
       // (tile dt = 4 i + e holds the dims 64 i + 4 r + e: a 16-byte piece feeds four tiles)
       const uint32_t pv_key = lane_number(4u * g);
+      if constexpr (kHalf) {  // (the sums of V are kept times 2^15: small probabilities keep their bits)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) p[t][i] *= kPScale;
+      }
+      if (half_block) {
+        half8_t ph[kPParts];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float left = p[j / 4][j % 4];
+#pragma unroll
+          for (int q = 0; q < kPParts; ++q) {
+            const _Float16 part = (_Float16)left;
+            ph[q][j] = part;
+            left -= (float)part;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < kVPieces; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            uint32_t pair[4];  // dim e of the pieces of keys 2 q, 2 q + 1
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const uint4& v0 = vraw[2 * q * kVPieces + i];
+              const uint4& v1 = vraw[(2 * q + 1) * kVPieces + i];
+              pair[q] = __builtin_amdgcn_perm(e < 2 ? v1.x : v1.y, e < 2 ? v0.x : v0.y,
+                                              e % 2 ? 0x07060302u : 0x05040100u);
+            }
+            const half8_t vh = __builtin_bit_cast(half8_t, make_uint4(pair[0], pair[1], pair[2], pair[3]));
+#pragma unroll
+            for (int q = kPParts - 1; q >= 0; --q)
+              acc[rb][4 * i + e] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[q], acc[rb][4 * i + e], 0, 0, 0);
+          }
+      } else
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
 #pragma unroll
@@ -569,6 +721,41 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     }
     if (kAhead && more) request_v(kb + (uint32_t)WAVES);
     wave_sync();  // the block's rows have been read: the next block may be parked
+  }
+  };
+  if constexpr (!kHalf) {
+    walk(std::integral_constant<int, kNever>{});
+  } else {
+    bool plain = kSplitQ && slot_columns(c_lo) != 32u;  // no block of fp16 keys
+    if (!plain) {
+      walk(std::integral_constant<int, sizeof(XT) == 2 ? kAlways : kSlotBlocks>{});
+      bool nan = false;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        bool here = run_l[rb] != run_l[rb];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) here = here || acc[rb][dt][i] != acc[rb][dt][i];
+        nan = nan || (here && row0 + (uint32_t)(16 * rb + r) < query);
+      }
+      // (parts of a value meet an infinity of the state as 0 * inf, the value itself does not: once more
+      // without them)
+      plain = __any(nan);
+      if (plain && kAhead && (uint32_t)wave < blocks) {
+        request_k((uint32_t)wave);
+        request_v((uint32_t)wave);
+      }
+    }
+    if (plain) walk(std::integral_constant<int, kNever>{});
+  }
+  if constexpr (kHalf) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= 1.0f / kPScale;
   }
 
   // The chunk's own K / V rows of this block go to the state slots when asked for (the first query
@@ -660,7 +847,6 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 
 // ------------------------------------------------------------------------------ decode
 
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 // Value of lane `src` (0..15) of the caller's 16-lane row, in every lane of that row.

@@ -913,3 +913,79 @@ def test_decode_takes_this_steps_rows_at_any_element(gpu_ctx, shift, past):
         assert np.array_equal(results[0], other)
     for b in [dq, dk, dv, out, ws] + plain + moved:
         b.free()
+
+
+def attention_in_64_bits(q, k, v, past, scale):
+    """One head, no window: rows of q over keys 0 .. past + row."""
+    q, k, v = (a.astype(np.float64) for a in (q, k, v))
+    out = np.empty_like(q)
+    with np.errstate(invalid="ignore"):
+        for r in range(q.shape[0]):
+            s = (k[:past + r + 1] @ q[r]) * scale * scale
+            p = np.exp(s - s.max())
+            out[r] = (p[:, None] * v[:past + r + 1]).sum(axis=0) / p.sum()
+    return out
+
+
+def chunk_over_fp16_state(ctx, q, ik, iv, sk, sv, past, scale):
+    m, depth = q.shape
+    bufs = [ctx.upload(np.ascontiguousarray(a)) for a in (q, ik, iv, sk, sv)]
+    out = ctx.zeros(q.nbytes)
+    ctx.attention_chunk(*bufs, out, batch=1, heads=1, kv_heads=1, chunk_rows=m, depth=depth,
+                        capacity=sk.shape[0], window=0, half_scale=scale, past=past, query=m,
+                        io_dtype=ka.dtype_code(q.dtype), kv_dtype=ka.F16)
+    return out.download(q.dtype, q.shape)
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+@pytest.mark.parametrize("past", [31, 32, 33, 320])
+@pytest.mark.parametrize("io", [np.float32, np.float16])
+def test_chunks_over_an_fp16_state_keep_the_bits_of_f32(gpu_ctx, depth, past, io):
+    """Blocks of 32 fp16 keys run with fp16 operands (the queries and the probabilities in parts): no
+    further from 64 bits than f32 operands are, for rows of 1e4 and of 1e-7 beside ordinary ones, a row
+    with entries eight decades apart, and probabilities down to 2^-30.  f32 operands: every product of
+    a score is rounded three times, 3 * 2^-24 of sum |q k| scale^2 at most, which moves a probability by
+    as much of itself; the rest (exponential, sums over the keys) stays below 2^-20."""
+    rng = np.random.default_rng(depth + past)
+    m, scale = 18, float(np.float32(np.sqrt(1.0 / np.sqrt(float(depth)))))
+    q, ik, iv = (rng.normal(size=(m, depth)).astype(io) for _ in range(3))
+    sk, sv = (rng.normal(size=(past + m + 14, depth)).astype(np.float16) for _ in range(2))
+    if io == np.float32:
+        q[3] *= 1e-7
+        q[4, ::2] *= 1e-8
+        q[5] *= 1e4
+    got = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale)
+    k = np.concatenate([sk[:past].astype(io).astype(np.float64), ik.astype(np.float64)])
+    v = np.concatenate([sv[:past].astype(np.float64), iv.astype(np.float64)])
+    want = attention_in_64_bits(q, k, v, past, scale)
+    moved = 3 * 2.0 ** -24 * (np.abs(q.astype(np.float64)) @ np.abs(k).T).max(axis=1) * scale * scale + 2.0 ** -20
+    bound = 2 * moved[:, None] * np.abs(v).max() + (2.0 ** -10 * np.abs(want) + 1e-7 if io == np.float16 else 0.0)
+    assert np.all(np.abs(got.astype(np.float64) - want) <= bound)
+    if io == np.float32:       # ordinary rows: measured 2.0e-7 to 4.3e-7, f32 operands 3.0e-7 to 7.0e-7
+        rows = [r for r in range(m) if r not in (3, 4, 5)]
+        assert np.linalg.norm(got[rows] - want[rows]) <= 6e-7 * np.linalg.norm(want[rows])
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+@pytest.mark.parametrize("io", [np.float32, np.float16])
+def test_infinities_in_an_fp16_state_reach_what_they_reach_in_f32(gpu_ctx, depth, io):
+    """A key whose score is -inf has no weight, a value of inf is the infinity of its dim, alone: parts of
+    a query or of a probability that are zero (here q of few bits, and the row whose largest probability
+    is 1) do not turn either into a NaN."""
+    rng = np.random.default_rng(depth)
+    past, m, scale = 96, 17, 0.25
+    q = np.abs(rng.integers(1, 3, size=(m, depth))).astype(io)
+    ik, iv = (rng.normal(size=(m, depth)).astype(io) for _ in range(2))
+    sk, sv = (rng.normal(size=(past + m, depth)).astype(np.float16) for _ in range(2))
+    sk[40, 5] = -np.inf
+    sv[70, 9] = np.inf
+    sv[3, 11] = -np.inf
+    got = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale)
+    k = np.concatenate([sk[:past].astype(np.float64), ik.astype(np.float64)])
+    v = np.concatenate([sv[:past].astype(np.float64), iv.astype(np.float64)])
+    want = attention_in_64_bits(q, k, v, past, scale)
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.isposinf(want[:, 9]).all()
+    assert np.array_equal(np.isneginf(got), np.isneginf(want)) and np.isneginf(want[:, 11]).all()
+    rest = np.delete(np.arange(depth), (9, 11))
+    assert np.all(np.abs(got[:, rest].astype(np.float64) - want[:, rest]) <=
+                  1e-5 + (2e-3 if io == np.float16 else 0.0))
