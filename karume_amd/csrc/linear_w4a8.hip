@@ -708,39 +708,51 @@ void linear_w4a8_tall_kernel(
   // (rows tid / 4 + 128 i)
   const uint32_t arow0 = tid >> 3, aunit = (tid & 7u) * 16u;
   const uint32_t brow0 = tid >> 2, bunit = (tid & 3u) * 16u;
-  const ST* ssrc = scales + (size_t)min(n0 + (uint32_t)(tid < BN ? tid : 0), n - 1) * groups;
+  // 32-bit offsets from bases that are the same for the whole workgroup: a stage's addresses take no
+  // vector instructions (a tile's 128 rows of x lie within 4 GiB, see the dispatch).  A K that ends inside
+  // a stage: the lanes past it re-read the row's start; their groups are fused with a zero scale.
+  const uint8_t* const a_tile = xq + (size_t)m0 * k;
+  const uint8_t* const b_tile = w + (size_t)n0 * (k >> 1);
+  const ST* const s_tile = scales + (size_t)n0 * groups;
+  uint32_t a_row[kAUnits], b_row[kBUnits];
+#pragma unroll
+  for (int i = 0; i < kAUnits; ++i) a_row[i] = min(arow0 + (T / 8) * i, m - 1 - m0) * k + aunit;
+#pragma unroll
+  for (int i = 0; i < kBUnits; ++i) b_row[i] = min(brow0 + (T / 4) * i, n - 1 - n0) * (k >> 1) + bunit;
+  const uint32_t s_row = min((uint32_t)(tid < BN ? tid : 0), n - 1 - n0) * groups;
 
   struct Staged {
     uint4 a[kAUnits];
     uint4 b[kBUnits];
     ST s[kGroupsPerStage];
   };
-  auto load_stage = [&](uint32_t stage, Staged& d) {
-    const uint32_t a_at = stage * kStage + aunit, b_at = stage * (kStage / 2) + bunit;
-    const uint32_t a_off = a_at < k ? a_at : 0u, b_off = b_at < (k >> 1) ? b_at : 0u;
+  auto load_stage = [&](uint32_t asked, Staged& d) {
+    const uint32_t stage = min(asked, stages - 1u);  // (past the last one: again, unused)
+    const uint8_t* const a_at = a_tile + (size_t)stage * kStage;
+    const uint8_t* const b_at = b_tile + (size_t)stage * (kStage / 2);
+    const bool past = GSH < 7 && stage * kStage + kStage > k;
+    const uint32_t a_back = past && stage * kStage + aunit >= k ? stage * kStage + aunit : 0u;
+    const uint32_t b_back = past && stage * (kStage / 2) + bunit >= (k >> 1) ? stage * (kStage / 2) + bunit : 0u;
 #pragma unroll
     for (int i = 0; i < kAUnits; ++i)
       d.a[i] = *reinterpret_cast<const uint4*>(
-          xq + (size_t)min(m0 + arow0 + (T / 8) * i, m - 1) * k + a_off);
+          GSH < 7 ? a_tile + (a_row[i] + stage * kStage - a_back) : a_at + a_row[i]);
 #pragma unroll
     for (int i = 0; i < kBUnits; ++i)
       d.b[i] = *reinterpret_cast<const uint4*>(
-          w + (size_t)min(n0 + brow0 + (T / 4) * i, n - 1) * (k >> 1) + b_off);
+          GSH < 7 ? b_tile + (b_row[i] + stage * (kStage / 2) - b_back) : b_at + b_row[i]);
 #pragma unroll
-    for (int j = 0; j < kGroupsPerStage; ++j) {
-      const uint32_t code = stage * kStage + (j << GSH);
-      d.s[j] = ssrc[(code < k ? code : 0u) >> GSH];
-    }
+    for (int j = 0; j < kGroupsPerStage; ++j)
+      d.s[j] = s_tile[s_row + min(stage * kGroupsPerStage + j, groups - 1u)];
   };
-  auto park_stage = [&](uint32_t stage, int buf, const Staged& d) {
-    const uint32_t keep = stage * kStage + aunit < k ? 0xFFFFFFFFu : 0u;
+  auto park_stage = [&](int buf, const Staged& d) {
 #pragma unroll
     for (int i = 0; i < kAUnits; ++i) {
       uint4 v;
-      v.x = __builtin_amdgcn_perm(d.a[i].y, d.a[i].x, 0x06040200u) & keep;
-      v.y = __builtin_amdgcn_perm(d.a[i].y, d.a[i].x, 0x07050301u) & keep;
-      v.z = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x06040200u) & keep;
-      v.w = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x07050301u) & keep;
+      v.x = __builtin_amdgcn_perm(d.a[i].y, d.a[i].x, 0x06040200u);
+      v.y = __builtin_amdgcn_perm(d.a[i].y, d.a[i].x, 0x07050301u);
+      v.z = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x06040200u);
+      v.w = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x07050301u);
       *reinterpret_cast<uint4*>(&s_a[buf][(arow0 + (T / 8) * i) * kRowA + aunit]) = v;
     }
 #pragma unroll
@@ -763,7 +775,7 @@ void linear_w4a8_tall_kernel(
 
   Staged staged;
   load_stage(0, staged);
-  park_stage(0, 0, staged);
+  park_stage(0, staged);
   __syncthreads();
 
   const uint32_t a_base = (uint32_t)((wm * 64 + frag_row) * kRowA + kHalfA * frag_h);
@@ -838,7 +850,7 @@ void linear_w4a8_tall_kernel(
         }
       }
     }
-    park_stage(stage + 1, buf ^ 1, staged);
+    park_stage(buf ^ 1, staged);
     __syncthreads();
   };
   for (uint32_t stage = 0; stage < stages; ++stage) run_stage(stage, (int)(stage & 1u));
@@ -899,7 +911,7 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
     // x 4096 709 and 130).
     const uint64_t cus = (uint64_t)ctx->num_cus;
     const uint64_t tall_tiles = (uint64_t)((m + 127) / 128) * n_blocks;
-    if (shift == 5 || ((shift == 6 || shift == 7) && tall_tiles * 5 >= cus * 3)) {
+    if (k <= (1u << 24) && (shift == 5 || ((shift == 6 || shift == 7) && tall_tiles * 5 >= cus * 3))) {
       const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
       const uint64_t small_rounds = ((uint64_t)small_m * small_n + cus - 1) / cus;
       const bool small =
