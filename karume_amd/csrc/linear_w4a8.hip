@@ -911,11 +911,22 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
     // x 4096 709 and 130).
     const uint64_t cus = (uint64_t)ctx->num_cus;
     const uint64_t tall_tiles = (uint64_t)((m + 127) / 128) * n_blocks;
-    if (k <= (1u << 24) && (shift == 5 || ((shift == 6 || shift == 7) && tall_tiles * 5 >= cus * 3))) {
+    // Fewer tall tiles than that: 64 x 256 tiles of the other kernel, or 64 x 128 where those would leave a
+    // quarter of the chip without work.  What would be 64 x 256 tiles goes to the 64 x 128 ones here in
+    // groups of 64 (four tiles' sums and eight groups' factors spilled there: 376 x 10350 x 3968 375 us, 54
+    // here; 79 x 24856 x 704 56 and 17; 36 shapes 0.12 to 0.35) and in groups of 128 from a second round
+    // on (347 x 11674 x 3072 55.6 and 41.1, 209 x 17856 x 1024 30.5 and 21.7; one round 0.90 to 1.13 of
+    // their time, 402 x 7336 x 7296 62.6 there, 70.7 here).
+    const uint64_t wide_tiles = (uint64_t)((m + 63) / 64) * n_blocks;
+    const bool wide = wide_tiles * 4 >= cus * 3;
+    const bool few_tall = tall_tiles * 5 < cus * 3;
+    const bool takes = shift == 5 || (shift == 6 && (!few_tall || wide)) ||
+                       (shift == 7 && (!few_tall || wide_tiles > cus));
+    if (k <= (1u << 24) && takes) {
       const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
       const uint64_t small_rounds = ((uint64_t)small_m * small_n + cus - 1) / cus;
       const bool small =
-          shift == 5 || small_rounds * 115 < (tall_tiles + cus - 1) / cus * 400;
+          shift == 5 || few_tall || small_rounds * 115 < (tall_tiles + cus - 1) / cus * 400;
       const uint32_t mb = small ? small_m : (m + 127) / 128, nb = small ? small_n : n_blocks;
       const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * mb;
       if (blocks <= 0x7fffffffull) {
@@ -934,8 +945,7 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
       }
     }
     const uint32_t m_blocks = (m + 63) / 64;
-    // 64 x 256 tiles, or 64 x 128 when those would leave a quarter of the chip without work
-    const bool narrow = (uint64_t)m_blocks * n_blocks * 4 < (uint64_t)ctx->num_cus * 3;
+    const bool narrow = !wide || shift == 6;
     const uint32_t nb = narrow ? (n + 127) / 128 : n_blocks;
     const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * m_blocks;
     if (shift > 5 && blocks <= 0x7fffffffull) {
@@ -945,7 +955,7 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
                      ptr<const uint8_t>(w), ps, pb, po, m, n, k, shift, m_blocks, nb)
 #define KRM_W4A8_TILE_G(GSH) \
   do { if (narrow) KRM_W4A8_TILE(GSH, 1); else KRM_W4A8_TILE(GSH, 2); } while (0)
-      if (shift == 6) KRM_W4A8_TILE_G(6);
+      if (shift == 6) KRM_W4A8_TILE(6, 1);
       else if (shift == 7) KRM_W4A8_TILE_G(7);
       else if (shift == 8) KRM_W4A8_TILE_G(8);
       else KRM_W4A8_TILE_G(0);

@@ -226,6 +226,22 @@ def test_w4a8_small_tiles_of_a_chip_that_tall_ones_leave_idle(gpu_ctx, m, n, k, 
     assert_exact(got, want, (m, n, k))
 
 
+@pytest.mark.parametrize("scale_f16", [True, False])
+@pytest.mark.parametrize("m, n, k, group", [
+    (65, 24500, 192, 64), (65, 24321, 64, 64), (130, 16400, 320, 64),   # the first that leave 64 x 256 tiles
+    (65, 24320, 192, 64),                                               # the last in 64 x 128 tiles over 256 codes
+    (100, 33025, 128, 128), (70, 33000, 384, 128), (65, 32768, 384, 128)])   # more than a round, and one
+def test_w4a8_between_the_tiles_of_few_and_of_many(gpu_ctx, m, n, k, group, scale_f16):
+    """Both sides of the lines between the two kernels, K of one group and K that ends inside a stage."""
+    rng = np.random.default_rng(m * 7 + n)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, group, scale_f16=scale_f16)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    bias = rng.normal(size=n).astype(np.float32)
+    got = run_w4a8(gpu_ctx, x, packed, scale, bias, n, k, group)
+    want = oracle.linear_w4a8(x, packed, np.asarray(scale, dtype=np.float32), bias, n, k, group)
+    assert_exact(got, want, (m, n, k))
+
+
 def test_w4a8_rows_do_not_depend_on_the_batch(gpu_ctx):
     rng = np.random.default_rng(3)
     n, k, group = 512, 4096, 128
