@@ -397,3 +397,26 @@ def test_probe_exchange_is_bounded_and_clean(gpu_ctx):
     with pytest.raises(ka.GpuValidationError):
         gpu_ctx.probe_exchange(work, 1000, 10)
     work.free()
+
+
+@pytest.mark.parametrize("n,k,g", [(8200, 2080, 32), (12000, 1152, 128), (9000, 576, 64), (16001, 832, 64),
+                                   (1772, 4672, 32), (30000, 96, 32)])
+@pytest.mark.parametrize("scale_type", [np.float16, np.float32])
+def test_few_fp16_rows_have_the_same_bits_in_every_batch(gpu_ctx, n, k, g, scale_type):
+    """2 to 16 fp16 rows on either side of the line between the GEMV and the tiles that split K: a row
+    does not depend on its batch, and every result is the oracle's to one fp16 ulp."""
+    rng = np.random.default_rng(n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    scale = scale.astype(scale_type)
+    x = rng.normal(size=(16, k)).astype(np.float16)
+    bias = rng.normal(size=n).astype(np.float16)
+    whole = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g)
+    for rows in (slice(0, 2), slice(3, 8), slice(7, 16)):
+        part = run_linear(gpu_ctx, x[rows], packed, scale, bias, n, k, g)
+        assert np.array_equal(part.view(np.uint16), whole[rows].view(np.uint16)), rows
+    cols = np.unique(np.concatenate([[0, 1, n - 2, n - 1], rng.choice(n, size=200)]))
+    want = oracle.linear_i4(x.astype(np.float32), packed.reshape(n, k // 2)[cols].reshape(-1),
+                            scale[cols].astype(np.float32), bias[cols].astype(np.float32), len(cols), k, g)
+    got = whole[:, cols].astype(np.float32)
+    # an fp16 ulp of the result beside the f32 sums (3e-5 of the row's typical product sum)
+    assert np.all(np.abs(got - want) <= 2.0 ** -10 * np.abs(want) + 4e-5)
