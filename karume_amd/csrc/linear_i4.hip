@@ -664,6 +664,8 @@ __device__ inline void slot_store(void* slot, int32_t is_f16, size_t i, float v)
 //  same x, which for f32 is four times the bytes of the two weight rows it meets; wave s
 //  prepares step s once (norm weight applied) and parks it in LDS for the others, after all
 //  weight requests are out.
+//  NSTEP == kStagedRows: any K, several rows of x brought to LDS by the workgroup.
+constexpr int kStagedRows = -1;
 template <typename XT, int MB, int NSTEP>
 constexpr bool share_x_in_lds() {
   return MB == 1 && NSTEP > 0;
@@ -685,6 +687,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x >> 6;
   constexpr bool XLDS = share_x_in_lds<XT, MB, NSTEP>();
+  constexpr bool kStageRows = NSTEP == kStagedRows && !NORM && !DECODE_ROW;
   // Four waves a workgroup (the launch below).  A wave whose rows lie past N stays: it re-reads
   // the last row and stores nothing, so no branch stands between the kernel's entry and its
   // loads (an early exit made the pointer arguments wait for the row test).
@@ -897,6 +900,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
           fetch_x(step, b, regs);
           consume(step, all_w[step], all_s[step], b, regs);
         }
+      }
+    }
+  } else if constexpr (kStageRows) {
+    // Several rows of x: every wave meets all of them at every step, and a lane's 32 elements of a row lie
+    // apart from its neighbours' (a load touched 64 lines).  The workgroup brings kRows rows of a step
+    // at a time to LDS instead, eight neighbouring elements a lane, the next ones on their way while these
+    // are used; rows past M are left out.  The arithmetic of a row is the same.  us before / now: 2 rows
+    // 2497 x 7040 16.1 / 8.5, 4 rows 11492 x 2112 32.5 / 22.2, 5 rows 1265 x 3072 25.9 / 15.6, 6 rows 4590 x
+    // 2560 34.4 / 28.7, 8 rows 680 x 5184 24.3 / 11.6, 2309 x 3584 29.7 / 20.4.
+    constexpr int kRows = MB < 4 ? MB : 4;
+    constexpr int kUnits = sizeof(Regs) / 16;
+    __shared__ uint4 s_rows[2][kRows][kUnits * kWave];
+    const uint32_t steps = (k + kStepElems - 1) / kStepElems;
+    uint32_t cur_w[ROWS][VEC], nxt_w[ROWS][VEC];
+    float cur_s[ROWS], nxt_s[ROWS];
+    using Quarter = typename Acts<XT>::template Raw<1, false>;
+    Quarter raw[kRows];
+    auto request_rows = [&](uint32_t step, uint32_t first) {
+      const uint32_t q_k0 = step * kStepElems + wave * 512 + lane * 8;
+      const uint32_t q_kc = q_k0 < k ? q_k0 : 0u;
+#pragma unroll
+      for (int i = 0; i < kRows; ++i)
+        Acts<XT>::template request<1, false>(x + (size_t)min(first + i, m - 1) * k + q_kc, nullptr, raw[i]);
+    };
+    auto park_rows = [&](uint32_t buf) {  // (units as in the shared row above)
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) {
+        typename Acts<XT>::template Regs<1> part;
+        Acts<XT>::template finish<1, false>(raw[i], true, part, squares[0]);
+        constexpr int kQuarterUnits = sizeof(part) / 16;
+        uint4 units[kQuarterUnits];
+        __builtin_memcpy(units, &part, sizeof(part));
+#pragma unroll
+        for (int j = 0; j < kQuarterUnits; ++j)
+          s_rows[buf][i][((lane & 3) * kQuarterUnits + j) * kWave + wave * 16 + (lane >> 2)] = units[j];
+      }
+    };
+    request_rows(0, 0);
+    fetch(0, cur_w, cur_s);
+    park_rows(0);
+    __syncthreads();
+    uint32_t buf = 0;
+    for (uint32_t step = 0; step < steps; ++step) {
+      fetch(step + 1 < steps ? step + 1 : step, nxt_w, nxt_s);
+#pragma unroll
+      for (int b0 = 0; b0 < MB; b0 += kRows) {
+        if (b0 > 0 && (uint32_t)b0 >= m) break;
+        const bool last = (uint32_t)(b0 + kRows) >= m;  // of the step
+        request_rows(last ? (step + 1 < steps ? step + 1 : step) : step, last ? 0u : b0 + kRows);
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+          uint4 units[kUnits];
+#pragma unroll
+          for (int u = 0; u < kUnits; ++u) units[u] = s_rows[buf][i][u * kWave + lane];
+          Regs regs;
+          __builtin_memcpy(&regs, units, sizeof(Regs));
+          consume(step, cur_w, cur_s, b0 + i, regs);
+        }
+        buf ^= 1u;
+        park_rows(buf);
+        __syncthreads();
+      }
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) cur_w[r][j] = nxt_w[r][j];
+        cur_s[r] = nxt_s[r];
       }
     }
   } else {
@@ -1136,6 +1206,12 @@ template <typename XT, typename ST, int MB, int ROWS, int VEC>
 int32_t pick_steps(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias, krm_buf out,
                    uint32_t m, uint32_t n, uint32_t k, uint32_t group_shift,
                    const GemvFusion& fuse) {
+  // 2 to 8 rows of f32 x over a step of K and more: through LDS.  (A K below a step leaves most lanes of
+  // the staging idle: 7 rows 12116 x 960 31 us, 38 staged; sixteen rows' sums beside it spill: 13 rows
+  // 8614 x 8960 322 us, 951.  fp16 x has half the lines: 4 rows 422 x 2496 6.4 us, 6.6.)
+  if constexpr (VEC == 4 && MB > 1 && MB <= 8 && sizeof(XT) == 4)
+    if (k >= 2048 && !fuse.norm_weight && !fuse.positions)
+      return launch_gemv<XT, ST, MB, ROWS, VEC, kStagedRows>(ctx, x, w, scales, bias, out, m, n, k, group_shift, fuse);
   // Rows short enough to hold in registers are requested whole (VEC == 4: 2048 codes a step).
   if constexpr (VEC == 4 && MB == 1) {
     const uint32_t steps = (k + 2047) / 2048;

@@ -420,3 +420,26 @@ def test_few_fp16_rows_have_the_same_bits_in_every_batch(gpu_ctx, n, k, g, scale
     got = whole[:, cols].astype(np.float32)
     # an fp16 ulp of the result beside the f32 sums (3e-5 of the row's typical product sum)
     assert np.all(np.abs(got - want) <= 2.0 ** -10 * np.abs(want) + 4e-5)
+
+
+@pytest.mark.parametrize("n,k,g", [(7, 2048, 64), (130, 2080, 32), (1000, 4128, 32), (37, 6272, 128),
+                                   (2100, 2176, 128)])
+@pytest.mark.parametrize("scale_type", [np.float16, np.float32])
+def test_several_f32_rows_brought_to_lds_have_the_bits_of_one_row(gpu_ctx, n, k, g, scale_type):
+    """2 to 8 rows of f32 x over a K of a step and more: the bits of a row alone (K of one step, of a
+    last step that is nearly empty; blocks of rows that are cut off; rows of N past the last)."""
+    rng = np.random.default_rng(n * 3 + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    scale = scale.astype(scale_type)
+    x = rng.normal(size=(8, k)).astype(np.float32)
+    x[2, 5] = np.inf                     # stays in its row
+    x[6, k - 1] = np.nan
+    bias = rng.normal(size=n).astype(np.float32)
+    alone = [run_linear(gpu_ctx, x[r:r + 1], packed, scale, bias, n, k, g)[0] for r in range(8)]
+    for m in (2, 3, 4, 5, 7, 8):
+        got = run_linear(gpu_ctx, x[:m], packed, scale, bias, n, k, g)
+        for r in range(m):
+            if r == 6:
+                assert np.isnan(got[r]).all()
+            else:
+                assert np.array_equal(got[r].view(np.uint32), alone[r].view(np.uint32)), (m, r)
