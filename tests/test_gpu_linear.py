@@ -443,3 +443,17 @@ def test_several_f32_rows_brought_to_lds_have_the_bits_of_one_row(gpu_ctx, n, k,
                 assert np.isnan(got[r]).all()
             else:
                 assert np.array_equal(got[r].view(np.uint32), alone[r].view(np.uint32)), (m, r)
+
+
+@pytest.mark.parametrize("n,k,g", [(70, 1152, 32), (300, 2048, 64), (1000, 4160, 64), (33, 8320, 128)])
+@pytest.mark.parametrize("m", [9, 12, 13, 16])
+def test_nine_to_sixteen_f32_rows_have_the_bits_of_one_row(gpu_ctx, n, k, g, m):
+    """One launch of sixteen rows or two of eight and the rest: the bits of a row alone."""
+    rng = np.random.default_rng(n + k + m)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    bias = rng.normal(size=n).astype(np.float32)
+    got = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g)
+    for r in (0, 7, 8, m - 1):
+        alone = run_linear(gpu_ctx, x[r:r + 1], packed, scale, bias, n, k, g)
+        assert np.array_equal(got[r:r + 1].view(np.uint32), alone.view(np.uint32)), r
