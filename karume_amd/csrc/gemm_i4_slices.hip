@@ -35,7 +35,7 @@
 // kXThree is bounded by the vector ALUs (11 operations a pair of x, 10 a word of weights, both at
 // every step; tiles of up to four columns share x).  Groups of 32, against the GEMV over blocks of 16
 // rows (in brackets: hi + lo planes, which lost the small entries of a row beside a large one): 77 x
-// 3000 x 2080 13.8 us, 210 (13.8); 17 rows of it 10.1, 45.5 (10.2); 128 x 2048 x 2048 11.2, 156 (12.0);
+// 3000 x 2080 12.9 us, 210 (13.8); 17 rows of it 10.1, 45.5 (10.2); 128 x 2048 x 2048 11.2, 156 (12.0);
 // 32 x 4096 x 8192 29, - (25); 512 x 4096 x 4096 77, 1969 (81); 512 x 11008 x 4096 215, 5594 (214); in
 // groups of 16 277, 2427 (332).  Error against 64 bits (2-norm,
 // normal x): 77 x 3000 x 2080 in groups of 32 9.5e-8, the GEMV 1.24e-7; 40 x 1000 x 4096 in groups of
