@@ -188,8 +188,9 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // (22 bits of p, 2^-39 where it is small), products are exact, sums f32, scale^2 multiplies the f32 sum.
 // Error against 64 bits (2-norm, f32 queries, normal values; f32 operands before): D = 64 behind 1024
 // 2.4e-7 (3.7e-7), D = 128 2.8e-7 (4.7e-7), D = 256 3.5e-7 (6.2e-7).  A part of zero beside an infinity
-// of the state is a NaN that the value itself would not give: a wave whose walk leaves a NaN walks again
-// with f32 operands.  With g = lane / 16:
+// of the state is a NaN that the value itself would not give, and 2^15 times a sum of this step's f32 rows
+// can be infinite where the sum is not: a wave whose walk leaves a value that is not finite walks again with
+// f32 operands and without the factor.  With g = lane / 16:
 //   S^T = K Q^T    two tiles of 16 keys; A = the K tile (row = key, lane group g walks dims
 //                  g D/4 ..), B = Q^T (column = query row): a lane ends up with the scores of
 //                  ONE query row (lane % 16) against keys 16 t + 4 g + i (t < 2, i < 4), so the
@@ -609,7 +610,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 #pragma unroll
       for (int i = 0; i < kQuarter / 4; ++i) {
         float qs[4];
-        if constexpr (kQDirect) {  // (the walk behind a NaN)
+        if constexpr (kQDirect) {  // (the second walk)
           const uint32_t row = min(row0 + (uint32_t)(16 * rb + r), a.chunk_rows - 1);
           const float4 v = load4_f32<XT>(q + ((size_t)z * a.chunk_rows + row) * D + g * kQuarter + 4 * i);
           qs[0] = v.x * a.scale; qs[1] = v.y * a.scale; qs[2] = v.z * a.scale; qs[3] = v.w * a.scale;
@@ -669,7 +670,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
         for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= alpha;
       // (tile dt = 4 i + e holds the dims 64 i + 4 r + e: a 16-byte piece feeds four tiles)
       const uint32_t pv_key = lane_number(4u * g);
-      if constexpr (kHalf) {  // (the sums of V are kept times 2^15: small probabilities keep their bits)
+      if constexpr (kMode != kNever) {  // (the sums of V are kept times 2^15: small probabilities keep their bits)
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -729,33 +730,32 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     bool plain = kSplitQ && slot_columns(c_lo) != 32u;  // no block of fp16 keys
     if (!plain) {
       walk(std::integral_constant<int, sizeof(XT) == 2 ? kAlways : kSlotBlocks>{});
-      bool nan = false;
+      bool lost = false;
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         bool here = run_l[rb] != run_l[rb];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) here = here || acc[rb][dt][i] != acc[rb][dt][i];
-        nan = nan || (here && row0 + (uint32_t)(16 * rb + r) < query);
+          for (int i = 0; i < 4; ++i) here = here || !(fabsf(acc[rb][dt][i]) < INFINITY);
+        lost = lost || (here && row0 + (uint32_t)(16 * rb + r) < query);
       }
-      // (parts of a value meet an infinity of the state as 0 * inf, the value itself does not: once more
-      // without them)
-      plain = __any(nan);
+      // (parts of a value meet an infinity of the state as 0 * inf, the value itself does not; 2^15 takes
+      // sums of this step's f32 rows past f32's range from 1e34 on: once more without either)
+      plain = __any(lost);
       if (plain && kAhead && (uint32_t)wave < blocks) {
         request_k((uint32_t)wave);
         request_v((uint32_t)wave);
       }
     }
     if (plain) walk(std::integral_constant<int, kNever>{});
-  }
-  if constexpr (kHalf) {
+    const float unscale = plain ? 1.0f : 1.0f / kPScale;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= 1.0f / kPScale;
+        for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= unscale;
   }
 
   // The chunk's own K / V rows of this block go to the state slots when asked for (the first query

@@ -989,3 +989,29 @@ def test_infinities_in_an_fp16_state_reach_what_they_reach_in_f32(gpu_ctx, depth
     rest = np.delete(np.arange(depth), (9, 11))
     assert np.all(np.abs(got[:, rest].astype(np.float64) - want[:, rest]) <=
                   1e-5 + (2e-3 if io == np.float16 else 0.0))
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+@pytest.mark.parametrize("past", [8, 40, 96])
+@pytest.mark.parametrize("infinite", [False, True])
+def test_large_f32_rows_of_a_chunk_beside_an_fp16_state(gpu_ctx, depth, past, infinite):
+    """This step's f32 value rows of 1e36 stay finite beside an fp16 state, also where an infinity of the
+    state sends the wave over its keys once more.  |v| <= 3e36 over at most 116 keys: no sum reaches
+    f32's largest.  The bound is that of f32 operands: a score's product is rounded three times, which moves
+    a probability by 3 * 2^-24 of sum |q k| scale^2; exponential and sums stay below 2^-20."""
+    rng = np.random.default_rng(depth + past)
+    m, scale = 20, float(np.float32(np.sqrt(1.0 / np.sqrt(float(depth)))))
+    q, ik = (rng.normal(size=(m, depth)).astype(np.float32) for _ in range(2))
+    iv = (np.clip(rng.normal(size=(m, depth)), -3, 3) * 1e36).astype(np.float32)
+    sk, sv = (rng.normal(size=(past + m, depth)).astype(np.float16) for _ in range(2))
+    if infinite:
+        sv[3, 9] = np.inf
+    got = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale).astype(np.float64)
+    k = np.concatenate([sk[:past].astype(np.float64), ik.astype(np.float64)])
+    v = np.concatenate([sv[:past].astype(np.float64), iv.astype(np.float64)])
+    want = attention_in_64_bits(q, k, v, past, scale)
+    if infinite:
+        assert np.isposinf(got[:, 9]).all()
+        got, want, v = (np.delete(a, 9, axis=1) for a in (got, want, v))
+    moved = 3 * 2.0 ** -24 * (np.abs(q.astype(np.float64)) @ np.abs(k).T).max(axis=1) * scale * scale + 2.0 ** -20
+    assert np.all(np.abs(got - want) <= 2 * moved[:, None] * np.abs(v).max())
