@@ -158,16 +158,32 @@ __device__ inline void finish_pair(float v0, float v1, uint32_t row, uint32_t co
   }
 }
 
-// Four elements next to each other, as wide as they are aligned (`quads_aligned` below).
+// Four elements next to each other, as wide as they are aligned (`quads_aligned` below), as they lie in
+// memory (fp16: the first eight bytes).  They become numbers where they are used: a conversion waits for its
+// load, and so for everything that was asked for in front of it.
 template <typename T>
-__device__ inline float4 load_quad(const T* p) {
+__device__ inline void load_quad(uint4& to, const T* p) {
   if constexpr (sizeof(T) == 4) {
-    return *reinterpret_cast<const float4*>(p);
+    to = *reinterpret_cast<const uint4*>(p);
   } else {
     const uint2 raw = *reinterpret_cast<const uint2*>(p);
+    to.x = raw.x; to.y = raw.y;
+  }
+}
+template <typename T>
+__device__ inline float4 quad_f32(const uint4& raw) {
+  if constexpr (sizeof(T) == 4) {
+    return make_float4(__uint_as_float(raw.x), __uint_as_float(raw.y), __uint_as_float(raw.z),
+                       __uint_as_float(raw.w));
+  } else {
     const half2_t a = __builtin_bit_cast(half2_t, raw.x), b = __builtin_bit_cast(half2_t, raw.y);
     return make_float4((float)a.x, (float)a.y, (float)b.x, (float)b.y);
   }
+}
+// Two elements at any element's alignment likewise.
+template <typename T>
+__device__ inline void load_pair(uint4& to, const T* p) {
+  __builtin_memcpy(&to, p, 2 * sizeof(T));
 }
 template <typename T>
 __device__ inline void store_pair(T* p, float v0, float v1) {
@@ -192,13 +208,13 @@ __device__ inline void store_quad(T* p, float v0, float v1, float v2, float v3) 
 // product reads from memory, asked for while the sums are still on their way through LDS, and the
 // same arithmetic as finish_pair behind them.
 struct QuadAhead {
-  float4 bias, residual;
+  uint4 bias, residual;   // (load_quad; a silu's residual: load_pair)
   float2 cos[2], sin[2];  // mode 2: of dims j, j + 1 and of j + D/2, j + 1 + D/2
 };
 template <typename T>
 __device__ inline void fetch_quad(QuadAhead& q, uint32_t row, uint32_t col, uint32_t n, int32_t pos,
                                   const T* bias, const RowsFusion& fuse) {
-  if (bias) q.bias = load_quad<T>(bias + col);
+  if (bias) load_quad<T>(q.bias, bias + col);
   const T* residual = static_cast<const T*>(fuse.residual);
   if (fuse.mode == 2) {
     const uint32_t half = fuse.depth >> 1, pair = col >> 1;
@@ -210,11 +226,9 @@ __device__ inline void fetch_quad(QuadAhead& q, uint32_t row, uint32_t col, uint
       q.sin[1] = *reinterpret_cast<const float2*>(fuse.sin_table + t + half);
     }
   } else if (residual && fuse.mode == 0) {
-    q.residual = load_quad<T>(residual + (size_t)row * n + col);
+    load_quad<T>(q.residual, residual + (size_t)row * n + col);
   } else if (residual) {
-    const size_t at = (size_t)row * (n >> 1) + (col >> 1);
-    q.residual.x = to_f32<T>(residual[at]);
-    q.residual.y = to_f32<T>(residual[at + 1]);
+    load_pair<T>(q.residual, residual + (size_t)row * (n >> 1) + (col >> 1));
   }
 }
 template <typename T>
@@ -222,16 +236,21 @@ __device__ inline void finish_quad(float4 v, const QuadAhead& q, uint32_t row, u
                                    uint32_t m, uint32_t n, int32_t pos, bool bias, T* out,
                                    const RowsFusion& fuse) {
   if (bias) {
-    v.x += q.bias.x; v.y += q.bias.y; v.z += q.bias.z; v.w += q.bias.w;
+    const float4 b = quad_f32<T>(q.bias);
+    v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
   }
   if (fuse.mode == 0) {
     if (fuse.residual) {
-      v.x += q.residual.x; v.y += q.residual.y; v.z += q.residual.z; v.w += q.residual.w;
+      const float4 r = quad_f32<T>(q.residual);
+      v.x += r.x; v.y += r.y; v.z += r.z; v.w += r.w;
     }
     store_quad<T>(out + (size_t)row * n + col, v.x, v.y, v.z, v.w);
   } else if (fuse.mode == 1) {
     float a = silu_times(v.x, v.y), b = silu_times(v.z, v.w);
-    if (fuse.residual) { a += q.residual.x; b += q.residual.y; }
+    if (fuse.residual) {
+      const float4 r = quad_f32<T>(q.residual);
+      a += r.x; b += r.y;
+    }
     store_pair<T>(out + (size_t)row * (n >> 1) + (col >> 1), a, b);
   } else {
     // what a separate linear would have stored, then the rotation

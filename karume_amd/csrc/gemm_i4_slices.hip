@@ -152,14 +152,18 @@ struct SliceGeometry {
   static constexpr int kSumTiles = MT * NT * 4096 <= kArea ? NT : kArea / (MT * 4096);
 };
 
+// Bits of the kernel's `flags`: element types, and whether the end reads anything in quads (kFetches), rope
+// positions among it (kRope).
+constexpr uint32_t kScaleF16 = 1, kIoF16 = 2, kFetches = 4, kRope = 8;
+
 template <int XKIND, int MT, int NT, int STEPS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_i4_slices_kernel(
     // (the leading 14 dwords of the arguments arrive in scalar registers with the wave)
     const uint8_t* __restrict__ x,  // [m][k], but kXSplit: [m][k / 32][hi, lo][32] fp16
     const uint8_t* __restrict__ w, const uint8_t* __restrict__ scales, uint32_t row_begin,
-    uint32_t row_end, uint32_t n, uint32_t k, uint32_t group_shift, uint32_t m_blocks, uint32_t tiles, uint32_t scale_f16_arg,
-    uint32_t io_f16, uint32_t m, SliceTail tail) {
+    uint32_t row_end, uint32_t n, uint32_t k, uint32_t group_shift, uint32_t m_blocks, uint32_t tiles, uint32_t flags,
+    uint32_t m, SliceTail tail) {
   using G = SliceGeometry<XKIND, MT, NT, STEPS>;
   constexpr int kPlanes = G::kPlanes, kStage = G::kStage, kRowBytes = G::kRowBytes;
   constexpr int kLanesPerRow = kRowBytes / 16, kRowsPerLoad = 64 / kLanesPerRow;
@@ -223,7 +227,7 @@ void gemm_i4_slices_kernel(
   // start and used behind its last step.  Smaller groups: the scales of a unit travel with its
   // weights, entry e * 32 NT + column.
   const uint32_t groups = k >> group_shift;
-  const bool scale_f16 = scale_f16_arg != 0;
+  const bool scale_f16 = (flags & kScaleF16) != 0;
   const uint32_t scale_size = scale_f16 ? 2u : 4u;
   constexpr int kSOff = STEPS == 8 ? NT : G::kSLoads;
   uint32_t s_off[kSOff];
@@ -404,8 +408,13 @@ void gemm_i4_slices_kernel(
       if (quad_at((int)threadIdx.x + 512 * i, t0, quads, &row, &col)) pos[i] = tail.fuse.positions[row];
     }
   };
-  const bool fetches = tail.quads && (tail.fuse.mode == 2 || tail.bias || tail.fuse.residual);
-  if (fetches && tail.fuse.mode == 2) fetch_positions(0);
+  // (Decided by a word that arrives with the wave.  Read from `tail`, which does not, the decision stood in
+  // front of the first stages; and fp16 that became f32 where it was asked for kept the K loop waiting for
+  // every stage on its way.  64 to 256 rows, n and k of 256 to 2048, fp16, us with both / without, cold weights:
+  // 64 x 256 x 256 in groups of 64 3.7 / 3.3, 64 x 1024 x 1024 4.84 / 4.40, 128 x 2048 x 1024 5.05 / 4.61; 104
+  // products without rope take 0.85 to 0.98 of the time.)
+  const bool fetches = (flags & kFetches) != 0, io_f16 = (flags & kIoF16) != 0;
+  if ((flags & kRope) != 0) fetch_positions(0);
   QuadAhead ahead[kMostItems];
   float inv[kMostItems];
   auto fetch = [&](int t0) {
@@ -428,7 +437,9 @@ void gemm_i4_slices_kernel(
   if (k0 < k1) {
     const uint32_t stages = (k1 - k0 + kStage - 1u) / kStage;
     constexpr int kStages = kBlock / kStage;  // of a flush block
-    // At most the stages younger than g (and, `more`, other loads) are on their way.
+    // At most the stages younger than g (and, `more`, other loads) are on their way.  (What the end of the
+    // kernel fetches ahead is not counted, as its loads differ from wave to wave: the first waits then ask for
+    // as many loads of a younger stage.)
     auto wait_for = [&](uint32_t g, auto more_tag) {
       constexpr int MORE = decltype(more_tag)::value;
       const uint32_t left = min((uint32_t)(DX - 1), stages - 1u - g);
@@ -510,7 +521,7 @@ void gemm_i4_slices_kernel(
     constexpr int quads = 8 * kTiles, kItems = (BM * quads + 511) / 512;
     const T* const bias = static_cast<const T*>(tail.bias);
     T* const out = static_cast<T*>(tail.out);
-    if (t0 > 0 && fetches && tail.fuse.mode == 2) fetch_positions(t0);
+    if (t0 > 0 && (flags & kRope) != 0) fetch_positions(t0);
     if ((!kFetchFirst || t0 > 0) && (fetches || XKIND == kXSplit)) fetch(t0);
     float* sums = reinterpret_cast<float*>(area);
     if (t0 > 0) __syncthreads();
@@ -582,11 +593,14 @@ template <int XKIND, int MT, int NT, int STEPS>
 int32_t launch_slices(krm_ctx* ctx, const SliceCall& c) {
   const uint32_t m_blocks = (c.row_end - c.row_begin + 32 * MT - 1) / (32 * MT);
   const uint32_t tiles = m_blocks * ((c.n + 32 * NT - 1) / (32 * NT));
+  uint32_t flags = (c.scale_f16 ? kScaleF16 : 0u) | (c.io_f16 ? kIoF16 : 0u);
+  if (c.tail.quads && (c.tail.fuse.mode == 2 || c.tail.bias || c.tail.fuse.residual)) flags |= kFetches;
+  if ((flags & kFetches) && c.tail.fuse.mode == 2) flags |= kRope;
   gemm_i4_slices_kernel<XKIND, MT, NT, STEPS>
       <<<dim3(((tiles + 7) / 8) * 8), dim3(512), 0, ctx->stream>>>(
           static_cast<const uint8_t*>(c.x), static_cast<const uint8_t*>(c.w),
           static_cast<const uint8_t*>(c.scales), c.row_begin, c.row_end, c.n, c.k, c.group_shift,
-          m_blocks, tiles, c.scale_f16, c.io_f16, c.m, c.tail);
+          m_blocks, tiles, flags, c.m, c.tail);
   return launched(ctx, "gemm_i4_slices_kernel");
 }
 

@@ -617,3 +617,33 @@ def test_rope_of_a_fused_projection_by_quads_and_by_pairs(gpu_ctx, io, m, heads,
         assert np.array_equal(a.view(bits), b.view(bits))
     assert np.isnan(got[0][0][:, m // 2]).all() and np.isfinite(got[0][2]).all()
     assert np.isfinite(np.delete(got[0][0], m // 2, 1)).all()
+
+
+@pytest.mark.parametrize("io", [ka.F16, ka.F32])
+@pytest.mark.parametrize("m,n,k", [(17, 8, 64), (40, 96, 576), (128, 2048, 256)])
+def test_the_residual_of_a_silu_is_read_at_any_element(gpu_ctx, io, m, n, k):
+    """Two residuals are read at once, wherever they lie: the same bits from a buffer that is a whole number of
+    pairs and from one that is an element off, with `out` aligned in both."""
+    rng = np.random.default_rng(m + n)
+    io_np = np.float32 if io == ka.F32 else np.float16
+    packed, _codes, scales = helpers.synthetic_int4(rng, n, k, 64)
+    x, residual = rng.normal(size=(m, k)).astype(io_np), rng.normal(size=m * n // 2).astype(io_np)
+    dx, dw, ds = map(gpu_ctx.upload, (x, packed, scales))
+    zero = gpu_ctx.zeros(m * n // 2 * np.dtype(io_np).itemsize)
+    gpu_ctx.linear_i4_rows(dx, dw, ds, zero, m, n, k, 64, io_dtype=io, scale_dtype=ka.F16,
+                           compute=ka.COMPUTE_F32, epilogue=ka.EPILOGUE_SILU_PAIRS)
+    product = zero.download(io_np, (m, n // 2)).astype(np.float64)
+    got = []
+    for shift in (0, 1):
+        res = gpu_ctx.upload(np.concatenate([np.zeros(shift, dtype=io_np), residual]))
+        out = gpu_ctx.zeros(m * n // 2 * np.dtype(io_np).itemsize)
+        gpu_ctx.linear_i4_rows(dx, dw, ds, out, m, n, k, 64, residual=res.offset(shift * np.dtype(io_np).itemsize),
+                               io_dtype=io, scale_dtype=ka.F16, compute=ka.COMPUTE_F32,
+                               epilogue=ka.EPILOGUE_SILU_PAIRS)
+        got.append(out.download(io_np, (m, n // 2)))
+    bits = np.uint32 if io == ka.F32 else np.uint16
+    assert np.array_equal(got[0].view(bits), got[1].view(bits))
+    # (the product rounded to `io` here, not in the kernel; then one rounding of the sum)
+    eps = 2.0 ** -22 if io == ka.F32 else 2.0 ** -10
+    want = product + residual.reshape(m, n // 2)
+    assert np.all(np.abs(got[0] - want) <= eps * (np.abs(product) + np.abs(want)) + 1e-7)
