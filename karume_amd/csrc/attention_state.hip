@@ -183,11 +183,13 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // takes blocks w, w + WAVES, ...  Products and sums are f32's.  Rows of f32 (the state's, or this step's
 // beside an fp16 state) run on v_mfma_f32_16x16x4_f32 with the generic kernel's operand roundings: q *
 // scale and k * scale are rounded before the product.  Blocks of fp16 rows run on
-// v_mfma_f32_16x16x32_f16, sixteen times that rate, with no fewer bits: K and V are fp16 as they are, q is
-// fp16 or three fp16 parts of the row times a power of two (33 bits), a probability two parts of p 2^15
-// (22 bits of p, 2^-39 where it is small), products are exact, sums f32, scale^2 multiplies the f32 sum.
-// Error against 64 bits (2-norm, f32 queries, normal values; f32 operands before): D = 64 behind 1024
-// 2.4e-7 (3.7e-7), D = 128 2.8e-7 (4.7e-7), D = 256 3.5e-7 (6.2e-7).  A part of zero beside an infinity
+// v_mfma_f32_16x16x32_f16, sixteen times that rate: K and V are fp16 as they are, q is fp16 or three fp16 parts
+// of the row times a power of two (33 bits below the row's largest magnitude), a probability from 2^-16 on three
+// parts of p 2^15 (all its bits; a block with a smaller one multiplies V with f32 operands), products are exact,
+// sums f32, scale^2 multiplies the f32 sum.
+// Error against 64 bits (2-norm, f32 queries, normal values; all in f32 operands): D = 64 behind 1024
+// 2.6e-7 (3.9e-7), D = 128 2.8e-7 (4.6e-7), D = 256 3.6e-7 (6.5e-7); queries four times as large 5.6e-7 (9.1e-7),
+// 7.1e-7 (1.3e-6), 8.5e-7 (1.7e-6).  A part of zero beside an infinity
 // of the state is a NaN that the value itself would not give, and 2^15 times a sum of this step's f32 rows
 // can be infinite where the sum is not: a wave whose walk leaves a value that is not finite walks again with
 // f32 operands and without the factor.  With g = lane / 16:
@@ -209,9 +211,11 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // rows a workgroup (not 32) so that a 128-row chunk of 32 heads is 256 workgroups, one per CU.
 // What bounds f32 rows is their matrix rate with two waves a SIMD to cover softmax and waits (D = 64,
 // r = 8, 128 rows behind 1024: 8 us of MFMA), fp16 rows the vector instructions of softmax and operands.
-// us with f32 operands / with fp16 ones, 128 rows behind 1024 and 512 behind 2048: fp16 D = 64 19.6 /
-// 10.1, 120 / 50; D = 128, r = 4 34.7 / 17.5, 236 / 102; D = 256 72 / 33, 148 / 64; f32 queries D = 64
-// 21.6 / 15.3, 132 / 75; D = 128 38.5 / 22.1, 267 / 140; D = 256 77 / 46, 161 / 97.  Before those f32
+// us with f32 operands / with fp16 ones / with fp16 ones where blocks hold probabilities below 2^-16 (queries
+// four times as large), 128 rows behind 1024 and 512 behind 2048: fp16 D = 64 21.3 / 11.8 / 15.8, 123 / 60 / 85; D =
+// 128, r = 4 34.1 / 17.9 / 25.3, 236 / 107 / 164; D = 256 71 / 34 / 55, 148 / 69 / 109; f32 queries D = 64 22.0 / 16.5 /
+// 19.1, 131 / 83 / 112; D = 128 38.2 / 22.3 / 29.8, 267 / 142 / 204; D = 256 76 / 47 / 68, 161 / 103 / 140.  (Two parts
+// for every probability, 22 bits and nothing below 2^-40, took 0 to 9 % less.)  Before those f32
 // forms, with V parked as well, rows looked up one by one (two element types: a wait at each), expf and no
 // requests ahead, us before / with f32 operands: the case of 8 us of MFMA
 // 22.7 / 19.3; fp16, D = 128, r = 4: 49.4 / 32.6; f32 over fp16 slots 106.5 / 36.8; D = 256, r = 8
@@ -300,8 +304,10 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   // State rows of fp16 are products of fp16 operands: see `half_block` below.
   constexpr bool kHalf = sizeof(ST) == 2;
   constexpr int kHalfRow = D + 8;             // halves of a parked row
-  constexpr int kPParts = 2;
-  constexpr float kPScale = 32768.0f;
+  // A probability from 2^-16 on is three fp16 parts of p 2^15, all its 24 bits: below that the last of them
+  // lie under fp16's smallest step, and a block that holds such a probability takes f32 operands.
+  constexpr int kPParts = 3;
+  constexpr float kPScale = 32768.0f, kPLeast = 1.0f / 65536.0f;
   constexpr int kQParts = sizeof(XT) == 2 ? 1 : 3, kSteps = D / 32;
   __shared__ __align__(16) float s_k[WAVES][32 * kRow];
   constexpr bool kSplitQ = kHalf && sizeof(XT) == 4;
@@ -676,7 +682,16 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 #pragma unroll
           for (int i = 0; i < 4; ++i) p[t][i] *= kPScale;
       }
-      if (half_block) {
+      bool half_sums = half_block;
+      if (kMode != kNever && half_block) {
+        uint32_t least = 0xffffffffu;  // (of the bits less one: a zero comes out on top)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) least = min(least, __float_as_uint(p[t][i]) - 1u);
+        half_sums = !__any(least < __float_as_uint(kPLeast * kPScale) - 1u);
+      }
+      if (half_sums) {
         half8_t ph[kPParts];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {

@@ -942,8 +942,9 @@ def chunk_over_fp16_state(ctx, q, ik, iv, sk, sv, past, scale):
 @pytest.mark.parametrize("io", [np.float32, np.float16])
 def test_chunks_over_an_fp16_state_keep_the_bits_of_f32(gpu_ctx, depth, past, io):
     """Blocks of 32 fp16 keys run with fp16 operands (the queries and the probabilities in parts): no
-    further from 64 bits than f32 operands are, for rows of 1e4 and of 1e-7 beside ordinary ones, a row
-    with entries eight decades apart, and probabilities down to 2^-30.  f32 operands: every product of
+    further from 64 bits than f32 operands are, for rows of 1e4 and of 1e-7 beside ordinary ones and a row
+    with entries eight decades apart (a small probability shows where it alone has a value:
+    test_small_probabilities_over_an_fp16_state_keep_their_bits).  f32 operands: every product of
     a score is rounded three times, 3 * 2^-24 of sum |q k| scale^2 at most, which moves a probability by
     as much of itself; the rest (exponential, sums over the keys) stays below 2^-20."""
     rng = np.random.default_rng(depth + past)
@@ -1015,3 +1016,32 @@ def test_large_f32_rows_of_a_chunk_beside_an_fp16_state(gpu_ctx, depth, past, in
         got, want, v = (np.delete(a, 9, axis=1) for a in (got, want, v))
     moved = 3 * 2.0 ** -24 * (np.abs(q.astype(np.float64)) @ np.abs(k).T).max(axis=1) * scale * scale + 2.0 ** -20
     assert np.all(np.abs(got - want) <= 2 * moved[:, None] * np.abs(v).max())
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+@pytest.mark.parametrize("past", [32, 33, 96])
+@pytest.mark.parametrize("lowest", [-11.0, -40.0, -80.0])
+@pytest.mark.parametrize("io", [np.float32, np.float16])
+def test_small_probabilities_over_an_fp16_state_keep_their_bits(gpu_ctx, depth, past, lowest, io):
+    """Eight keys of the state score down to `lowest` under the rest, and each alone has a value in its dim: the
+    dim shows that key's probability, however small.  (From 2^-16 = e^-11.1 on a probability is three fp16 parts,
+    below that an f32 operand.)  Scores are exact, one product with 1.  Exponentials are within 2^-22 in the
+    dim and in the sum, and about 20 sums and products round once each; fp16 results once more."""
+    rng = np.random.default_rng(depth + past)
+    m = 18
+    q = np.zeros((m, depth), dtype=io)
+    q[:, :8] = rng.uniform(lowest, -0.5, size=(m, 8)).astype(io)
+    q[:, 0] = lowest
+    ins = np.zeros((m, depth), dtype=io)
+    sk, sv = (np.zeros((past + m, depth), dtype=np.float16) for _ in range(2))
+    keys = rng.choice(past, size=8, replace=False)
+    sk[keys, np.arange(8)] = 1.0
+    sv[keys, np.arange(8)] = 32768.0
+    got = chunk_over_fp16_state(gpu_ctx, q, ins, ins, sk, sv, past, 1.0).astype(np.float64)
+    p = np.exp(q[:, :8].astype(np.float64))
+    want = 32768.0 * p / (p.sum(axis=1) + past - 8 + np.arange(1, m + 1))[:, None]
+    bound = (2 * 2.0 ** -22 + 20 * 2.0 ** -24) * want
+    if io == np.float16:
+        bound = bound + 2.0 ** -11 * want + 2.0 ** -25
+    assert np.all(np.abs(got[:, :8] - want) <= bound)
+    assert not got[:, 8:].any()
