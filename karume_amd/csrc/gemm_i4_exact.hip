@@ -21,13 +21,14 @@
 //   - scales come in blocks of two or four stages, neighbouring lanes taking neighbouring groups of a
 //     column: one scale a lane from 64 columns cost 2048 clk a stage of a 4800-clk stage;
 //   - hi and lo are written once, by a pass of their own, and not again by each of the n / 512 column
-//     tiles, which took the K loop over the register file (272 bytes of spills a lane);
+//     tiles, which took the K loop over the register file;
 //   - the K loop is one basic block of eight steps, each step's products beside the reads and conversion
 //     of the next step's operands, one barrier a stage.
-// us, before (stages staged through registers, split in the loop) / now, without bias, fp16 scales: f32
-// 512 x 11008 x 4096 120 / 94, 512 x 4096 x 11008 118 / 101 (before: on the K-splitting tiles), in groups of 64
-// 249 x 23257 x 1152 0.83 of the time; fp16 512 x 11008 x 4096 60.8 / 58.4, in groups of 64 70.6 / 64.6, 348 x
-// 8164 x 4608 0.90 of the time.  About 20 us of each are not the K loop: launch 7, first loads 3, the
+// us, before (stages staged through registers, f32 x split in the loop; f32 512 x 4096 x 11008 in groups of 128: on
+// the K-splitting tiles) / now, in replayed recordings over four weights, no bias, fp16 scales, groups of 128 and
+// of 64: f32 512 x 11008 x 4096 119 / 96 and 126 / 100, 512 x 4096 x 11008 117 / 101 and 177 / 106, 348 x 8164 x 4608
+// 88 / 69 and 96 / 73; fp16 512 x 11008 x 4096 72 / 65 and 77 / 66, 348 x 8164 x 4608 49 / 44 and 52 / 45.  (512 x
+// 11008 x 4096 over one weight, fp16: 66 / 56.)  About 20 us of each are not the K loop: launch 7, first loads 3, the
 // partials of shared tiles 8.
 #include "gemm_i4_deal.h"
 #include "gemm_i4_rows.h"
@@ -402,30 +403,33 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
       if (merge) {  // every other partial of the tile is complete; the sum is taken in K order
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
+          auto partial = [&](uint32_t u, float16_t (&part)[2]) {
+            if (u == v) {
+              part[0] = total[mt][0];
+              part[1] = total[mt][1];
+              return;
+            }
+            const float4_t* src = reinterpret_cast<const float4_t*>(
+                deal.partials + (size_t)slot_of(u) * kPartialFloats) + mt * 8 * 512 + here;
+            float4_t p[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) p[i] = observe4(src + i * 512);
+            landed(p);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) part[i >> 2][4 * (i & 3) + e] = p[i][e];
+          };
+          // (the first one outside the loop: a sum that its first turn set was kept over the tiles, in scratch)
           float16_t sum[2];
-          for (uint32_t u = first; u <= last; ++u) {
-            float16_t part[2] = {total[mt][0], total[mt][1]};
-            if (u != v) {
-              const float4_t* src = reinterpret_cast<const float4_t*>(
-                  deal.partials + (size_t)slot_of(u) * kPartialFloats) + mt * 8 * 512 + here;
-              float4_t p[8];
+          partial(first, sum);
+          for (uint32_t u = first + 1u; u <= last; ++u) {
+            float16_t part[2];
+            partial(u, part);
 #pragma unroll
-              for (int i = 0; i < 8; ++i) p[i] = observe4(src + i * 512);
-              landed(p);
+            for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-              for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) part[i >> 2][4 * (i & 3) + e] = p[i][e];
-            }
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-              if (u == first) {
-                sum[nt] = part[nt];
-              } else {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sum[nt][r] += part[nt][r];
-              }
-            }
+              for (int r = 0; r < 16; ++r) sum[nt][r] += part[nt][r];
           }
           store_rows(mt, sum);
         }
@@ -463,14 +467,15 @@ bool plan_exact(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group
   if (!split && (spt < 10 || units < 9 * cus)) return false;
   if (units < 12 * cus) {
     // Fewer than twelve stages a workgroup: the K-splitting tiles of gemm_i4_slices.hip, unless
-    // their estimate is clearly above this form's, {fixed, a stage} in us, fitted over 16 shapes each
-    // (rms 5 to 8 %).  Over 192 shapes of 65 to 512 rows the f32 class takes 0.95 of the time that it took
+    // their estimate is clearly above this form's, {fixed, a stage} in us, fitted over 16 to 30 shapes each
+    // (rms 5 to 8 %).  (f32 x in groups of 64 had {37.1, 3.35} while the sum of its partials lay in scratch: over 60
+    // shapes 0.88 of that time, 1.01 at worst; 440 x 11375 x 1536 68 / 50, 306 x 9645 x 3840 96 / 66.)  Over 192 shapes of 65 to 512 rows the f32 class takes 0.95 of the time that it took
     // with its hi and lo made in the loop, 1.02 at worst.
     struct Fit {
       float fixed, stage;
     };
     const bool wide_groups = group >= 128;
-    const Fit f = split ? (wide_groups ? Fit{25.3f, 3.33f} : Fit{37.1f, 3.35f})
+    const Fit f = split ? (wide_groups ? Fit{25.3f, 3.33f} : Fit{27.0f, 3.54f})
                         : (wide_groups ? Fit{16.4f, 2.26f} : Fit{15.4f, 2.47f});
     const float here = f.fixed + f.stage * ((float)units / (float)cus);
     if (here > 0.92f * slices_estimate_us(ctx, m, n, k, group, !split, split)) return false;
