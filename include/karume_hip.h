@@ -163,8 +163,9 @@ int32_t krm_dequant_i4(krm_ctx* ctx, krm_buf w, krm_buf scales, krm_buf out_f32,
  *   out    [m, n]  io_dtype
  * group must be a power of two >= 16 dividing k (docs/ir-v1.md:135-150).
  * The kernel is a pure function of (m, n, k, group, dtypes, compute); for m <= 16 a row of
- * `out` does not depend on the other rows in the call (same reduction order for every m; fp16 rows
- * in batches of 2 to 16: one row alone agrees to the rounding of its fp16 result). */
+ * `out` does not depend on the other rows in the call (same reduction order for every m; but fp16
+ * rows in groups of 128 and more with k a multiple of 256 have one order in batches of 2 to 16 and
+ * another alone, which agree to the rounding of the fp16 result). */
 int32_t krm_linear_i4(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                       krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                       int32_t io_dtype, int32_t scale_dtype, int32_t compute);

@@ -716,14 +716,6 @@ float slices_estimate_us(const krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k,
   return f.call + (float)rounds * (t.fixed + f.round + f.factor * t.per_1024 * (float)k * (1.0f / 1024));
 }
 
-float slices_few_rows_us(const krm_ctx* ctx, uint32_t n, uint32_t k, uint32_t group) {
-  uint64_t rounds = 0;
-  const TileCost t = group >= 128  ? cheapest_tile<kX16, 8>(ctx, 32, n, k, &rounds)
-                     : group == 64 ? cheapest_tile<kX16, 4>(ctx, 32, n, k, &rounds)
-                                   : cheapest_tile<kX16, 2>(ctx, 32, n, k, &rounds);
-  return (float)rounds * (t.fixed + t.per_1024 * (float)k * (1.0f / 1024));
-}
-
 // Any shape with K a multiple of 32 (at least 64), any group size of the format and 16-byte
 // aligned rows.  *handled = false (nothing launched) otherwise.
 int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,

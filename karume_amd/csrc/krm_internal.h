@@ -119,8 +119,6 @@ inline T* ptr(krm_buf address) {
 // What a product of the K-splitting tiles takes (gemm_i4_slices.hip).
 float slices_estimate_us(const krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                          bool half_x, bool split);
-// The costs between its tiles, for up to 32 rows of fp16 x.
-float slices_few_rows_us(const krm_ctx* ctx, uint32_t n, uint32_t k, uint32_t group);
 
 // What the K-splitting MFMA GEMM (gemm_i4_slices.hip) does with a finished sum besides storing it.
 struct RowsFusion {

@@ -1410,21 +1410,6 @@ int32_t linear_i4_gemm_f16(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, k
                            krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                            int32_t io_dtype, int32_t scale_dtype);
 
-// Whether 2 to 16 fp16 rows take the tiles that split K (gemm_i4_slices.hip: the same exact products, f32
-// sums and scaling on the matrix cores) and not the GEMV, whose vector ALUs do every row's products.  What
-// has matrix instructions in the GEMV (groups of 128, whole steps of 256) stays there, as do groups of 16,
-// which have a form that keeps up.  The line depends on the shape alone, so that a row has the same bits
-// in every batch of 2 to 16, and lies where two rows, which gain the least, do not lose by it: the tiles'
-// estimated time against a fixed part and one in n * k.  us on the GEMV / here: 16 rows 28437 x 512 in groups
-// of 64 54.5 / 7.2, 11 rows 7970 x 4416 in groups of 64 48 / 11, 9 rows 21833 x 3712 in groups of 128 89 /
-// 16, 5 rows 27304 x 3584 in groups of 32 63 / 29, 2 rows 11442 x 512 in groups of 64 6.5 / 5.5; below the
-// line 2 rows 933 x 4608 6.7 / 9.5, 13 rows 1772 x 4672 24.7 / 9.5.
-static bool few_rows_on_slices(const krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
-                               int32_t io_dtype) {
-  if (m < 2 || io_dtype != KRM_F16 || group < 32 || (k % 256 == 0 && group >= 128)) return false;
-  return 2.0f + 1.15f * slices_few_rows_us(ctx, n, k, group) < 4.0f + 0.3e-6f * (float)n * (float)k;
-}
-
 }  // namespace krm
 
 extern "C" {
@@ -1448,15 +1433,9 @@ int32_t krm_linear_i4(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_bu
                        aligned(scales, dtype_bytes(scale_dtype)) &&
                        aligned(bias, dtype_bytes(io_dtype)),
               "krm_linear_i4: x must be 16-byte aligned, w 4-byte aligned");
-  bool handled = false;
-  if (m <= 16) {
-    if (few_rows_on_slices(ctx, m, n, k, group, io_dtype)) {
-      KRM_TRY(linear_i4_gemm_slices(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
-                                    compute, RowsFusion{}, &handled, io_dtype));
-      if (handled) return KRM_OK;
-    }
+  if (m <= 16)
     return linear_i4_gemv(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype);
-  }
+  bool handled = false;
   KRM_TRY(linear_i4_gemm_exact(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
                                scale_dtype, compute, &handled));
   if (handled) return KRM_OK;

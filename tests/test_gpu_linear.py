@@ -403,8 +403,8 @@ def test_probe_exchange_is_bounded_and_clean(gpu_ctx):
                                    (1772, 4672, 32), (30000, 96, 32)])
 @pytest.mark.parametrize("scale_type", [np.float16, np.float32])
 def test_few_fp16_rows_have_the_same_bits_in_every_batch(gpu_ctx, n, k, g, scale_type):
-    """2 to 16 fp16 rows on either side of the line between the GEMV and the tiles that split K: a row
-    does not depend on its batch, and every result is the oracle's to one fp16 ulp."""
+    """2 to 16 fp16 rows where the GEMV has no matrix instructions: a row does not depend on its batch, and
+    every result is the oracle's to one fp16 ulp."""
     rng = np.random.default_rng(n + k)
     packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
     scale = scale.astype(scale_type)
@@ -457,3 +457,28 @@ def test_nine_to_sixteen_f32_rows_have_the_bits_of_one_row(gpu_ctx, n, k, g, m):
     for r in (0, 7, 8, m - 1):
         alone = run_linear(gpu_ctx, x[r:r + 1], packed, scale, bias, n, k, g)
         assert np.array_equal(got[r:r + 1].view(np.uint32), alone.view(np.uint32)), r
+
+
+@pytest.mark.parametrize("n,k,g", [(8200, 2080, 32), (12000, 1152, 128), (9000, 576, 64), (16001, 832, 64),
+                                   (1772, 4672, 32), (30000, 96, 32), (4096, 4096, 64)])
+@pytest.mark.parametrize("scale_type", [np.float16, np.float32])
+def test_few_fp16_rows_have_the_bits_of_one_row_alone(gpu_ctx, n, k, g, scale_type):
+    """fp16 rows without matrix instructions in the GEMV (groups below 128, or a K that is no multiple of 256):
+    one reduction order for one row and for 2 to 16, and for the fused entry point without a fusion."""
+    rng = np.random.default_rng(n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    scale = scale.astype(scale_type)
+    x = rng.normal(size=(16, k)).astype(np.float16)
+    bias = rng.normal(size=n).astype(np.float16)
+    alone = [run_linear(gpu_ctx, x[r:r + 1], packed, scale, bias, n, k, g).view(np.uint16) for r in (0, 3, 15)]
+    for m in (2, 5, 9, 16):
+        got = run_linear(gpu_ctx, x[:m], packed, scale, bias, n, k, g).view(np.uint16)
+        for r, want in zip((0, 3, 15), alone):
+            assert r >= m or np.array_equal(got[r:r + 1], want), (m, r)
+        buffers = [gpu_ctx.upload(a) for a in (x[:m], packed, scale, bias)]
+        out = gpu_ctx.alloc(m * n * 2)
+        gpu_ctx.linear_i4_fused(*buffers[:3], out, m, n, k, g, bias=buffers[3], io_dtype=ka.F16,
+                                scale_dtype=ka.dtype_code(scale.dtype))
+        assert np.array_equal(out.download(np.uint16, (m, n)), got), m
+        for b in buffers + [out]:
+            b.free()
