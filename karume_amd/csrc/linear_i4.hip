@@ -687,7 +687,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) voi
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x >> 6;
   constexpr bool XLDS = share_x_in_lds<XT, MB, NSTEP>();
-  constexpr bool kStageRows = NSTEP == kStagedRows && !NORM && !DECODE_ROW;
+  constexpr bool kStageRows = NSTEP == kStagedRows;
   // Four waves a workgroup (the launch below).  A wave whose rows lie past N stays: it re-reads
   // the last row and stores nothing, so no branch stands between the kernel's entry and its
   // loads (an early exit made the pointer arguments wait for the row test).
@@ -1193,7 +1193,7 @@ int32_t launch_gemv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf 
     }
   }
   if (fuse.positions) return fail(ctx, KRM_ERR_VALIDATION, "decode row: one row, even row count");
-  if constexpr (NSTEP <= kFusedSteps) {
+  if constexpr (NSTEP <= kFusedSteps && NSTEP != kStagedRows) {
     if (fuse.norm_weight) KRM_GEMV_LAUNCH(true, false); else KRM_GEMV_LAUNCH(false, false);
   } else {  // (pick_steps)
     KRM_GEMV_LAUNCH(false, false);

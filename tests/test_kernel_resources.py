@@ -52,3 +52,10 @@ def test_no_other_kernel_uses_scratch_memory(kernels):
 def test_every_form_that_may_spill_does(kernels):
     spilling = {n for n, k in kernels.items() if kernel_resources.scratch(k) > 0}
     assert [p for p in SPILL if not any(n.startswith(p) for n in spilling)] == []
+
+
+def test_rows_of_the_gemv_brought_to_lds_are_built_without_a_norm(kernels):
+    """Rows of x in LDS (a step count of -1) are picked without a norm alone: no other instance is built."""
+    staged = [arguments(n) for n in kernels if n.startswith("gemv_i4_kernel<") and arguments(n)[5] == "-1"]
+    assert len(staged) == 12
+    assert {(a[6], a[7]) for a in staged} == {("false", "false")}
