@@ -23,13 +23,12 @@
 // two LDS copies (distinct objects, so fragment reads may pass the parking writes), the
 // dequantisation of chunk c + 1 interleaved with the MFMAs of chunk c, one barrier a chunk.
 #include "gemm_i4_deal.h"
+#include "i4_codes.h"
 
 using namespace krm;
 
 namespace {
 
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
 // A K chunk of KC codes is staged per pass; rows are padded by 16 bytes so the 16-byte
@@ -68,13 +67,6 @@ __device__ inline _Float16 scale_from_bits<__half>(uint32_t bits) {
 template <>
 __device__ inline _Float16 scale_from_bits<float>(uint32_t bits) {
   return (_Float16)__uint_as_float(bits);
-}
-
-// (a & mask) | bits in one VALU op (the compiler emits two when both constants are literals).
-__device__ inline uint32_t and_or(uint32_t a, uint32_t mask, uint32_t bits) {
-  uint32_t d;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(mask), "v"(bits));
-  return d;
 }
 
 // 8 codes of a word -> 8 fp16 values (u - 8) * scale, order (c0,c4,c1,c5,c2,c6,c3,c7).
@@ -888,23 +880,6 @@ void gemm_i4_f16_dealt_kernel(const XT* __restrict__ x, const uint8_t* __restric
 // (the C layout keeps the column in lane % 32, so the scale is one value per lane and column
 // tile).  Stages, LDS layout, the (tile, stage) deal over the CUs and the ordered merge of the
 // partials are those of the kernel above.
-// 8 codes of a word -> 8 fp16 integers (u - 8), order (c0,c4,c1,c5,c2,c6,c3,c7).
-__device__ inline uint4 ints_word(uint32_t word) {
-  const uint32_t magic = 0x64006400u;  // (1024, 1024)
-  const half2_t off_lo = {(_Float16)1032.0f, (_Float16)1032.0f};
-  const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-  const half2_t off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
-  const uint32_t upper = word >> 8;
-  const half2_t q0 = __builtin_bit_cast(half2_t, and_or(word, 0x000F000Fu, magic)) - off_lo;
-  const half2_t q1 = __builtin_elementwise_fma(
-      __builtin_bit_cast(half2_t, and_or(word, 0x00F000F0u, magic)), sixteenth, off_hi);
-  const half2_t q2 = __builtin_bit_cast(half2_t, and_or(upper, 0x000F000Fu, magic)) - off_lo;
-  const half2_t q3 = __builtin_elementwise_fma(
-      __builtin_bit_cast(half2_t, and_or(upper, 0x00F000F0u, magic)), sixteenth, off_hi);
-  return make_uint4(__builtin_bit_cast(uint32_t, q0), __builtin_bit_cast(uint32_t, q1),
-                    __builtin_bit_cast(uint32_t, q2), __builtin_bit_cast(uint32_t, q3));
-}
-
 template <typename XT, typename ST>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ w,
@@ -1024,7 +999,7 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
           for (int nt = 0; nt < WN; ++nt) {
             const uint32_t word = j == 0 ? braw[nt].x : j == 1 ? braw[nt].y : j == 2 ? braw[nt].z
                                                                                     : braw[nt].w;
-            const half8_t b = __builtin_bit_cast(half8_t, ints_word(word));
+            const half8_t b = ints_paired(word);
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {

@@ -3,52 +3,15 @@
 // happens to a finished pair of columns.
 #pragma once
 
-#include "krm_internal.h"
+#include "i4_codes.h"
 
 namespace krm {
 namespace {
 
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
-template <typename T>
-__device__ inline float to_f32(T v);
-template <>
-__device__ inline float to_f32<float>(float v) { return v; }
-template <>
-__device__ inline float to_f32<__half>(__half v) { return __half2float(v); }
-template <typename T>
-__device__ inline T from_f32(float v);
-template <>
-__device__ inline float from_f32<float>(float v) { return v; }
-template <>
-__device__ inline __half from_f32<__half>(float v) { return __float2half_rn(v); }
-
-// (a & mask) | bits in one VALU op (the compiler emits two when both constants are literals).
-__device__ inline uint32_t and_or(uint32_t a, uint32_t mask, uint32_t bits) {
-  uint32_t d;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(mask), "v"(bits));
-  return d;
-}
-
-// 8 codes of a word -> 8 fp16 integers (u - 8).  1024 + u (or 1024 + 16 u) is built in the fp16
-// mantissa, one packed op removes the offset.
-// Order (c0,c4,c1,c5,c2,c6,c3,c7): two ops a pair, for activations stored in the same order.
-__device__ inline half8_t ints_paired(uint32_t word) {
-  const uint32_t magic = 0x64006400u;  // (1024, 1024)
-  const half2_t off_lo = {(_Float16)1032.0f, (_Float16)1032.0f};
-  const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-  const half2_t off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
-  const uint32_t upper = word >> 8;
-  const half2_t q0 = __builtin_bit_cast(half2_t, and_or(word, 0x000F000Fu, magic)) - off_lo;
-  const half2_t q1 = __builtin_elementwise_fma(
-      __builtin_bit_cast(half2_t, and_or(word, 0x00F000F0u, magic)), sixteenth, off_hi);
-  const half2_t q2 = __builtin_bit_cast(half2_t, and_or(upper, 0x000F000Fu, magic)) - off_lo;
-  const half2_t q3 = __builtin_elementwise_fma(
-      __builtin_bit_cast(half2_t, and_or(upper, 0x00F000F0u, magic)), sixteenth, off_hi);
-  return half8_t{q0.x, q0.y, q1.x, q1.y, q2.x, q2.y, q3.x, q3.y};
-}
+// 8 codes of a word -> 8 fp16 integers in their own order (ints_paired: the order of activations stored
+// as (x0,x4,x1,x5,x2,x6,x3,x7)).
 // Natural order c0..c7, as (u - 8) / 1024 (the sum over K is multiplied by 1024 at the end): the
 // even and the odd codes of the word are masked apart where they are and a byte of each becomes a pair
 // of fp16 subnormals, u 2^-24 and 16 u 2^-24, which one packed fma scales and offsets exactly (ten

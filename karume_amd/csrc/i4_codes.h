@@ -1,0 +1,58 @@
+// Element types as f32, and packed int4 codes as fp16 integers: what every int4 product shares.
+#pragma once
+
+#include "krm_internal.h"
+
+namespace krm {
+namespace {
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+
+template <typename T>
+__device__ inline float to_f32(T v);
+template <>
+__device__ inline float to_f32<float>(float v) { return v; }
+template <>
+__device__ inline float to_f32<__half>(__half v) { return __half2float(v); }
+template <typename T>
+__device__ inline T from_f32(float v);
+template <>
+__device__ inline float from_f32<float>(float v) { return v; }
+template <>
+__device__ inline __half from_f32<__half>(float v) { return __float2half_rn(v); }
+
+// (a & mask) | bits in one VALU op: the compiler splits it in two when both constants are
+// literals, because this ISA's three-operand encodings take no literal.
+__device__ inline uint32_t and_or(uint32_t a, uint32_t mask, uint32_t bits) {
+  uint32_t d;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(mask), "v"(bits));
+  return d;
+}
+
+// Eight codes of one u32 as four fp16 pairs holding the exact integers (u - 8): pair i = (code i,
+// code i+4).  1024 + u is built in the fp16 mantissa, then the offset is removed with one packed op;
+// codes in the upper nibble of a byte arrive as 1024 + 16u.  Two ops a pair, for activations stored in
+// the same order.
+__device__ inline void codes_to_half2(uint32_t word, half2_t (&q)[4]) {
+  const uint32_t magic = 0x64006400u;  // (1024.0, 1024.0)
+  const half2_t off_lo = {(_Float16)1032.0f, (_Float16)1032.0f};
+  const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
+  const half2_t off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
+  const uint32_t upper = word >> 8;
+  q[0] = __builtin_bit_cast(half2_t, and_or(word, 0x000F000Fu, magic)) - off_lo;
+  q[1] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(word, 0x00F000F0u, magic)),
+                                   sixteenth, off_hi);
+  q[2] = __builtin_bit_cast(half2_t, and_or(upper, 0x000F000Fu, magic)) - off_lo;
+  q[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(upper, 0x00F000F0u, magic)),
+                                   sixteenth, off_hi);
+}
+// The same as one operand of a matrix instruction: (c0,c4,c1,c5,c2,c6,c3,c7).
+__device__ inline half8_t ints_paired(uint32_t word) {
+  half2_t q[4];
+  codes_to_half2(word, q);
+  return half8_t{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+}
+
+}  // namespace
+}  // namespace krm

@@ -14,15 +14,13 @@
 // reduction order therefore differs from the reference's (results agree within a stated
 // tolerance, not bitwise) but depends on (K, group) only — never on M, N or the launch — so a
 // row of x gives the same bits whether it is run alone or in a batch.
-#include "krm_internal.h"
+#include "i4_codes.h"
 
 #include <cmath>
 
 using namespace krm;
 
 namespace {
-
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 // ------------------------------------------------------------------------------------ dequant
 
@@ -121,31 +119,6 @@ __device__ inline float wave_sum4(float a, float b, float c, float d, int lane) 
   const float p1 = (odd ? d : c) + dpp_from<0xB1>(odd ? c : d);  // even lanes: c, odd lanes: d
   const float q = (high ? p1 : p0) + dpp_from<0x4E>(high ? p0 : p1);
   return wave_sum_tail(q);
-}
-
-// Eight codes of one u32 as four fp16 pairs holding the exact integers (u - 8):
-// pair i = (code i, code i+4).  1024 + u is built in the fp16 mantissa, then the offset is
-// removed with one packed op; codes in the upper nibble of a byte arrive as 1024 + 16u.
-// (a & mask) | bits in one VALU op: the compiler splits it in two when both constants are
-// literals, because this ISA's three-operand encodings take no literal.
-__device__ inline uint32_t and_or(uint32_t a, uint32_t mask, uint32_t bits) {
-  uint32_t d;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(mask), "v"(bits));
-  return d;
-}
-
-__device__ inline void codes_to_half2(uint32_t word, half2_t (&q)[4]) {
-  const uint32_t magic = 0x64006400u;  // (1024.0, 1024.0)
-  const half2_t off_lo = {(_Float16)1032.0f, (_Float16)1032.0f};
-  const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-  const half2_t off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
-  const uint32_t upper = word >> 8;
-  q[0] = __builtin_bit_cast(half2_t, and_or(word, 0x000F000Fu, magic)) - off_lo;
-  q[1] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(word, 0x00F000F0u, magic)),
-                                   sixteenth, off_hi);
-  q[2] = __builtin_bit_cast(half2_t, and_or(upper, 0x000F000Fu, magic)) - off_lo;
-  q[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(upper, 0x00F000F0u, magic)),
-                                   sixteenth, off_hi);
 }
 
 // Eight consecutive fp16 activations (x0..x7 in four dwords) regrouped to match
@@ -601,20 +574,6 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_tiles_kernel(
     step(tile + gridDim.x, 1, odd);
   }
 }
-
-
-template <typename T>
-__device__ inline float to_f32(T v);
-template <>
-__device__ inline float to_f32<float>(float v) { return v; }
-template <>
-__device__ inline float to_f32<__half>(__half v) { return __half2float(v); }
-template <typename T>
-__device__ inline T from_f32(float v);
-template <>
-__device__ inline float from_f32<float>(float v) { return v; }
-template <>
-__device__ inline __half from_f32<__half>(float v) { return __float2half_rn(v); }
 
 // Optional work fused around the dot products (all null / 0 = the plain linear op).
 struct GemvFusion {
