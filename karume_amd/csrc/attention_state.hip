@@ -185,8 +185,8 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // scale and k * scale are rounded before the product.  Blocks of fp16 rows run on
 // v_mfma_f32_16x16x32_f16, sixteen times that rate: K and V are fp16 as they are, q is fp16 or three fp16 parts
 // of the row times a power of two (33 bits below the row's largest magnitude), a probability from 2^-16 on three
-// parts of p 2^15 (all its bits; a block with a smaller one multiplies V with f32 operands), products are exact,
-// sums f32, scale^2 multiplies the f32 sum.
+// parts of p 2^15 (all its bits; a row with a smaller one in the block multiplies V with f32 operands there),
+// products are exact, sums f32, scale^2 multiplies the f32 sum.
 // Error against 64 bits (2-norm, f32 queries, normal values; all in f32 operands): D = 64 behind 1024
 // 2.6e-7 (3.9e-7), D = 128 2.8e-7 (4.6e-7), D = 256 3.6e-7 (6.5e-7); queries four times as large 5.6e-7 (9.1e-7),
 // 7.1e-7 (1.3e-6), 8.5e-7 (1.7e-6).  A part of zero beside an infinity
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   constexpr bool kHalf = sizeof(ST) == 2;
   constexpr int kHalfRow = D + 8;             // halves of a parked row
   // A probability from 2^-16 on is three fp16 parts of p 2^15, all its 24 bits: below that the last of them
-  // lie under fp16's smallest step, and a block that holds such a probability takes f32 operands.
+  // lie under fp16's smallest step, and a row with such a probability takes f32 operands in that block.
   constexpr int kPParts = 3;
   constexpr float kPScale = 32768.0f, kPLeast = 1.0f / 65536.0f;
   constexpr int kQParts = sizeof(XT) == 2 ? 1 : 3, kSteps = D / 32;
@@ -682,16 +682,40 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 #pragma unroll
           for (int i = 0; i < 4; ++i) p[t][i] *= kPScale;
       }
-      bool half_sums = half_block;
+      // Rows with such a small probability in the block take f32 operands, the others of the sixteen see zeros
+      // there: a row's sums do not depend on its neighbours.
+      bool small = !half_block, some_small = small, all_small = small;
       if (kMode != kNever && half_block) {
         uint32_t least = 0xffffffffu;  // (of the bits less one: a zero comes out on top)
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int i = 0; i < 4; ++i) least = min(least, __float_as_uint(p[t][i]) - 1u);
-        half_sums = !__any(least < __float_as_uint(kPLeast * kPScale) - 1u);
+        small = least < __float_as_uint(kPLeast * kPScale) - 1u;
+        const uint64_t lanes = __ballot(small);  // (a row's keys lie in four lanes)
+        some_small = lanes != 0;
+        if (some_small) {
+          const uint64_t pairs = lanes | lanes >> 32;
+          const uint32_t rows = (uint32_t)(pairs | pairs >> 16) & 0xffffu;
+          small = (rows >> r & 1u) != 0;
+          all_small = rows == 0xffffu;
+        }
       }
-      if (half_sums) {
+      if (some_small)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float weight = small ? p[j / 4][j % 4] : 0.f;
+        p[j / 4][j % 4] = small ? 0.f : p[j / 4][j % 4];
+#pragma unroll
+        for (int i = 0; i < kVPieces; ++i) {
+          const float4 v4 = element4(vraw[j * kVPieces + i], pv_key + v_step(j), slots);
+          const float vf[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[rb][4 * i + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[e], weight, acc[rb][4 * i + e], 0, 0, 0);
+        }
+      }
+      if (!all_small) {
         half8_t ph[kPParts];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -721,18 +745,6 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
               acc[rb][4 * i + e] =
                   __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[q], acc[rb][4 * i + e], 0, 0, 0);
           }
-      } else
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-#pragma unroll
-        for (int i = 0; i < kVPieces; ++i) {
-          const float4 v4 = element4(vraw[j * kVPieces + i], pv_key + v_step(j), slots);
-          const float vf[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            acc[rb][4 * i + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[e], p[j / 4][j % 4],
-                                                                     acc[rb][4 * i + e], 0, 0, 0);
-        }
       }
     }
     if (kAhead && more) request_v(kb + (uint32_t)WAVES);

@@ -1045,3 +1045,22 @@ def test_small_probabilities_over_an_fp16_state_keep_their_bits(gpu_ctx, depth, 
         bound = bound + 2.0 ** -11 * want + 2.0 ** -25
     assert np.all(np.abs(got[:, :8] - want) <= bound)
     assert not got[:, 8:].any()
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+@pytest.mark.parametrize("past", [32, 33, 320])
+@pytest.mark.parametrize("io", [np.float32, np.float16])
+def test_a_row_over_an_fp16_state_has_the_same_bits_beside_a_steep_row(gpu_ctx, depth, past, io):
+    """A query whose probabilities are small (its scores spread over hundreds) takes f32 operands for them; the
+    rows beside it in a block of sixteen keep their bits."""
+    rng = np.random.default_rng(depth + past)
+    m, scale = 20, float(np.float32(np.sqrt(1.0 / np.sqrt(float(depth)))))
+    q, ik, iv = (rng.normal(size=(m, depth)).astype(io) for _ in range(3))
+    sk, sv = (rng.normal(size=(past + m, depth)).astype(np.float16) for _ in range(2))
+    q *= io(0.5)
+    alone = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale)
+    q[5] *= io(100)
+    beside = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale)
+    rest = np.delete(np.arange(m), 5)
+    assert np.isfinite(beside).all() and not np.array_equal(alone[5], beside[5])
+    assert alone[rest].tobytes() == beside[rest].tobytes()
