@@ -191,8 +191,8 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // 2.6e-7 (3.9e-7), D = 128 2.8e-7 (4.6e-7), D = 256 3.6e-7 (6.5e-7); queries four times as large 5.6e-7 (9.1e-7),
 // 7.1e-7 (1.3e-6), 8.5e-7 (1.7e-6).  A part of zero beside an infinity
 // of the state is a NaN that the value itself would not give, and 2^15 times a sum of this step's f32 rows
-// can be infinite where the sum is not: a wave whose walk leaves a value that is not finite walks again with
-// f32 operands and without the factor.  With g = lane / 16:
+// can be infinite where the sum is not: a row whose sums are not finite is formed anew with f32 operands and
+// without the factor, alone.  With g = lane / 16:
 //   S^T = K Q^T    two tiles of 16 keys; A = the K tile (row = key, lane group g walks dims
 //                  g D/4 ..), B = Q^T (column = query row): a lane ends up with the scores of
 //                  ONE query row (lane % 16) against keys 16 t + 4 g + i (t < 2, i < 4), so the
@@ -314,6 +314,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   __shared__ __align__(16) __half s_q[kSplitQ ? kQParts * kRows * kHalfRow : 8];  // the parts of Q
   __shared__ float s_factor[kSplitQ ? kRows : 1];                                // scale^2 2^-e of a row
   __shared__ float s_m[WAVES][kRows], s_l[WAVES][kRows];
+  __shared__ uint32_t s_lost[WAVES];
 
   const uint32_t z = blockIdx.x, row0 = blockIdx.y * (uint32_t)kRows;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -751,40 +752,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     wave_sync();  // the block's rows have been read: the next block may be parked
   }
   };
-  if constexpr (!kHalf) {
-    walk(std::integral_constant<int, kNever>{});
-  } else {
-    bool plain = kSplitQ && slot_columns(c_lo) != 32u;  // no block of fp16 keys
-    if (!plain) {
-      walk(std::integral_constant<int, sizeof(XT) == 2 ? kAlways : kSlotBlocks>{});
-      bool lost = false;
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        bool here = run_l[rb] != run_l[rb];
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) here = here || !(fabsf(acc[rb][dt][i]) < INFINITY);
-        lost = lost || (here && row0 + (uint32_t)(16 * rb + r) < query);
-      }
-      // (parts of a value meet an infinity of the state as 0 * inf, the value itself does not; 2^15 takes
-      // sums of this step's f32 rows past f32's range from 1e34 on: once more without either)
-      plain = __any(lost);
-      if (plain && kAhead && (uint32_t)wave < blocks) {
-        request_k((uint32_t)wave);
-        request_v((uint32_t)wave);
-      }
-    }
-    if (plain) walk(std::integral_constant<int, kNever>{});
-    const float unscale = plain ? 1.0f : 1.0f / kPScale;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[rb][dt][i] *= unscale;
-  }
-
+  // The end of a turn: the waves' states are merged, the rows `due` and not `lost` in any wave written, the
+  // chunk's own rows stored by the first turn.  Returns the rows lost in any wave.
+  auto finish = [&](uint32_t due, uint32_t lost, bool first) __attribute__((always_inline)) -> uint32_t {
   // The chunk's own K / V rows of this block go to the state slots when asked for (the first query
   // head of each kv plane does it; asked for here, stored behind the merge).  Without a window no
   // reader of this launch touches them: slot rows are read for columns < past only, these are
@@ -796,13 +766,14 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     const uint32_t i = min((uint32_t)tid + j * kBlock, (uint32_t)kQUnits - 1u);
     const uint32_t row = min(row0 + i / kPieces, query - 1u);
     const size_t src = ((size_t)kv_plane * a.chunk_rows + row) * D + 4 * (i % kPieces);
-    if (append) {
+    if (append && first) {
       own_k[j] = load4_raw<XT>(ins_k + src);
       own_v[j] = load4_raw<XT>(ins_v + src);
     }
   }
 
   // the wave's state: (max, sum) per query row and O[row][d] in its own area
+  if (kHalf && lane == 0) s_lost[wave] = lost;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     for (int x = 16; x <= 32; x <<= 1) {
@@ -823,6 +794,11 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   }
   __syncthreads();
 
+  if constexpr (kHalf) {
+#pragma unroll
+    for (int wv = 0; wv < WAVES; ++wv) lost |= s_lost[wv];
+  }
+
   // merge of the waves, wave order: a row's dims dealt over the threads of its block of 16 rows (a
   // workgroup of two waves takes two rounds)
   constexpr uint32_t kUnits = kBlock < 256u ? 256u : kBlock;
@@ -841,7 +817,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       total_l = fmaf(wgt[wv], s_l[wv][rr], total_l);
     }
     const float inv = 1.0f / total_l;
-    if (row < a.chunk_rows) {
+    if (row < a.chunk_rows && (!kHalf || (due & ~lost) >> rr & 1u)) {
 #pragma unroll
       for (int e = 0; e < kPer; ++e) {
         float o = 0.f;
@@ -857,7 +833,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     }
    }
   }
-  if (append) {
+  if (append && first) {
 #pragma unroll
     for (int j = 0; j < kQPer; ++j) {
       const uint32_t i = (uint32_t)tid + j * kBlock, row = row0 + i / kPieces;
@@ -870,6 +846,46 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       st_f32<ST>(slot_v, dst + 2, vv.z); st_f32<ST>(slot_v, dst + 3, vv.w);
     }
   }
+  return lost;
+  };
+
+  // One turn writes every row.  Over an fp16 state a row whose sums are not finite in some wave is written by a
+  // second turn, with f32 operands and without the factor: parts of a value meet an infinity of the state
+  // as 0 * inf, the value itself does not, and 2^15 takes sums of this step's f32 rows past f32's range from
+  // 1e34 on.  The other rows keep what the first turn wrote, whatever stands beside them.
+  constexpr uint32_t kEvery = 0xffffffffu;  // a bit for each row of the workgroup
+  uint32_t due = kEvery;
+  bool first = true;
+  if constexpr (kHalf) {
+    if (!kSplitQ || slot_columns(c_lo) == 32u) {  // (else there is no block of fp16 keys)
+      walk(std::integral_constant<int, sizeof(XT) == 2 ? kAlways : kSlotBlocks>{});
+      uint32_t lost = 0;  // of the wave's rows
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        bool here = !(fabsf(run_l[rb]) < INFINITY);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            here = here || !(fabsf(acc[rb][dt][i]) < INFINITY);
+            acc[rb][dt][i] *= 1.0f / kPScale;
+          }
+        const uint64_t lanes = __ballot(here && row0 + (uint32_t)(16 * rb + r) < query);
+        const uint64_t pairs = lanes | lanes >> 32;
+        lost |= ((uint32_t)(pairs | pairs >> 16) & 0xffffu) << (16 * rb);
+      }
+      due = finish(kEvery, lost, true);
+      if (due == 0) return;  // (the same rows in every thread)
+      first = false;
+      __syncthreads();  // the waves' states have been read: their areas take key blocks again
+      if (kAhead && (uint32_t)wave < blocks) {
+        request_k((uint32_t)wave);
+        request_v((uint32_t)wave);
+      }
+    }
+  }
+  walk(std::integral_constant<int, kNever>{});
+  finish(due, 0u, first);
 }
 
 // ------------------------------------------------------------------------------ decode

@@ -1064,3 +1064,22 @@ def test_a_row_over_an_fp16_state_has_the_same_bits_beside_a_steep_row(gpu_ctx, 
     rest = np.delete(np.arange(m), 5)
     assert np.isfinite(beside).all() and not np.array_equal(alone[5], beside[5])
     assert alone[rest].tobytes() == beside[rest].tobytes()
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+@pytest.mark.parametrize("past", [32, 33, 320])
+@pytest.mark.parametrize("io", [np.float32, np.float16])
+@pytest.mark.parametrize("entry", [np.nan, np.inf])
+def test_a_row_over_an_fp16_state_has_the_same_bits_beside_a_row_that_is_not_finite(gpu_ctx, depth, past, io, entry):
+    """A row whose sums are not finite is formed once more with f32 operands, alone: the rows beside it in a block
+    of sixteen keep their bits."""
+    rng = np.random.default_rng(depth + past)
+    m, scale = 20, float(np.float32(np.sqrt(1.0 / np.sqrt(float(depth)))))
+    q, ik, iv = (rng.normal(size=(m, depth)).astype(io) for _ in range(3))
+    sk, sv = (rng.normal(size=(past + m, depth)).astype(np.float16) for _ in range(2))
+    alone = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale)
+    q[5, 3] = io(entry)
+    beside = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale)
+    rest = np.delete(np.arange(m), 5)
+    assert np.isnan(beside[5]).all() and np.isfinite(beside[rest]).all()
+    assert alone[rest].tobytes() == beside[rest].tobytes()
