@@ -184,12 +184,13 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // beside an fp16 state) run on v_mfma_f32_16x16x4_f32 with the generic kernel's operand roundings: q *
 // scale and k * scale are rounded before the product.  Blocks of fp16 rows run on
 // v_mfma_f32_16x16x32_f16, sixteen times that rate: K and V are fp16 as they are, q is fp16 or three fp16 parts
-// of the row times a power of two (33 bits below the row's largest magnitude), a probability from 2^-16 on three
-// parts of p 2^15 (all its bits; a row with a smaller one in the block multiplies V with f32 operands there),
-// products are exact, sums f32, scale^2 multiplies the f32 sum.
+// of the row times powers of two (all bits of an entry down to 2^-36 of the row's largest magnitude; a row with
+// smaller ones is formed with f32 operands), a probability from 2^-16 on three parts of p 2^15 (all its bits; a row
+// with a smaller one in the block multiplies V with f32 operands there), products are exact, sums f32, scale^2
+// multiplies the f32 sum.
 // Error against 64 bits (2-norm, f32 queries, normal values; all in f32 operands): D = 64 behind 1024
-// 2.6e-7 (3.9e-7), D = 128 2.8e-7 (4.6e-7), D = 256 3.6e-7 (6.5e-7); queries four times as large 5.6e-7 (9.1e-7),
-// 7.1e-7 (1.3e-6), 8.5e-7 (1.7e-6).  A part of zero beside an infinity
+// 2.3e-7 (3.6e-7), D = 128 2.4e-7 (4.4e-7), D = 256 3.1e-7 (6.3e-7); queries four times as large 4.6e-7 (9.0e-7),
+// 6.3e-7 (1.2e-6), 7.9e-7 (1.7e-6).  A part of zero beside an infinity
 // of the state is a NaN that the value itself would not give, and 2^15 times a sum of this step's f32 rows
 // can be infinite where the sum is not: a row whose sums are not finite is formed anew with f32 operands and
 // without the factor, alone.  With g = lane / 16:
@@ -211,12 +212,12 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // rows a workgroup (not 32) so that a 128-row chunk of 32 heads is 256 workgroups, one per CU.
 // What bounds f32 rows is their matrix rate with two waves a SIMD to cover softmax and waits (D = 64,
 // r = 8, 128 rows behind 1024: 8 us of MFMA), fp16 rows the vector instructions of softmax and operands.
-// us with f32 operands / with fp16 ones / with fp16 ones where blocks hold probabilities below 2^-16 (queries
-// four times as large), 128 rows behind 1024 and 512 behind 2048: fp16 D = 64 21.3 / 11.8 / 15.8, 123 / 60 / 85; D =
-// 128, r = 4 34.1 / 17.9 / 25.3, 236 / 107 / 164; D = 256 71 / 34 / 55, 148 / 69 / 109; f32 queries D = 64 22.0 / 16.5 /
-// 19.1, 131 / 83 / 112; D = 128 38.2 / 22.3 / 29.8, 267 / 142 / 204; D = 256 76 / 47 / 68, 161 / 103 / 140.  (Two parts
-// for every probability, 22 bits and nothing below 2^-40, took 0 to 9 % less.)  Before those f32
-// forms, with V parked as well, rows looked up one by one (two element types: a wait at each), expf and no
+// us with f32 operands / with fp16 ones / with fp16 ones where rows hold probabilities below 2^-16 (queries
+// four times as large), 128 rows behind 1024 and 512 behind 2048: fp16 D = 64 19.1 / 10.5 / 15.2, 118 / 53 / 89; D =
+// 128, r = 4 32 / 17 / 25, 234 / 106 / 166; D = 256, 16 heads, r = 8 71 / 36 / 56, 272 / 133 / 216; f32 queries D = 64
+// 20.8 / 14.8 / 19.0, 130 / 80 / 115; D = 128 36 / 21 / 29, 265 / 140 / 207; D = 256 76 / 50 / 70, 302 / 196 / 275.
+// (Two parts for every probability, 22 bits and nothing below 2^-40, and q's parts at one scale took 0 to 11 %
+// less.)  Before those f32 forms, with V parked as well, rows looked up one by one (two element types: a wait at each), expf and no
 // requests ahead, us before / with f32 operands: the case of 8 us of MFMA
 // 22.7 / 19.3; fp16, D = 128, r = 4: 49.4 / 32.6; f32 over fp16 slots 106.5 / 36.8; D = 256, r = 8
 // (two waves then, four now that LDS holds K alone): 172 / 71.
@@ -309,6 +310,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
   constexpr int kPParts = 3;
   constexpr float kPScale = 32768.0f, kPLeast = 1.0f / 65536.0f;
   constexpr int kQParts = sizeof(XT) == 2 ? 1 : 3, kSteps = D / 32;
+  constexpr float kQNext = 2048.0f;
   __shared__ __align__(16) float s_k[WAVES][32 * kRow];
   constexpr bool kSplitQ = kHalf && sizeof(XT) == 4;
   __shared__ __align__(16) __half s_q[kSplitQ ? kQParts * kRows * kHalfRow : 8];  // the parts of Q
@@ -489,8 +491,11 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       const uint32_t i = (uint32_t)tid + j * kBlock;
       float4 v = raw4_f32<XT>(qraw[j]);
       if (split) {
-        // The row times 2^e, its largest magnitude in [2^13, 2^14), as three fp16 parts (33 bits).  A
-        // row lies in kPieces neighbouring lanes.
+        // The row times 2^e, its largest magnitude in [2^13, 2^14), as three fp16 parts, each what the one
+        // before it leaves times 2^11: all 24 bits of an entry down to 2^-36 of the largest, in sums of their
+        // own that are put together at the end (at one scale the parts ended at 2^-24, and entries below 2^-14
+        // of the largest lost bits).  A row with an entry that they do not hold gets a NaN for its factor, and
+        // with it the second turn.  A row lies in kPieces neighbouring lanes.
         float top = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 #pragma unroll
         for (int off = 1; off < kPieces; off <<= 1) top = fmaxf(top, __shfl_xor(top, off, kWave));
@@ -503,18 +508,25 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
           down = __uint_as_float((uint32_t)(127 - power) << 23);
         }
         float left[4] = {v.x * up, v.y * up, v.z * up, v.w * up};  // exact: a power of two
-        if (i < (uint32_t)kQUnits) {
-          if (i % kPieces == 0) s_factor[i / kPieces] = a.scale * a.scale * down;
+        __half parts[kQParts][4];
+        bool whole = true;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
 #pragma unroll
           for (int p = 0; p < kQParts; ++p) {
-            __half* to = s_q + (p * kRows + i / kPieces) * kHalfRow + 4 * (i % kPieces);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const __half part = __float2half_rn(left[e]);
-              to[e] = part;
-              left[e] -= __half2float(part);
-            }
+            parts[p][e] = __float2half_rn(left[e]);
+            left[e] = (left[e] - __half2float(parts[p][e])) * kQNext;
           }
+          whole = whole && left[e] == 0.f;
+        }
+        const uint64_t row_lanes = (kPieces == 64 ? ~0ull : (1ull << (kPieces % 64)) - 1ull) << (lane & ~(kPieces - 1));
+        whole = (~__ballot(whole) & row_lanes) == 0;
+        if (i < (uint32_t)kQUnits) {
+          if (i % kPieces == 0) s_factor[i / kPieces] = whole ? a.scale * a.scale * down : NAN;
+#pragma unroll
+          for (int p = 0; p < kQParts; ++p)
+            __builtin_memcpy(__builtin_assume_aligned(
+                s_q + (p * kRows + i / kPieces) * kHalfRow + 4 * (i % kPieces), 8), parts[p], 8);
         }
       }
       v.x *= a.scale; v.y *= a.scale; v.z *= a.scale; v.w *= a.scale;
@@ -593,6 +605,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
       if (half_block) {
         const __half* keys = reinterpret_cast<const __half*>(mk) + r * kHalfRow + 8 * g;
         const float factor = kQDirect ? a.scale * a.scale : s_factor[kSplitQ ? 16 * rb + r : 0];
+        float4v_t sums[kQParts][2];  // of a part of q each
+#pragma unroll
+        for (int p = 0; p < kQParts; ++p) sums[p][0] = sums[p][1] = st[0];
 #pragma unroll
         for (int i = 0; i < kSteps; ++i) {
           half8_t qs[kQParts];
@@ -605,14 +620,19 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
           for (int t = 0; t < 2; ++t) {
             const half8_t kh = *reinterpret_cast<const half8_t*>(keys + 16 * t * kHalfRow + 32 * i);
 #pragma unroll
-            for (int p = kQParts - 1; p >= 0; --p)
-              st[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qs[p], st[t], 0, 0, 0);
+            for (int p = 0; p < kQParts; ++p)
+              sums[p][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qs[p], sums[p][t], 0, 0, 0);
           }
         }
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) st[t][i] *= factor;
+          for (int i = 0; i < 4; ++i) {
+            float sum = sums[kQParts - 1][t][i];
+#pragma unroll
+            for (int p = kQParts - 2; p >= 0; --p) sum = fmaf(sum, 1.0f / kQNext, sums[p][t][i]);
+            st[t][i] = sum * factor;
+          }
       } else
 #pragma unroll
       for (int i = 0; i < kQuarter / 4; ++i) {

@@ -1083,3 +1083,26 @@ def test_a_row_over_an_fp16_state_has_the_same_bits_beside_a_row_that_is_not_fin
     rest = np.delete(np.arange(m), 5)
     assert np.isnan(beside[5]).all() and np.isfinite(beside[rest]).all()
     assert alone[rest].tobytes() == beside[rest].tobytes()
+
+
+@pytest.mark.parametrize("depth", [64, 128, 256])
+@pytest.mark.parametrize("past", [32, 96])
+@pytest.mark.parametrize("power", [12, 20, 30, 60])
+def test_small_entries_of_an_f32_query_over_an_fp16_state_keep_their_bits(gpu_ctx, depth, past, power):
+    """An entry of 2^power stands where every key is zero, so that the others decide the scores: they keep the bits
+    that f32 operands keep (a product is rounded three times: 3 * 2^-24 of sum |q k|; exponential and sums
+    stay below 2^-20).  Down to 2^-36 of the largest they fit three fp16 parts, below that the row takes f32
+    operands."""
+    rng = np.random.default_rng(depth + past)
+    m = 18
+    q, ik, iv = (rng.normal(size=(m, depth)).astype(np.float32) for _ in range(3))
+    sk, sv = (rng.normal(size=(past + m, depth)).astype(np.float16) for _ in range(2))
+    q[::2, 0] = 2.0 ** power
+    sk[:, 0] = ik[:, 0] = 0.0
+    scale = float(np.float32(np.sqrt(1.0 / np.sqrt(float(depth)))))
+    got = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale).astype(np.float64)
+    k = np.concatenate([sk[:past].astype(np.float64), ik.astype(np.float64)])
+    v = np.concatenate([sv[:past].astype(np.float64), iv.astype(np.float64)])
+    want = attention_in_64_bits(q, k, v, past, scale)
+    moved = 3 * 2.0 ** -24 * (np.abs(q.astype(np.float64)) @ np.abs(k).T).max(axis=1) * scale * scale + 2.0 ** -20
+    assert np.all(np.abs(got - want) <= 2 * moved[:, None] * np.abs(v).max())
