@@ -633,28 +633,50 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
             for (int p = kQParts - 2; p >= 0; --p) sum = fmaf(sum, 1.0f / kQNext, sums[p][t][i]);
             st[t][i] = sum * factor;
           }
-      } else
-#pragma unroll
-      for (int i = 0; i < kQuarter / 4; ++i) {
-        float qs[4];
-        if constexpr (kQDirect) {  // (the second walk)
-          const uint32_t row = min(row0 + (uint32_t)(16 * rb + r), a.chunk_rows - 1);
-          const float4 v = load4_f32<XT>(q + ((size_t)z * a.chunk_rows + row) * D + g * kQuarter + 4 * i);
-          qs[0] = v.x * a.scale; qs[1] = v.y * a.scale; qs[2] = v.z * a.scale; qs[3] = v.w * a.scale;
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) qs[j] = qf[rb][4 * i + j];
-        }
-        float kf[2][4];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-          *reinterpret_cast<float4*>(kf[t]) =
-              *reinterpret_cast<const float4*>(&mk[(16 * t + r) * kRow + g * kQuarter + 4 * i]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
+      } else {
+        // The keys' next piece is read beside the products of this one where it gains (f32 rows, D = 64, 128
+        // rows behind 1024 17.7 us left to the compiler, 17.5 so; D = 256 70.8 and 69.9; D = 128, 512 behind
+        // 2048 234 and 235).
+        constexpr bool kKeysAhead = !kHalf && D != 128;
+        auto read_keys = [&](int i, float (&to)[2][4]) {
 #pragma unroll
           for (int t = 0; t < 2; ++t)
-            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][j], qs[j], st[t], 0, 0, 0);
+            *reinterpret_cast<float4*>(to[t]) =
+                *reinterpret_cast<const float4*>(&mk[(16 * t + r) * kRow + g * kQuarter + 4 * i]);
+        };
+        float next[2][4];
+        if constexpr (kKeysAhead) {
+          read_keys(0, next);
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < kQuarter / 4; ++i) {
+          float qs[4];
+          if constexpr (kQDirect) {  // (the second walk)
+            const uint32_t row = min(row0 + (uint32_t)(16 * rb + r), a.chunk_rows - 1);
+            const float4 v = load4_f32<XT>(q + ((size_t)z * a.chunk_rows + row) * D + g * kQuarter + 4 * i);
+            qs[0] = v.x * a.scale; qs[1] = v.y * a.scale; qs[2] = v.z * a.scale; qs[3] = v.w * a.scale;
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) qs[j] = qf[rb][4 * i + j];
+          }
+          float kf[2][4];
+          if constexpr (kKeysAhead) {
+            __builtin_memcpy(kf, next, sizeof(kf));
+            if (i + 1 < kQuarter / 4) read_keys(i + 1, next);
+          } else {
+            read_keys(i, kf);
+          }
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+              st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t][j], qs[j], st[t], 0, 0, 0);
+          if constexpr (kKeysAhead) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+          }
+        }
       }
       // this lane: query row 16 rb + r, keys 16 t + 4 g + i
       // (uniform: a block that every one of these rows sees whole needs no mask)
