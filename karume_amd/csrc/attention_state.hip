@@ -217,8 +217,8 @@ __global__ __launch_bounds__(kThreads) void attention_generic_kernel(
 // 128, r = 4 32 / 17 / 25, 234 / 106 / 166; D = 256, 16 heads, r = 8 71 / 36 / 56, 272 / 133 / 216; f32 queries D = 64
 // 20.8 / 14.8 / 19.0, 130 / 80 / 115; D = 128 36 / 21 / 29, 265 / 140 / 207; D = 256 76 / 50 / 70, 302 / 196 / 275.
 // (Two parts for every probability, 22 bits and nothing below 2^-40, and q's parts at one scale took 0 to 11 %
-// less.)  Before those f32 forms, with V parked as well, rows looked up one by one (two element types: a wait at each), expf and no
-// requests ahead, us before / with f32 operands: the case of 8 us of MFMA
+// less.)  Before those f32 forms, with V parked as well, rows looked up one by one (two element types: a wait
+// at each), expf and no requests ahead, us before / with f32 operands: the case of 8 us of MFMA
 // 22.7 / 19.3; fp16, D = 128, r = 4: 49.4 / 32.6; f32 over fp16 slots 106.5 / 36.8; D = 256, r = 8
 // (two waves then, four now that LDS holds K alone): 172 / 71.
 typedef float float4v_t __attribute__((ext_vector_type(4)));

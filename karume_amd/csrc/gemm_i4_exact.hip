@@ -469,8 +469,9 @@ bool plan_exact(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group
     // Fewer than twelve stages a workgroup: the K-splitting tiles of gemm_i4_slices.hip, unless
     // their estimate is clearly above this form's, {fixed, a stage} in us, fitted over 16 to 30 shapes each
     // (rms 5 to 8 %).  (f32 x in groups of 64 had {37.1, 3.35} while the sum of its partials lay in scratch: over 60
-    // shapes 0.88 of that time, 1.01 at worst; 440 x 11375 x 1536 68 / 50, 306 x 9645 x 3840 96 / 66.)  Over 192 shapes of 65 to 512 rows the f32 class takes 0.95 of the time that it took
-    // with its hi and lo made in the loop, 1.02 at worst.
+    // shapes 0.88 of that time, 1.01 at worst; 440 x 11375 x 1536 68 / 50, 306 x 9645 x 3840 96 / 66.)  Over 192
+    // shapes of 65 to 512 rows the f32 class takes 0.95 of the time that it took with its hi and lo made in the
+    // loop, 1.02 at worst.
     struct Fit {
       float fixed, stage;
     };
