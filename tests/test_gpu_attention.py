@@ -1106,3 +1106,34 @@ def test_small_entries_of_an_f32_query_over_an_fp16_state_keep_their_bits(gpu_ct
     want = attention_in_64_bits(q, k, v, past, scale)
     moved = 3 * 2.0 ** -24 * (np.abs(q.astype(np.float64)) @ np.abs(k).T).max(axis=1) * scale * scale + 2.0 ** -20
     assert np.all(np.abs(got - want) <= 2 * moved[:, None] * np.abs(v).max())
+
+
+@pytest.mark.parametrize("io", [np.float32, np.float16])
+@pytest.mark.parametrize("infinite", [False, True])
+def test_two_row_blocks_a_workgroup_have_the_bits_of_one_over_an_fp16_state(gpu_ctx, io, infinite):
+    """512 heads of 20 rows are workgroups of two blocks of sixteen rows, one head two workgroups: the same bits, also
+    for a steep row, a row that is not finite (alone in the second turn) and, with an infinity in the state, rows
+    that all take the second turn."""
+    rng = np.random.default_rng(int(infinite))
+    heads, m, depth, past, scale = 512, 20, 64, 96, 0.5
+    q, ik, iv = (rng.normal(size=(m, depth)).astype(io) for _ in range(3))
+    sk, sv = (rng.normal(size=(past + m, depth)).astype(np.float16) for _ in range(2))
+    q[2] *= io(50)
+    q[17] *= io(50)
+    q[18, 3] = np.nan
+    if infinite:
+        sv[40, 9] = np.inf
+    one = chunk_over_fp16_state(gpu_ctx, q, ik, iv, sk, sv, past, scale)
+    bufs = [gpu_ctx.upload(np.ascontiguousarray(a)) for a in (np.broadcast_to(q, (heads, m, depth)), ik, iv, sk, sv)]
+    out = gpu_ctx.zeros(heads * q.nbytes)
+    gpu_ctx.attention_chunk(*bufs, out, batch=1, heads=heads, kv_heads=1, chunk_rows=m, depth=depth,
+                            capacity=past + m, window=0, half_scale=scale, past=past, query=m,
+                            io_dtype=ka.dtype_code(q.dtype), kv_dtype=ka.F16)
+    many = out.download(q.dtype, (heads, m, depth))
+    finite = np.delete(np.arange(m), 18)
+    assert np.isnan(one[18]).all() and np.isnan(many[:, 18]).all()
+    assert np.isfinite(one[finite, 9]).any() != infinite  # (a steep row's zero times the infinity is a NaN)
+    if infinite:
+        one, many = np.delete(one, 9, axis=1), np.delete(many, 9, axis=2)
+    assert np.isfinite(one[finite]).all()
+    assert all(head[finite].tobytes() == one[finite].tobytes() for head in many)
