@@ -547,6 +547,103 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
 
   float run_m[RB], run_l[RB];
   float4v_t acc[RB][DT];
+  // The end of a turn: the waves' states are merged, the rows `due` and not `lost` in any wave written, the
+  // chunk's own rows stored by the first turn.  Returns the rows lost in any wave.
+  auto finish = [&](uint32_t due, uint32_t lost, bool first) __attribute__((always_inline)) -> uint32_t {
+  // The chunk's own K / V rows of this block go to the state slots when asked for (the first query
+  // head of each kv plane does it; asked for here, stored behind the merge).  Without a window no
+  // reader of this launch touches them: slot rows are read for columns < past only, these are
+  // rows past + row.
+  const bool append = (flags & KRM_CHUNK_APPEND) && z % (a.heads / a.kv_heads) == 0;
+  uint4 own_k[kQPer], own_v[kQPer];
+#pragma unroll
+  for (int j = 0; j < kQPer; ++j) {
+    const uint32_t i = min((uint32_t)tid + j * kBlock, (uint32_t)kQUnits - 1u);
+    const uint32_t row = min(row0 + i / kPieces, query - 1u);
+    const size_t src = ((size_t)kv_plane * a.chunk_rows + row) * D + 4 * (i % kPieces);
+    if (append && first) {
+      own_k[j] = load4_raw<XT>(ins_k + src);
+      own_v[j] = load4_raw<XT>(ins_v + src);
+    }
+  }
+
+  // the wave's state: (max, sum) per query row and O[row][d] in its own area
+  if (kHalf && lane == 0) s_lost[wave] = lost;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    for (int x = 16; x <= 32; x <<= 1) {
+      const Exchanged both = exchange(run_l[rb], run_l[rb], x);
+      run_l[rb] = both.clear + both.set;
+    }
+    if (g == 0) {
+      s_m[wave][16 * rb + r] = run_m[rb];
+      s_l[wave][16 * rb + r] = run_l[rb];
+    }
+#pragma unroll
+    for (int i = 0; i < kVPieces; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)  // register j of tiles 4 i + 0..3: dims 64 i + 16 g + 4 j + 0..3
+        *reinterpret_cast<float4*>(&mk[(16 * rb + r) * kRow + 64 * i + 16 * g + 4 * j]) =
+            make_float4(acc[rb][4 * i][j], acc[rb][4 * i + 1][j], acc[rb][4 * i + 2][j],
+                        acc[rb][4 * i + 3][j]);
+  }
+  __syncthreads();
+
+  if constexpr (kHalf) {
+#pragma unroll
+    for (int wv = 0; wv < WAVES; ++wv) lost |= s_lost[wv];
+  }
+
+  // merge of the waves, wave order: a row's dims dealt over the threads of its block of 16 rows (a
+  // workgroup of two waves takes two rounds)
+  constexpr uint32_t kUnits = kBlock < 256u ? 256u : kBlock;
+  for (uint32_t unit = tid; unit < kUnits; unit += kBlock) {
+   for (uint32_t rb = 0; rb < (uint32_t)RB; ++rb) {
+    constexpr int kPer = 16 * D / (int)kUnits, kParts = D / kPer;
+    const uint32_t rr = 16u * rb + unit / kParts, d0 = (unit % kParts) * kPer;
+    const uint32_t row = row0 + rr;
+    float top = s_m[0][rr];
+#pragma unroll
+    for (int wv = 1; wv < WAVES; ++wv) top = fmaxf(top, s_m[wv][rr]);  // finite: the own column
+    float wgt[WAVES], total_l = 0.f;
+#pragma unroll
+    for (int wv = 0; wv < WAVES; ++wv) {
+      wgt[wv] = expf(s_m[wv][rr] - top);
+      total_l = fmaf(wgt[wv], s_l[wv][rr], total_l);
+    }
+    const float inv = 1.0f / total_l;
+    if (row < a.chunk_rows && (!kHalf || (due & ~lost) >> rr & 1u)) {
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) {
+        float o = 0.f;
+#pragma unroll
+        for (int wv = 0; wv < WAVES; ++wv) o = fmaf(wgt[wv], s_k[wv][rr * kRow + d0 + e], o);
+        float value = row < query ? o * inv : 0.0f;
+        if (out_f16 && sizeof(XT) == 4) value = rounded_f32(value);  // the f32 result, rounded again
+        if (out_f16)
+          st_f32<__half>(reinterpret_cast<__half*>(out), out_index(row, d0 + e), value);
+        else
+          st_f32<XT>(out, out_index(row, d0 + e), value);
+      }
+    }
+   }
+  }
+  if (append && first) {
+#pragma unroll
+    for (int j = 0; j < kQPer; ++j) {
+      const uint32_t i = (uint32_t)tid + j * kBlock, row = row0 + i / kPieces;
+      if (i >= (uint32_t)kQUnits || row >= query) continue;
+      const size_t dst = ((size_t)kv_plane * a.capacity + past + row) * D + 4 * (i % kPieces);
+      const float4 kv = raw4_f32<XT>(own_k[j]), vv = raw4_f32<XT>(own_v[j]);
+      st_f32<ST>(slot_k, dst, kv.x); st_f32<ST>(slot_k, dst + 1, kv.y);
+      st_f32<ST>(slot_k, dst + 2, kv.z); st_f32<ST>(slot_k, dst + 3, kv.w);
+      st_f32<ST>(slot_v, dst, vv.x); st_f32<ST>(slot_v, dst + 1, vv.y);
+      st_f32<ST>(slot_v, dst + 2, vv.z); st_f32<ST>(slot_v, dst + 3, vv.w);
+    }
+  }
+  return lost;
+  };
+
   // One walk over the wave's key blocks: kNever, kAlways or (f32 queries: this step's own rows are f32)
   // kSlotBlocks with fp16 operands.
   enum { kNever, kAlways, kSlotBlocks };
@@ -635,7 +732,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
           }
       } else {
         // The keys' next piece is read beside the products of this one where it gains (f32 rows, D = 64, 128
-        // rows behind 1024 17.7 us left to the compiler, 17.5 so; D = 256 70.8 and 69.9; D = 128, 512 behind
+        // rows behind 1024 17.7 us left to the compiler, 17.5 so; D = 256 70.8 and 68.8; D = 128, 512 behind
         // 2048 234 and 235).
         constexpr bool kKeysAhead = !kHalf && D != 128;
         auto read_keys = [&](int i, float (&to)[2][4]) {
@@ -794,103 +891,6 @@ __global__ __launch_bounds__(64 * WAVES) void attention_rows_kernel(
     wave_sync();  // the block's rows have been read: the next block may be parked
   }
   };
-  // The end of a turn: the waves' states are merged, the rows `due` and not `lost` in any wave written, the
-  // chunk's own rows stored by the first turn.  Returns the rows lost in any wave.
-  auto finish = [&](uint32_t due, uint32_t lost, bool first) __attribute__((always_inline)) -> uint32_t {
-  // The chunk's own K / V rows of this block go to the state slots when asked for (the first query
-  // head of each kv plane does it; asked for here, stored behind the merge).  Without a window no
-  // reader of this launch touches them: slot rows are read for columns < past only, these are
-  // rows past + row.
-  const bool append = (flags & KRM_CHUNK_APPEND) && z % (a.heads / a.kv_heads) == 0;
-  uint4 own_k[kQPer], own_v[kQPer];
-#pragma unroll
-  for (int j = 0; j < kQPer; ++j) {
-    const uint32_t i = min((uint32_t)tid + j * kBlock, (uint32_t)kQUnits - 1u);
-    const uint32_t row = min(row0 + i / kPieces, query - 1u);
-    const size_t src = ((size_t)kv_plane * a.chunk_rows + row) * D + 4 * (i % kPieces);
-    if (append && first) {
-      own_k[j] = load4_raw<XT>(ins_k + src);
-      own_v[j] = load4_raw<XT>(ins_v + src);
-    }
-  }
-
-  // the wave's state: (max, sum) per query row and O[row][d] in its own area
-  if (kHalf && lane == 0) s_lost[wave] = lost;
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    for (int x = 16; x <= 32; x <<= 1) {
-      const Exchanged both = exchange(run_l[rb], run_l[rb], x);
-      run_l[rb] = both.clear + both.set;
-    }
-    if (g == 0) {
-      s_m[wave][16 * rb + r] = run_m[rb];
-      s_l[wave][16 * rb + r] = run_l[rb];
-    }
-#pragma unroll
-    for (int i = 0; i < kVPieces; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)  // register j of tiles 4 i + 0..3: dims 64 i + 16 g + 4 j + 0..3
-        *reinterpret_cast<float4*>(&mk[(16 * rb + r) * kRow + 64 * i + 16 * g + 4 * j]) =
-            make_float4(acc[rb][4 * i][j], acc[rb][4 * i + 1][j], acc[rb][4 * i + 2][j],
-                        acc[rb][4 * i + 3][j]);
-  }
-  __syncthreads();
-
-  if constexpr (kHalf) {
-#pragma unroll
-    for (int wv = 0; wv < WAVES; ++wv) lost |= s_lost[wv];
-  }
-
-  // merge of the waves, wave order: a row's dims dealt over the threads of its block of 16 rows (a
-  // workgroup of two waves takes two rounds)
-  constexpr uint32_t kUnits = kBlock < 256u ? 256u : kBlock;
-  for (uint32_t unit = tid; unit < kUnits; unit += kBlock) {
-   for (uint32_t rb = 0; rb < (uint32_t)RB; ++rb) {
-    constexpr int kPer = 16 * D / (int)kUnits, kParts = D / kPer;
-    const uint32_t rr = 16u * rb + unit / kParts, d0 = (unit % kParts) * kPer;
-    const uint32_t row = row0 + rr;
-    float top = s_m[0][rr];
-#pragma unroll
-    for (int wv = 1; wv < WAVES; ++wv) top = fmaxf(top, s_m[wv][rr]);  // finite: the own column
-    float wgt[WAVES], total_l = 0.f;
-#pragma unroll
-    for (int wv = 0; wv < WAVES; ++wv) {
-      wgt[wv] = expf(s_m[wv][rr] - top);
-      total_l = fmaf(wgt[wv], s_l[wv][rr], total_l);
-    }
-    const float inv = 1.0f / total_l;
-    if (row < a.chunk_rows && (!kHalf || (due & ~lost) >> rr & 1u)) {
-#pragma unroll
-      for (int e = 0; e < kPer; ++e) {
-        float o = 0.f;
-#pragma unroll
-        for (int wv = 0; wv < WAVES; ++wv) o = fmaf(wgt[wv], s_k[wv][rr * kRow + d0 + e], o);
-        float value = row < query ? o * inv : 0.0f;
-        if (out_f16 && sizeof(XT) == 4) value = rounded_f32(value);  // the f32 result, rounded again
-        if (out_f16)
-          st_f32<__half>(reinterpret_cast<__half*>(out), out_index(row, d0 + e), value);
-        else
-          st_f32<XT>(out, out_index(row, d0 + e), value);
-      }
-    }
-   }
-  }
-  if (append && first) {
-#pragma unroll
-    for (int j = 0; j < kQPer; ++j) {
-      const uint32_t i = (uint32_t)tid + j * kBlock, row = row0 + i / kPieces;
-      if (i >= (uint32_t)kQUnits || row >= query) continue;
-      const size_t dst = ((size_t)kv_plane * a.capacity + past + row) * D + 4 * (i % kPieces);
-      const float4 kv = raw4_f32<XT>(own_k[j]), vv = raw4_f32<XT>(own_v[j]);
-      st_f32<ST>(slot_k, dst, kv.x); st_f32<ST>(slot_k, dst + 1, kv.y);
-      st_f32<ST>(slot_k, dst + 2, kv.z); st_f32<ST>(slot_k, dst + 3, kv.w);
-      st_f32<ST>(slot_v, dst, vv.x); st_f32<ST>(slot_v, dst + 1, vv.y);
-      st_f32<ST>(slot_v, dst + 2, vv.z); st_f32<ST>(slot_v, dst + 3, vv.w);
-    }
-  }
-  return lost;
-  };
-
   // One turn writes every row.  Over an fp16 state a row whose sums are not finite in some wave is written by a
   // second turn, with f32 operands and without the factor: parts of a value meet an infinity of the state
   // as 0 * inf, the value itself does not, and 2^15 takes sums of this step's f32 rows past f32's range from
