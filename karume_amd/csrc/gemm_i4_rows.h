@@ -4,6 +4,7 @@
 #pragma once
 
 #include "i4_codes.h"
+#include "lds_stream.h"
 
 namespace krm {
 namespace {
@@ -38,27 +39,6 @@ __device__ inline half8_t ints_natural(uint32_t word) {
 // counted by hand (vector memory operations of a wave complete in order).  Nothing else of the K
 // loop loads from memory through the compiler.
 
-// 16 bytes a lane from base + offset to LDS at lds + 16 * lane.
-__device__ inline void stream_to_lds(uint32_t lds, uint32_t offset, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds),
-               "v"(offset), "s"(base)
-               : "memory");
-}
-// The same for a dword or a zero-extended ushort a lane, to LDS at lds + 4 * lane.
-__device__ inline void stream_word_to_lds(uint32_t lds, uint32_t offset, const void* base, bool half) {
-  if (half)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" ::"s"(lds),
-                 "v"(offset), "s"(base)
-                 : "memory");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds),
-                 "v"(offset), "s"(base)
-                 : "memory");
-}
-template <int N>
-__device__ inline void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 // silu(gate) * up with the roundings of the decode row's epilogue
 __device__ inline float silu_times(float gate, float up) {
   const float t = __builtin_amdgcn_exp2f(-fabsf(gate) * 1.4426950408889634f);

@@ -23,7 +23,7 @@
 // two's-complement nibble in the upper half of a byte reads as the signed byte 16 * q; the
 // integer dot products therefore run on bytes 16 * q (two ops per four codes, no sign
 // extension) and the exact factor 16 is shifted out of the group sum before it is converted.
-#include "krm_internal.h"
+#include "lds_stream.h"
 
 namespace {
 
@@ -662,14 +662,20 @@ void linear_w4a8_tile_kernel(
   }
 }
 
-// The same staging with a 128 x 256 workgroup tile, wave = 64 x 64 (or 64 x 128 and 64 x 32, four
-// waves), for groups of 32, 64 or 128
-// codes.  Four 32 x 32 tiles per wave would need 64 int32 and 64 f32 accumulators at once, more
-// than two waves per SIMD leave room for, so the work is ordered by group: the group's weight
-// words are expanded once (both column tiles, all MFMA steps of the group), then each row tile
-// in turn runs its two MFMA chains over the group and is fused into its f32 accumulators — 32
-// int32 accumulators live at a time, and the expansion is shared by the two row tiles.
-// (Groups of 32 in the smaller tile only, see the dispatch.)
+// 64 x 128 tiles of four waves of 64 x 32, several a CU, or 128 x 256 ones of eight waves of 64 x 64, for groups
+// of 32, 64 or 128 codes (32 in the smaller tile only, see the dispatch).  The work is ordered by group: the
+// group's weight words are expanded once, then each row tile in turn runs its MFMA chains over the group
+// and is fused into its f32 accumulators, so that one row tile's int32 sums live at a time.
+//
+// Bound by the vector ALUs beside the matrix pipe, 32 subtractions and 32 fmas a group and wave against 8
+// MFMAs, and at its end by the writes of all tiles, which the chip holds at once (512 x 11008: 6 us).
+// Stages go from memory to LDS directly, two ahead of the one that is read.  Staged through registers, one
+// ahead, a stage of 512 x 11008 x 4096 took 2283 clk: 281 to ask for the next one, 640 of products, 1218 of
+// waiting for it (a scale a lane touched 64 lines: 445 of them) and parking it, 143 at the barrier.  Now
+// 1551: 299, 1139, 45, 68.  us with the quantiser's launch, before / now, fp16 scales unless noted: 512 x 11008 x
+// 4096 51.4 / 46.6, in groups of 64 60.6 / 55.0, of 32 105 / 83, with f32 scales (whose quotient by 16 was
+// tested in every group) 56.8 / 47.9; 2048 x 11008 x 4096 166 / 157; 20 x 20000 x 1024 in groups of 32 18.2 / 15.1;
+// 500 x 600 x 8000 in groups of 32, f32 scales 112 / 72.
 template <typename ST, int GSH, int WM, int NW, int WN>
 __global__ __launch_bounds__(64 * WM * NW) __attribute__((amdgpu_waves_per_eu(2, WN == 2 ? 2 : 4)))
 void linear_w4a8_tall_kernel(
@@ -678,90 +684,77 @@ void linear_w4a8_tall_kernel(
     uint32_t m, uint32_t n, uint32_t k, uint32_t m_blocks, uint32_t n_blocks) {
   static_assert(GSH >= 5 && GSH <= 7, "groups of 32, 64 or 128 codes");
   static_assert(GSH > 5 || WN == 1, "two column tiles of groups of 32 spill");
-  constexpr int T = 64 * WM * NW, MT = 2;
+  constexpr int kWaves = WM * NW, MT = 2;
   constexpr int BM = 64 * WM, BN = 32 * WN * NW;
   constexpr int kStage = 128;                          // codes per LDS stage
-  constexpr int kRowA = kStage + 16, kRowB = kStage / 2 + 16;
   constexpr int kGroupsPerStage = kStage >> GSH;       // 4, 2 or 1
   constexpr int kStepsPerGroup = 1 << (GSH - 5);       // MFMA steps of 32 codes: 1, 2 or 4
-  constexpr int kAUnits = BM * (kStage / 16) / T;      // 16-byte units of xq per thread
-  constexpr int kBUnits = BN * (kStage / 32) / T;      // and of packed weights
-  __shared__ __align__(16) uint8_t s_a[2][BM * kRowA];
-  __shared__ __align__(16) uint8_t s_b[2][BN * kRowB];
-  __shared__ __align__(16) float s_s[2][BN][kGroupsPerStage];
+  constexpr int kDepth = 3;                            // stages in LDS: one is read, two are on their way
+  constexpr int kXBytes = BM * kStage, kWBytes = BN * kStage / 2;
+  constexpr int kXLoads = kXBytes / 1024 / kWaves, kWLoads = kWBytes / 1024 / kWaves;  // of a wave and stage
+  // Scales come in blocks of stages, neighbouring lanes on neighbouring groups of a column: a load costs
+  // by the lines that it touches.  Two blocks in LDS: one is read, one is filled.
+  constexpr int kBlock = GSH == 7 ? 4 : 2, kEntries = kBlock * kGroupsPerStage;
+  constexpr int kSBytes = BN * kEntries * 4, kSLoads = kSBytes / 256 / kWaves;  // of a wave and block
+  __shared__ __align__(1024) uint8_t s_x[kDepth * kXBytes];
+  __shared__ __align__(1024) uint8_t s_w[kDepth * kWBytes];
+  __shared__ __align__(1024) uint8_t s_s[2 * kSBytes];
 
   const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
   const uint32_t mb = slot % m_blocks, nb = (slot / m_blocks) * 8u + xcd;
   if (nb >= n_blocks) return;  // the whole workgroup leaves before any barrier
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / NW, wn = wave % NW;
-  const int frag_row = lane & 31, frag_h = lane >> 5;
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t wm = wave / NW, wn = wave % NW;
+  const uint32_t frag_row = lane & 31u, frag_h = lane >> 5;
   const uint32_t m0 = mb * BM, n0 = nb * BN;
   const uint32_t groups = k >> GSH;
   const uint32_t chunks_total = k >> 6;
-  // bytes of a step's codes that a half of the wave takes: a step of a 64-code chunk is 16 codes of
-  // each half of it, of a group of 32 the two halves of the group
-  constexpr int kHalfA = GSH == 5 ? 16 : 32, kHalfB = GSH == 5 ? 8 : 16;
   const uint32_t stages = (k + kStage - 1) / kStage;
 
-  // staging roles: xq rows in 8 units of 16 bytes (rows tid / 8 + 64 i), weight rows in 4
-  // (rows tid / 4 + 128 i)
-  const uint32_t arow0 = tid >> 3, aunit = (tid & 7u) * 16u;
-  const uint32_t brow0 = tid >> 2, bunit = (tid & 3u) * 16u;
-  // 32-bit offsets from bases that are the same for the whole workgroup: a stage's addresses take no
-  // vector instructions (a tile's 128 rows of x lie within 4 GiB, see the dispatch).  A K that ends inside
-  // a stage: the lanes past it re-read the row's start; their groups are fused with a zero scale.
-  const uint8_t* const a_tile = xq + (size_t)m0 * k;
-  const uint8_t* const b_tile = w + (size_t)n0 * (k >> 1);
-  const ST* const s_tile = scales + (size_t)n0 * groups;
-  uint32_t a_row[kAUnits], b_row[kBUnits];
-#pragma unroll
-  for (int i = 0; i < kAUnits; ++i) a_row[i] = min(arow0 + (T / 8) * i, m - 1 - m0) * k + aunit;
-#pragma unroll
-  for (int i = 0; i < kBUnits; ++i) b_row[i] = min(brow0 + (T / 4) * i, n - 1 - n0) * (k >> 1) + bunit;
-  const uint32_t s_row = min((uint32_t)(tid < BN ? tid : 0), n - 1 - n0) * groups;
-
-  struct Staged {
-    uint4 a[kAUnits];
-    uint4 b[kBUnits];
-    ST s[kGroupsPerStage];
+  // A stage in LDS: rows of xq of 128 bytes, of weights of 64, their 16-byte pieces turned by the row number
+  // so that the rows of a fragment spread over all banks.  A load of a wave brings eight rows of xq
+  // or sixteen of weights.  32-bit offsets from bases that are the same for the whole workgroup (a
+  // tile's 128 rows of x lie within 4 GiB, see the dispatch).
+  const uint8_t* const x_tile = xq + (size_t)m0 * k;
+  const uint8_t* const w_tile = w + (size_t)n0 * (k >> 1);
+  const uint8_t* const s_tile = reinterpret_cast<const uint8_t*>(scales + (size_t)n0 * groups);
+  auto lds_address = [](const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p;
   };
-  auto load_stage = [&](uint32_t asked, Staged& d) {
-    const uint32_t stage = min(asked, stages - 1u);  // (past the last one: again, unused)
-    const uint8_t* const a_at = a_tile + (size_t)stage * kStage;
-    const uint8_t* const b_at = b_tile + (size_t)stage * (kStage / 2);
-    const bool past = GSH < 7 && stage * kStage + kStage > k;
-    const uint32_t a_back = past && stage * kStage + aunit >= k ? stage * kStage + aunit : 0u;
-    const uint32_t b_back = past && stage * (kStage / 2) + bunit >= (k >> 1) ? stage * (kStage / 2) + bunit : 0u;
+  const uint32_t x_lds = lds_address(s_x) + wave * 1024u, w_lds = lds_address(s_w) + wave * 1024u;
+  const uint32_t s_lds = lds_address(s_s) + wave * 256u;
+  uint32_t x_row[kXLoads], w_row[kWLoads];
 #pragma unroll
-    for (int i = 0; i < kAUnits; ++i)
-      d.a[i] = *reinterpret_cast<const uint4*>(
-          GSH < 7 ? a_tile + (a_row[i] + stage * kStage - a_back) : a_at + a_row[i]);
+  for (uint32_t i = 0; i < kXLoads; ++i) x_row[i] = min((wave + kWaves * i) * 8u + lane / 8u, m - 1u - m0) * k;
 #pragma unroll
-    for (int i = 0; i < kBUnits; ++i)
-      d.b[i] = *reinterpret_cast<const uint4*>(
-          GSH < 7 ? b_tile + (b_row[i] + stage * (kStage / 2) - b_back) : b_at + b_row[i]);
+  for (uint32_t i = 0; i < kWLoads; ++i)
+    w_row[i] = min((wave + kWaves * i) * 16u + lane / 4u, n - 1u - n0) * (k >> 1);
+  // (row >> 1) & 7 of a load's rows of xq; the number of loads between a wave's own is even
+  static_assert(kWaves % 2 == 0, "a wave's loads begin at rows of one parity of eight");
+  const uint32_t x_piece = ((lane & 7u) ^ (((wave & 1u) * 4u + lane / 16u) & 7u)) * 16u;
+  const uint32_t w_piece = ((lane & 3u) ^ ((lane >> 4) & 3u)) * 16u;  // (row >> 2) & 3
+  auto request_scales = [&](uint32_t block) {
 #pragma unroll
-    for (int j = 0; j < kGroupsPerStage; ++j)
-      d.s[j] = s_tile[s_row + min(stage * kGroupsPerStage + j, groups - 1u)];
+    for (uint32_t i = 0; i < kSLoads; ++i) {
+      const uint32_t entry = (wave + kWaves * i) * 64u + lane;
+      const uint32_t col = min(entry / kEntries, n - 1u - n0);
+      const uint32_t g = min(block * kEntries + entry % kEntries, groups - 1u);
+      stream_word_to_lds(s_lds + (block & 1u) * kSBytes + kWaves * 256u * i, (col * groups + g) * (uint32_t)sizeof(ST),
+                         s_tile, sizeof(ST) == 2);
+    }
   };
-  auto park_stage = [&](int buf, const Staged& d) {
+  // (past the last stage: the last one again, unused; past K: its last codes again, whose groups are fused
+  // with a zero scale)
+  auto request = [&](uint32_t asked, uint32_t buf) {
+    const uint32_t stage = min(asked, stages - 1u);
+    const uint32_t x_at = min(stage * kStage + x_piece, k - 16u);
+    const uint32_t w_at = min(stage * (kStage / 2) + w_piece, (k >> 1) - 16u);
 #pragma unroll
-    for (int i = 0; i < kAUnits; ++i) {
-      uint4 v;
-      v.x = __builtin_amdgcn_perm(d.a[i].y, d.a[i].x, 0x06040200u);
-      v.y = __builtin_amdgcn_perm(d.a[i].y, d.a[i].x, 0x07050301u);
-      v.z = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x06040200u);
-      v.w = __builtin_amdgcn_perm(d.a[i].w, d.a[i].z, 0x07050301u);
-      *reinterpret_cast<uint4*>(&s_a[buf][(arow0 + (T / 8) * i) * kRowA + aunit]) = v;
-    }
+    for (uint32_t i = 0; i < kXLoads; ++i)
+      stream_to_lds(x_lds + buf * kXBytes + kWaves * 1024u * i, x_row[i] + x_at, x_tile);
 #pragma unroll
-    for (int i = 0; i < kBUnits; ++i)
-      *reinterpret_cast<uint4*>(&s_b[buf][(brow0 + (T / 4) * i) * kRowB + bunit]) = d.b[i];
-    if (tid < BN) {
-#pragma unroll
-      for (int j = 0; j < kGroupsPerStage; ++j) s_s[buf][tid][j] = scale_f32<ST>(&d.s[j], 0);
-    }
+    for (uint32_t i = 0; i < kWLoads; ++i)
+      stream_to_lds(w_lds + buf * kWBytes + kWaves * 1024u * i, w_row[i] + w_at, w_tile);
   };
 
   float accf[MT][WN][16];
@@ -771,55 +764,71 @@ void linear_w4a8_tall_kernel(
     for (int nt = 0; nt < WN; ++nt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) accf[mt][nt][r] = 0.f;
-  const v16i_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  // Sums start from 1.5 * 2^23 as a float's bits: a sum of 2^21 at most stays in its last 22 bits, and one
+  // subtraction makes it a float (a conversion takes twice a subtraction's time).
+  static_assert(GSH <= 7, "a group's sum of 16 xq q fits 22 bits");
+  constexpr int kMagicBits = 0x4B400000;
+  constexpr float kMagic = 12582912.0f;
+  v16i_t magic;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) magic[r] = kMagicBits;
 
-  Staged staged;
-  load_stage(0, staged);
-  park_stage(0, staged);
-  __syncthreads();
+  request_scales(0);
+  request(0, 0);
+  request(1, 1);
 
-  const uint32_t a_base = (uint32_t)((wm * 64 + frag_row) * kRowA + kHalfA * frag_h);
-  const uint32_t b_base = (uint32_t)((wn * 32 * WN + frag_row) * kRowB + kHalfB * frag_h);
-  auto run_stage = [&](uint32_t stage, int buf) {
-    load_stage(stage + 1, staged);
-    __builtin_amdgcn_sched_barrier(0);  // the requests stay a stage ahead of their use
+  // Fragment addresses.  A step of 32 codes takes 16 of each half of the wave, neighbours in memory: in a chunk
+  // of 64 codes step s takes the codes 32 h + 16 s .., in a group of 32 the codes 16 h ...  (Pieces
+  // of a row are told apart by exclusive or: their place is a power of two's bits.)
+  const uint32_t x_frag = (wm * 64u + frag_row) * 128u + (((GSH == 5 ? frag_h : 2u * frag_h) ^ ((frag_row >> 1) & 7u)) * 16u);
+  const uint32_t w_frag = (wn * 32u * WN + frag_row) * 64u +
+                          (((GSH == 5 ? 0u : frag_h) ^ ((frag_row >> 2) & 3u)) * 16u) + (GSH == 5 ? 8u * frag_h : 0u);
+  const uint32_t s_frag = (wn * 32u * WN + frag_row) * (kEntries * 4u);
+  // eight codes, two per byte, as bytes of 16 q in their order
+  auto expand = [](uint32_t word0, uint32_t word1) {
+    v4i_t b;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t word = i ? word1 : word0;
+      const uint32_t even = ((word << 4) ^ 0x80808080u) & 0xF0F0F0F0u, odd = (word ^ 0x88888888u) & 0xF0F0F0F0u;
+      b[2 * i] = (int)__builtin_amdgcn_perm(odd, even, 0x05010400u);
+      b[2 * i + 1] = (int)__builtin_amdgcn_perm(odd, even, 0x07030602u);
+    }
+    return b;
+  };
+  auto run_stage = [&](uint32_t stage, const uint32_t buf) {
+    // this stage has landed in every wave (the next one's loads may be on their way), and the one before
+    // it has been read
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kXLoads + kWLoads) : "memory");
+    if (stage % kBlock == 0) request_scales(stage / kBlock + 1u);
+    request(stage + 2u, (buf + 2u) % kDepth);
+    const uint8_t* const xs_at = s_x + buf * kXBytes;
+    const uint8_t* const ws_at = s_w + buf * kWBytes;
+    const uint8_t* const ss_at = s_s + (stage / kBlock & 1u) * kSBytes + s_frag + stage % kBlock * (kGroupsPerStage * 4u);
 #pragma unroll
     for (int gi = 0; gi < kGroupsPerStage; ++gi) {
       // codes 0 .. (1 << GSH) - 1 of the group = MFMA steps 0 .. kStepsPerGroup - 1;
       // step st lies in chunk (gi << GSH) / 64 + st / 2, half st % 2
-      const int first_chunk_in_stage = (gi << GSH) >> 6;
-      const bool valid = GSH == 5 ? stage * 4u + gi < groups
-                                  : stage * 2u + first_chunk_in_stage < chunks_total;
+      const int first_chunk = (gi << GSH) >> 6;
+      const bool valid = GSH == 7 || (GSH == 5 ? stage * 4u + gi < groups : stage * 2u + first_chunk < chunks_total);
       v4i_t bexp[WN][kStepsPerGroup];
       float mult[WN];
 #pragma unroll
       for (int nt = 0; nt < WN; ++nt) {
+        if constexpr (GSH == 5) {
+          const uint2 words = *reinterpret_cast<const uint2*>(ws_at + ((w_frag + nt * 2048) ^ (16 * gi)));
+          bexp[nt][0] = expand(words.x, words.y);
+        } else {
 #pragma unroll
-        for (int cc = 0; cc < kStepsPerGroup / 2; ++cc) {
-          const uint4 braw = *reinterpret_cast<const uint4*>(
-              &s_b[buf][b_base + nt * 32 * kRowB + 32 * (first_chunk_in_stage + cc)]);
-          const uint32_t words[4] = {braw.x, braw.y, braw.z, braw.w};
-#pragma unroll
-          for (int s = 0; s < 2; ++s) {
-            v4i_t b;
-            b[0] = (int)(((words[2 * s] << 4) ^ 0x80808080u) & 0xF0F0F0F0u);
-            b[1] = (int)((words[2 * s] ^ 0x88888888u) & 0xF0F0F0F0u);
-            b[2] = (int)(((words[2 * s + 1] << 4) ^ 0x80808080u) & 0xF0F0F0F0u);
-            b[3] = (int)((words[2 * s + 1] ^ 0x88888888u) & 0xF0F0F0F0u);
-            bexp[nt][2 * cc + s] = b;
+          for (int cc = 0; cc < kStepsPerGroup / 2; ++cc) {
+            const uint4 words = *reinterpret_cast<const uint4*>(
+                ws_at + ((w_frag + nt * 2048) ^ (32 * (first_chunk + cc))));
+            bexp[nt][2 * cc] = expand(words.x, words.y);
+            bexp[nt][2 * cc + 1] = expand(words.z, words.w);
           }
         }
-        if constexpr (GSH == 5) {
-          const uint2 words = *reinterpret_cast<const uint2*>(
-              &s_b[buf][b_base + nt * 32 * kRowB + 16 * gi]);
-          bexp[nt][0][0] = (int)(((words.x << 4) ^ 0x80808080u) & 0xF0F0F0F0u);
-          bexp[nt][0][1] = (int)((words.x ^ 0x88888888u) & 0xF0F0F0F0u);
-          bexp[nt][0][2] = (int)(((words.y << 4) ^ 0x80808080u) & 0xF0F0F0F0u);
-          bexp[nt][0][3] = (int)((words.y ^ 0x88888888u) & 0xF0F0F0F0u);
-        }
-        const float ws = s_s[buf][wn * 32 * WN + nt * 32 + frag_row][gi];
-        // an fp16 scale / 16 is exact in f32; an f32 scale may not be (subnormal quotient):
-        // then the sums are shifted instead (below)
+        const uint32_t bits = *reinterpret_cast<const uint32_t*>(ss_at + nt * (32 * kEntries * 4) + 4 * gi);
+        const float ws = sizeof(ST) == 2 ? (float)__builtin_bit_cast(_Float16, (uint16_t)bits) : __uint_as_float(bits);
         mult[nt] = valid ? ws : 0.f;  // past K: accf + 0 * 0
       }
 #pragma unroll
@@ -827,33 +836,35 @@ void linear_w4a8_tall_kernel(
         v16i_t acc[WN];
 #pragma unroll
         for (int st = 0; st < kStepsPerGroup; ++st) {
-          const v4i_t a = *reinterpret_cast<const v4i_t*>(
-              &s_a[buf][a_base + mt * 32 * kRowA +
-                        (GSH == 5 ? 32 * gi
-                                  : 64 * (first_chunk_in_stage + st / 2) + 16 * (st & 1))]);
+          const uint32_t piece = GSH == 5 ? 2 * gi : 4 * (first_chunk + st / 2) + (st & 1);
+          const v4i_t a = *reinterpret_cast<const v4i_t*>(xs_at + ((x_frag + mt * 4096) ^ (16 * piece)));
 #pragma unroll
           for (int nt = 0; nt < WN; ++nt)
-            acc[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bexp[nt][st],
-                                                            st == 0 ? zero : acc[nt], 0, 0, 0);
+            acc[nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, bexp[nt][st], st == 0 ? magic : acc[nt], 0, 0, 0);
         }
 #pragma unroll
         for (int nt = 0; nt < WN; ++nt) {
+          // a sum of 16 xq q: the 16 is divided out of an fp16 scale, which leaves it exact in f32, or (an f32
+          // scale's quotient may be subnormal) out of the sum, exact as well
           const float ws16 = mult[nt] * 0.0625f;
-          const bool exact = sizeof(ST) == 2 || __all(ws16 * 16.0f == mult[nt]);
-          const float factor = exact ? ws16 : mult[nt];
-          const int down = exact ? 0 : 4;
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int32_t sum = sizeof(ST) == 2 ? acc[nt][r] : acc[nt][r] >> down;
-            accf[mt][nt][r] = fmaf((float)sum, factor, accf[mt][nt][r]);
+            const float biased = __uint_as_float((uint32_t)acc[nt][r]);
+            accf[mt][nt][r] = sizeof(ST) == 2 ? fmaf(biased - kMagic, ws16, accf[mt][nt][r])
+                                              : fmaf(fmaf(biased, 0.0625f, -0.0625f * kMagic), mult[nt], accf[mt][nt][r]);
           }
         }
       }
     }
-    park_stage(buf ^ 1, staged);
-    __syncthreads();
   };
-  for (uint32_t stage = 0; stage < stages; ++stage) run_stage(stage, (int)(stage & 1u));
+  for (uint32_t stage = 0; stage < stages; stage += kDepth) {
+    run_stage(stage, 0);
+    if (stage + 1u >= stages) break;
+    run_stage(stage + 1u, 1);
+    if (stage + 2u >= stages) break;
+    run_stage(stage + 2u, 2);
+  }
+  wait_vm<0>();  // what was asked for past the end
 
 #pragma unroll
   for (int nt = 0; nt < WN; ++nt) {
@@ -898,35 +909,26 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
   }
   if (m > 8 && group >= 32 && group <= kMaxGroupTimes16 && aligned(xq, 16) && aligned(w, 16)) {
     const uint32_t n_blocks = (n + 255) / 256;
-    // 128 x 256 tiles for groups of 64 / 128 when they still cover most of the chip, or 64 x 128 ones
-    // of four waves, several to a CU, when their finer grain makes fewer rounds of a CU's work: a
-    // quarter of a tall tile each, at 1.15 of its time per output (less is shared).  us before / now,
-    // the quantiser's launch included: 512 x 11008 x 4096 57.3 / 51, in groups of 64 72 / 62; 200 x
-    // 20000 x 4096 59 / 54; 300 x 14000 x 2048 in groups of 64 42 / 33; where the tall ones fill whole
-    // rounds (2048 x 11008 x 4096 181, 256 x 32000 x 2048 41) they stay.
+    // Tiles that stream their stages to LDS: more of 64 x 128 than CUs, in groups of 64 and 128.  Up to one a CU
+    // its chain of stages is what takes the time, and the kernel below (eight waves, 256 codes a stage) is as
+    // good: 512 x 4096 x 4096 28.9 us here, 27.8 there, in groups of 64 34.0 and 31.1; 128 x 4096 x 4096 24.8
+    // and 23.6; 512 x 4096 x 11008 55.9 and 57.6.  From there on 300 x 7000 x 8192 53.1 and 74.1, 350 x 6500 x 3072
+    // 27.9 and 37.1, in groups of 64 31.1 and 40.4, 128 x 32000 x 4096 39.0 and 42.0, 64 x 33000 x 1024 15.8 and 19.4.
     // Groups of 32 always come here and always take the 64 x 128 tiles: the generic kernel re-reads both
-    // operands for every output (512 x 11008 x 4096 50785 / 116 us, 197 x 1655 x 9600 7716 / 120, 20 x
-    // 20000 x 1024 914 / 19, 9 x 300 x 512 11.7 / 11.8), and a 128 x 256 tile of four groups a stage does
-    // not fit the registers (206 spilled: 2048 x 11008 x 4096 1907 us, 352 in 64 x 128 tiles; 2048 x 4096
-    // x 4096 709 and 130).
+    // operands for every output (512 x 11008 x 4096 50785 us, 82 here), and a 128 x 256 tile of four groups a
+    // stage does not fit the registers.
     const uint64_t cus = (uint64_t)ctx->num_cus;
-    const uint64_t tall_tiles = (uint64_t)((m + 127) / 128) * n_blocks;
-    // Fewer tall tiles than that: 64 x 256 tiles of the other kernel, or 64 x 128 where those would leave a
-    // quarter of the chip without work.  What would be 64 x 256 tiles goes to the 64 x 128 ones here in
-    // groups of 64 (four tiles' sums and eight groups' factors spilled there: 376 x 10350 x 3968 375 us, 54
-    // here; 79 x 24856 x 704 56 and 17; 36 shapes 0.12 to 0.35) and in groups of 128 from a second round
-    // on (347 x 11674 x 3072 55.6 and 41.1, 209 x 17856 x 1024 30.5 and 21.7; one round 0.90 to 1.13 of
-    // their time, 402 x 7336 x 7296 62.6 there, 70.7 here).
-    const uint64_t wide_tiles = (uint64_t)((m + 63) / 64) * n_blocks;
-    const bool wide = wide_tiles * 4 >= cus * 3;
-    const bool few_tall = tall_tiles * 5 < cus * 3;
-    const bool takes = shift == 5 || (shift == 6 && (!few_tall || wide)) ||
-                       (shift == 7 && (!few_tall || wide_tiles > cus));
-    if (k <= (1u << 24) && takes) {
-      const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
-      const uint64_t small_rounds = ((uint64_t)small_m * small_n + cus - 1) / cus;
-      const bool small =
-          shift == 5 || few_tall || small_rounds * 115 < (tall_tiles + cus - 1) / cus * 400;
+    const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
+    const uint64_t small_tiles = (uint64_t)small_m * small_n;
+    if (k <= (1u << 24) && (shift == 5 || (shift <= 7 && small_tiles > cus))) {
+      // 128 x 256 tiles in groups of 64 and 128 where they cover most of the chip and the 64 x 128 ones, a
+      // quarter of one each at 1.08 of its time per output (less is shared), make no fewer rounds of a CU's
+      // work.  us, 64 x 128 / 128 x 256: 512 x 11008 x 4096 48.8 / 54.3, 2048 x 11008 x 4096 162.3 / 165.8, 768 x
+      // 11008 x 2048 45.0 / 63.7; 512 x 16384 x 4096 64.5 / 59.4, 256 x 32000 x 2048 39.6 / 37.3, 1024 x 8192 x
+      // 4096 in groups of 64 79.2 / 72.6.
+      const uint64_t tall_tiles = (uint64_t)((m + 127) / 128) * n_blocks;
+      const uint64_t small_rounds = (small_tiles + cus - 1) / cus, tall_rounds = (tall_tiles + cus - 1) / cus;
+      const bool small = shift == 5 || tall_tiles * 5 < cus * 3 || small_rounds * 108 < tall_rounds * 400;
       const uint32_t mb = small ? small_m : (m + 127) / 128, nb = small ? small_n : n_blocks;
       const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * mb;
       if (blocks <= 0x7fffffffull) {
@@ -944,8 +946,9 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
         return launched(ctx, "linear_w4a8_tall_kernel");
       }
     }
+    // 64 x 256 tiles in larger groups, or 64 x 128 where those would leave a quarter of the chip without work
     const uint32_t m_blocks = (m + 63) / 64;
-    const bool narrow = !wide || shift == 6;
+    const bool narrow = shift <= 7 || (uint64_t)m_blocks * n_blocks * 4 < cus * 3;
     const uint32_t nb = narrow ? (n + 127) / 128 : n_blocks;
     const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * m_blocks;
     if (shift > 5 && blocks <= 0x7fffffffull) {
@@ -956,7 +959,7 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
 #define KRM_W4A8_TILE_G(GSH) \
   do { if (narrow) KRM_W4A8_TILE(GSH, 1); else KRM_W4A8_TILE(GSH, 2); } while (0)
       if (shift == 6) KRM_W4A8_TILE(6, 1);
-      else if (shift == 7) KRM_W4A8_TILE_G(7);
+      else if (shift == 7) KRM_W4A8_TILE(7, 1);
       else if (shift == 8) KRM_W4A8_TILE_G(8);
       else KRM_W4A8_TILE_G(0);
 #undef KRM_W4A8_TILE_G

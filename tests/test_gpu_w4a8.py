@@ -359,3 +359,26 @@ def test_w4a8_fused_call_special_rows_and_ties(gpu_ctx):
         alone = run_w4a8_fused(gpu_ctx, x[row:row + 1], packed, scale, None, n, k, group,
                                work=False)
         assert_exact(alone[0], want[row], ("alone", row))
+
+
+@pytest.mark.parametrize("scale_f16", [True, False])
+@pytest.mark.parametrize("m, n, k, group", [
+    (65, 16500, 128, 128), (65, 16500, 256, 128), (70, 16500, 384, 128), (65, 16500, 640, 128), (65, 16500, 1152, 128),
+    (65, 16500, 64, 64), (66, 16500, 448, 64), (65, 16500, 576, 64), (129, 30000, 640, 128), (129, 30000, 320, 64),
+    (9, 129, 32, 32), (65, 300, 352, 32), (65, 300, 672, 32)])
+def test_w4a8_stages_and_scale_blocks_of_the_streamed_tiles(gpu_ctx, m, n, k, group, scale_f16):
+    """One to nine stages of 128 codes (three lie in LDS at a time, scales in blocks of two or four), a K that
+    ends inside a stage; the largest sums a group can have, and f32 scales whose sixteenth is subnormal."""
+    rng = np.random.default_rng(m + n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, group, scale_f16)
+    packed, scale = packed.copy(), scale.copy()
+    packed[::7] = 0            # codes -8 all along
+    packed[3::7] = 0xFF        # codes 7
+    if not scale_f16:
+        scale[1::5] = np.float32(2.0) ** rng.integers(-149, -120, size=scale[1::5].shape)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[0], x[m - 1] = 1.0, -1.0  # xq = 127 and -127 all along
+    bias = rng.normal(size=n).astype(np.float32)
+    got = run_w4a8(gpu_ctx, x, packed, scale, bias, n, k, group)
+    want = oracle.linear_w4a8(x, packed, np.asarray(scale, dtype=np.float32), bias, n, k, group)
+    assert_exact(got, want, (m, n, k, group))
