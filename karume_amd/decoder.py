@@ -447,6 +447,9 @@ class LlamaDecoderSession:
         also does the step's bookkeeping and the next step's embedding."""
         g, c, b, io = self.gpu, self.config, self.buf, self.io_dtype
         d = c.d_model
+        rows_form = m > 16 and self.fuse_decode and self._rows_form_covers(m)
+        if rows_form and lengths is None and last_row is not None:
+            m = min(m, (query + 31) // 32 * 32)  # rows past the last valid one's tile are not formed
         if step_end is None:
             g.embedding(self.embedding, ids if ids is not None else b["ids"], b["h"], m, c.vocab,
                         d, F16, io)
@@ -455,8 +458,8 @@ class LlamaDecoderSession:
             return
         if step_end is not None:
             raise ExecutionError("the fused step exit needs the fused one-row launches")
-        if m > 16 and self.fuse_decode and self._rows_form_covers(m):
-            self._forward_rows(context, m, past, query, lengths)
+        if rows_form:
+            self._forward_rows(context, m, past, query, lengths, last_row)
             self._head(last_row, m)
             return
         pending = {}   # owner layer -> (k rows, v rows) whose appends wait for the last reader
@@ -563,11 +566,13 @@ class LlamaDecoderSession:
                 and all(sp["hd"] % 32 == 0 for sp in self.spec) and m <= 65536)
 
     def _forward_rows(self, context: GenerationContext, m: int, past: int, query: int,
-                      lengths: Optional[DeviceBuffer]) -> None:
-        """A chunk of m > 16 rows, 7 launches a layer: the [q; k; v] projection writes roped,
+                      lengths: Optional[DeviceBuffer], last_row: Optional[int]) -> None:
+        """m > 16 rows of a chunk, 7 launches a layer: the [q; k; v] projection writes roped,
         head-major q / k / v, the attention writes row-major and appends the chunk's K / V rows,
         the o and down projections add the residual in place, the gate/up projection applies
-        silu * up.  (A KV-sharing layer projects and rotates q alone, in two launches.)"""
+        silu * up.  (A KV-sharing layer projects and rotates q alone, in two launches.)  Behind the
+        last layer's attention only the tile of 32 rows with `last_row` goes on (all without one):
+        a row's bits do not depend on the rows beside it."""
         from .runtime import EPILOGUE_SILU_PAIRS
         g, c, b, io = self.gpu, self.config, self.buf, self.io_dtype
         d, group, compute = c.d_model, c.group_size, self.prefill_compute
@@ -637,19 +642,25 @@ class LlamaDecoderSession:
                 if last_reader:
                     self._append_pair(context, owner, pending.pop(owner), m, past, query, lengths)
                 g.transpose_01(b["att"], b["att2"], c.heads, m, depth, io)
+            first, rows = 0, m
+            if last_row is not None and li + 1 == c.layers and m > 32:
+                first, rows = min(last_row // 32 * 32, m - 32), 32
             lin = lw["o"]
-            g.linear_i4_rows(b["att2"], lin.w, lin.s, b["h"], m, lin.n, lin.k, group,
-                             residual=b["h"], io_dtype=io, scale_dtype=lin.scale_dtype,
-                             compute=compute, x_dtype=F16 if att_half else io)
-            g.rms_norm_cast(b["h"], lw["ffn_norm"], b["xn"], m, d, c.rms_eps, io, xd)
+            o_xd = F16 if att_half else io
+            h = b["h"].offset(first * d * self.eb)
+            att = b["att2"].offset(first * lin.k * (2 if o_xd == F16 else self.eb))
+            g.linear_i4_rows(att, lin.w, lin.s, h, rows, lin.n, lin.k, group,
+                             residual=h, io_dtype=io, scale_dtype=lin.scale_dtype,
+                             compute=compute, x_dtype=o_xd)
+            g.rms_norm_cast(h, lw["ffn_norm"], b["xn"], rows, d, c.rms_eps, io, xd)
             lin = lw["gate_up"]
             # (fp16 in and out: silu(gate) * up is computed on the f32 sums and rounded once)
-            g.linear_i4_rows(b["xn"], lin.w, lin.s, b["act"], m, lin.n, lin.k, group,
+            g.linear_i4_rows(b["xn"], lin.w, lin.s, b["act"], rows, lin.n, lin.k, group,
                              io_dtype=xd, scale_dtype=lin.scale_dtype, compute=compute,
                              epilogue=EPILOGUE_SILU_PAIRS)
             lin = lw["down"]
-            g.linear_i4_rows(b["act"], lin.w, lin.s, b["h"], m, lin.n, lin.k, group,
-                             residual=b["h"], io_dtype=io, scale_dtype=lin.scale_dtype,
+            g.linear_i4_rows(b["act"], lin.w, lin.s, h, rows, lin.n, lin.k, group,
+                             residual=h, io_dtype=io, scale_dtype=lin.scale_dtype,
                              compute=compute, x_dtype=xd)
 
     def _replay_max_past(self, context: GenerationContext) -> int:

@@ -876,3 +876,33 @@ def test_sessions_that_take_turns_on_one_context_equal_plain_launches(gpu_ctx):
         context.dispose()
     for session in sessions:
         session.close()
+
+
+@pytest.mark.parametrize("kv,compute", [(ka.F32, ka.COMPUTE_F32), (ka.F16, ka.COMPUTE_F16)])
+@pytest.mark.parametrize("chunk,query", [(128, 1), (128, 32), (128, 33), (128, 96), (100, 70), (100, 97),
+                                         (128, 128), (40, 17), (20, 20)])
+def test_last_row_runs_form_only_the_rows_that_count(gpu_ctx, chunk, query, kv, compute):
+    """A run that returns the last valid row alone leaves out the rows past its tile and, behind the last layer's
+    attention, the other tiles: state, logits and token against the run that returns every row."""
+    config = LlamaConfig(layers=2, d_model=512, ffn=768, heads=8, kv_heads=2, vocab=640)
+    session = LlamaDecoderSession(gpu_ctx, random_weights(config, seed=2), io_dtype=ka.F32, kv_dtype=kv,
+                                  chunk_length=chunk, prefill_compute=compute)
+    ids = np.random.default_rng(chunk + query).integers(0, config.vocab, size=(1, chunk)).astype(np.int32)
+    pos = np.arange(chunk, dtype=np.int32).reshape(1, chunk)
+    runs = []
+    for last_row in (query - 1, None):
+        context = session.create_generation_context(capacity=256, chunk_length=chunk)
+        token, logits = session.run(ids, pos, last_row, context=context, query_length=query, want_logits=True)
+        state = [b.download(np.uint32, (b.nbytes // 4,)) for b in context.slots_k + context.slots_v]
+        runs.append((token[0, -1 if last_row is not None else query - 1, 0],
+                     logits[0] if last_row is not None else logits[0, query - 1], state))
+        context.dispose()
+    session.close()
+    for one, all_rows in zip(runs[0][2], runs[1][2]):
+        assert np.array_equal(one, all_rows)
+    # (the head of one row and of all rows: f32 sums in another order, or x rounded to fp16 in that class)
+    scale = float(np.abs(runs[1][1]).max())
+    assert np.abs(runs[0][1] - runs[1][1]).max() <= (2e-3 if compute == ka.COMPUTE_F16 else 2e-5) * scale
+    top = np.sort(runs[1][1])
+    if top[-1] - top[-2] > 4e-3 * scale:
+        assert runs[0][0] == runs[1][0]
