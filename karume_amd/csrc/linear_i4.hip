@@ -17,6 +17,7 @@
 #include "i4_codes.h"
 
 #include <cmath>
+#include <type_traits>
 
 using namespace krm;
 
@@ -301,7 +302,17 @@ struct Acts<float> {
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-template <typename ST, int CHUNKS, int KW>
+// Scales of groups of 128: those of a chunk's two halves are neighbours, and so are the chunks of a share.  A load
+// costs by the lines it touches, sixteen of sixteen rows, and one scale at a time there were as many of
+// them as of the weights.  One load a share (a pair a chunk where a share may end early), us before / now: 16 rows
+// 11008 x 4096 10.1 / 8.5, 4096 x 4096 5.7 / 5.2, 6000 x 4096 8.2 / 6.7, 28000 x 6144 26.9 / 22.7, 4096 x 8192 f32 scales
+// 10.7 / 9.4, 2000 x 10240 10.9 / 9.5; 2 rows 32000 x 4096 19.5 / 15.0; 12 rows 20000 x 2304 10.1 / 9.6.
+template <typename ST, int CHUNKS>
+struct __attribute__((packed, aligned(4))) ChunkScales {
+  ST of[CHUNKS][2];
+};
+
+template <typename ST, int CHUNKS, bool GROUPS_128, int KW>
 __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_kernel(
     const __half* __restrict__ x, const uint32_t* __restrict__ w, const ST* __restrict__ scales,
     const __half* __restrict__ bias, __half* __restrict__ out, uint32_t m, uint32_t n, uint32_t k,
@@ -345,10 +356,16 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_kernel(
   };
   auto fetch_w = [&](uint32_t chunk, Weights& c) {
     const uint32_t kc = chunk * kChunk;
+    if constexpr (!GROUPS_128) {
+      c.scale[0] = load_scale<ST>(sptr, (k_first + kc) >> group_shift);
+      c.scale[1] = load_scale<ST>(sptr, (k_first + kc + 128) >> group_shift);
+    } else if constexpr (CHUNKS == 0) {
+      const auto pair = *reinterpret_cast<const ChunkScales<ST, 1>*>(sptr + ((k_first + kc) >> 7));
+      c.scale[0] = to_f32<ST>(pair.of[0][0]);
+      c.scale[1] = to_f32<ST>(pair.of[0][1]);
+    }
     c.words[0] = *reinterpret_cast<const uint4*>(wptr + (kc >> 3));
     c.words[1] = *reinterpret_cast<const uint4*>(wptr + (kc >> 3) + 16);
-    c.scale[0] = load_scale<ST>(sptr, (k_first + kc) >> group_shift);
-    c.scale[1] = load_scale<ST>(sptr, (k_first + kc + 128) >> group_shift);
   };
   const int load_row = lane >> 5, load_piece = lane & 31;
   auto fetch_x = [&](uint32_t chunk, Acts& c) {
@@ -403,12 +420,18 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_kernel(
     Weights wq[CHUNKS];
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) fetch_w(c, wq[c]);
+    ChunkScales<ST, CHUNKS> share;
+    if constexpr (GROUPS_128) share = *reinterpret_cast<const ChunkScales<ST, CHUNKS>*>(sptr + (k_first >> 7));
     __builtin_amdgcn_sched_barrier(0);
     park_x(xa[0], 0);
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
       if (c + 2 < CHUNKS) fetch_x(c + 2, xa[c & 1]);       // slot of the chunk parked last pass
       if (c + 1 < CHUNKS) park_x(xa[(c + 1) & 1], (c + 1) & 1);
+      if constexpr (GROUPS_128) {
+        wq[c].scale[0] = to_f32<ST>(share.of[c][0]);
+        wq[c].scale[1] = to_f32<ST>(share.of[c][1]);
+      }
       consume(wq[c], c & 1);
     }
   } else {
@@ -454,8 +477,9 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_kernel(
 // share of x in registers (32 a chunk, read through one LDS strip).  One tile a workgroup fetched
 // and parked all of x (16 K fp16: four times the tile's weights) for every tile, one workgroup a CU
 // at a time (its strips filled the LDS).  Same sums in the same order.  What bounds it now is the
-// weights' stream behind the first round trip.
-template <typename ST, int CHUNKS, bool EVEN, int KW>
+// weights' stream behind the first round trip: three tiles on their way took longer than two (16 rows 11008 x
+// 4096 9.7 us, 8.5), the waves' first ones arrive later.
+template <typename ST, int CHUNKS, bool EVEN, bool GROUPS_128, int KW>
 __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_tiles_kernel(
     const __half* __restrict__ x, const uint32_t* __restrict__ w, const ST* __restrict__ scales,
     const __half* __restrict__ bias, __half* __restrict__ out, uint32_t m, uint32_t n, uint32_t k,
@@ -479,19 +503,27 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_tiles_kernel(
   const uint32_t tiles = (n + 15) / 16;
   struct Tile {
     uint4 words[CHUNKS][2];  // pieces g and 4 + g of the row's 32 words
-    ST scale[CHUNKS][2];     // (as loaded: a conversion here would wait inside the branch)
+    ChunkScales<ST, CHUNKS> scale;  // (as loaded: a conversion here would wait inside the branch)
   };
   auto fetch_tile = [&](uint32_t tile, Tile& t) {
     const uint32_t row = min(tile * 16 + r16, n - 1);  // rows past N re-read the last row, unused
     const uint32_t* wrow = w + (size_t)row * (k >> 3) + 4 * g;
     const ST* srow = scales + (size_t)row * (k >> group_shift);
+    if constexpr (GROUPS_128 && EVEN)
+      t.scale = *reinterpret_cast<const ChunkScales<ST, CHUNKS>*>(srow + (k_first >> 7));
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
       const uint32_t at = chunk_k0(c);
       t.words[c][0] = *reinterpret_cast<const uint4*>(wrow + (at >> 3));
       t.words[c][1] = *reinterpret_cast<const uint4*>(wrow + (at >> 3) + 16);
-      t.scale[c][0] = srow[at >> group_shift];
-      t.scale[c][1] = srow[(at + 128) >> group_shift];
+      if constexpr (!GROUPS_128) {
+        t.scale.of[c][0] = srow[at >> group_shift];
+        t.scale.of[c][1] = srow[(at + 128) >> group_shift];
+      } else if constexpr (!EVEN) {  // (the whole of an uneven share may pass the row's end)
+        const auto pair = *reinterpret_cast<const ChunkScales<ST, 1>*>(srow + (at >> 7));
+        t.scale.of[c][0] = pair.of[0][0];
+        t.scale.of[c][1] = pair.of[0][1];
+      }
     }
   };
 
@@ -543,8 +575,8 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_tiles_kernel(
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          total[i] = fmaf(half_sum[0][i], (float)own.scale[c][0], total[i]);
-          total[i] = fmaf(half_sum[1][i], (float)own.scale[c][1], total[i]);
+          total[i] = fmaf(half_sum[0][i], (float)own.scale.of[c][0], total[i]);
+          total[i] = fmaf(half_sum[1][i], (float)own.scale.of[c][1], total[i]);
         }
       }
     if (tile + 2u * gridDim.x < tiles) fetch_tile(tile + 2u * gridDim.x, own);
@@ -1275,51 +1307,52 @@ static int32_t gemv_dispatch(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
       uint32_t group_shift = 0;
       while ((1u << group_shift) < group) ++group_shift;
       const uint32_t blocks = (n + 15) / 16, share = (k / 256 + 7) / 8;
-      // (measured, 16 rows, us before / now: N = 11008, K = 4096 13.7 / 10.0; N = 32000, K = 2048
-      // 15.2 / 11.5; N = 9000, K = 5632 16.3 / 12.2.  Up to a tile a CU, or four chunks a wave and more: the kernel above.)
+      auto by_scales = [&](auto launch) {
+        if (scale_dtype == KRM_F16 && group == 128) launch(__half{}, std::true_type{});
+        else if (scale_dtype == KRM_F16) launch(__half{}, std::false_type{});
+        else if (group == 128) launch(float{}, std::true_type{});
+        else launch(float{}, std::false_type{});
+      };
+      // (measured, 16 rows, us in the kernel above / here: N = 11008, K = 4096 13.7 / 10.0; N = 32000, K = 2048
+      // 15.2 / 11.5; N = 9000, K = 5632 16.3 / 12.2, before both read scales together.  Up to a tile a CU, or four chunks a wave and more: the kernel above.)
       if (k >= 2048 && share <= 3 && blocks > (uint32_t)ctx->num_cus) {
-#define KRM_MFMA_TILES(ST, CH, EVEN)                                                           \
-  gemv_i4_mfma_tiles_kernel<ST, CH, EVEN, 8><<<dim3(ctx->num_cus), dim3(512), 0, ctx->stream>>>( \
+#define KRM_MFMA_TILES(ST, CH, EVEN, G128)                                                     \
+  gemv_i4_mfma_tiles_kernel<ST, CH, EVEN, G128, 8>                                             \
+      <<<dim3(ctx->num_cus), dim3(512), 0, ctx->stream>>>(                                     \
       ptr<const __half>(x), ptr<const uint32_t>(w), ptr<const ST>(scales),                     \
       ptr<const __half>(bias), ptr<__half>(out), m, n, k, group_shift)
-        auto launch = [&](auto scale_tag) {
+        auto launch = [&](auto scale_tag, auto groups_128) {
           using ST = decltype(scale_tag);
+          constexpr bool kG128 = decltype(groups_128)::value;
           const bool even = k % 2048 == 0;
-          if (share == 1) KRM_MFMA_TILES(ST, 1, true);
-          else if (share == 2 && even) KRM_MFMA_TILES(ST, 2, true);
-          else if (share == 2) KRM_MFMA_TILES(ST, 2, false);
-          else if (even) KRM_MFMA_TILES(ST, 3, true);
-          else KRM_MFMA_TILES(ST, 3, false);
+          if (share == 1) KRM_MFMA_TILES(ST, 1, true, kG128);
+          else if (share == 2 && even) KRM_MFMA_TILES(ST, 2, true, kG128);
+          else if (share == 2) KRM_MFMA_TILES(ST, 2, false, kG128);
+          else if (even) KRM_MFMA_TILES(ST, 3, true, kG128);
+          else KRM_MFMA_TILES(ST, 3, false, kG128);
         };
-        if (scale_dtype == KRM_F16) launch(__half{}); else launch(float{});
+        by_scales(launch);
 #undef KRM_MFMA_TILES
         return launched(ctx, "gemv_i4_mfma_tiles_kernel");
       }
-#define KRM_MFMA_GEMV(ST, CH, KW)                                                              \
-  gemv_i4_mfma_kernel<ST, CH, KW><<<dim3(blocks), dim3(KW * 64), 0, ctx->stream>>>(            \
+#define KRM_MFMA_GEMV(CH, KW)                                                                  \
+  gemv_i4_mfma_kernel<ST, CH, kG128, KW><<<dim3(blocks), dim3(KW * 64), 0, ctx->stream>>>(     \
       ptr<const __half>(x), ptr<const uint32_t>(w), ptr<const ST>(scales),                     \
       ptr<const __half>(bias), ptr<__half>(out), m, n, k, group_shift)
-  // eight waves a workgroup (two per SIMD) when K gives each at least one chunk
-#define KRM_MFMA_GEMV_BY_K(ST)                         \
-  switch (k % 1024 ? 0u : k / 1024) {                  \
-    case 1: KRM_MFMA_GEMV(ST, 1, 4); break;            \
-    case 2: KRM_MFMA_GEMV(ST, 1, 8); break;            \
-    case 4: KRM_MFMA_GEMV(ST, 2, 8); break;            \
-    case 8: KRM_MFMA_GEMV(ST, 4, 8); break;            \
-    default:                                           \
-      if (k >= 2048) {                                 \
-        KRM_MFMA_GEMV(ST, 0, 8);                       \
-      } else {                                         \
-        KRM_MFMA_GEMV(ST, 0, 4);                       \
-      }                                                \
-      break;                                           \
-  }
-      if (scale_dtype == KRM_F16) {
-        KRM_MFMA_GEMV_BY_K(__half)
-      } else {
-        KRM_MFMA_GEMV_BY_K(float)
-      }
-#undef KRM_MFMA_GEMV_BY_K
+      // eight waves a workgroup (two per SIMD) when K gives each at least one chunk
+      by_scales([&](auto scale_tag, auto groups_128) {
+        using ST = decltype(scale_tag);
+        constexpr bool kG128 = decltype(groups_128)::value;
+        switch (k % 1024 ? 0u : k / 1024) {
+          case 1: KRM_MFMA_GEMV(1, 4); break;
+          case 2: KRM_MFMA_GEMV(1, 8); break;
+          case 4: KRM_MFMA_GEMV(2, 8); break;
+          case 8: KRM_MFMA_GEMV(4, 8); break;
+          default:
+            if (k >= 2048) KRM_MFMA_GEMV(0, 8); else KRM_MFMA_GEMV(0, 4);
+            break;
+        }
+      });
 #undef KRM_MFMA_GEMV
       return launched(ctx, "gemv_i4_mfma_kernel");
     }

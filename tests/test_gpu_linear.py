@@ -482,3 +482,33 @@ def test_few_fp16_rows_have_the_bits_of_one_row_alone(gpu_ctx, n, k, g, scale_ty
         assert np.array_equal(out.download(np.uint16, (m, n)), got), m
         for b in buffers + [out]:
             b.free()
+
+
+@pytest.mark.parametrize("scale_type", [np.float16, np.float32])
+@pytest.mark.parametrize("m, n, k", [(2, 40, 1024), (16, 33, 2048), (5, 17, 4096), (16, 16, 8192), (3, 50, 768),
+                                     (16, 20, 2304), (7, 24, 5120), (16, 4112, 2048), (9, 4225, 4096),
+                                     (16, 4500, 6144), (4, 4128, 2304), (16, 4100, 4352), (2, 4700, 5888)])
+def test_scales_of_a_share_read_together(gpu_ctx, m, n, k, scale_type):
+    """Batched fp16 rows in groups of 128, whose scales a wave reads at once (every form of the shares of K, a tile
+    a workgroup and several), at a scale address of no more than four bytes' alignment: one fp16 ulp and
+    the GEMV's gate against the oracle, and the bits of the same weights in groups of 256 (neighbouring groups of
+    128 share a scale here)."""
+    rng = np.random.default_rng(n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, 128, scale_type is np.float16)
+    scale[:, 1::2] = scale[:, 0::2]
+    scale = scale.astype(scale_type)
+    x = rng.normal(size=(m, k)).astype(np.float16)
+    want = oracle.linear_i4(x.astype(np.float32), packed, scale.astype(np.float32), np.zeros(n, dtype=np.float32),
+                            n, k, 128)
+    dx, dw, out = gpu_ctx.upload(x), gpu_ctx.upload(packed), gpu_ctx.alloc(m * n * 2)
+    skewed = np.concatenate([np.zeros(4 // scale.itemsize, dtype=scale_type), scale.reshape(-1)])
+    ds, d256 = gpu_ctx.upload(skewed), gpu_ctx.upload(np.ascontiguousarray(scale[:, ::2]))
+    got = []
+    for at, group in ((ds.offset(4), 128), (d256, 256)):
+        gpu_ctx.linear_i4(dx, dw, at, None, out, m, n, k, group, ka.F16, ka.dtype_code(scale.dtype))
+        got.append(out.download(np.uint16, (m, n)))
+    for b in (dx, dw, ds, d256, out):
+        b.free()
+    assert np.array_equal(got[0], got[1])
+    ulp = np.spacing(np.abs(want).astype(np.float16)).astype(np.float32)
+    assert np.all(np.abs(got[0].view(np.float16).astype(np.float32) - want) <= ulp + 4e-5)
