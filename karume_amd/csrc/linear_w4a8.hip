@@ -460,8 +460,8 @@ __global__ __launch_bounds__(256) void linear_w4a8_rows_kernel(
 //  * Every stage issues the same loads in the same order whatever K is (addresses past K are
 //    clamped, chunks past K multiply zeros and are fused with a zero scale): a branch around a
 //    load would make the compiler's wait counts assume the worst path.
-// GSH = log2(group) for groups of 64, 128, 256 (group boundaries known at compile time);
-// GSH = 0: any larger group (a whole number of stages).
+// GSH = 8: groups of 256, a stage each (64 and 128: linear_w4a8_tall_kernel); GSH = 0: any larger group (a
+// whole number of stages).
 // Workgroup ids are dealt so that the row blocks of a column block run on one XCD.
 // (Weights loaded straight from global memory into the operand registers, without LDS, were
 // measured 1.5 x slower: a lane's own 16 bytes of its own row make every quad of lanes touch
@@ -662,8 +662,8 @@ void linear_w4a8_tile_kernel(
   }
 }
 
-// 64 x 128 tiles of four waves of 64 x 32, several a CU, or 128 x 256 ones of eight waves of 64 x 64, for groups
-// of 32, 64 or 128 codes (32 in the smaller tile only, see the dispatch).  The work is ordered by group: the
+// 64 x 128 tiles of four waves of 64 x 32, several a CU, or of eight waves of 32 x 32, and 128 x 256 tiles of eight
+// waves of 64 x 64, for groups of 32, 64 or 128 codes (32 in the smaller tile only, see the dispatch).  The work is ordered by group: the
 // group's weight words are expanded once, then each row tile in turn runs its MFMA chains over the group
 // and is fused into its f32 accumulators, so that one row tile's int32 sums live at a time.
 //
@@ -676,7 +676,7 @@ void linear_w4a8_tile_kernel(
 // 4096 51.4 / 46.6, in groups of 64 60.6 / 55.0, of 32 105 / 83, with f32 scales (whose quotient by 16 was
 // tested in every group) 56.8 / 47.9; 2048 x 11008 x 4096 166 / 157; 20 x 20000 x 1024 in groups of 32 18.2 / 15.1;
 // 500 x 600 x 8000 in groups of 32, f32 scales 112 / 72.
-template <typename ST, int GSH, int WM, int NW, int WN>
+template <typename ST, int GSH, int WM, int NW, int WN, int MT>
 __global__ __launch_bounds__(64 * WM * NW) __attribute__((amdgpu_waves_per_eu(2, WN == 2 ? 2 : 4)))
 void linear_w4a8_tall_kernel(
     const uint8_t* __restrict__ xq, const float* __restrict__ xs, const uint8_t* __restrict__ w,
@@ -684,8 +684,8 @@ void linear_w4a8_tall_kernel(
     uint32_t m, uint32_t n, uint32_t k, uint32_t m_blocks, uint32_t n_blocks) {
   static_assert(GSH >= 5 && GSH <= 7, "groups of 32, 64 or 128 codes");
   static_assert(GSH > 5 || WN == 1, "two column tiles of groups of 32 spill");
-  constexpr int kWaves = WM * NW, MT = 2;
-  constexpr int BM = 64 * WM, BN = 32 * WN * NW;
+  constexpr int kWaves = WM * NW;
+  constexpr int BM = 32 * MT * WM, BN = 32 * WN * NW;
   constexpr int kStage = 128;                          // codes per LDS stage
   constexpr int kGroupsPerStage = kStage >> GSH;       // 4, 2 or 1
   constexpr int kStepsPerGroup = 1 << (GSH - 5);       // MFMA steps of 32 codes: 1, 2 or 4
@@ -780,7 +780,7 @@ void linear_w4a8_tall_kernel(
   // Fragment addresses.  A step of 32 codes takes 16 of each half of the wave, neighbours in memory: in a chunk
   // of 64 codes step s takes the codes 32 h + 16 s .., in a group of 32 the codes 16 h ...  (Pieces
   // of a row are told apart by exclusive or: their place is a power of two's bits.)
-  const uint32_t x_frag = (wm * 64u + frag_row) * 128u + (((GSH == 5 ? frag_h : 2u * frag_h) ^ ((frag_row >> 1) & 7u)) * 16u);
+  const uint32_t x_frag = (wm * 32u * MT + frag_row) * 128u + (((GSH == 5 ? frag_h : 2u * frag_h) ^ ((frag_row >> 1) & 7u)) * 16u);
   const uint32_t w_frag = (wn * 32u * WN + frag_row) * 64u +
                           (((GSH == 5 ? 0u : frag_h) ^ ((frag_row >> 2) & 3u)) * 16u) + (GSH == 5 ? 8u * frag_h : 0u);
   const uint32_t s_frag = (wn * 32u * WN + frag_row) * (kEntries * 4u);
@@ -874,7 +874,7 @@ void linear_w4a8_tall_kernel(
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const uint32_t row = m0 + wm * 64 + mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4);
+        const uint32_t row = m0 + wm * 32 * MT + mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4);
         if (row < m && col < n) out[(size_t)row * n + col] = fmaf(accf[mt][nt][r], xs[row], b);
       }
   }
@@ -909,18 +909,21 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
   }
   if (m > 8 && group >= 32 && group <= kMaxGroupTimes16 && aligned(xq, 16) && aligned(w, 16)) {
     const uint32_t n_blocks = (n + 255) / 256;
-    // Tiles that stream their stages to LDS: more of 64 x 128 than CUs, in groups of 64 and 128.  Up to one a CU
-    // its chain of stages is what takes the time, and the kernel below (eight waves, 256 codes a stage) is as
-    // good: 512 x 4096 x 4096 28.9 us here, 27.8 there, in groups of 64 34.0 and 31.1; 128 x 4096 x 4096 24.8
-    // and 23.6; 512 x 4096 x 11008 55.9 and 57.6.  From there on 300 x 7000 x 8192 53.1 and 74.1, 350 x 6500 x 3072
-    // 27.9 and 37.1, in groups of 64 31.1 and 40.4, 128 x 32000 x 4096 39.0 and 42.0, 64 x 33000 x 1024 15.8 and 19.4.
-    // Groups of 32 always come here and always take the 64 x 128 tiles: the generic kernel re-reads both
-    // operands for every output (512 x 11008 x 4096 50785 us, 82 here), and a 128 x 256 tile of four groups a
-    // stage does not fit the registers.
+    // Groups of 32, 64 and 128: tiles that stream their stages to LDS.  us there (groups of 32: in 64 x 128 tiles
+    // staged through registers; 64 and 128: in the kernel below, which larger groups take) / here: 300 x 7000 x
+    // 8192 74.1 / 53.1, 350 x 6500 x 3072 37.1 / 27.9, in groups of 64 40.4 / 31.1, 128 x 32000 x 4096 42.0 / 39.0, 64 x
+    // 33000 x 1024 19.4 / 15.8.  Up to one 64 x 128 tile a CU a tile's chain of stages is what takes the time:
+    // there eight waves of 32 x 32 instead of four of 64 x 32, us before / in four / in eight: 512 x 4096 x 4096 27.5 /
+    // 28.9 / 26.9, in groups of 64 31.1 / 34.0 / 29.2, 128 x 4096 x 4096 23.6 / 24.8 / 22.4, 64 x 4096 x 11008 50.8 /
+    // 50.8 / 47.3, 500 x 600 x 8000 in groups of 32, f32 scales 112 / 72 / 57, 20 x 20000 x 1024 17.7 / 15.1 / 12.6.
+    // (Six stages on their way instead of three 23.6 for 22.4; a stage's operands read beside the products of the
+    // stage before it, or half of the waves asking behind their products: no change.)
+    // Groups of 32 always take the 64 x 128 tiles: a 128 x 256 tile of four groups a stage does not fit
+    // the registers.
     const uint64_t cus = (uint64_t)ctx->num_cus;
     const uint32_t small_m = (m + 63) / 64, small_n = (n + 127) / 128;
     const uint64_t small_tiles = (uint64_t)small_m * small_n;
-    if (k <= (1u << 24) && (shift == 5 || (shift <= 7 && small_tiles > cus))) {
+    if (k <= (1u << 24) && shift <= 7) {
       // 128 x 256 tiles in groups of 64 and 128 where they cover most of the chip and the 64 x 128 ones, a
       // quarter of one each at 1.08 of its time per output (less is shared), make no fewer rounds of a CU's
       // work.  us, 64 x 128 / 128 x 256: 512 x 11008 x 4096 48.8 / 54.3, 2048 x 11008 x 4096 162.3 / 165.8, 768 x
@@ -932,15 +935,18 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
       const uint32_t mb = small ? small_m : (m + 127) / 128, nb = small ? small_n : n_blocks;
       const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * mb;
       if (blocks <= 0x7fffffffull) {
-#define KRM_W4A8_TALL(GSH, WM, WN)                                                             \
-  hipLaunchKernelGGL((linear_w4a8_tall_kernel<ST, GSH, WM, 4, WN>), dim3((uint32_t)blocks),    \
+#define KRM_W4A8_TALL(GSH, WM, WN, MT)                                                         \
+  hipLaunchKernelGGL((linear_w4a8_tall_kernel<ST, GSH, WM, 4, WN, MT>), dim3((uint32_t)blocks),    \
                      dim3(256 * WM), 0, ctx->stream, ptr<const uint8_t>(xq), pxs,              \
                      ptr<const uint8_t>(w), ps, pb, po, m, n, k, mb, nb)
-        if (small) {
-          if (shift == 5) KRM_W4A8_TALL(5, 1, 1);
-          else if (shift == 6) KRM_W4A8_TALL(6, 1, 1); else KRM_W4A8_TALL(7, 1, 1);
+        if (small_tiles <= cus) {
+          if (shift == 5) KRM_W4A8_TALL(5, 2, 1, 1);
+          else if (shift == 6) KRM_W4A8_TALL(6, 2, 1, 1); else KRM_W4A8_TALL(7, 2, 1, 1);
+        } else if (small) {
+          if (shift == 5) KRM_W4A8_TALL(5, 1, 1, 2);
+          else if (shift == 6) KRM_W4A8_TALL(6, 1, 1, 2); else KRM_W4A8_TALL(7, 1, 1, 2);
         } else {
-          if (shift == 6) KRM_W4A8_TALL(6, 2, 2); else KRM_W4A8_TALL(7, 2, 2);
+          if (shift == 6) KRM_W4A8_TALL(6, 2, 2, 2); else KRM_W4A8_TALL(7, 2, 2, 2);
         }
 #undef KRM_W4A8_TALL
         return launched(ctx, "linear_w4a8_tall_kernel");
@@ -948,19 +954,17 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
     }
     // 64 x 256 tiles in larger groups, or 64 x 128 where those would leave a quarter of the chip without work
     const uint32_t m_blocks = (m + 63) / 64;
-    const bool narrow = shift <= 7 || (uint64_t)m_blocks * n_blocks * 4 < cus * 3;
+    const bool narrow = (uint64_t)m_blocks * n_blocks * 4 < cus * 3;
     const uint32_t nb = narrow ? (n + 127) / 128 : n_blocks;
     const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * m_blocks;
-    if (shift > 5 && blocks <= 0x7fffffffull) {
+    if (shift > 7 && blocks <= 0x7fffffffull) {
 #define KRM_W4A8_TILE(GSH, WN)                                                                 \
   hipLaunchKernelGGL((linear_w4a8_tile_kernel<ST, GSH, 1, WN>), dim3((uint32_t)blocks),        \
                      dim3(512), 0, ctx->stream, ptr<const uint8_t>(xq), pxs,                  \
                      ptr<const uint8_t>(w), ps, pb, po, m, n, k, shift, m_blocks, nb)
 #define KRM_W4A8_TILE_G(GSH) \
   do { if (narrow) KRM_W4A8_TILE(GSH, 1); else KRM_W4A8_TILE(GSH, 2); } while (0)
-      if (shift == 6) KRM_W4A8_TILE(6, 1);
-      else if (shift == 7) KRM_W4A8_TILE(7, 1);
-      else if (shift == 8) KRM_W4A8_TILE_G(8);
+      if (shift == 8) KRM_W4A8_TILE_G(8);
       else KRM_W4A8_TILE_G(0);
 #undef KRM_W4A8_TILE_G
 #undef KRM_W4A8_TILE

@@ -365,7 +365,10 @@ def test_w4a8_fused_call_special_rows_and_ties(gpu_ctx):
 @pytest.mark.parametrize("m, n, k, group", [
     (65, 16500, 128, 128), (65, 16500, 256, 128), (70, 16500, 384, 128), (65, 16500, 640, 128), (65, 16500, 1152, 128),
     (65, 16500, 64, 64), (66, 16500, 448, 64), (65, 16500, 576, 64), (129, 30000, 640, 128), (129, 30000, 320, 64),
-    (9, 129, 32, 32), (65, 300, 352, 32), (65, 300, 672, 32)])
+    (9, 129, 32, 32), (65, 300, 352, 32), (65, 300, 672, 32), (65, 16385, 352, 32),
+    # no more tiles than CUs
+    (64, 128, 128, 128), (65, 129, 384, 128), (9, 300, 640, 128), (130, 200, 1152, 128), (33, 100, 64, 64),
+    (200, 300, 448, 64), (31, 129, 576, 64), (64, 32768, 256, 128)])
 def test_w4a8_stages_and_scale_blocks_of_the_streamed_tiles(gpu_ctx, m, n, k, group, scale_f16):
     """One to nine stages of 128 codes (three lie in LDS at a time, scales in blocks of two or four), a K that
     ends inside a stage; the largest sums a group can have, and f32 scales whose sixteenth is subnormal."""
