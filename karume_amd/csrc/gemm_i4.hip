@@ -668,7 +668,7 @@ void gemm_i4_f16_dealt_kernel(const XT* __restrict__ x, const uint8_t* __restric
   uint32_t v = blockIdx.x;
   if ((gridDim.x & 7u) == 0) v = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const uint32_t my_begin = deal_begin(deal, v);
-  uint32_t left = deal.units_lo + (v < deal.extra ? 1u : 0u);
+  uint32_t left = deal_units(deal, v);
 
   // The tiles of the range are taken last to first: a range usually ends with the first stages
   // of a tile and begins with the last stages of the one before, so every workgroup then walks
@@ -912,7 +912,7 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
   uint32_t v = blockIdx.x;
   if ((gridDim.x & 7u) == 0) v = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const uint32_t my_begin = deal_begin(deal, v);
-  uint32_t left = deal.units_lo + (v < deal.extra ? 1u : 0u);
+  uint32_t left = deal_units(deal, v);
 
   while (left > 0) {
     const uint32_t range_end = my_begin + left;

@@ -7,18 +7,28 @@
 namespace krm {
 namespace {
 
+// One span of units dealt over all workgroups, in contiguous ranges that differ by one unit, or (tile_groups
+// > 0) the units of each tile dealt so over workgroups of its own.
 struct UnitDeal {
   uint32_t stages_per_tile;
-  uint32_t units_lo, extra;  // workgroup v owns units_lo + (v < extra) units from deal_begin(v)
+  uint32_t tile_groups;
+  uint32_t units_lo, extra;  // workgroup i of a span owns units_lo + (i < extra) units
   float* partials;           // [2 * workgroups] slots of 128 x 256 floats
   uint32_t* tickets;         // one counter per tile, kTicketStride words apart, zero at rest
 };
-__host__ __device__ inline uint32_t deal_begin(const UnitDeal& d, uint32_t v) {
-  return v * d.units_lo + (v < d.extra ? v : d.extra);
+// (a division by what only the launch knows is twenty instructions: none where there is one span)
+__device__ inline uint32_t deal_begin(const UnitDeal& d, uint32_t v) {
+  const uint32_t tile = d.tile_groups ? v / d.tile_groups : 0u, i = v - tile * d.tile_groups;
+  return tile * d.stages_per_tile + i * d.units_lo + (i < d.extra ? i : d.extra);
+}
+__device__ inline uint32_t deal_units(const UnitDeal& d, uint32_t v) {
+  const uint32_t i = d.tile_groups ? v % d.tile_groups : v;
+  return d.units_lo + (i < d.extra ? 1u : 0u);
 }
 __device__ inline uint32_t deal_owner(const UnitDeal& d, uint32_t unit) {
+  const uint32_t tile = d.tile_groups ? unit / d.stages_per_tile : 0u, at = unit - tile * d.stages_per_tile;
   const uint32_t big = d.extra * (d.units_lo + 1u);
-  return unit < big ? unit / (d.units_lo + 1u) : d.extra + (unit - big) / d.units_lo;
+  return tile * d.tile_groups + (at < big ? at / (d.units_lo + 1u) : d.extra + (at - big) / d.units_lo);
 }
 constexpr uint32_t kPartialFloats = 128u * 256u;
 

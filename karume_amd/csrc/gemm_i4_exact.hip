@@ -133,10 +133,11 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
     w_at[c] = (wn * 64u + frag_row) * 64u + (((2u * c + frag_h) ^ w_turn) * 16u);
   const uint32_t s_at = (wn * 64u + frag_row) * (G::kEntries * 4u);
 
-  uint32_t v = blockIdx.x;
-  if ((gridDim.x & 7u) == 0) v = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  // (workgroups are dealt to the eight XCDs in turn: neighbouring ranges lie on one)
+  const uint32_t xcd = blockIdx.x & 7u;
+  const uint32_t v = xcd * (gridDim.x >> 3) + min(xcd, gridDim.x & 7u) + (blockIdx.x >> 3);
   const uint32_t my_begin = deal_begin(deal, v);
-  uint32_t left = deal.units_lo + (v < deal.extra ? 1u : 0u);
+  uint32_t left = deal_units(deal, v);
 
   // The tiles of the range are taken last to first: a range usually ends with the first stages of a
   // tile and begins with the last stages of the one before, so every workgroup walks K upwards from
@@ -487,12 +488,33 @@ bool plan_exact(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group
   if ((uint64_t)((m + 31) / 32) * ((n + 31) / 32) <= 6 * cus) return false;
   if (tiles * 8 < cus) return false;  // a tile shared by more than eight workgroups
   if (!ctx->gemm_partials) return false;
-  grid = (uint32_t)cus;
   deal.stages_per_tile = spt;
-  deal.units_lo = (uint32_t)(units / cus);
-  deal.extra = (uint32_t)(units % cus);
   deal.partials = ctx->gemm_partials;
   deal.tickets = ctx->tickets;
+  // Workgroups of a tile's own, as many as the CUs give each tile: some walk more stages than with all units
+  // dealt evenly, but none ends two tiles, each end a partial written and some of them merged behind the last
+  // workgroup's.  That is worth up to five stages of one workgroup a tile, which exchanges nothing, four and a half
+  // of several; two that share a tile of hi and lo, whose stages take longest, gained nothing.  us dealt
+  // evenly / so (more stages): fp16 512 x 4096 x 11008 61.8 / 58.6 (0.5), 113 x 14557 x 7168 47.9 / 44.5 (0), 333 x 6000 x
+  // 4992 40.3 / 38.9 (2), 280 x 10758 x 6592 71.0 / 68.3 (3.7), 348 x 8164 x 4608 43.2 / 42.7 (4.5), 346 x 7484 x 5120 43.5 /
+  // 46.3 (5.9), one a tile 228 x 25350 x 3072 51.1 / 47.5 (5.3), 512 x 11008 x 4096 55.7 / 58.6 (10.5); hi and lo 512 x
+  // 4096 x 11008 102.8 / 99.8 (0.5), 131 x 14091 x 8320 98.8 / 93.2 (0.7), 275 x 6187 x 6784 72.5 / 71.8 (4.5), one a
+  // tile 200 x 27000 x 2048 62.9 / 60.5 (2.8), two 286 x 12123 x 4352 74.9 / 76.5 (1.1).
+  const uint32_t sharers = (uint32_t)(cus / tiles);
+  if (sharers > 0) {
+    const float more = (float)((spt + sharers - 1) / sharers) - (float)units / (float)cus;
+    if (more <= (sharers == 1 ? 5.4f : sharers > 2 ? 4.7f : split ? 0.6f : 4.6f)) {
+      grid = sharers * (uint32_t)tiles;
+      deal.tile_groups = sharers;
+      deal.units_lo = spt / sharers;
+      deal.extra = spt % sharers;
+      return true;
+    }
+  }
+  grid = (uint32_t)cus;
+  deal.tile_groups = 0;
+  deal.units_lo = (uint32_t)(units / cus);
+  deal.extra = (uint32_t)(units % cus);
   return true;
 }
 

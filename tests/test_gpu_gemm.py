@@ -545,6 +545,14 @@ def test_unit_dealt_products_at_the_edges_of_their_tiles(gpu_ctx, m, n, k, g, mo
     assert np.all(err <= bound), float(np.max(err / bound))
 
 
+@pytest.mark.parametrize("m,n,k,g,mode", [(228, 25350, 3072, 128, "f16"), (200, 26999, 2048, 128, "f32"),  # one a tile
+                                          (280, 10758, 6592, 64, "f16"), (333, 6001, 4992, 64, "f16"),   # two, three
+                                          (250, 8190, 6272, 128, "f32"), (300, 5000, 8192, 128, "f32")])  # four, five
+def test_tiles_with_workgroups_of_their_own(gpu_ctx, m, n, k, g, mode):
+    """One to five workgroups share a tile and no other, in equal and in unequal parts of its K."""
+    test_unit_dealt_products_at_the_edges_of_their_tiles(gpu_ctx, m, n, k, g, mode)
+
+
 @pytest.mark.parametrize("io", [ka.F16, ka.F32])
 @pytest.mark.parametrize("compute", [ka.COMPUTE_F16, ka.COMPUTE_F32])
 @pytest.mark.parametrize("m,n,k,silu", [(17, 4, 64, False), (33, 64, 128, True), (50, 96, 576, False),
