@@ -1036,7 +1036,7 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
       for (int r = 0; r < 16; ++r) {
         const uint32_t local = mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4);
         const uint32_t row = m0 + local;
-        if (row < m && col < n) store_out<XT>(out, (size_t)row * n + col, sum[r] + b);
+        if (row < m && col < n) store_out<XT>(out, (size_t)row * n + col, sum[r] * 1024.0f + b);
       }
     };
 

@@ -358,7 +358,7 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
         for (int r = 0; r < 16; ++r) {
           const uint32_t local = o_row + mt * 32 + 8 * (r / 4) + (r % 4);
           float value = sum[nt][r];
-          value *= PLANES == 2 ? s_inv[local] : 1024.0f;  // exact: a power of two
+          value *= PLANES == 2 ? s_inv[local] : 1024.0f;  // exact: a power of two (s_inv has the 1024 in it)
           if (whole || (m0 + local < m && col < n))
             out[(size_t)(m0 + local) * n + col] = from_f32<T>(value + add);
         }

@@ -47,10 +47,23 @@ __device__ inline void codes_to_half2(uint32_t word, half2_t (&q)[4]) {
   q[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(upper, 0x00F000F0u, magic)),
                                    sixteenth, off_hi);
 }
-// The same as one operand of a matrix instruction: (c0,c4,c1,c5,c2,c6,c3,c7).
+// The same pairs as (u - 8) / 1024, exact, where the sum is multiplied by 1024 at the end: a code at the bottom
+// of its half is the fp16 subnormal u 2^-24, one four bits up 16 u 2^-24, and one packed fma scales and offsets
+// it.  Nine ops of which five take half the time of a packed one: a mask (v_and_b32, 2.4 clk a wave beside
+// others, v_and_or_b32 4.4) needs no bits set beside it.
+__device__ inline void codes_over_1024(uint32_t word, half2_t (&q)[4]) {
+  const half2_t low = {(_Float16)16384.0f, (_Float16)16384.0f}, high = {(_Float16)1024.0f, (_Float16)1024.0f};
+  const half2_t offset = {(_Float16)-0.0078125f, (_Float16)-0.0078125f};
+  const uint32_t upper = word >> 8;
+  q[0] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, word & 0x000F000Fu), low, offset);
+  q[1] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, word & 0x00F000F0u), high, offset);
+  q[2] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, upper & 0x000F000Fu), low, offset);
+  q[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, upper & 0x00F000F0u), high, offset);
+}
+// The same as one operand of a matrix instruction: (c0,c4,c1,c5,c2,c6,c3,c7), each (u - 8) / 1024.
 __device__ inline half8_t ints_paired(uint32_t word) {
   half2_t q[4];
-  codes_to_half2(word, q);
+  codes_over_1024(word, q);
   return half8_t{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
 }
 
