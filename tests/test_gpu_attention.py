@@ -660,6 +660,41 @@ def test_varlen_planned_on_the_device_is_recordable(gpu_ctx):
         b.free()
 
 
+@pytest.mark.parametrize("nseq", [1, 62, 63, 64, 65, 127, 128, 300])
+def test_varlen_plan_tables_past_a_wave(gpu_ctx, nseq):
+    """The tables of a plan, by steps of 64 sequences: offsets as given, splits of 128 columns summed before each
+    sequence (one up to 512 columns); one wrong offset anywhere leaves no splits and raises the fault word."""
+    rng = np.random.default_rng(nseq)
+    rows = rng.choice([0, 1, 511, 512, 513, 2000], size=nseq)
+    cu = np.concatenate([[3], 3 + np.cumsum(rows)]).astype(np.int32)
+    total = int(cu[-1])
+    max_splits = gpu_ctx.attention_varlen_max_splits(nseq, 128, ka.F16, total)
+    chunks = -(-rows // 128)
+    prefix = np.concatenate([[0], np.cumsum(np.where(chunks <= 4, 1, chunks))])
+    cu_dev, plan = gpu_ctx.alloc(cu.nbytes), gpu_ctx.alloc(gpu_ctx.attention_varlen_plan_bytes(nseq))
+
+    def tables(offsets, total_rows, splits):
+        cu_dev.upload(offsets)
+        plan.upload(np.full(2 * (nseq + 1) + 1, -7, dtype=np.int32))
+        gpu_ctx.attention_varlen_plan(cu_dev, plan, nseq=nseq, depth=128, kv_dtype=ka.F16,
+                                      total_rows=total_rows, max_splits=splits)
+        got = plan.download(np.int32, (2 * (nseq + 1) + 1,))
+        return got[:nseq + 1], got[nseq + 1:-1], got[-1]
+
+    got_cu, got_prefix, fault = tables(cu, total, max_splits)
+    assert (got_cu == cu).all() and (got_prefix == prefix).all() and fault == 0
+    broken = [(cu, total - 1, max_splits), (cu, total, int(prefix[-1]) - 1)]
+    for at in sorted({0, nseq // 2, nseq}):
+        wrong = cu.copy()
+        wrong[at] = -1 if at < nseq else cu[at - 1] - 1
+        broken.append((wrong, total, max_splits))
+    for offsets, total_rows, splits in broken:
+        got_cu, got_prefix, fault = tables(offsets, total_rows, splits)
+        assert (got_cu == offsets).all() and not got_prefix.any() and fault == 1
+    for b in (cu_dev, plan):
+        b.free()
+
+
 @pytest.mark.parametrize("io,kv", [(np.float32, np.float32), (np.float16, np.float16),
                                    (np.float32, np.float16)])
 @pytest.mark.parametrize("dyn", [False, True])
