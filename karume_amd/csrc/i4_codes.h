@@ -60,6 +60,15 @@ __device__ inline void codes_over_1024(uint32_t word, half2_t (&q)[4]) {
   q[2] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, upper & 0x000F000Fu), low, offset);
   q[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, upper & 0x00F000F0u), high, offset);
 }
+// Eight consecutive fp16 activations (x0..x7 in four dwords) regrouped to match
+// codes_to_half2: pair i = (x_i, x_{i+4}).
+__device__ inline void pair_activations(const uint4& raw, half2_t (&p)[4]) {
+  p[0] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.z, raw.x, 0x05040100u));
+  p[1] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.z, raw.x, 0x07060302u));
+  p[2] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.w, raw.y, 0x05040100u));
+  p[3] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.w, raw.y, 0x07060302u));
+}
+
 // The same as one operand of a matrix instruction: (c0,c4,c1,c5,c2,c6,c3,c7), each (u - 8) / 1024.
 __device__ inline half8_t ints_paired(uint32_t word) {
   half2_t q[4];

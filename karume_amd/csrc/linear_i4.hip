@@ -1,5 +1,5 @@
 // int4 group-quantised `linear` for gfx950: the dequant kernel (bit-exact gate) and the
-// bandwidth-bound GEMV used for M <= 16 rows of activations.
+// bandwidth-bound GEMV used for M <= 16 rows of activations (plain ones of 2 and more: gemv_i4_rows.hip).
 //
 // Semantics follow the reference's linear op with i4 weights
 // (packages/runtime/src/kernels/linear.ts:34-64, body packages/runtime/src/kernels/gemm.ts:
@@ -120,15 +120,6 @@ __device__ inline float wave_sum4(float a, float b, float c, float d, int lane) 
   const float p1 = (odd ? d : c) + dpp_from<0xB1>(odd ? c : d);  // even lanes: c, odd lanes: d
   const float q = (high ? p1 : p0) + dpp_from<0x4E>(high ? p0 : p1);
   return wave_sum_tail(q);
-}
-
-// Eight consecutive fp16 activations (x0..x7 in four dwords) regrouped to match
-// codes_to_half2: pair i = (x_i, x_{i+4}).
-__device__ inline void pair_activations(const uint4& raw, half2_t (&p)[4]) {
-  p[0] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.z, raw.x, 0x05040100u));
-  p[1] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.z, raw.x, 0x07060302u));
-  p[2] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.w, raw.y, 0x05040100u));
-  p[3] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.w, raw.y, 0x07060302u));
 }
 
 template <typename XT>
@@ -1300,15 +1291,25 @@ int32_t pick_vec(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bia
 
 namespace krm {
 
+// 2 to 16 rows with the bits of one row alone (gemv_i4_rows.hip).
+int32_t linear_i4_gemv_rows(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias, krm_buf out, uint32_t m,
+                            uint32_t n, uint32_t k, uint32_t group, int32_t io_dtype, int32_t scale_dtype, bool* handled);
+
 // Rows M <= 16: the GEMV above.  Declared in gemm_i4.hip's dispatcher too.
 static int32_t gemv_dispatch(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, const GemvFusion& fuse) {
+  const bool plain = !fuse.norm_weight && !fuse.residual && !fuse.pair_silu && !fuse.positions;
+  const bool on_mfma = plain && io_dtype == KRM_F16 && m >= 2 && k % 256 == 0 && group >= 128 && aligned(w, 16) &&
+                       aligned(x, 16) && aligned(scales, 4);
+  if (plain && !on_mfma) {
+    bool handled = false;
+    KRM_TRY(linear_i4_gemv_rows(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype, &handled));
+    if (handled) return KRM_OK;
+  }
   if (io_dtype == KRM_F16) {
     // batched fp16 rows on the matrix cores (plain op only)
-    const bool plain = !fuse.norm_weight && !fuse.residual && !fuse.pair_silu && !fuse.positions;
-    if (plain && m >= 2 && k % 256 == 0 && group >= 128 && aligned(w, 16) && aligned(x, 16) &&
-        aligned(scales, 4)) {
+    if (on_mfma) {
       uint32_t group_shift = 0;
       while ((1u << group_shift) < group) ++group_shift;
       const uint32_t blocks = (n + 15) / 16, share = (k / 256 + 7) / 8;
@@ -1373,17 +1374,6 @@ static int32_t gemv_dispatch(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
 int32_t linear_i4_gemv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                        krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                        int32_t io_dtype, int32_t scale_dtype) {
-  // 9 to 16 rows of f32 x: eight and the rest, a launch each (a row's bits are the same).  Sixteen rows' sums
-  // leave the one-launch form too few registers, and eight rows over a K of a step and more are brought
-  // to LDS.  us in one launch / in two, over 70 shapes: 9 rows 703 x 10240 77 / 21, 12 rows 1836 x 9472 152 / 45,
-  // 16 rows 1350 x 9088 144 / 64, 11 rows 29237 x 10112 1043 / 396, at worst 0.93; a K below a step 9 rows 14803 x
-  // 1152 83 / 49, 12 rows 3458 x 1152 24.7 / 21.1, but 13 rows and more 1.01 to 1.08.
-  if (io_dtype == KRM_F32 && m > 8 && m <= 16 && (k >= 2048 || m <= 12) && k % 32 == 0 && group % 32 == 0 &&
-      aligned(w, 16)) {
-    KRM_TRY(gemv_dispatch(ctx, x, w, scales, bias, out, 8, n, k, group, io_dtype, scale_dtype, GemvFusion{}));
-    return gemv_dispatch(ctx, x + (size_t)8 * k * 4, w, scales, bias, out + (size_t)8 * n * 4, m - 8, n, k, group,
-                         io_dtype, scale_dtype, GemvFusion{});
-  }
   return gemv_dispatch(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
                        GemvFusion{});
 }

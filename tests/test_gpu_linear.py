@@ -512,3 +512,42 @@ def test_scales_of_a_share_read_together(gpu_ctx, m, n, k, scale_type):
     assert np.array_equal(got[0], got[1])
     ulp = np.spacing(np.abs(want).astype(np.float16)).astype(np.float32)
     assert np.all(np.abs(got[0].view(np.float16).astype(np.float32) - want) <= ulp + 4e-5)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("n,k,g,scale_type,offset", [
+    (1030, 32, 32, np.float32, 0), (6200, 96, 32, np.float16, 0), (1025, 2048, 128, np.float16, 1),
+    (1040, 4160, 32, np.float32, 3), (6145, 2144, 32, np.float16, 1), (20011, 160, 32, np.float16, 0),
+    (9000, 1088, 64, np.float32, 0), (17, 8256, 64, np.float16, 0), (64, 6272, 128, np.float32, 1),
+    (20, 65536, 32, np.float32, 0), (1, 1152, 32, np.float16, 0)])
+def test_dealt_rows_have_the_bits_of_one_row_alone(gpu_ctx, dtype, n, k, g, scale_type, offset):
+    """2 to 16 rows in every form they are dealt in (a wave has 64 or 16 rows of W, 1 to 8 of x, one to four quads of
+    segments): K of one segment, of a part of a quad, of a step and past it; N off the tile; scales that are not
+    aligned, or too many for LDS.  Bits of each row alone, also where x has infinities, zeros and subnormals."""
+    rng = np.random.default_rng(n + k)
+    packed = rng.integers(0, 2**32, size=n * k // 8, dtype=np.uint32)
+    scale = (rng.random(size=n * (k // g) + offset) * .02 + .001).astype(scale_type)
+    bias = rng.normal(size=n).astype(dtype)
+    x = rng.normal(size=(16, k)).astype(dtype)
+    x[1] *= dtype(1e-7 if dtype == np.float16 else 1e-42)
+    x[2, ::3] = 0
+    x[3, k // 2] = np.inf
+    d_w, d_s, d_b = gpu_ctx.upload(packed), gpu_ctx.upload(scale), gpu_ctx.upload(bias)
+    at = d_s.offset(offset * scale.itemsize)
+    io, sd = ka.dtype_code(np.dtype(dtype)), ka.dtype_code(np.dtype(scale_type))
+
+    def run(rows):
+        d_x, out = gpu_ctx.upload(np.ascontiguousarray(rows)), gpu_ctx.alloc(len(rows) * n * rows.itemsize)
+        gpu_ctx.linear_i4(d_x, d_w, at, d_b, out, len(rows), n, k, g, io, sd, ka.COMPUTE_F32)
+        got = out.download(dtype, (len(rows), n))
+        d_x.free()
+        out.free()
+        return got
+
+    alone = np.concatenate([run(x[r:r + 1]) for r in range(16)])
+    for m in (2, 3, 4, 5, 7, 9, 12, 16):
+        got = run(x[:m])
+        same = (got == alone[:m]) | (np.isnan(got) & np.isnan(alone[:m]))
+        assert same.all() and (np.signbit(got) == np.signbit(alone[:m]))[~np.isnan(got)].all(), m
+    for b in (d_w, d_s, d_b):
+        b.free()
