@@ -41,7 +41,11 @@ __device__ inline float block_sum(float v, float* scratch) {
 // packages/runtime/src/kernels/rms-norm.ts:35-91 (no mean subtraction; weight is f32).
 // OT: the type the result is stored in (XT, or fp16 beside f32 rows: a copy for a consumer
 // that would round the f32 result to fp16 anyway).
-template <typename XT, typename OT = XT>
+// KEEP > 0: rows up to KEEP * 256 elements stay in registers, one trip to memory: all loads are unconditional (elements
+// past the row are its last one and not counted), because a branch around each made them trips in a row.  us before / now,
+// f32 to fp16: 128 rows of 2048 2.72 / 2.40, 128 of 512 2.60 / 2.05, 64 of 896 2.58 / 2.14 (an empty launch of a replay is
+// 1.8); 512 rows of 11008, which walked their row twice in the form for any length, 24.0 / 6.3 (f32 27.4 / 7.5).
+template <typename XT, typename OT, int KEEP>
 __global__ __launch_bounds__(kThreads) void rms_norm_kernel(const XT* __restrict__ x,
                                                            const float* __restrict__ weight,
                                                            OT* __restrict__ out, uint32_t dim,
@@ -50,37 +54,38 @@ __global__ __launch_bounds__(kThreads) void rms_norm_kernel(const XT* __restrict
   const size_t base = (size_t)blockIdx.x * dim;
   // the fp16 copy of an f32 row is the f32 result rounded again, never a product rounded once
   auto keep_f32 = [](float v) { return sizeof(OT) == sizeof(XT) ? v : rounded_f32(v); };
-  constexpr int kKeep = 16;  // rows up to 4096 elements stay in registers: one trip to memory
-  if (dim <= (uint32_t)(kThreads * kKeep)) {
-    float v[kKeep], wv[kKeep];
+  if constexpr (KEEP > 0) {
+    float v[KEEP], wv[KEEP];
 #pragma unroll
-    for (int j = 0; j < kKeep; ++j) {
-      const uint32_t i = threadIdx.x + j * kThreads;
-      v[j] = i < dim ? ld<XT>(x, base + i) : 0.f;
-      wv[j] = i < dim ? weight[i] : 0.f;
+    for (int j = 0; j < KEEP; ++j) {
+      const uint32_t i = min(threadIdx.x + j * kThreads, dim - 1);
+      v[j] = ld<XT>(x, base + i);
+      wv[j] = weight[i];
     }
     float squares = 0.f;  // the same elements in the same order as the loop below
 #pragma unroll
-    for (int j = 0; j < kKeep; ++j)
-      if (threadIdx.x + j * kThreads < dim) squares = fmaf(v[j], v[j], squares);
+    for (int j = 0; j < KEEP; ++j) {
+      const float sum = fmaf(v[j], v[j], squares);
+      squares = threadIdx.x + j * kThreads < dim ? sum : squares;
+    }
     const float total = block_sum(squares, scratch);
     const float inv = 1.0f / sqrtf(total / (float)dim + eps);
 #pragma unroll
-    for (int j = 0; j < kKeep; ++j) {
+    for (int j = 0; j < KEEP; ++j) {
       const uint32_t i = threadIdx.x + j * kThreads;
       if (i < dim) st<OT>(out, base + i, keep_f32(v[j] * inv * wv[j]));
     }
-    return;
+  } else {
+    float squares = 0.f;
+    for (uint32_t i = threadIdx.x; i < dim; i += kThreads) {
+      const float v = ld<XT>(x, base + i);
+      squares = fmaf(v, v, squares);
+    }
+    const float total = block_sum(squares, scratch);
+    const float inv = 1.0f / sqrtf(total / (float)dim + eps);
+    for (uint32_t i = threadIdx.x; i < dim; i += kThreads)
+      st<OT>(out, base + i, keep_f32(ld<XT>(x, base + i) * inv * weight[i]));
   }
-  float squares = 0.f;
-  for (uint32_t i = threadIdx.x; i < dim; i += kThreads) {
-    const float v = ld<XT>(x, base + i);
-    squares = fmaf(v, v, squares);
-  }
-  const float total = block_sum(squares, scratch);
-  const float inv = 1.0f / sqrtf(total / (float)dim + eps);
-  for (uint32_t i = threadIdx.x; i < dim; i += kThreads)
-    st<OT>(out, base + i, keep_f32(ld<XT>(x, base + i) * inv * weight[i]));
 }
 
 // Half-split RoPE with the cos / sin rows looked up by absolute position:
@@ -392,6 +397,20 @@ inline unsigned grid_for(size_t total) {
     }                                                 \
   } while (0)
 
+template <typename XT, typename OT>
+static void launch_rms_norm(krm_ctx* ctx, krm_buf x, krm_buf weight, krm_buf out, uint32_t rows, uint32_t dim,
+                            float eps) {
+  auto launch = [&](auto kernel) {
+    kernel<<<dim3(rows), dim3(kThreads), 0, ctx->stream>>>(ptr<const XT>(x), ptr<const float>(weight), ptr<OT>(out),
+                                                           dim, eps);
+  };
+  if (dim <= 4 * kThreads) launch(rms_norm_kernel<XT, OT, 4>);
+  else if (dim <= 8 * kThreads) launch(rms_norm_kernel<XT, OT, 8>);
+  else if (dim <= 16 * kThreads) launch(rms_norm_kernel<XT, OT, 16>);
+  else if (dim <= 48 * kThreads) launch(rms_norm_kernel<XT, OT, 48>);
+  else launch(rms_norm_kernel<XT, OT, 0>);
+}
+
 extern "C" {
 
 int32_t krm_rms_norm(krm_ctx* ctx, krm_buf x, krm_buf weight_f32, krm_buf out, uint32_t rows,
@@ -401,12 +420,8 @@ int32_t krm_rms_norm(krm_ctx* ctx, krm_buf x, krm_buf weight_f32, krm_buf out, u
   KRM_REQUIRE(ctx, dim >= 1 && std::isfinite(eps), "krm_rms_norm: dim %u / eps", dim);
   if (rows == 0) return KRM_OK;
   KRM_REQUIRE(ctx, x && weight_f32 && out, "krm_rms_norm: NULL buffer");
-  KRM_IO_DISPATCH(io_dtype,
-                  (rms_norm_kernel<float><<<dim3(rows), dim3(kThreads), 0, ctx->stream>>>(
-                      ptr<const float>(x), ptr<const float>(weight_f32), ptr<float>(out), dim, eps)),
-                  (rms_norm_kernel<__half><<<dim3(rows), dim3(kThreads), 0, ctx->stream>>>(
-                      ptr<const __half>(x), ptr<const float>(weight_f32), ptr<__half>(out), dim,
-                      eps)));
+  KRM_IO_DISPATCH(io_dtype, (launch_rms_norm<float, float>(ctx, x, weight_f32, out, rows, dim, eps)),
+                  (launch_rms_norm<__half, __half>(ctx, x, weight_f32, out, rows, dim, eps)));
   return launched(ctx, "rms_norm_kernel");
 }
 
@@ -420,8 +435,7 @@ int32_t krm_rms_norm_cast(krm_ctx* ctx, krm_buf x, krm_buf weight_f32, krm_buf o
   KRM_REQUIRE(ctx, dim >= 1 && std::isfinite(eps), "krm_rms_norm_cast: dim %u / eps", dim);
   if (rows == 0) return KRM_OK;
   KRM_REQUIRE(ctx, x && weight_f32 && out, "krm_rms_norm_cast: NULL buffer");
-  rms_norm_kernel<float, __half><<<dim3(rows), dim3(kThreads), 0, ctx->stream>>>(
-      ptr<const float>(x), ptr<const float>(weight_f32), ptr<__half>(out), dim, eps);
+  launch_rms_norm<float, __half>(ctx, x, weight_f32, out, rows, dim, eps);
   return launched(ctx, "rms_norm_kernel");
 }
 

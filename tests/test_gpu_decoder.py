@@ -26,6 +26,23 @@ def test_rms_norm_golden_and_random(gpu_ctx):
     assert ok, (fails, max_abs)
 
 
+@pytest.mark.parametrize("dim", [1, 255, 1024, 1025, 2048, 2049, 4096, 4097, 12288, 12289])
+def test_rms_norm_at_the_lengths_kept_in_registers(gpu_ctx, dim):
+    """Rows at the edges of each form; the tolerance of a row of 2048 above (a thread adds up to 48 squares)."""
+    rng = np.random.default_rng(dim)
+    x, w = rng.normal(size=(3, dim)).astype(np.float32), rng.normal(size=dim).astype(np.float32)
+    dx, dw = gpu_ctx.upload(x), gpu_ctx.upload(w)
+    out, out16 = gpu_ctx.alloc(x.nbytes), gpu_ctx.alloc(x.nbytes // 2)
+    gpu_ctx.rms_norm(dx, dw, out, 3, dim, 1e-5)
+    gpu_ctx.rms_norm_cast(dx, dw, out16, 3, dim, 1e-5)
+    got = out.download(np.float32, x.shape)
+    ok, fails, max_abs, _ = oracle.allclose(got, oracle.rms_norm(x, w, 1e-5), atol=1e-6, rtol=1e-5)
+    assert ok, (fails, max_abs)
+    assert out16.download(np.float16, x.shape).tobytes() == got.astype(np.float16).tobytes()
+    for b in (dx, dw, out, out16):
+        b.free()
+
+
 def test_rope_silu_add_embedding_argmax(gpu_ctx):
     rng = np.random.default_rng(1)
     rows, heads, d, table = 5, 3, 8, 16
