@@ -880,11 +880,12 @@ void gemm_i4_f16_dealt_kernel(const XT* __restrict__ x, const uint8_t* __restric
 // (the C layout keeps the column in lane % 32, so the scale is one value per lane and column
 // tile).  Stages, LDS layout, the (tile, stage) deal over the CUs and the ordered merge of the
 // partials are those of the kernel above.
-template <typename XT, typename ST>
+// OT: of the bias and the result (f32 beside fp16 x: rows that were rounded before).
+template <typename XT, typename OT, typename ST>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__ w,
-                          const ST* __restrict__ scales, const XT* __restrict__ bias,
-                          XT* __restrict__ out, uint32_t m, uint32_t n, uint32_t k,
+                          const ST* __restrict__ scales, const OT* __restrict__ bias,
+                          OT* __restrict__ out, uint32_t m, uint32_t n, uint32_t k,
                           uint32_t group_shift, uint32_t m_blocks, UnitDeal deal) {
   constexpr int MT = 2, WN = 2, T = 512;
   constexpr int BM = 64, BN = 512;
@@ -1031,12 +1032,12 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
 
     auto store_block = [&](int mt, int nt, const float16_t& sum) {
       const uint32_t col = n0 + wn * 64 + nt * 32 + frag_row;
-      const float b = (bias && col < n) ? bias_f32<XT>(bias, col) : 0.f;
+      const float b = (bias && col < n) ? bias_f32<OT>(bias, col) : 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const uint32_t local = mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4);
         const uint32_t row = m0 + local;
-        if (row < m && col < n) store_out<XT>(out, (size_t)row * n + col, sum[r] * 1024.0f + b);
+        if (row < m && col < n) store_out<OT>(out, (size_t)row * n + col, sum[r] * 1024.0f + b);
       }
     };
 
@@ -1283,14 +1284,14 @@ int32_t pick_tile(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bi
   return launch<XT, ST, 1, 1, 64, 1, 1>(ctx, x, w, scales, bias, out, m, n, k, group_shift);
 }
 
-template <typename XT, typename ST>
+template <typename XT, typename OT, typename ST>
 int32_t launch_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias, krm_buf out,
                      uint32_t m, uint32_t n, uint32_t k, uint32_t group_shift, uint32_t grid,
                      const UnitDeal& deal) {
   KRM_TRY(needs_serial_scratch(ctx, "the unit-dealt GEMM"));
-  gemm_i4_staged_kernel<XT, ST><<<dim3(grid), dim3(512), 0, ctx->stream>>>(
-      ptr<const XT>(x), ptr<const uint8_t>(w), ptr<const ST>(scales), ptr<const XT>(bias),
-      ptr<XT>(out), m, n, k, group_shift, (m + 63) / 64, deal);
+  gemm_i4_staged_kernel<XT, OT, ST><<<dim3(grid), dim3(512), 0, ctx->stream>>>(
+      ptr<const XT>(x), ptr<const uint8_t>(w), ptr<const ST>(scales), ptr<const OT>(bias),
+      ptr<OT>(out), m, n, k, group_shift, (m + 63) / 64, deal);
   return launched(ctx, "gemm_i4_staged_kernel");
 }
 
@@ -1298,12 +1299,19 @@ int32_t launch_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_bu
 
 namespace krm {
 
+// Whether f32 x of this shape, rounded to fp16, comes to the staged tiles (buffers aligned, main stream).
+bool gemm_staged_takes_f32(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group) {
+  uint32_t grid = 0;
+  UnitDeal deal{};
+  return group >= 64 && plan_staged(ctx, m, n, k, group, false, grid, deal);
+}
+
 // The exact-integer GEMM with x in fp16 for shapes whose (tile, stage) units cover the chip; sets
 // *handled = false (and launches nothing) for every other shape.
 int32_t linear_i4_gemm_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
-                             bool* handled) {
+                             bool* handled, int32_t x_dtype) {
   *handled = false;
   if (compute == KRM_COMPUTE_F32 && io_dtype == KRM_F32) return KRM_OK;
   if (group < 64 || k % 32 != 0 || !aligned(w, 16) || !aligned(x, 16)) return KRM_OK;
@@ -1312,18 +1320,22 @@ int32_t linear_i4_gemm_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales
   // (a side branch of a graph has no scratch: there the K-splitting tiles, which need none with fp16
   // operands, take these shapes too)
   if (ctx->stream != ctx->main_stream) return KRM_OK;
-  if (!plan_staged(ctx, m, n, k, group, io_dtype == KRM_F16, grid, deal)) return KRM_OK;
+  if (!plan_staged(ctx, m, n, k, group, x_dtype == KRM_F16, grid, deal)) return KRM_OK;
   uint32_t group_shift = 0;
   while ((1u << group_shift) < group) ++group_shift;
   *handled = true;
-#define KRM_STAGED(XT, ST) \
-  return launch_staged<XT, ST>(ctx, x, w, scales, bias, out, m, n, k, group_shift, grid, deal)
+#define KRM_STAGED(XT, OT, ST) \
+  return launch_staged<XT, OT, ST>(ctx, x, w, scales, bias, out, m, n, k, group_shift, grid, deal)
   if (io_dtype == KRM_F16) {
-    if (scale_dtype == KRM_F16) KRM_STAGED(__half, __half);
-    KRM_STAGED(__half, float);
+    if (scale_dtype == KRM_F16) KRM_STAGED(__half, __half, __half);
+    KRM_STAGED(__half, __half, float);
   }
-  if (scale_dtype == KRM_F16) KRM_STAGED(float, __half);
-  KRM_STAGED(float, float);
+  if (x_dtype == KRM_F16) {
+    if (scale_dtype == KRM_F16) KRM_STAGED(__half, float, __half);
+    KRM_STAGED(__half, float, float);
+  }
+  if (scale_dtype == KRM_F16) KRM_STAGED(float, float, __half);
+  KRM_STAGED(float, float, float);
 #undef KRM_STAGED
 }
 

@@ -5,7 +5,7 @@
 // (packages/runtime/src/kernels/linear.ts:34-64, packages/runtime/src/kernels/gemm.ts:1187-1237).
 // The weights enter the matrix cores as the exact integers (u - 8) in fp16 and the group scale
 // multiplies the f32 sum of a group afterwards — the arithmetic of the GEMV, on MFMA.  Two forms of x:
-//   PLANES 1  fp16 x: one MFMA a step;
+//   PLANES 1  fp16 x (f32 x that was rounded before: f32 bias and result): one MFMA a step;
 //   PLANES 2  f32 x as x * 2^e = hi + lo, both fp16, |x * 2^e - (hi + lo)| <= 2^-23 |x * 2^e| (e per
 //             row, chosen so that the row's largest magnitude lands in [2^13, 2^14): no overflow, and
 //             small entries keep an absolute resolution of 2^-38 of the row's maximum), written once by
@@ -534,26 +534,35 @@ int32_t launch_exact(krm_ctx* ctx, const ExactCall& c, uint32_t grid, const Unit
   return launched(ctx, "gemm_i4_exact_kernel");
 }
 
-template <typename ST, bool HALF>
+// T: of the bias and the result (f32 beside fp16 x: rows that were rounded before).
+template <typename T, typename ST, bool HALF>
 int32_t pick_exact(krm_ctx* ctx, const ExactCall& c, bool split, uint32_t grid, const UnitDeal& deal) {
-  if (split) return launch_exact<float, ST, 2, HALF, 1>(ctx, c, grid, deal);
-  return exact_rows(c.m, c.n, false) == 64 ? launch_exact<__half, ST, 1, HALF, 1>(ctx, c, grid, deal)
-                                           : launch_exact<__half, ST, 1, HALF, 2>(ctx, c, grid, deal);
+  if constexpr (sizeof(T) == 4)
+    if (split) return launch_exact<T, ST, 2, HALF, 1>(ctx, c, grid, deal);
+  return exact_rows(c.m, c.n, false) == 64 ? launch_exact<T, ST, 1, HALF, 1>(ctx, c, grid, deal)
+                                           : launch_exact<T, ST, 1, HALF, 2>(ctx, c, grid, deal);
 }
 
 }  // namespace
 
 namespace krm {
 
+// Whether fp16 x of this shape comes here (buffers aligned, main stream).
+bool gemm_exact_takes_half(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group) {
+  uint32_t grid = 0;
+  UnitDeal deal{};
+  return group >= 64 && (uint64_t)k * 256 <= 0xffffffffull && plan_exact(ctx, m, n, k, group, false, grid, deal);
+}
+
 // The exact-integer GEMM of fp16 x and of the f32 class for shapes whose (tile, stage) units cover the
 // chip; sets *handled = false (and launches nothing) for every other shape.
 int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
-                             bool* handled) {
+                             bool* handled, int32_t x_dtype) {
   *handled = false;
   const bool split = compute == KRM_COMPUTE_F32 && io_dtype == KRM_F32;
-  if (!split && io_dtype != KRM_F16) return KRM_OK;
+  if (!split && x_dtype != KRM_F16) return KRM_OK;
   if (group < 64 || !aligned(w, 16) || !aligned(x, 16)) return KRM_OK;
   // (a side branch of a graph has no scratch: there the K-splitting tiles, which need none with fp16
   // operands, take these shapes too; the f32 class is refused there)
@@ -582,7 +591,7 @@ int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
       c.m = rows;
       plan_exact(ctx, rows, n, k, group, split, grid, deal);
     }
-    c.x = ptr<const uint8_t>(x) + (size_t)r * k * dtype_bytes(io_dtype);
+    c.x = ptr<const uint8_t>(x) + (size_t)r * k * dtype_bytes(x_dtype);
     c.w = ptr<const uint8_t>(w);
     c.scales = ptr<const uint8_t>(scales);
     c.bias = ptr<const void>(bias);
@@ -598,15 +607,17 @@ int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
       KRM_TRY(launched(ctx, "split_rows_kernel"));
       c.x = static_cast<const uint8_t*>(ctx->x_planes);
     }
-    const bool half_groups = group == 64;
-    int32_t status;
-    if (scale_dtype == KRM_F16)
-      status = half_groups ? pick_exact<__half, true>(ctx, c, split, grid, deal)
-                           : pick_exact<__half, false>(ctx, c, split, grid, deal);
+    auto by_group = [&](auto io, auto scale) {
+      using T = decltype(io);
+      using ST = decltype(scale);
+      return group == 64 ? pick_exact<T, ST, true>(ctx, c, split, grid, deal)
+                         : pick_exact<T, ST, false>(ctx, c, split, grid, deal);
+    };
+    const bool half_scales = scale_dtype == KRM_F16;
+    if (io_dtype == KRM_F16)
+      KRM_TRY(half_scales ? by_group(__half{}, __half{}) : by_group(__half{}, float{}));
     else
-      status = half_groups ? pick_exact<float, true>(ctx, c, split, grid, deal)
-                           : pick_exact<float, false>(ctx, c, split, grid, deal);
-    KRM_TRY(status);
+      KRM_TRY(half_scales ? by_group(float{}, __half{}) : by_group(float{}, float{}));
   }
   return KRM_OK;
 }

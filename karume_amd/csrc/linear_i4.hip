@@ -1381,14 +1381,15 @@ int32_t linear_i4_gemv(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_b
 // MFMA GEMMs for M > 16: exact integer weights dealt by units (gemm_i4_exact.hip; short ranges of
 // products with fp16 x and f32 x rounded to fp16: gemm_i4.hip) or with K split inside a workgroup
 // (gemm_i4_slices.hip); fp16 weights (gemm_i4.hip).
+// x_dtype: fp16 beside an io_dtype of f32 are rows that were rounded before.
 int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                              krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                              int32_t io_dtype, int32_t scale_dtype, int32_t compute,
-                             bool* handled);
+                             bool* handled, int32_t x_dtype);
 int32_t linear_i4_gemm_staged(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                               krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                               int32_t io_dtype, int32_t scale_dtype, int32_t compute,
-                              bool* handled);
+                              bool* handled, int32_t x_dtype);
 int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                             krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                             int32_t io_dtype, int32_t scale_dtype, int32_t compute,
@@ -1396,8 +1397,50 @@ int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales
 int32_t linear_i4_gemm_f16(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias,
                            krm_buf out, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
                            int32_t io_dtype, int32_t scale_dtype);
+bool gemm_exact_takes_half(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group);
+bool gemm_staged_takes_f32(krm_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t group);
 
 }  // namespace krm
+
+// f32 rows rounded to fp16, eight codes a thread.
+__global__ __launch_bounds__(256) void round_rows_kernel(const uint4* __restrict__ x, uint4* __restrict__ out,
+                                                         uint32_t pieces) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= pieces) return;
+  const uint4 a = x[2 * (size_t)i], b = x[2 * (size_t)i + 1];
+  auto pack = [](uint32_t lo, uint32_t hi) {
+    return __builtin_bit_cast(uint32_t, half2_t{(_Float16)__uint_as_float(lo), (_Float16)__uint_as_float(hi)});
+  };
+  out[i] = make_uint4(pack(a.x, a.y), pack(a.z, a.w), pack(b.x, b.y), pack(b.z, b.w));
+}
+
+// f32 x of a product in fp16: its rows rounded once into the context's scratch (*rows) where that costs less than it
+// gives, instead of by every tile that reads them; otherwise *rows = x.
+static int32_t round_rows(krm_ctx* ctx, krm_buf x, krm_buf w, uint32_t m, uint32_t n, uint32_t k, uint32_t group,
+                          krm_buf* rows) {
+  *rows = x;
+  const uint64_t pieces = (uint64_t)m * k / 8;
+  // what the tiles on fp16 x take, or the scratch does not hold; a side branch of a graph has none
+  if (k % 32 != 0 || k < 64 || !aligned(w, 16) || pieces * 16 > kPlaneBytes || !ctx->x_planes ||
+      ctx->stream != ctx->main_stream)
+    return KRM_OK;
+  // A launch, x once more and the f32 result of a form that is quicker with fp16.  us before / now: where fp16 x goes to
+  // the unit-dealt products 512 x 11008 x 4096 70.2 / 65.4, 199 x 19207 x 4160 74.3 / 66.2, 248 x 4516 x 7040 44.4 / 32.4;
+  // to the K-splitting tiles from an estimated gain on 148 x 4751 x 6656 in groups of 64 46.5 / 33.5, 463 x 5555 x 3200
+  // 52.9 / 38.6, 104 x 11345 x 2432 20.0 / 17.4, 110 x 7290 x 5312 in groups of 32 44.2 / 32.1.  Below it 323 x 758 x 6400
+  // 20.5 / 21.0, 266 x 7717 x 1280 23.1 / 24.1, 174 x 1936 x 3456 10.8 / 11.2, 103 x 5143 x 1024 6.7 / 8.7; and the tiles
+  // staged through registers round what they read as quickly: 338 x 18849 x 1280 39.4 / 41.2, 303 x 21592 x 512 27.1 / 28.8.
+  if (!gemm_exact_takes_half(ctx, m, n, k, group)) {
+    if (gemm_staged_takes_f32(ctx, m, n, k, group)) return KRM_OK;
+    const float gain = slices_estimate_us(ctx, m, n, k, group, false, false) -
+                       slices_estimate_us(ctx, m, n, k, group, true, false);
+    if (gain < (group >= 128 ? 4.4f : 5.0f) + (float)pieces * (8 * 1.2e-6f)) return KRM_OK;
+  }
+  round_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, ctx->stream>>>(
+      ptr<const uint4>(x), static_cast<uint4*>(ctx->x_planes), (uint32_t)pieces);
+  *rows = (krm_buf)reinterpret_cast<uintptr_t>(ctx->x_planes);
+  return launched(ctx, "round_rows_kernel");
+}
 
 extern "C" {
 
@@ -1423,14 +1466,20 @@ int32_t krm_linear_i4(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_bu
   if (m <= 16)
     return linear_i4_gemv(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype);
   bool handled = false;
-  KRM_TRY(linear_i4_gemm_exact(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
-                               scale_dtype, compute, &handled));
+  krm_buf rows = x;
+  int32_t x_dtype = io_dtype;
+  if (compute == KRM_COMPUTE_F16 && io_dtype == KRM_F32) {
+    KRM_TRY(round_rows(ctx, x, w, m, n, k, group, &rows));
+    if (rows != x) x_dtype = KRM_F16;
+  }
+  KRM_TRY(linear_i4_gemm_exact(ctx, rows, w, scales, bias, out, m, n, k, group, io_dtype,
+                               scale_dtype, compute, &handled, x_dtype));
   if (handled) return KRM_OK;
-  KRM_TRY(linear_i4_gemm_staged(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,
-                                scale_dtype, compute, &handled));
+  KRM_TRY(linear_i4_gemm_staged(ctx, rows, w, scales, bias, out, m, n, k, group, io_dtype,
+                                scale_dtype, compute, &handled, x_dtype));
   if (handled) return KRM_OK;
-  KRM_TRY(linear_i4_gemm_slices(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
-                                compute, RowsFusion{}, &handled, io_dtype));
+  KRM_TRY(linear_i4_gemm_slices(ctx, rows, w, scales, bias, out, m, n, k, group, io_dtype, scale_dtype,
+                                compute, RowsFusion{}, &handled, x_dtype));
   if (handled) return KRM_OK;
   if (compute == KRM_COMPUTE_F16)
     return linear_i4_gemm_f16(ctx, x, w, scales, bias, out, m, n, k, group, io_dtype,

@@ -627,6 +627,30 @@ def test_rope_of_a_fused_projection_by_quads_and_by_pairs(gpu_ctx, io, m, heads,
     assert np.isfinite(np.delete(got[0][0], m // 2, 1)).all()
 
 
+# (unit-dealt tiles of 128 x 256 and of 64 x 512; tiles staged through registers; tiles that split K)
+@pytest.mark.parametrize("m,n,k,g", [(348, 8164, 4608, 128), (199, 19207, 4160, 64), (64, 25001, 8128, 64),
+                                     (463, 5555, 3200, 128), (104, 8583, 1152, 128), (148, 4751, 6656, 64),
+                                     (113, 6077, 2112, 32)])
+def test_f32_rows_rounded_to_fp16_once(gpu_ctx, m, n, k, g):
+    """f32 x in fp16 arithmetic with its rows rounded by a pass of their own: the gate of the exact-operand kernels
+    on the rounded x, f32 bias and result; a magnitude past fp16 is infinite, and so is its row's result."""
+    rng = np.random.default_rng(m + n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    scale = scale.astype(np.float32 if m % 2 else np.float16)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[m - 1, k - 1] = 7e4
+    bias = rng.normal(size=n).astype(np.float32)
+    with np.errstate(over="ignore"):
+        seen = x.astype(np.float16).astype(np.float32)
+    got = run_linear(gpu_ctx, x, packed, scale, bias, n, k, g, compute=ka.COMPUTE_F16)
+    assert not np.isfinite(got[m - 1]).any()
+    cols = np.unique(np.concatenate([rng.choice(n, size=64), [0, 255, 256, 511, 512, n - 2, n - 1]]))
+    want = sampled_oracle(seen[:-1], packed, scale.astype(np.float32), bias, n, k, g, cols)
+    bound = row_gate(seen[:-1]) + 1e-5 * np.abs(want)
+    err = np.abs(got[:-1, cols].astype(np.float64) - want)
+    assert np.all(err <= bound), float(np.max(err / bound))
+
+
 @pytest.mark.parametrize("io", [ka.F16, ka.F32])
 @pytest.mark.parametrize("m,n,k", [(17, 8, 64), (40, 96, 576), (128, 2048, 256)])
 def test_the_residual_of_a_silu_is_read_at_any_element(gpu_ctx, io, m, n, k):
