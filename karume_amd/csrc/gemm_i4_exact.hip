@@ -601,9 +601,8 @@ int32_t linear_i4_gemm_exact(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales,
     while ((1u << c.group_shift) < group) ++c.group_shift;
     c.row_scale = ctx->row_scales;
     if (split) {
-      split_rows_kernel<<<dim3(c.m), dim3(512), 0, ctx->stream>>>(
-          reinterpret_cast<const float*>(c.x), static_cast<uint4*>(ctx->x_planes), ctx->row_scales, k,
-          deal.stages_per_tile * 128u);
+      launch_split_rows(ctx, reinterpret_cast<const float*>(c.x), static_cast<uint4*>(ctx->x_planes), ctx->row_scales,
+                        c.m, k, deal.stages_per_tile * 128u);
       KRM_TRY(launched(ctx, "split_rows_kernel"));
       c.x = static_cast<const uint8_t*>(ctx->x_planes);
     }

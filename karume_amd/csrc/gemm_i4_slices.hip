@@ -760,9 +760,8 @@ int32_t linear_i4_gemm_slices(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales
   c.tail.row_scale = ctx->row_scales;
   for (uint64_t first = 0; first < m; first += fit) {
     const uint32_t rows = (uint32_t)(m - first < fit ? m - first : fit);
-    split_rows_kernel<<<dim3(rows), dim3(512), 0, ctx->stream>>>(
-        ptr<const float>(x) + first * k, reinterpret_cast<uint4*>(ctx->gemm_partials),
-        ctx->row_scales + 2 * first, k, k);
+    launch_split_rows(ctx, ptr<const float>(x) + first * k, reinterpret_cast<uint4*>(ctx->gemm_partials),
+                      ctx->row_scales + 2 * first, rows, k, k);
     KRM_TRY(launched(ctx, "split_rows_kernel"));
     c.x = reinterpret_cast<const uint8_t*>(ctx->gemm_partials);
     c.row_begin = (uint32_t)first;

@@ -627,6 +627,22 @@ def test_rope_of_a_fused_projection_by_quads_and_by_pairs(gpu_ctx, io, m, heads,
     assert np.isfinite(np.delete(got[0][0], m // 2, 1)).all()
 
 
+@pytest.mark.parametrize("k", [64, 2048, 2112, 4096, 4160, 8192, 8256, 16384, 16448])
+def test_hi_and_lo_of_rows_of_any_length(gpu_ctx, k):
+    """The lengths at which the pass that splits f32 rows has other threads: every row at the gate of its class, the
+    largest magnitude in its last piece."""
+    rng = np.random.default_rng(k)
+    m, n, g = 18, 70, 64
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[::2, k - 1] = 300
+    got = run_linear(gpu_ctx, x, packed, scale, None, n, k, g, compute=ka.COMPUTE_F32)
+    want = sampled_oracle(x, packed, scale.astype(np.float32), np.zeros(n, np.float32), n, k, g, np.arange(n))
+    bound = row_gate(x) + 1e-5 * np.abs(want)
+    err = np.abs(got.astype(np.float64) - want)
+    assert np.all(err <= bound), float(np.max(err / bound))
+
+
 # (unit-dealt tiles of 128 x 256 and of 64 x 512; tiles staged through registers; tiles that split K)
 @pytest.mark.parametrize("m,n,k,g", [(348, 8164, 4608, 128), (199, 19207, 4160, 64), (64, 25001, 8128, 64),
                                      (463, 5555, 3200, 128), (104, 8583, 1152, 128), (148, 4751, 6656, 64),
