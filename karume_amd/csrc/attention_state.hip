@@ -1043,6 +1043,9 @@ struct DecodeArgs {
   uint32_t* tickets;         // arrival counter (sequence, head unit) at index * kTicketStride, zero between launches
   uint32_t* lengths;         // single sequence: device {past, query, fault} or null
   uint32_t capacity;         // single sequence: slot rows (checked against device lengths)
+  uint32_t splits;           // that the grid and the workspace are sized for
+  uint32_t units;            // kv heads * head_groups
+  uint32_t folded;           // the grid is (8 units, splits / 8, batch), else (splits, units, batch)
 };
 
 // Columns are walked in chunks of kDecodeIter * G rows (G = 256 / lanes-per-row groups, each
@@ -1123,8 +1126,16 @@ void attention_decode_kernel(
   const int tid = threadIdx.x;
   const int sub = tid % LPR;   // which 16 bytes of the row
   const int group = tid / LPR;
-  const uint32_t hk = blockIdx.y / a.head_groups;
-  const uint32_t head0 = hk * a.repeat + (blockIdx.y - hk * a.head_groups) * R;  // first head
+  // Workgroups that share a split's rows (head groups of a kv head) follow each other on one XCD, whose L2 then has
+  // the rows for all of them: workgroups go to the eight XCDs in turn.  (Splits and head groups as the two sides of the grid:
+  // the same XCD where the splits are a multiple of eight, every XCD reading every row elsewhere.)  us before / now:
+  // f32 32 heads of 8, D = 128, 4000 columns (63 splits) 17.3 / 12.1, 600 8.4 / 6.8; 8 heads of 2 11.7 / 8.3; 8 heads of 1,
+  // D = 256, 4000 20.9 / 14.7, fp16 12.2 / 8.6, ragged 25 sequences up to 2602 51.2 / 43.9; fp16 32 of 8, D = 128, 4095 (32
+  // splits) 8.71 / 8.48.
+  const uint32_t unit = a.folded ? blockIdx.x >> 3 : blockIdx.y;
+  const uint32_t hk = unit / a.head_groups;
+  const uint32_t at_split = a.folded ? blockIdx.y * 8u + ((blockIdx.x - hk) & 7u) : blockIdx.x;
+  const uint32_t head0 = hk * a.repeat + (unit - hk * a.head_groups) * R;  // first head
 
   // The rows of a chunk as they arrive: K pieces (row-owner layout, or the MFMA A-operand
   // layout: piece tile*4 + t) and V pieces (row-owner layout).
@@ -1186,7 +1197,7 @@ void attention_decode_kernel(
     early = a.lengths != nullptr && a.window == 0;
     if (early) {
       const size_t base = (size_t)blockIdx.z * a.slot_batch_stride + (size_t)hk * a.slot_plane_stride;
-      const uint32_t want = blockIdx.x * (kSplitChunks * (uint32_t)kChunkCols);
+      const uint32_t want = at_split * (kSplitChunks * (uint32_t)kChunkCols);
       const uint32_t c_begin = want < a.capacity ? want : a.capacity - 1u;
       const uint32_t room = a.capacity - c_begin;
       request_rows(slot_k + base, slot_v + base, 0u, c_begin,
@@ -1200,7 +1211,7 @@ void attention_decode_kernel(
   uint32_t seq, split, nsplit, first_split;
   uint32_t past, row_base;
   if constexpr (RAGGED) {
-    // The last sequence whose first split is <= blockIdx.x, 64 sequences at a time: every lane
+    // The last sequence whose first split is <= at_split, 64 sequences at a time: every lane
     // asks for one sequence's entries at once, so the tables cost one round trip (a binary search
     // cost log2(nseq) of them in a row, 0.6 us each, in front of the first row's address).
     uint32_t first_of = 0, next_of = 0, row_of = 0, row_end_of = 0;
@@ -1211,8 +1222,8 @@ void attention_decode_kernel(
       next_of = (uint32_t)a.split_prefix[i + 1];
       row_of = (uint32_t)a.cu_rows[i];
       row_end_of = (uint32_t)a.cu_rows[i + 1];
-      const uint64_t mine = __ballot(base + (uint32_t)lane < a.nseq && first_of <= blockIdx.x &&
-                                     blockIdx.x < next_of);
+      const uint64_t mine = __ballot(base + (uint32_t)lane < a.nseq && first_of <= at_split &&
+                                     at_split < next_of);
       if (mine) {
         const int owner = __builtin_ctzll(mine);
         seq = base + owner;
@@ -1226,7 +1237,7 @@ void attention_decode_kernel(
     }
     first_split = first_of;
     nsplit = next_of - first_of;
-    split = blockIdx.x - first_split;
+    split = at_split - first_split;
     row_base = row_of;
     past = row_end_of - row_of;
   } else {
@@ -1236,13 +1247,13 @@ void attention_decode_kernel(
     past = p32;
     row_base = 0;
     nsplit = decode_splits(past - window_low(a.window, past), kChunkCols);
-    split = blockIdx.x;
+    split = at_split;
     // The grid and the workspace were sized on the host for the longest past the launch may
     // see.  A replay whose device-side past needs more splits than that would never complete a
     // ticket round and would index partials beyond the workspace: raise the fault word and
     // leave everything untouched instead.
-    if (nsplit > gridDim.x) {
-      if (a.lengths && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) a.lengths[2] = 1u;
+    if (nsplit > a.splits) {
+      if (a.lengths && at_split == 0 && unit == 0 && tid == 0) a.lengths[2] = 1u;
       return;
     }
     if (split >= nsplit) return;  // the grid is sized for the longest past it may see
@@ -1595,7 +1606,7 @@ void attention_decode_kernel(
   // on this target, and a device-scope one writes the whole L2 back.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  uint32_t* ticket = &a.tickets[(size_t)(seq * gridDim.y + blockIdx.y) * kTicketStride];
+  uint32_t* ticket = &a.tickets[(size_t)(seq * a.units + unit) * kTicketStride];
   if (tid == 0)
     s_ticket = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
@@ -1685,8 +1696,8 @@ __global__ void clear_tickets_kernel(uint32_t* tickets, uint32_t count) {
 template <typename XT, typename ST, int R, int LPR, bool RAGGED>
 int32_t launch_decode(krm_ctx* ctx, const DecodeLaunch& L) {
   attention_decode_kernel<XT, ST, R, LPR, RAGGED>
-      <<<dim3(L.grid_x, L.args.kv_heads * L.args.head_groups, L.grid_z), dim3(kThreads), 0,
-         ctx->stream>>>(
+      <<<L.args.folded ? dim3(8 * L.args.units, (L.grid_x + 7) / 8, L.grid_z) : dim3(L.grid_x, L.args.units, L.grid_z),
+         dim3(kThreads), 0, ctx->stream>>>(
           ptr<const XT>(L.q), ptr<const XT>(L.ins_k), ptr<const XT>(L.ins_v),
           ptr<const ST>(L.slot_k), ptr<const ST>(L.slot_v), ptr<XT>(L.out), L.ws_ml, L.ws_acc,
           L.args);
@@ -1735,6 +1746,10 @@ int32_t decode_dispatch(krm_ctx* ctx, DecodeLaunch& L, uint32_t repeat, uint32_t
 
   L.args.repeat = repeat;
   L.args.head_groups = repeat / per_block;
+  L.args.splits = L.grid_x;
+  L.args.units = L.args.kv_heads * L.args.head_groups;
+  // (one split: the head groups lie on neighbouring XCDs, and seven of eight workgroups of the other grid had no work)
+  L.args.folded = L.grid_x > 1 && L.args.head_groups > 1 && (L.grid_x + 7) / 8 <= 65535 ? 1u : 0u;
   const uint64_t counters = (uint64_t)L.args.nseq * L.args.kv_heads * L.args.head_groups;
   if ((uint64_t)L.args.kv_heads * L.args.head_groups > 65535 || counters > L.ticket_slots)
     return fail(ctx, KRM_ERR_VALIDATION, "decode attention: B * H = %llu exceeds %u",

@@ -660,6 +660,19 @@ def test_varlen_planned_on_the_device_is_recordable(gpu_ctx):
         b.free()
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,depth,past,window", [
+    (1, 12, 3, 128, 641, 0), (2, 20, 5, 128, 1100, 0), (1, 24, 12, 64, 2300, 0), (3, 8, 1, 256, 600, 0),
+    (1, 18, 9, 128, 3000, 1100)])
+def test_decode_of_splits_that_share_rows_on_an_xcd(gpu_ctx, batch, heads, kv_heads, depth, past, window):
+    """Several splits and several head groups a kv head (the folded grid): splits no multiple of eight, kv heads
+    past eight, a batch, a window; the class's gate against the oracle."""
+    case = StateCase("folded", batch, heads, kv_heads, 1, depth, window or past + 1, window, past, 1)
+    x = random_state_inputs(case, seed=past, f16_values=False)
+    got = run_attention(gpu_ctx, case, x)
+    ok, fails, max_abs, worst = oracle.allclose(got, oracle_state_attention(case, x), atol=STATE_ATOL, rtol=0)
+    assert ok, (fails, max_abs, worst)
+
+
 @pytest.mark.parametrize("nseq", [1, 62, 63, 64, 65, 127, 128, 300])
 def test_varlen_plan_tables_past_a_wave(gpu_ctx, nseq):
     """The tables of a plan, by steps of 64 sequences: offsets as given, splits of 128 columns summed before each
