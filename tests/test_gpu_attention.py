@@ -660,6 +660,16 @@ def test_varlen_planned_on_the_device_is_recordable(gpu_ctx):
         b.free()
 
 
+@pytest.mark.parametrize("splits", [5, 8, 9, 16, 24, 25, 32, 33, 40, 57, 64])
+def test_decode_merges_any_number_of_splits(gpu_ctx, splits):
+    """Passes of 32 partials, short ones in blocks of eight: the class's gate against the oracle."""
+    case = StateCase("splits", 1, 2, 1, 1, 128, splits * 64 + 1, 0, splits * 64, 1)  # f32: 64 columns a split
+    x = random_state_inputs(case, seed=splits, f16_values=False)
+    got = run_attention(gpu_ctx, case, x)
+    ok, fails, max_abs, worst = oracle.allclose(got, oracle_state_attention(case, x), atol=STATE_ATOL, rtol=0)
+    assert ok, (fails, max_abs, worst)
+
+
 @pytest.mark.parametrize("batch,heads,kv_heads,depth,past,window", [
     (1, 12, 3, 128, 641, 0), (2, 20, 5, 128, 1100, 0), (1, 24, 12, 64, 2300, 0), (3, 8, 1, 256, 600, 0),
     (1, 18, 9, 128, 3000, 1100)])
