@@ -28,9 +28,9 @@
 // What bounds it: what the second-level cache delivers to a CU (tiles of 64 x 96: 2 * 64 + 96 / 2
 // bytes a code), then the conversion of the weights on the vector ALUs (10 operations a word, 9 beside hi + lo planes).
 // Measured on cold weights, fp16 x (f32 class in brackets), against the kernel that loaded through
-// registers, one 32 x 32 or 32 x 64 tile a workgroup: 128 x 2560 x 2048 6.6 us, 9.6 before (11.8,
-// 14.5); 128 x 2048 x 2048 5.4, 7.0 (10.1, 12.5); 128 x 11264 x 2048 15.1, 27.0 (25.9, 38.6); 128 x
-// 2048 x 5632 10.6, 13.0 (19.7, 26.2).
+// registers, one 32 x 32 or 32 x 64 tile a workgroup: 128 x 2560 x 2048 6.6 us, 9.6 before (11.0,
+// 14.5); 128 x 2048 x 2048 5.4, 7.0 (10.1, 12.5); 128 x 11264 x 2048 15.1, 27.0 (22.6, 38.6); 128 x
+// 2048 x 5632 10.6, 13.0 (19.0, 26.2).
 //
 // kXThree is bounded by the vector ALUs (11 operations a pair of x, 10 a word of weights, both at
 // every step; tiles of up to four columns share x).  Groups of 32, against the GEMV over blocks of 16

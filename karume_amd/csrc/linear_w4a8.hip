@@ -50,11 +50,12 @@ __device__ inline bool is_nan_bits(float v) {
 // ------------------------------------------------------------------------- quantize_rows
 //
 // One workgroup per row (grid-stride over rows): |x| maximum with NaN propagation, then the
-// quotients.  Rows of up to 256 * 4 * kQuantCache elements stay in registers between the two
+// quotients.  Rows of up to THREADS * 4 * HELD elements stay in registers between the two
 // (one trip to memory, all loads in flight together); longer rows are read twice.  x / s is the
 // correctly rounded f32 division, so the codes equal the CPU formula's for every input, also
-// next to a rounding tie.
-constexpr int kQuantCache = 12;  // float4 per thread: rows of up to 12288 elements
+// next to a rounding tie.  Threads as many as leave each one to three quads: the quotients of a row are a
+// chain of one workgroup.  us with 256 threads of up to twelve quads / so: 512 x 4096 4.5 / 4.1, 512 x 11008 7.9 / 6.7, 128 x
+// 5632 4.4 / 3.7, 16 x 4096 3.6 / 3.0, 9 x 1024 2.6 / 2.35, 512 x 16384 14.4 / 9.5.
 
 // x / s must be the correctly rounded quotient only where it decides the code: t = x * (1 / s)
 // (1 / s correctly rounded) lies within 2.3e-5 of it for |x / s| <= 127.5, so when t is further
@@ -85,18 +86,19 @@ __device__ inline uint32_t quantize4(const float4& v, float s, float inv_s) {
   return packed;
 }
 
-__global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restrict__ x,
+template <uint32_t THREADS, int HELD>
+__global__ __launch_bounds__(THREADS) void quantize_rows_kernel(const float* __restrict__ x,
                                                             uint32_t* __restrict__ xq,
                                                             float* __restrict__ xs,
                                                             uint32_t rows, uint32_t dim) {
-  __shared__ float s_max[4];
-  __shared__ uint32_t s_nan[4];
+  __shared__ float s_max[THREADS / 64];
+  __shared__ uint32_t s_nan[THREADS / 64];
   const uint32_t quads = dim >> 2;
-  const bool cached = quads <= 256u * kQuantCache;
+  const bool cached = quads <= THREADS * HELD;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (uint32_t row = blockIdx.x; row < rows; row += gridDim.x) {
     const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * dim);
-    float4 cache[kQuantCache];
+    float4 cache[HELD];
     float amax = 0.f;
     bool nan = false;
     auto fold = [&](const float4& v) {
@@ -109,16 +111,16 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restr
     };
     if (cached) {
 #pragma unroll
-      for (int i = 0; i < kQuantCache; ++i) {
-        if (256u * i >= quads) break;  // uniform: the row ends before this stride
-        const uint32_t at = threadIdx.x + 256u * i;
+      for (int i = 0; i < HELD; ++i) {
+        if (THREADS * i >= quads) break;  // uniform: the row ends before this stride
+        const uint32_t at = threadIdx.x + THREADS * i;
         cache[i] = xr[at < quads ? at : 0u];  // past the row: its first quad again, not folded
       }
 #pragma unroll
-      for (int i = 0; i < kQuantCache; ++i)
-        if (threadIdx.x + 256u * i < quads) fold(cache[i]);
+      for (int i = 0; i < HELD; ++i)
+        if (threadIdx.x + THREADS * i < quads) fold(cache[i]);
     } else {
-      for (uint32_t i = threadIdx.x; i < quads; i += 256) fold(xr[i]);
+      for (uint32_t i = threadIdx.x; i < quads; i += THREADS) fold(xr[i]);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
@@ -128,8 +130,12 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restr
       s_nan[wave] = wave_nan ? 1u : 0u;
     }
     __syncthreads();
-    amax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-    const bool row_nan = (s_nan[0] | s_nan[1] | s_nan[2] | s_nan[3]) != 0u;
+    bool row_nan = false;
+#pragma unroll
+    for (uint32_t w = 0; w < THREADS / 64; ++w) {
+      amax = fmaxf(amax, s_max[w]);
+      row_nan = row_nan || s_nan[w] != 0u;
+    }
     float s = fmaxf(amax * (float)(1.0 / 127.0), kF32Tiny);
     if (row_nan) s = __uint_as_float(0x7fc00000u);
     if (threadIdx.x == 0) xs[row] = s;
@@ -137,12 +143,12 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restr
     uint32_t* qr = xq + (size_t)row * quads;
     if (cached) {
 #pragma unroll
-      for (int i = 0; i < kQuantCache; ++i) {
-        const uint32_t at = threadIdx.x + 256u * i;
+      for (int i = 0; i < HELD; ++i) {
+        const uint32_t at = threadIdx.x + THREADS * i;
         if (at < quads) qr[at] = quantize4(cache[i], s, inv_s);
       }
     } else {
-      for (uint32_t i = threadIdx.x; i < quads; i += 256) qr[i] = quantize4(xr[i], s, inv_s);
+      for (uint32_t i = threadIdx.x; i < quads; i += THREADS) qr[i] = quantize4(xr[i], s, inv_s);
     }
     __syncthreads();  // s_max / s_nan are rewritten by the next row
   }
@@ -673,7 +679,7 @@ void linear_w4a8_tile_kernel(
 // ahead, a stage of 512 x 11008 x 4096 took 2283 clk: 281 to ask for the next one, 640 of products, 1218 of
 // waiting for it (a scale a lane touched 64 lines: 445 of them) and parking it, 143 at the barrier.  Now
 // 1551: 299, 1139, 45, 68.  us with the quantiser's launch, before / now, fp16 scales unless noted: 512 x 11008 x
-// 4096 51.4 / 46.6, in groups of 64 60.6 / 55.0, of 32 105 / 83, with f32 scales (whose quotient by 16 was
+// 4096 51.4 / 46.6 (45.9 with the quantiser's threads by length), in groups of 64 60.6 / 55.0, of 32 105 / 83, with f32 scales (whose quotient by 16 was
 // tested in every group) 56.8 / 47.9; 2048 x 11008 x 4096 166 / 157; 20 x 20000 x 1024 in groups of 32 18.2 / 15.1;
 // 500 x 600 x 8000 in groups of 32, f32 scales 112 / 72.
 template <typename ST, int GSH, int WM, int NW, int WN, int MT>
@@ -1024,9 +1030,15 @@ extern "C" int32_t krm_quantize_rows(krm_ctx* ctx, krm_buf x, krm_buf xq, krm_bu
   KRM_REQUIRE(ctx, aligned(x, 16) && aligned(xq, 4) && aligned(xs, 4),
               "quantize_rows: x needs 16-byte, xq and xs 4-byte alignment");
   const uint32_t blocks = rows < (1u << 16) ? rows : (1u << 16);
-  hipLaunchKernelGGL(quantize_rows_kernel, dim3(blocks), dim3(256), 0, ctx->stream,
-                     krm::ptr<const float>(x), krm::ptr<uint32_t>(xq), krm::ptr<float>(xs), rows,
-                     dim);
+  auto launch = [&](auto kernel, uint32_t threads) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, ctx->stream, krm::ptr<const float>(x), krm::ptr<uint32_t>(xq),
+                       krm::ptr<float>(xs), rows, dim);
+  };
+  if (dim <= 1024) launch(quantize_rows_kernel<256, 1>, 256);
+  else if (dim <= 2048) launch(quantize_rows_kernel<512, 1>, 512);
+  else if (dim <= 4096) launch(quantize_rows_kernel<512, 2>, 512);
+  else if (dim <= 8192) launch(quantize_rows_kernel<1024, 2>, 1024);
+  else launch(quantize_rows_kernel<1024, 3>, 1024);
   return krm::launched(ctx, "quantize_rows_kernel");
 }
 

@@ -72,6 +72,18 @@ def test_quantize_matches_oracle_rows_of_different_size(gpu_ctx):
     assert float(s[3]) == 1.1754943508222875e-38 and not q[3].any()
 
 
+@pytest.mark.parametrize("dim", [4, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196, 12288, 12292])
+def test_quantize_at_the_lengths_kept_in_registers(gpu_ctx, dim):
+    """Rows at the edges of each number of threads; the largest magnitude, then a NaN, in the last quad."""
+    x = np.random.default_rng(dim).normal(size=(3, dim)).astype(np.float32)
+    x[1, dim - 1] = 50
+    x[2, dim - 2] = np.nan
+    q, s = run_quantize(gpu_ctx, x)
+    want_q, want_s = oracle.quantize_rows(x, dim)
+    assert_exact(s, want_s, "scale")
+    assert_exact(q, want_q, "codes")
+
+
 def test_quantize_propagates_nan_and_inf_to_the_row_scale(gpu_ctx):
     rows, dim = 4, 8
     x = helpers.seeded(rows * dim, helpers.SIGNED_A8).reshape(rows, dim)
