@@ -221,7 +221,7 @@ __global__ __launch_bounds__(kMaxUnits * 64) void gemv_i4_rows_kernel(
       for (uint32_t j = 0; j < kQuad; ++j) sums[r][j] = 0.f;
     for (uint32_t step = 0; segment_of(step, position, 0) < segments; ++step) {
       const uint32_t own = segment_of(step, position, own_sub);
-      wait_vm<0>();
+      wait_streamed_and_read();  // (the other half of the ring, which is filled next, was read a stage ago)
       if (segment_of(step + 1, position, 0) < segments) {
         request(position, step + 1, buf ^ 1u);
       } else {

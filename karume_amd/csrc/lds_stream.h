@@ -27,6 +27,9 @@ template <int N>
 __device__ inline void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// Everything streamed has landed, and everything this wave read from LDS has arrived: what is asked for behind it
+// may land where it read.  (A read's own wait stands at its first use, which may come later.)
+__device__ inline void wait_streamed_and_read() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 
 }  // namespace
 }  // namespace krm
