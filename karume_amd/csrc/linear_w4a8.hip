@@ -466,8 +466,8 @@ __global__ __launch_bounds__(256) void linear_w4a8_rows_kernel(
 //  * Every stage issues the same loads in the same order whatever K is (addresses past K are
 //    clamped, chunks past K multiply zeros and are fused with a zero scale): a branch around a
 //    load would make the compiler's wait counts assume the worst path.
-// GSH = 8: groups of 256, a stage each (64 and 128: linear_w4a8_tall_kernel); GSH = 0: any larger group (a
-// whole number of stages).
+// GSH = log2(group) for groups of 64, 128 (up to a K of 2^24: linear_w4a8_tall_kernel) and 256; GSH = 0: any
+// larger group (a whole number of stages).
 // Workgroup ids are dealt so that the row blocks of a column block run on one XCD.
 // (Weights loaded straight from global memory into the operand registers, without LDS, were
 // measured 1.5 x slower: a lane's own 16 bytes of its own row make every quad of lanes touch
@@ -958,19 +958,24 @@ int32_t launch_w4a8(krm_ctx* ctx, krm_buf xq, krm_buf xs, krm_buf w, krm_buf sca
         return launched(ctx, "linear_w4a8_tall_kernel");
       }
     }
-    // 64 x 256 tiles in larger groups, or 64 x 128 where those would leave a quarter of the chip without work
+    // 64 x 256 tiles in larger groups, and in groups of 64 and 128 past a K of 2^24, whose rows the tiles above
+    // do not reach with 32-bit offsets (64 x 256 x 16777472: 491 and 242 ms in the form for any shape, 127 and 102
+    // here); 64 x 128 where those would leave a quarter of the chip without work, and in groups of 64 (four tiles'
+    // sums and eight groups' factors spill).
     const uint32_t m_blocks = (m + 63) / 64;
-    const bool narrow = (uint64_t)m_blocks * n_blocks * 4 < cus * 3;
+    const bool narrow = shift == 6 || (uint64_t)m_blocks * n_blocks * 4 < cus * 3;
     const uint32_t nb = narrow ? (n + 127) / 128 : n_blocks;
     const uint64_t blocks = (uint64_t)((nb + 7) / 8) * 8u * m_blocks;
-    if (shift > 7 && blocks <= 0x7fffffffull) {
+    if (shift > 5 && blocks <= 0x7fffffffull) {
 #define KRM_W4A8_TILE(GSH, WN)                                                                 \
   hipLaunchKernelGGL((linear_w4a8_tile_kernel<ST, GSH, 1, WN>), dim3((uint32_t)blocks),        \
                      dim3(512), 0, ctx->stream, ptr<const uint8_t>(xq), pxs,                  \
                      ptr<const uint8_t>(w), ps, pb, po, m, n, k, shift, m_blocks, nb)
 #define KRM_W4A8_TILE_G(GSH) \
   do { if (narrow) KRM_W4A8_TILE(GSH, 1); else KRM_W4A8_TILE(GSH, 2); } while (0)
-      if (shift == 8) KRM_W4A8_TILE_G(8);
+      if (shift == 6) KRM_W4A8_TILE(6, 1);
+      else if (shift == 7) KRM_W4A8_TILE_G(7);
+      else if (shift == 8) KRM_W4A8_TILE_G(8);
       else KRM_W4A8_TILE_G(0);
 #undef KRM_W4A8_TILE_G
 #undef KRM_W4A8_TILE

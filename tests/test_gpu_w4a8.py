@@ -397,3 +397,27 @@ def test_w4a8_stages_and_scale_blocks_of_the_streamed_tiles(gpu_ctx, m, n, k, gr
     got = run_w4a8(gpu_ctx, x, packed, scale, bias, n, k, group)
     want = oracle.linear_w4a8(x, packed, np.asarray(scale, dtype=np.float32), bias, n, k, group)
     assert_exact(got, want, (m, n, k, group))
+
+
+@pytest.mark.parametrize("group", [64, 128])
+def test_w4a8_rows_longer_than_the_streamed_tiles_reach(gpu_ctx, group):
+    """A K past 2^24 and more than eight rows: codes and scales whose sums are exact in f32 in any order."""
+    m, n, k = 9, 5, (1 << 24) + 192
+    k -= k % group
+    rng = np.random.default_rng(group)
+    xq = rng.integers(-1, 2, size=(m, k), dtype=np.int8)
+    packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    scale = rng.choice(np.float32([0.5, 1, 2]), size=(n, k // group))
+    want = np.zeros((m, n), dtype=np.float64)
+    step = 1 << 20
+    for at in range(0, k, step):   # |sum of a block| < 2^24
+        two = packed[:, at // 2:(at + step) // 2]
+        q = np.stack([two & 15, two >> 4], axis=2).reshape(n, -1).astype(np.float32) - 8
+        q *= np.repeat(scale[:, at // group:(at + step) // group], group, axis=1)
+        want += xq[:, at:at + step].astype(np.float32) @ q.T
+    bufs = [gpu_ctx.upload(a) for a in (xq, np.ones(m, dtype=np.float32), packed, scale)]
+    out = gpu_ctx.alloc(m * n * 4)
+    gpu_ctx.linear_w4a8(*bufs, None, out, m, n, k, group)
+    assert np.array_equal(out.download(np.float32, (m, n)).astype(np.float64), want)
+    for b in bufs + [out]:
+        b.free()

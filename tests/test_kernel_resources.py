@@ -38,6 +38,12 @@ def test_tiles_of_w4a8_groups_up_to_128_keep_their_state_in_registers(kernels):
         assert kernel_resources.scratch(kernel) == 0, name
 
 
+def test_w4a8_groups_of_64_and_128_have_tiles_for_any_k(kernels):
+    """Past a K of 2^24 the tiles above do not reach all rows with their offsets of 32 bits."""
+    tiles = {(arguments(n)[1], arguments(n)[3]) for n in kernels if n.startswith("linear_w4a8_tile_kernel<")}
+    assert tiles == {("6", "1")} | {(group, wide) for group in ("7", "8", "0") for wide in ("1", "2")}
+
+
 # The forms that spill: the large f32-activation forms of the GEMM on fp16 weights (f32 x is rounded in the
 # loop, beside a 64 x 64 tile a wave).
 SPILL = ("gemm_i4_f16_kernel<float, __half, 2, 2, 64, 1, 4, true,",
