@@ -894,6 +894,7 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
   constexpr int kRowB = kStage / 2 + 16;
   constexpr int kAUnits = BM * (kStage / 8) / T;   // 2
   constexpr int kBUnits = BN * (kStage / 32) / T;  // 4
+  constexpr bool kWhole = sizeof(ST) == 4 && sizeof(OT) == 4;  // the totals (see scales_whole)
   static_assert((size_t)BM * BN == kPartialFloats, "the partial slots hold one tile");
   __shared__ __align__(16) uint8_t s_a[2][BM * kRowA];
   __shared__ __align__(16) uint8_t s_b[2][BN * kRowB];
@@ -1000,7 +1001,7 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
           for (int nt = 0; nt < WN; ++nt) {
             const uint32_t word = j == 0 ? braw[nt].x : j == 1 ? braw[nt].y : j == 2 ? braw[nt].z
                                                                                     : braw[nt].w;
-            const half8_t b = ints_paired(word);
+            const half8_t b = ints_paired<true>(word);
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
@@ -1013,6 +1014,12 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
           }
         }
         if (c == 1 || half_stage_groups) {  // the scale group ends here
+          if constexpr (kWhole) {
+            if (scales_whole(ws)) {
+#pragma unroll
+              for (int i = 0; i < MT * WN; ++i) acc[i / WN][i % WN] *= 1024.0f;
+            }
+          }
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -1037,7 +1044,7 @@ void gemm_i4_staged_kernel(const XT* __restrict__ x, const uint8_t* __restrict__
       for (int r = 0; r < 16; ++r) {
         const uint32_t local = mt * 32 + 8 * (r / 4) + 4 * frag_h + (r % 4);
         const uint32_t row = m0 + local;
-        if (row < m && col < n) store_out<OT>(out, (size_t)row * n + col, sum[r] * 1024.0f + b);
+        if (row < m && col < n) store_out<OT>(out, (size_t)row * n + col, (kWhole ? sum[r] : sum[r] * 1024.0f) + b);
       }
     };
 

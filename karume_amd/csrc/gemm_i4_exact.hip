@@ -98,6 +98,10 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
                           T* __restrict__ out, UnitDeal deal, const float* __restrict__ row_scale) {
   using G = ExactGeometry<PLANES, HALF, WM>;
   constexpr int BM = G::BM, BN = G::BN, D = G::kDepth, X = G::kXLoads, W = G::kWLoads, S = G::kSLoads;
+  // The totals (see scales_whole).  hi and lo have whole weights for it, twelve operations a word instead of nine:
+  // 300 x 32000 x 2048 in groups of 64 102 -> 104 us (with the scales whole it spilled: 133).  f32 rows rounded before:
+  // 512 x 11008 x 4096 in groups of 64 76 -> 86 (as much as in the tiles that round), in groups of 128 73 -> 74.
+  constexpr bool kWhole = sizeof(ST) == 4 && sizeof(T) == 4, kWholeSums = kWhole && PLANES == 1;
   static_assert((size_t)BM * BN == kPartialFloats, "the partial slots hold one tile");
   __shared__ __align__(1024) uint8_t s_x[D * G::kXBytes];
   __shared__ __align__(1024) uint8_t s_w[D * G::kWBytes];
@@ -230,6 +234,7 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
 #pragma unroll
       for (int i = 0; i < 4; ++i) total[i >> 1][i & 1] = acc[i >> 1][i & 1] = zero16;
       float ws[2] = {0.f, 0.f};
+      bool scales_past = false;
       half8_t a[2][PLANES][2], b[2][2];
       uint4 words[2];
 
@@ -255,18 +260,31 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
           const uint32_t bits = *reinterpret_cast<const uint32_t*>(at + nt * (32 * G::kEntries * 4));
           ws[nt] = sizeof(ST) == 2 ? (float)__builtin_bit_cast(_Float16, (uint16_t)bits) : __uint_as_float(bits);
         }
+        if constexpr (kWholeSums) scales_past = scales_whole(ws);
       };
       auto convert = [&](int t, const uint4 (&from)[2], half8_t (&to)[2]) {
         const int j = t % 4;
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
           const uint32_t word = j == 0 ? from[nt].x : j == 1 ? from[nt].y : j == 2 ? from[nt].z : from[nt].w;
-          to[nt] = PLANES == 2 ? ints_paired(word) : ints_natural(word);
+          to[nt] = PLANES == 2 ? ints_paired<!kWhole>(word) : ints_natural(word);
         }
       };
-      auto flush = [&](int mt, int nt) {
+      // (inside a stage a branch for `whole_sums` cost registers and spilled: a multiplication there)
+      auto flush = [&](int mt, int nt, bool inside) {
+        const float factor = kWholeSums && inside && scales_past ? 1024.0f : 1.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) total[mt][nt][r] = fmaf(acc[mt][nt][r], ws[nt], total[mt][nt][r]);
+        for (int r = 0; r < 16; ++r)
+          total[mt][nt][r] = fmaf(kWholeSums && inside ? acc[mt][nt][r] * factor : acc[mt][nt][r], ws[nt], total[mt][nt][r]);
+      };
+      // in front of the other flushes
+      auto whole_sums = [&] {
+        if constexpr (kWholeSums) {
+          if (scales_past) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] *= 1024.0f;
+          }
+        }
       };
       // Step t of a stage whose operands are in registers; beside its products run the reads and the
       // conversion of the next step's operands (`next_x`, `next_words`: where they lie).
@@ -277,7 +295,7 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
         for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
           for (int mt = 0; mt < 2; ++mt) {
-            if (opens) flush(mt, nt);
+            if (opens) flush(mt, nt, t == 4);
 #pragma unroll
             for (int p = 0; p < PLANES; ++p)
               acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
@@ -301,6 +319,7 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
           const int next = (t & 1) ^ 1;
+          if (t == 0) whole_sums();
           if (t == 7) {
             // the next stage has landed, in every wave, and this one has been read
             stage_landed<(D - 2) * (X + W + S)>(__builtin_amdgcn_readfirstlane(stage + D - 1), s1);
@@ -324,6 +343,7 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
         const uint32_t x_base = buf * G::kXBytes;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
+          if (t == 0) whole_sums();
           if (t < 3) read_x(t + 1, x_base, a[(t & 1) ^ 1]);
           products(t);
           if (t == 1) read_scales(s1 - 1u - s0, slot, 0);
@@ -331,10 +351,11 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
         }
       }
       wait_vm<0>();  // what was asked for past the end
+      whole_sums();
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) flush(mt, nt);
+        for (int nt = 0; nt < 2; ++nt) flush(mt, nt, false);
     }
     __syncthreads();  // the LDS is free: the next tile's first stages come in beside what follows
     if (left > s1 - s0) request_first(locate(left - (s1 - s0)));
@@ -345,7 +366,7 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
     const uint32_t o_row = (G::WM == 2 ? (here >> 8) * 64u : 0u) + ((here & 63u) >> 5) * 4u;
     const uint32_t o_col = n0 + (G::WM == 2 ? (here >> 6) & 3u : here >> 6) * 64u + (here & 31u);
     if constexpr (PLANES == 2) {
-      if (here < BM) s_inv[here] = row_scale[2 * (size_t)min(m0 + here, m - 1u) + 1];
+      if (here < BM) s_inv[here] = row_scale[2 * (size_t)min(m0 + here, m - 1u) + 1] * (kWhole ? 1.0f : 1024.0f);
       __syncthreads();
     }
     auto store_rows = [&](int mt, const float16_t (&sum)[2]) {
@@ -358,7 +379,7 @@ void gemm_i4_exact_kernel(const uint8_t* __restrict__ x, const uint8_t* __restri
         for (int r = 0; r < 16; ++r) {
           const uint32_t local = o_row + mt * 32 + 8 * (r / 4) + (r % 4);
           float value = sum[nt][r];
-          value *= PLANES == 2 ? s_inv[local] : 1024.0f;  // exact: a power of two (s_inv has the 1024 in it)
+          if (PLANES == 2 || !kWhole) value *= PLANES == 2 ? s_inv[local] : 1024.0f;  // exact: a power of two
           if (whole || (m0 + local < m && col < n))
             out[(size_t)(m0 + local) * n + col] = from_f32<T>(value + add);
         }

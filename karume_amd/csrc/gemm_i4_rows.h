@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __res
   const float factor = __uint_as_float(up << 23);
   if (threadIdx.x == 0) {
     scale[2 * (size_t)blockIdx.x] = factor;
-    scale[2 * (size_t)blockIdx.x + 1] = __uint_as_float((down + 10u) << 23);  // (weights are (u - 8) / 1024)
+    scale[2 * (size_t)blockIdx.x + 1] = __uint_as_float(down << 23);
   }
   uint4* dst = planes + (size_t)blockIdx.x * (padded >> 2);
   auto split = [&](uint32_t p, const uint4& va, const uint4& vb) {

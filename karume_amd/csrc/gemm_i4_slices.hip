@@ -156,7 +156,9 @@ struct SliceGeometry {
 // positions among it (kRope).
 constexpr uint32_t kScaleF16 = 1, kIoF16 = 2, kFetches = 4, kRope = 8;
 
-template <int XKIND, int MT, int NT, int STEPS>
+// WHOLE: hi and lo beside f32 scales, totals of whole weights (see scales_whole; a branch beside each group's sums
+// cost fp16 scales 2 to 5 %, this form has the conversion of twelve operations a word).
+template <int XKIND, int MT, int NT, int STEPS, bool WHOLE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_i4_slices_kernel(
     // (the leading 14 dwords of the arguments arrive in scalar registers with the wave)
@@ -374,7 +376,7 @@ void gemm_i4_slices_kernel(
       for (int nt = 0; nt < NT; ++nt) {
         const uint32_t word = j == 0 ? words[nt].x : words[nt].y;
         const half8_t b = XKIND == kXThree ? sixteenths(word)
-                          : XKIND == kXSplit ? ints_paired(word) : ints_natural(word);
+                          : XKIND == kXSplit ? ints_paired<!WHOLE>(word) : ints_natural(word);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -560,7 +562,8 @@ void gemm_i4_slices_kernel(
           for (int wv = 0; wv < kWaves; ++wv) add(v, part[wv]);
         }
         if constexpr (XKIND == kXSplit) {  // exact: a power of two
-          v.x *= inv[i]; v.y *= inv[i]; v.z *= inv[i]; v.w *= inv[i];
+          const float back = WHOLE ? inv[i] : inv[i] * 1024.0f;
+          v.x *= back; v.y *= back; v.z *= back; v.w *= back;
         }
         if constexpr (XKIND != kXSplit) {  // the weights went in as sixteenths or 1024ths
           constexpr float kWhole = XKIND == kXThree ? 16.f : 1024.f;
@@ -596,8 +599,10 @@ int32_t launch_slices(krm_ctx* ctx, const SliceCall& c) {
   uint32_t flags = (c.scale_f16 ? kScaleF16 : 0u) | (c.io_f16 ? kIoF16 : 0u);
   if (c.tail.quads && (c.tail.fuse.mode == 2 || c.tail.bias || c.tail.fuse.residual)) flags |= kFetches;
   if ((flags & kFetches) && c.tail.fuse.mode == 2) flags |= kRope;
-  gemm_i4_slices_kernel<XKIND, MT, NT, STEPS>
-      <<<dim3(((tiles + 7) / 8) * 8), dim3(512), 0, ctx->stream>>>(
+  auto kernel = gemm_i4_slices_kernel<XKIND, MT, NT, STEPS, false>;
+  if constexpr (XKIND == kXSplit)
+    if (!c.scale_f16) kernel = gemm_i4_slices_kernel<XKIND, MT, NT, STEPS, true>;
+  kernel<<<dim3(((tiles + 7) / 8) * 8), dim3(512), 0, ctx->stream>>>(
           static_cast<const uint8_t*>(c.x), static_cast<const uint8_t*>(c.w),
           static_cast<const uint8_t*>(c.scales), c.row_begin, c.row_end, c.n, c.k, c.group_shift,
           m_blocks, tiles, flags, c.m, c.tail);

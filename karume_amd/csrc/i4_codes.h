@@ -60,6 +60,20 @@ __device__ inline void codes_over_1024(uint32_t word, half2_t (&q)[4]) {
   q[2] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, upper & 0x000F000Fu), low, offset);
   q[3] = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, upper & 0x00F000F0u), high, offset);
 }
+// Sums over K that stay 1024 times smaller until their end reach subnormal numbers 1024 times sooner: an fp16 scale
+// or result is far from there, an f32 scale beside an f32 result need not be.  There a group's scale is multiplied
+// by 1024, unless one of the wave's would leave f32's range by that: then (what is returned) its sums are, where they
+// are.
+template <int N>
+__device__ inline bool scales_whole(float (&scale)[N]) {
+  uint64_t past = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) past |= __builtin_amdgcn_ballot_w64(fabsf(scale[i]) >= 0x1p117f);
+  const float factor = past ? 1.0f : 1024.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) scale[i] *= factor;
+  return past != 0;
+}
 // Eight consecutive fp16 activations (x0..x7 in four dwords) regrouped to match
 // codes_to_half2: pair i = (x_i, x_{i+4}).
 __device__ inline void pair_activations(const uint4& raw, half2_t (&p)[4]) {
@@ -69,10 +83,12 @@ __device__ inline void pair_activations(const uint4& raw, half2_t (&p)[4]) {
   p[3] = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(raw.w, raw.y, 0x07060302u));
 }
 
-// The same as one operand of a matrix instruction: (c0,c4,c1,c5,c2,c6,c3,c7), each (u - 8) / 1024.
+// The same as one operand of a matrix instruction: (c0,c4,c1,c5,c2,c6,c3,c7), each (u - 8) / 1024 or (OVER false)
+// whole.
+template <bool OVER>
 __device__ inline half8_t ints_paired(uint32_t word) {
   half2_t q[4];
-  codes_over_1024(word, q);
+  if constexpr (OVER) codes_over_1024(word, q); else codes_to_half2(word, q);
   return half8_t{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
 }
 

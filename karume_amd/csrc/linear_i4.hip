@@ -562,7 +562,7 @@ __global__ __launch_bounds__(KW * 64) void gemv_i4_mfma_tiles_kernel(
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           const uint32_t word = (&own.words[c][s >> 2].x)[s & 3];
-          const half8_t b = ints_paired(word);
+          const half8_t b = ints_paired<true>(word);
           half_sum[s >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fx[c][s], b, half_sum[s >> 2], 0, 0, 0);
         }
 #pragma unroll

@@ -695,3 +695,45 @@ def test_the_residual_of_a_silu_is_read_at_any_element(gpu_ctx, io, m, n, k):
     eps = 2.0 ** -22 if io == ka.F32 else 2.0 ** -10
     want = product + residual.reshape(m, n // 2)
     assert np.all(np.abs(got[0] - want) <= eps * (np.abs(product) + np.abs(want)) + 1e-7)
+
+
+# (exact tiles of hi + lo and of rounded rows, in both group forms; tiles staged through registers; hi + lo of the
+# tiles that split K)
+@pytest.mark.parametrize("m,n,k,g,compute", [
+    (330, 11300, 448, 64, "f32"), (257, 7001, 2048, 128, "f32"), (333, 6001, 4992, 64, "f16"),
+    (348, 8164, 4608, 128, "f16"), (338, 18849, 1280, 128, "f16"), (330, 20011, 448, 64, "f16"),
+    (50, 96, 576, 64, "f32"), (33, 64, 512, 128, "f32"), (128, 2048, 1024, 64, "f32")])
+def test_f32_scales_keep_their_range(gpu_ctx, m, n, k, g, compute):
+    """Whole numbers in x and one f32 scale of 2^-145 for all codes: every sum is a whole number of them below 2^24
+    on the way, and so is the result, a subnormal or small normal f32, exactly.  (Totals kept 1024 times smaller
+    until their end would lose their last bits.)"""
+    rng = np.random.default_rng(m + n + k)
+    packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    scale = np.full((n, k // g), 2.0 ** -145, dtype=np.float32)
+    top = 1800 if compute == "f16" else 7000     # exact in fp16, in hi + lo
+    x = rng.integers(-top, top + 1, size=(m, k)).astype(np.float32)
+    got = run_linear(gpu_ctx, x, packed, scale, None, n, k, g,
+                     compute=ka.COMPUTE_F16 if compute == "f16" else ka.COMPUTE_F32)
+    cols = np.unique(np.concatenate([rng.choice(n, size=64), [0, n // 2, n - 1]]))
+    q = np.stack([packed[cols] & 15, packed[cols] >> 4], axis=2).reshape(len(cols), k).astype(np.float64) - 8
+    want = x.astype(np.float64) @ q.T
+    assert np.abs(want).max() < 2 ** 23
+    assert np.array_equal(got[:, cols].astype(np.float64) * 2.0 ** 145, want)
+
+
+@pytest.mark.parametrize("m,n,k,g", [(333, 6001, 4992, 64), (348, 8164, 4608, 128), (338, 18849, 1280, 128),
+                                     (330, 20011, 448, 64)])
+def test_f32_scales_of_both_ends_of_their_range(gpu_ctx, m, n, k, g):
+    """f32 rows rounded to fp16, columns with a scale of 2^118 beside columns with one of 2^-130, codes of zero in some
+    groups: whole numbers of a thousandth of the scale, exactly."""
+    rng = np.random.default_rng(m + n + k)
+    packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    packed[:, g // 2:g] = 0x88
+    scale = np.full((n, k // g), 2.0 ** 118, dtype=np.float32)
+    scale[1::2] = 2.0 ** -130
+    x = rng.integers(-60, 61, size=(m, k)).astype(np.float32) * np.float32(2.0 ** -10)
+    got = run_linear(gpu_ctx, x, packed, scale, None, n, k, g, compute=ka.COMPUTE_F16)
+    cols = np.unique(np.concatenate([rng.choice(n, size=64), [0, 1, n // 2, n - 2, n - 1]]))
+    q = np.stack([packed[cols] & 15, packed[cols] >> 4], axis=2).reshape(len(cols), k).astype(np.float64) - 8
+    want = (x.astype(np.float64) @ q.T) * scale[cols, 0].astype(np.float64)
+    assert np.abs(want).max() < 2.0 ** 127 and np.array_equal(got[:, cols].astype(np.float64), want)
