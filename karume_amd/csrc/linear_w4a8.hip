@@ -53,9 +53,9 @@ __device__ inline bool is_nan_bits(float v) {
 // quotients.  Rows of up to THREADS * 4 * HELD elements stay in registers between the two
 // (one trip to memory, all loads in flight together); longer rows are read twice.  x / s is the
 // correctly rounded f32 division, so the codes equal the CPU formula's for every input, also
-// next to a rounding tie.  Threads as many as leave each one to three quads: the quotients of a row are a
+// next to a rounding tie.  Threads as many as leave each a few quads: the quotients of a row are a
 // chain of one workgroup.  us with 256 threads of up to twelve quads / so: 512 x 4096 4.5 / 4.1, 512 x 11008 7.9 / 6.7, 128 x
-// 5632 4.4 / 3.7, 16 x 4096 3.6 / 3.0, 9 x 1024 2.6 / 2.35, 512 x 16384 14.4 / 9.5.
+// 5632 4.4 / 3.6, 16 x 4096 3.6 / 3.0, 9 x 1024 2.6 / 2.35, 512 x 16384 14.4 / 9.5.
 
 // x / s must be the correctly rounded quotient only where it decides the code: t = x * (1 / s)
 // (1 / s correctly rounded) lies within 2.3e-5 of it for |x / s| <= 127.5, so when t is further
@@ -1042,7 +1042,13 @@ extern "C" int32_t krm_quantize_rows(krm_ctx* ctx, krm_buf x, krm_buf xq, krm_bu
   if (dim <= 1024) launch(quantize_rows_kernel<256, 1>, 256);
   else if (dim <= 2048) launch(quantize_rows_kernel<512, 1>, 512);
   else if (dim <= 4096) launch(quantize_rows_kernel<512, 2>, 512);
-  else if (dim <= 8192) launch(quantize_rows_kernel<1024, 2>, 1024);
+  // (sixteen waves to a row have a place on a CU twice, and where few of a thread's quads are in the row they are
+  // there for little.  us with 1024 threads / so: 8192 x 4352 48.8 / 31.7, 2048 x 5632 16.2 / 13.1, 512 x 6144 5.5 / 4.9,
+  // 1 x 4352 3.45 / 3.33, 8192 x 8192 67.9 / 60.3, 512 x 8192 6.1 / 5.6, 1 x 8192 3.89 / 3.89; 8192 x 8448 74.0 / 67.0, 512 x
+  // 10240 6.65 / 6.35, but 256 x 10240 4.85 / 5.05, 2048 x 11008 22.4 / 23.2)
+  else if (dim <= 6144) launch(quantize_rows_kernel<512, 3>, 512);
+  else if (dim <= 8192) launch(quantize_rows_kernel<512, 4>, 512);
+  else if (dim <= 10240 && rows > 256) launch(quantize_rows_kernel<512, 6>, 512);
   else launch(quantize_rows_kernel<1024, 3>, 1024);
   return krm::launched(ctx, "quantize_rows_kernel");
 }

@@ -84,6 +84,18 @@ def test_quantize_at_the_lengths_kept_in_registers(gpu_ctx, dim):
     assert_exact(q, want_q, "codes")
 
 
+@pytest.mark.parametrize("rows", [3, 257])
+@pytest.mark.parametrize("dim", [6144, 6148, 10240, 10244])
+def test_quantize_where_threads_hold_three_to_six_quads(gpu_ctx, dim, rows):
+    """Rows at the edges of those forms, one of which many rows take: the largest magnitude in the last quad."""
+    x = np.random.default_rng(dim + rows).normal(size=(rows, dim)).astype(np.float32)
+    x[1::2, dim - 1] = 50
+    q, s = run_quantize(gpu_ctx, x)
+    want_q, want_s = oracle.quantize_rows(x, dim)
+    assert_exact(s, want_s, "scale")
+    assert_exact(q, want_q, "codes")
+
+
 def test_quantize_propagates_nan_and_inf_to_the_row_scale(gpu_ctx):
     rows, dim = 4, 8
     x = helpers.seeded(rows * dim, helpers.SIGNED_A8).reshape(rows, dim)

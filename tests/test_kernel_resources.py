@@ -44,6 +44,12 @@ def test_w4a8_groups_of_64_and_128_have_tiles_for_any_k(kernels):
     assert tiles == {("6", "1")} | {(group, wide) for group in ("7", "8", "0") for wide in ("1", "2")}
 
 
+def test_rows_to_quantize_have_threads_by_their_length(kernels):
+    """A thread has up to three quads more than it needs: not sixteen waves for rows that eight hold."""
+    forms = {tuple(int(a.rstrip("u")) for a in arguments(n)) for n in kernels if n.startswith("quantize_rows_kernel<")}
+    assert forms == {(256, 1), (512, 1), (512, 2), (512, 3), (512, 4), (512, 6), (1024, 3)}
+
+
 # The forms that spill: the large f32-activation forms of the GEMM on fp16 weights (f32 x is rounded in the
 # loop, beside a 64 x 64 tile a wave).
 SPILL = ("gemm_i4_f16_kernel<float, __half, 2, 2, 64, 1, 4, true,",
