@@ -43,6 +43,11 @@ def test_rms_norm_at_the_lengths_kept_in_registers(gpu_ctx, dim):
         b.free()
 
 
+@pytest.mark.parametrize("dim", [3072, 3073, 6144, 6145, 8192, 8193])
+def test_rms_norm_at_the_lengths_of_12_24_and_32_pieces(gpu_ctx, dim):
+    test_rms_norm_at_the_lengths_kept_in_registers(gpu_ctx, dim)
+
+
 def test_rope_silu_add_embedding_argmax(gpu_ctx):
     rng = np.random.default_rng(1)
     rows, heads, d, table = 5, 3, 8, 16

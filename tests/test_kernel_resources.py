@@ -50,6 +50,13 @@ def test_rows_to_quantize_have_threads_by_their_length(kernels):
     assert forms == {(256, 1), (512, 1), (512, 2), (512, 3), (512, 4), (512, 6), (1024, 3)}
 
 
+def test_norms_read_at_most_half_as_much_again_as_a_row_has(kernels):
+    """Pieces past a row are loads all the same: forms for rows of up to 4, 8, 12, 16, 24, 32 and 48 pieces."""
+    forms = {tuple(arguments(n)) for n in kernels if n.startswith("rms_norm_kernel<")}
+    types = (("float", "float"), ("__half", "__half"), ("float", "__half"))
+    assert forms == {(*t, kept) for t in types for kept in ("0", "4", "8", "12", "16", "24", "32", "48")}
+
+
 # The forms that spill: the large f32-activation forms of the GEMM on fp16 weights (f32 x is rounded in the
 # loop, beside a 64 x 64 tile a wave).
 SPILL = ("gemm_i4_f16_kernel<float, __half, 2, 2, 64, 1, 4, true,",
