@@ -1046,6 +1046,7 @@ struct DecodeArgs {
   uint32_t splits;           // that the grid and the workspace are sized for
   uint32_t units;            // kv heads * head_groups
   uint32_t folded;           // the grid is (8 units, splits / 8, batch), else (splits, units, batch)
+  uint32_t rest_batch, rest_head;  // folded: first XCD of the last splits, a batch entry and a kv head
 };
 
 // Columns are walked in chunks of kDecodeIter * G rows (G = 256 / lanes-per-row groups, each
@@ -1135,7 +1136,10 @@ void attention_decode_kernel(
   // splits) 8.71 / 8.48.
   const uint32_t unit = a.folded ? blockIdx.x >> 3 : blockIdx.y;
   const uint32_t hk = unit / a.head_groups;
-  const uint32_t at_split = a.folded ? blockIdx.y * 8u + ((blockIdx.x - hk) & 7u) : blockIdx.x;
+  // Each kv head's splits begin on the XCD behind the one before it; the last ones, fewer than eight, begin behind the
+  // last one of the head before, or some XCDs would have up to one more of every head.
+  const uint32_t first_xcd = blockIdx.y == a.splits >> 3 ? blockIdx.z * a.rest_batch + hk * a.rest_head : hk;
+  const uint32_t at_split = a.folded ? blockIdx.y * 8u + ((blockIdx.x - first_xcd) & 7u) : blockIdx.x;
   const uint32_t head0 = hk * a.repeat + (unit - hk * a.head_groups) * R;  // first head
 
   // The rows of a chunk as they arrive: K pieces (row-owner layout, or the MFMA A-operand
@@ -1777,6 +1781,10 @@ int32_t decode_dispatch(krm_ctx* ctx, DecodeLaunch& L, uint32_t repeat, uint32_t
   L.args.units = L.args.kv_heads * L.args.head_groups;
   // (one split: the head groups lie on neighbouring XCDs, and seven of eight workgroups of the other grid had no work)
   L.args.folded = L.grid_x > 1 && L.args.head_groups > 1 && (L.grid_x + 7) / 8 <= 65535 ? 1u : 0u;
+  // (eight kv heads share the XCDs evenly whatever the splits)
+  const bool even = L.args.kv_heads % 8 == 0;
+  L.args.rest_head = even ? 1u : L.grid_x % 8;
+  L.args.rest_batch = even ? 0u : L.args.kv_heads * (L.grid_x % 8);
   const uint64_t counters = (uint64_t)L.args.nseq * L.args.kv_heads * L.args.head_groups;
   if ((uint64_t)L.args.kv_heads * L.args.head_groups > 65535 || counters > L.ticket_slots)
     return fail(ctx, KRM_ERR_VALIDATION, "decode attention: B * H = %llu exceeds %u",

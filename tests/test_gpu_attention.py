@@ -683,6 +683,13 @@ def test_decode_of_splits_that_share_rows_on_an_xcd(gpu_ctx, batch, heads, kv_he
     assert ok, (fails, max_abs, worst)
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,depth,past", [(4, 12, 3, 128, 620), (3, 8, 2, 128, 1300),
+                                                             (3, 32, 4, 64, 1200), (2, 32, 8, 128, 700)])
+def test_decode_deals_the_last_splits_of_a_batch_over_all_xcds(gpu_ctx, batch, heads, kv_heads, depth, past):
+    """The folded grid's last row, which begins on another XCD for every batch entry and kv head."""
+    test_decode_of_splits_that_share_rows_on_an_xcd(gpu_ctx, batch, heads, kv_heads, depth, past, 0)
+
+
 @pytest.mark.parametrize("nseq", [1, 62, 63, 64, 65, 127, 128, 300])
 def test_varlen_plan_tables_past_a_wave(gpu_ctx, nseq):
     """The tables of a plan, by steps of 64 sequences: offsets as given, splits of 128 columns summed before each
