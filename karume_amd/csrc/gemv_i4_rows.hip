@@ -395,15 +395,16 @@ namespace krm {
 // 2 rows: where the one-row kernel's form is the slower one.  us there / here: f32 1093 x 1920 5.4 / 4.1, 4806 x 1152
 // 6.4 / 5.2, 7309 x 2560 8.4 / 7.7, 32000 x 4096 27.5 / 23.7, 1300 x 1024 4.2 / 3.9, but 1100 x 512 3.6 / 3.7, 701 x 576
 // 3.0 / 3.8, 1945 x 3328 4.8 / 5.3, 4096 x 4096 6.42 / 6.44; fp16 548 x 8064 4.6 / 5.9, 6085 x 3840 6.9 / 7.2.  3 fp16 rows
-// 422 x 2496 4.2 / 4.8, 3032 x 704 4.4 / 4.0.  3 f32 rows and 4 rows of either, all faster here: 4 rows 1955 x 3968 fp16
-// 6.3 / 5.2, 3 rows 428 x 4480 f32 6.7 / 6.1.
+// 422 x 2496 4.2 / 4.8, 2040 x 768 4.4 / 4.7, 1114 x 2016 4.9 / 4.5, 2453 x 544 5.1 / 4.7, 1977 x 3200 6.4 / 5.75, 3032
+// x 704 4.4 / 4.0.  4 fp16 rows 388 x 2208 4.5 / 5.2, 700 x 5632 5.75 / 6.2, 1000 x 1024 3.94 / 4.3, 1455 x 640 4.37 /
+// 4.69, 1932 x 512 4.44 / 4.30, 1740 x 1408 4.76 / 4.87, 1741 x 1600 4.92 / 4.74, 2152 x 640 5.4 / 5.0, 1955 x 3968 6.3 / 5.2.  3 f32 rows and more, all faster here: 428 x 4480 6.7 / 6.1.
 int32_t linear_i4_gemv_rows(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias, krm_buf out, uint32_t m,
                             uint32_t n, uint32_t k, uint32_t group, int32_t io_dtype, int32_t scale_dtype, bool* handled) {
   const bool f32 = io_dtype == KRM_F32;
   *handled = false;
   if (m < 2 || m > 16 || k % kSegment || group < kSegment || !aligned(w, 16)) return KRM_OK;
   if (m == 2 && (!f32 || n < (k < 2048 ? 1024u : 6144u) || (uint64_t)n * k < 1250000)) return KRM_OK;
-  if (m == 3 && !f32 && n < 1024) return KRM_OK;
+  if (!f32 && m <= 4 && (n < 1024 || (n < 2048 && k > 512 && k <= 1536))) return KRM_OK;
   if ((uint64_t)kWave * k > 0x7fffffffull || n > 0x7fffffffu / 16) return KRM_OK;  // offsets of 32 bits
   *handled = true;
   if (f32)
