@@ -2184,18 +2184,22 @@ __global__ __launch_bounds__(kWave) void varlen_plan_kernel(const int32_t* __res
     const bool ascending = lo >= 0 && hi >= lo;
     ok = ok && ascending;
     const uint32_t own = i < nseq && ascending ? decode_splits((uint64_t)(hi - lo), chunk_columns) : 0u;
+    // Sums through each lane: within rows of 16 lanes, then of the row before into odd rows, of the lower half into
+    // the upper one (operands of the vector ALU; six shuffles through LDS were 0.3 us of a plan and the attention
+    // behind it).
     uint32_t through = own;
-#pragma unroll
-    for (int step = 1; step < kWave; step *= 2) {
-      const uint32_t other = __shfl_up(through, step);
-      if ((int)lane >= step) through += other;
-    }
+    through += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)through, 0x111, 0xf, 0xf, false);  // row_shr:1
+    through += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)through, 0x112, 0xf, 0xf, false);
+    through += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)through, 0x114, 0xf, 0xf, false);
+    through += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)through, 0x118, 0xf, 0xf, false);
+    through += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)through, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    through += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)through, 0x143, 0xc, 0xf, false);  // row_bcast:31
     if (i <= nseq) {
       cu[i] = lo;
       prefix[i] = (int32_t)(before + through - own);
       if (i == nseq) ok = ok && (uint64_t)lo <= total_rows;
     }
-    before += (uint32_t)__shfl(through, kWave - 1);
+    before += (uint32_t)__builtin_amdgcn_readlane((int)through, kWave - 1);
   }
   ok = __all(ok) && before <= max_splits;
   if (!ok)  // no workgroup of the attention launch finds a split: nothing is read or written
