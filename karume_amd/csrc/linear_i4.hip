@@ -1193,9 +1193,10 @@ template <typename XT, typename ST, int MB, int ROWS, int VEC>
 int32_t pick_steps(krm_ctx* ctx, krm_buf x, krm_buf w, krm_buf scales, krm_buf bias, krm_buf out,
                    uint32_t m, uint32_t n, uint32_t k, uint32_t group_shift,
                    const GemvFusion& fuse) {
-  // 2 to 8 rows of f32 x over a step of K and more: through LDS.  (A K below a step leaves most lanes of
-  // the staging idle: 7 rows 12116 x 960 31 us, 38 staged; sixteen rows' sums beside it spill: 13 rows
-  // 8614 x 8960 322 us, 951.  fp16 x has half the lines: 4 rows 422 x 2496 6.4 us, 6.6.)
+  // 2 to 8 rows of f32 x over a step of K and more, with a residual or silu behind them or not dealt (gemv_i4_rows_plan.h):
+  // through LDS.  (Measured on plain rows, when all came here: a K below a step leaves most lanes of the staging
+  // idle, 7 rows 12116 x 960 31 us, 38 staged; sixteen rows' sums beside it spill, 13 rows 8614 x 8960 322 us, 951;
+  // fp16 x has half the lines, 4 rows 422 x 2496 6.4 us, 6.6.)
   if constexpr (VEC == 4 && MB > 1 && MB <= 8 && sizeof(XT) == 4)
     if (k >= 2048 && !fuse.norm_weight && !fuse.positions)
       return launch_gemv<XT, ST, MB, ROWS, VEC, kStagedRows>(ctx, x, w, scales, bias, out, m, n, k, group_shift, fuse);

@@ -301,3 +301,22 @@ def make_w4a8(case: W4a8Case, x_value=None):
     fn = (lambda i: x_value(i, case.m, case.k)) if x_value else SIGNED_A8
     x = seeded(case.m * case.k, fn).reshape(case.m, case.k)
     return x, packed, q, scale, bias
+
+
+# 2 to 16 rows of x, dealt by karume_amd/csrc/gemv_i4_rows_plan.h: bytes of an x, of a scale, m, n, k, group of a small
+# product for every form (SPAN, R, deal) that a size up to 32000 x 11008 takes, past one step of K where it can be.
+DEALT_ROWS = [
+    (2, 4, 16, 1539, 32, 32), (2, 2, 15, 1638, 2112, 64), (2, 4, 9, 19701, 32, 32), (2, 2, 9, 4111, 2176, 128),
+    (2, 4, 9, 8215, 2176, 128), (2, 4, 16, 14353, 32, 32), (2, 2, 16, 2085, 2112, 32),
+    (2, 2, 14, 8243, 2112, 64), (2, 4, 10, 16563, 160, 32), (2, 2, 10, 5472, 2112, 64),
+    (2, 4, 10, 11088, 2112, 64), (2, 4, 12, 16461, 160, 32), (2, 2, 12, 5500, 2176, 128),
+    (2, 4, 11, 11053, 2112, 64), (2, 4, 16, 4146, 544, 32), (2, 4, 16, 4126, 2144, 32),
+    (2, 2, 16, 12532, 2112, 64), (2, 2, 5, 33, 2144, 32), (2, 2, 16, 259, 3104, 32), (2, 2, 16, 516, 3200, 64),
+    (2, 4, 16, 702, 3712, 128), (2, 4, 15, 1656, 2240, 64), (4, 4, 16, 1794, 32, 32),
+    (4, 4, 15, 1032, 2112, 32), (4, 2, 2, 16600, 2112, 64), (4, 4, 9, 19678, 32, 32), (4, 2, 9, 3287, 2112, 64),
+    (4, 2, 9, 8208, 2176, 128), (4, 2, 16, 14342, 32, 32), (4, 4, 15, 2058, 2112, 64),
+    (4, 4, 11, 8216, 2112, 64), (4, 4, 10, 17297, 160, 32), (4, 4, 9, 5450, 2176, 32),
+    (4, 4, 9, 10913, 2112, 64), (4, 2, 11, 16436, 160, 32), (4, 2, 11, 5588, 2112, 64),
+    (4, 4, 11, 10894, 2112, 32), (4, 2, 16, 4120, 544, 32), (4, 4, 15, 4108, 2176, 64),
+    (4, 4, 16, 12405, 2112, 64), (4, 2, 3, 33, 2144, 32), (4, 2, 16, 260, 3616, 32), (4, 4, 16, 517, 3136, 64),
+    (4, 2, 16, 693, 3680, 32), (4, 2, 15, 1025, 2432, 128)]

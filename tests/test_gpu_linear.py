@@ -426,8 +426,9 @@ def test_few_fp16_rows_have_the_same_bits_in_every_batch(gpu_ctx, n, k, g, scale
                                    (2100, 2176, 128)])
 @pytest.mark.parametrize("scale_type", [np.float16, np.float32])
 def test_several_f32_rows_brought_to_lds_have_the_bits_of_one_row(gpu_ctx, n, k, g, scale_type):
-    """2 to 8 rows of f32 x over a K of a step and more: the bits of a row alone (K of one step, of a
-    last step that is nearly empty; blocks of rows that are cut off; rows of N past the last)."""
+    """2 to 8 rows of f32 x over a K of a step and more, from 3 rows on dealt, 2 by shape: the bits of a row alone (K of
+    one step, of a last step that is nearly empty; blocks of rows that are cut off; rows of N past the last).  (Rows
+    brought to LDS: 2 of them here, and what follows a fusion below.)"""
     rng = np.random.default_rng(n * 3 + k)
     packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
     scale = scale.astype(scale_type)
@@ -445,10 +446,43 @@ def test_several_f32_rows_brought_to_lds_have_the_bits_of_one_row(gpu_ctx, n, k,
                 assert np.array_equal(got[r].view(np.uint32), alone[r].view(np.uint32)), (m, r)
 
 
+@pytest.mark.parametrize("scale_type", [np.float16, np.float32])
+@pytest.mark.parametrize("n,k,g", [(66, 2048, 64), (130, 2080, 32), (2100, 2176, 128), (38, 6272, 128)])
+@pytest.mark.parametrize("silu", [False, True])
+def test_several_f32_rows_of_a_fusion_have_the_bits_of_one_row(gpu_ctx, silu, n, k, g, scale_type):
+    """2 to 16 rows of f32 x over a K of a step and more with a residual or silu pairs behind them (blocks of 2, 4 and 8
+    rows brought to LDS, 9 and more not): the bits of the same call on a row alone, an infinity in its row only."""
+    rng = np.random.default_rng(n + k)
+    packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
+    scale = scale.astype(scale_type)
+    n_out = n // 2 if silu else n
+    x = rng.normal(size=(16, k)).astype(np.float32)
+    x[2, 5] = np.inf
+    residual, bias = rng.normal(size=(16, n_out)).astype(np.float32), rng.normal(size=n).astype(np.float32)
+    bufs = [gpu_ctx.upload(a) for a in (x, packed, scale, residual, bias)]
+    dx, dw, ds, dr, db = bufs
+    out = gpu_ctx.alloc(16 * n_out * 4)
+
+    def run(first, m):
+        gpu_ctx.linear_i4_fused(dx.offset(first * k * 4), dw, ds, out, m, n, k, g, bias=db,
+                                residual=None if silu else dr.offset(first * n_out * 4), scale_dtype=ka.dtype_code(scale.dtype),
+                                epilogue=ka.EPILOGUE_SILU_PAIRS if silu else ka.EPILOGUE_NONE)
+        return out.download(np.float32, (m, n_out))
+
+    alone = np.concatenate([run(r, 1) for r in range(16)])
+    assert np.isfinite(np.delete(alone, 2, axis=0)).all()
+    for m in (2, 3, 4, 5, 8, 9, 16):
+        got = run(0, m)
+        same = (got.view(np.uint32) == alone[:m].view(np.uint32)) | (np.isnan(got) & np.isnan(alone[:m]))
+        assert same.all(), (m, np.argwhere(~same)[:3])
+    for b in bufs + [out]:
+        b.free()
+
+
 @pytest.mark.parametrize("n,k,g", [(70, 1152, 32), (300, 2048, 64), (1000, 4160, 64), (33, 8320, 128)])
 @pytest.mark.parametrize("m", [9, 12, 13, 16])
 def test_nine_to_sixteen_f32_rows_have_the_bits_of_one_row(gpu_ctx, n, k, g, m):
-    """One launch of sixteen rows or two of eight and the rest: the bits of a row alone."""
+    """Nine rows and more, which are dealt: the bits of a row alone."""
     rng = np.random.default_rng(n + k + m)
     packed, _q, scale = helpers.synthetic_int4(rng, n, k, g)
     x = rng.normal(size=(m, k)).astype(np.float32)
@@ -521,9 +555,9 @@ def test_scales_of_a_share_read_together(gpu_ctx, m, n, k, scale_type):
     (9000, 1088, 64, np.float32, 0), (17, 8256, 64, np.float16, 0), (64, 6272, 128, np.float32, 1),
     (20, 65536, 32, np.float32, 0), (1, 1152, 32, np.float16, 0)])
 def test_dealt_rows_have_the_bits_of_one_row_alone(gpu_ctx, dtype, n, k, g, scale_type, offset):
-    """2 to 16 rows in every form they are dealt in (a wave has 64 or 16 rows of W, 1 to 8 of x, one to four quads of
-    segments): K of one segment, of a part of a quad, of a step and past it; N off the tile; scales that are not
-    aligned, or too many for LDS.  Bits of each row alone, also where x has infinities, zeros and subnormals."""
+    """2 to 16 rows at the edges of what they are dealt by: K of one segment, of a part of a quad, of a step and past
+    it; N off the tile; scales that are not aligned, or too many for LDS.  Bits of each row alone, also where x has
+    infinities, zeros and subnormals.  (The forms: the test below.)"""
     rng = np.random.default_rng(n + k)
     packed = rng.integers(0, 2**32, size=n * k // 8, dtype=np.uint32)
     scale = (rng.random(size=n * (k // g) + offset) * .02 + .001).astype(scale_type)
@@ -550,4 +584,30 @@ def test_dealt_rows_have_the_bits_of_one_row_alone(gpu_ctx, dtype, n, k, g, scal
         same = (got == alone[:m]) | (np.isnan(got) & np.isnan(alone[:m]))
         assert same.all() and (np.signbit(got) == np.signbit(alone[:m]))[~np.isnan(got)].all(), m
     for b in (d_w, d_s, d_b):
+        b.free()
+
+
+@pytest.mark.parametrize("x_size,scale_size,m,n,k,g", helpers.DEALT_ROWS)
+def test_every_form_of_dealt_rows_has_the_bits_of_one_row_alone(gpu_ctx, x_size, scale_size, m, n, k, g):
+    """64 or 16 rows of W a wave, 1 to 8 of x, one, two or four quads of segments in turn (test_rows_plan.py holds the
+    list against the plan); infinities and subnormals stay in their rows."""
+    dtype, scale_type = (np.float32 if b == 4 else np.float16 for b in (x_size, scale_size))
+    rng = np.random.default_rng(m + n + k)
+    packed = rng.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
+    scale = (rng.random(size=(n, k // g)) * .02 + .001).astype(scale_type)
+    bias = rng.normal(size=n).astype(dtype)
+    x = rng.normal(size=(m, k)).astype(dtype)
+    x[0] *= dtype(1e-7 if x_size == 2 else 1e-42)
+    x[m - 1, k // 2] = np.inf
+    dw, ds, db, dx = (gpu_ctx.upload(a) for a in (packed, scale, bias, x))
+    out = gpu_ctx.alloc(m * n * x_size)
+    io, sd = ka.dtype_code(np.dtype(dtype)), ka.dtype_code(np.dtype(scale_type))
+    gpu_ctx.linear_i4(dx, dw, ds, db, out, m, n, k, g, io, sd)
+    got = out.download(dtype, (m, n))
+    for r in range(m):
+        gpu_ctx.linear_i4(dx.offset(r * k * x_size), dw, ds, db, out, 1, n, k, g, io, sd)
+        alone = out.download(dtype, (n,))
+        same = (got[r] == alone) & (np.signbit(got[r]) == np.signbit(alone))
+        assert (same | (np.isnan(got[r]) & np.isnan(alone))).all(), r
+    for b in (dw, ds, db, dx, out):
         b.free()
