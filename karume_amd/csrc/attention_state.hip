@@ -1045,8 +1045,9 @@ struct DecodeArgs {
   uint32_t capacity;         // single sequence: slot rows (checked against device lengths)
   uint32_t splits;           // that the grid and the workspace are sized for
   uint32_t units;            // kv heads * head_groups
-  uint32_t folded;           // the grid is (8 units, splits / 8, batch), else (splits, units, batch)
-  uint32_t rest_batch, rest_head;  // folded: first XCD of the last splits, a batch entry and a kv head
+  // Not 0: the grid is (8 units, splits / 8, batch), else (splits, units, batch).  Bits 4 and 8: XCDs by which the last
+  // splits of a kv head and of a batch entry begin behind those of the one before.
+  uint32_t folded;
 };
 
 // Columns are walked in chunks of kDecodeIter * G rows (G = 256 / lanes-per-row groups, each
@@ -1138,8 +1139,12 @@ void attention_decode_kernel(
   const uint32_t hk = unit / a.head_groups;
   // Each kv head's splits begin on the XCD behind the one before it; the last ones, fewer than eight, begin behind the
   // last one of the head before, or some XCDs would have up to one more of every head.
-  const uint32_t first_xcd = blockIdx.y == a.splits >> 3 ? blockIdx.z * a.rest_batch + hk * a.rest_head : hk;
-  const uint32_t at_split = a.folded ? blockIdx.y * 8u + ((blockIdx.x - first_xcd) & 7u) : blockIdx.x;
+  uint32_t at_split = blockIdx.x;
+  if (a.folded) {
+    const uint32_t first_xcd =
+        blockIdx.y == a.splits >> 3 ? blockIdx.z * (a.folded >> 8) + hk * (a.folded >> 4) : hk;  // (modulo eight)
+    at_split = blockIdx.y * 8u + ((blockIdx.x - first_xcd) & 7u);
+  }
   const uint32_t head0 = hk * a.repeat + (unit - hk * a.head_groups) * R;  // first head
 
   // The rows of a chunk as they arrive: K pieces (row-owner layout, or the MFMA A-operand
@@ -1780,11 +1785,12 @@ int32_t decode_dispatch(krm_ctx* ctx, DecodeLaunch& L, uint32_t repeat, uint32_t
   L.args.splits = L.grid_x;
   L.args.units = L.args.kv_heads * L.args.head_groups;
   // (one split: the head groups lie on neighbouring XCDs, and seven of eight workgroups of the other grid had no work)
-  L.args.folded = L.grid_x > 1 && L.args.head_groups > 1 && (L.grid_x + 7) / 8 <= 65535 ? 1u : 0u;
   // (eight kv heads share the XCDs evenly whatever the splits)
   const bool even = L.args.kv_heads % 8 == 0;
-  L.args.rest_head = even ? 1u : L.grid_x % 8;
-  L.args.rest_batch = even ? 0u : L.args.kv_heads * (L.grid_x % 8);
+  const uint32_t rest = L.grid_x % 8, behind_head = even ? 1u : rest, behind_batch = even ? 0u : L.args.kv_heads * rest % 8;
+  L.args.folded = L.grid_x > 1 && L.args.head_groups > 1 && (L.grid_x + 7) / 8 <= 65535
+                      ? 1u | behind_head << 4 | behind_batch << 8
+                      : 0u;
   const uint64_t counters = (uint64_t)L.args.nseq * L.args.kv_heads * L.args.head_groups;
   if ((uint64_t)L.args.kv_heads * L.args.head_groups > 65535 || counters > L.ticket_slots)
     return fail(ctx, KRM_ERR_VALIDATION, "decode attention: B * H = %llu exceeds %u",
