@@ -134,9 +134,10 @@ int32_t krm_graph_begin(krm_ctx* ctx);
  * main branch; while a side branch is selected they fail with KRM_ERR_VALIDATION and record
  * nothing: the decode attention when it splits the columns (more than four chunks),
  * krm_attention_varlen / _planned and every f32-class (KRM_COMPUTE_F32 with f32 x) MFMA product in
- * groups of 64 and more.  krm_linear_i4 of fp16 operands whose large products share tiles through
- * that scratch on the main branch takes the form without it on a side branch: the same class of
- * result, other bits for more than six 32 x 32 tiles of output a CU.  GEMVs (m <= 16), the fp16-operand
+ * groups of 64 and more.  krm_linear_i4 of fp16 x, or of f32 x under KRM_COMPUTE_F16, uses that
+ * scratch on the main branch only (large products share tiles through it; f32 rows may be rounded
+ * into it by a launch of their own) and takes the forms without it on a side branch: the same class
+ * of result, other bits for more than six 32 x 32 tiles of output a CU.  GEMVs (m <= 16), the fp16-operand
  * few-row products, krm_attention_state_noalloc (its own scratch: still one call at a time per
  * GPU) and the glue ops carry no such state. */
 int32_t krm_graph_branch(krm_ctx* ctx, uint32_t branch);
@@ -163,7 +164,9 @@ int32_t krm_dequant_i4(krm_ctx* ctx, krm_buf w, krm_buf scales, krm_buf out_f32,
  *   bias   [n]     io_dtype, or 0 for "no bias" (the reference always binds one; zeros)
  *   out    [m, n]  io_dtype
  * group must be a power of two >= 16 dividing k (docs/ir-v1.md:135-150).
- * The kernel is a pure function of (m, n, k, group, dtypes, compute); for m <= 16 a row of
+ * The kernel is a pure function of (m, n, k, group, dtypes, compute) on the main branch; for m > 16 a row
+ * of `out` may have other bits beside other rows (the form that a shape takes orders its sums, in groups
+ * of 64 and more past six 32 x 32 tiles of output a CU); for m <= 16 a row of
  * `out` does not depend on the other rows in the call (same reduction order for every m; but fp16
  * rows in groups of 128 and more with k a multiple of 256 have one order in batches of 2 to 16 and
  * another alone, which agree to the rounding of the fp16 result). */

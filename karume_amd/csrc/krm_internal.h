@@ -26,10 +26,12 @@ struct krm_ctx {
   // Scratch of the unit-dealt GEMM: two 128 x 256 f32 partials per CU (64 MiB on 256 CUs),
   // allocated with the context so that launches can be recorded into graphs.
   float* gemm_partials = nullptr;
-  // Per-row scales {2^e, 2^-e} of the f32-class prefill GEMM (kMaxSplitRows rows), written by
+  // Per-row scales {2^e, 2^-e} of the f32-class GEMMs with hi and lo planes (kMaxSplitRows rows), written by
   // a pre-pass of every such launch.
   float* row_scales = nullptr;
-  // fp16 planes of f32 activations, written by a pre-pass of every unit-dealt GEMM (kPlaneBytes).
+  // f32 activations in fp16, written by a launch in front of the product (kPlaneBytes): hi and lo planes for the
+  // unit-dealt GEMM of the f32 class, rounded rows for the products under KRM_COMPUTE_F16 that gain by it (unit-dealt and
+  // K-splitting).
   void* x_planes = nullptr;
   bool recording = false;  // between krm_graph_begin and krm_graph_end
   // Parallel branches of a recording (krm_graph_branch): `stream` is the stream launches go

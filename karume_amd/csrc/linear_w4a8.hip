@@ -679,9 +679,9 @@ void linear_w4a8_tile_kernel(
 // ahead, a stage of 512 x 11008 x 4096 took 2283 clk: 281 to ask for the next one, 640 of products, 1218 of
 // waiting for it (a scale a lane touched 64 lines: 445 of them) and parking it, 143 at the barrier.  Now
 // 1551: 299, 1139, 45, 68.  us with the quantiser's launch, before / now, fp16 scales unless noted: 512 x 11008 x
-// 4096 51.4 / 46.6 (45.9 with the quantiser's threads by length), in groups of 64 60.6 / 55.0, of 32 105 / 83, with f32 scales (whose quotient by 16 was
-// tested in every group) 56.8 / 47.9; 2048 x 11008 x 4096 166 / 157; 20 x 20000 x 1024 in groups of 32 18.2 / 15.1;
-// 500 x 600 x 8000 in groups of 32, f32 scales 112 / 72.
+// 4096 49.0 / 43.4 among other calls, in a replay of its own 56.6 / 50.1, there in groups of 64 67.3 / 59.3, of 32 112 /
+// 89, with f32 scales (whose quotient by 16 was tested in every group) 62.6 / 51.1; 2048 x 11008 x 4096 166 / 157;
+// 20 x 20000 x 1024 in groups of 32 18.2 / 15.1; 500 x 600 x 8000 in groups of 32, f32 scales 112 / 72.
 template <typename ST, int GSH, int WM, int NW, int WN, int MT>
 __global__ __launch_bounds__(64 * WM * NW) __attribute__((amdgpu_waves_per_eu(2, WN == 2 ? 2 : 4)))
 void linear_w4a8_tall_kernel(
